@@ -135,8 +135,8 @@ int pink_hip_get_som(pink_hip_ctx *ctx, float *host_som);
  * m_update_info (Trainer.h:302-303); the call then returns when they are there.
  * With bmu_out NULL and up to 128 KiB of images the call only copies the images into a
  * pinned buffer and returns (operator() returns nothing either); they are trained, in
- * order, a launch group (up to 64 images; 256 for small uint8 trainers) at a time: when the group is full or when any
- * other call on the context follows.  A loop of per-image calls then runs at the rate of
+ * order, a launch group (up to 64 images; 256 for small uint8 trainers) at a time: when the group is full, when some
+ * tens of images wait and the device is idle, or when any other call on the context follows.  A loop of per-image calls then runs at the rate of
  * the kernels (the rotation of a group is one launch), not of per-image launches and
  * round trips, and leaves the weights of training call by call.  pink_hip_get_som,
  * pink_hip_update_counts and pink_hip_synchronize wait for that work; an error in it is
@@ -149,9 +149,9 @@ int pink_hip_update_counts(pink_hip_ctx *ctx, uint32_t *host_counts_out);
  * asynchronous on the context's stream (see pink_hip_synchronize).  A small uint8 trainer
  * (at most 64 neurons, 32 variants, 2048 elements per neuron) trains a launch group of up
  * to 256 images in ONE launch whose blocks stay on the device and exchange one word per
- * image; the host waits for each such launch and learns from it whether every block saw
+ * image; the host waits for the call's launches and learns from them whether every block saw
  * the others in time (they do unless other work keeps the device's compute units busy for
- * seconds).  If not, nothing of the context has changed, the group is trained again with
+ * seconds).  If not, the launches behind the one that gave up changed nothing, their groups are trained again with
  * one launch per image, and the context stays with that form.  The environment variable
  * PINK_HIP_RESIDENT_TRAINER=0, read when a context is created, selects the one launch per
  * image from the start. */
@@ -160,8 +160,9 @@ int pink_hip_train_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n
 /* Mapper<...,true>::operator()(Data const&) (Mapper.h:181-208) for n_images images:
  * heatmap_out[i*N + n] = sqrt(min over rotations of the distance), already square-rooted
  * (Mapper.h:206); best_rot_out[i*N + n] = index of that rotation (may be NULL).
- * A call that brings 32 MB of images or more starts three helper threads in the context (kept until
- * pink_hip_destroy) that copy the input into pinned memory beside the calling thread. */
+ * A call that moves more than 1 MB of images or results (here and in pink_hip_get_som) shares 16 MB of pinned memory and
+ * five helper threads with the other contexts of the process; they exist from the first such call until the last context
+ * is destroyed. */
 int pink_hip_map(pink_hip_ctx *ctx, const float *host_images, uint32_t n_images,
                  float *host_heatmap_out, uint32_t *host_best_rot_out);
 int pink_hip_map_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images,

@@ -22,6 +22,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -1813,8 +1815,9 @@ __global__ __launch_bounds__(256) void k_train_small_u8(float *__restrict__ som,
 // Every wait is bounded: a wave that does not see all words within `spin_limit` polls raises `error` and marks its
 // block's slots, polling waves leave when they see such a mark, a block that leaves stops publishing, so every
 // block leaves.  The group's
-// results go to the OTHER buffers (weights, operand, norms); the host looks at `error` after the launch and only
-// then makes them the current ones, or trains the group again, image by image, from the untouched current ones.
+// results go to the OTHER buffers (weights, operand, norms), which the next launch takes as its current ones; launches
+// that follow one that gave up leave at once, so its inputs stay as they were.  The host looks at `error` after the last
+// of the launches it queued and trains the groups again, image by image, from the one that gave up.
 // ---------------------------------------------------------------------------------
 constexpr uint32_t kSlotStride = 16;                      // 64-bit words between two blocks' slots (128 bytes)
 constexpr uint32_t kSlotWords = 2 * 64 * kSlotStride;     // two sets of 64 slots
@@ -1827,7 +1830,8 @@ struct ResidentTrain {
     const uint32_t *variant;        // operand row -> variant index
     uint32_t *bmu_out;              // one per image
     unsigned long long *slots;
-    uint32_t *error;
+    uint32_t *error;                // 0, or the number (from 1) of the launch that gave up, among those the host has not checked yet
+    uint32_t launch;                // this launch's number
     uint32_t N, S, R, KS, nstored, images, tag0, spin_limit;
     uint32_t rot_stride, pb_stride, nb_stride;      // per image: floats, 16-byte words, norms
     VariantPair vp;
@@ -1988,7 +1992,7 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
                     __hip_atomic_store(a.slots + ((size_t)lane * 64 + n) * kSlotStride, (unsigned long long)kGaveUpTag << 32, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
                 if (lane == 0) {
-                    __hip_atomic_store(a.error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(a.error, a.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     s_bmu_f = make_uint2(0xffffffffu, 0u);
                 }
             } else {
@@ -2043,11 +2047,14 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
     if (tid == 0) a.na_next[n] = (long long)na;
 }
 
-// m_update_info[bmu]++ for the images of a group (Trainer.h:302-303), after a resident launch that went through.
-__global__ __launch_bounds__(256) void k_count_best_matches(const uint32_t *__restrict__ bmu, uint32_t images, uint32_t *__restrict__ counts)
+// m_update_info[bmu]++ for the images of a group (Trainer.h:302-303), behind a resident launch: nothing when that launch
+// or one before it gave up.  The error word goes to the host with it, which looks when it next waits for the stream.
+__global__ __launch_bounds__(256) void k_count_best_matches(const uint32_t *__restrict__ bmu, uint32_t images, uint32_t *__restrict__ counts,
+                                                            const uint32_t *__restrict__ error, uint32_t *__restrict__ host_error)
 {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < images) atomicAdd(&counts[bmu[t]], 1u);
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, e = *error;
+    if (t == 0) *host_error = e;
+    if (t < images && e == 0) atomicAdd(&counts[bmu[t]], 1u);
 }
 
 // Decode keys: distance (optionally square-rooted for the mapper, Mapper.h:206), exact
@@ -2080,9 +2087,10 @@ __global__ __launch_bounds__(256) void k_finalize(const unsigned long long *__re
 // ---------------------------------------------------------------------------------
 struct EventPair { hipEvent_t a, b; int cls; uint32_t launches; };
 
-// Host threads that copy one buffer into another side by side (the caller takes a part too): what carries a large
-// pageable input of a mapper into pinned memory faster than one thread can (a single thread moves about half of what the
-// PCIe link takes).  copy() returns when every part has been copied.
+// Host threads that copy one buffer into another side by side (the caller takes a part too): what carries large
+// pageable buffers into and out of pinned memory faster than one thread can (a single thread moves about half of what
+// the PCIe link takes, a quarter into pages it touches first).  copy() returns when every part has been copied.  Between
+// the pieces of one transfer, some tens of microseconds apart, the workers spin; after that they sleep.
 class HostCopyPool {
 public:
     explicit HostCopyPool(unsigned workers)
@@ -2094,7 +2102,7 @@ public:
         {
             std::lock_guard<std::mutex> lock(m_);
             stop_ = true;
-            ++generation_;
+            generation_.fetch_add(1, std::memory_order_release);
         }
         start_.notify_all();
         for (std::thread &t : threads_) t.join();
@@ -2102,17 +2110,17 @@ public:
     void copy(char *dst, const char *src, size_t bytes)
     {
         const size_t parts = threads_.size() + 1;
+        dst_ = dst; src_ = src; bytes_ = bytes;
+        each_ = ((bytes + parts - 1) / parts + 4095) & ~(size_t)4095;
+        pending_.store((unsigned)threads_.size(), std::memory_order_relaxed);
         {
             std::lock_guard<std::mutex> lock(m_);
-            dst_ = dst; src_ = src; bytes_ = bytes;
-            each_ = ((bytes + parts - 1) / parts + 4095) & ~(size_t)4095;
-            pending_ = (unsigned)threads_.size();
-            ++generation_;
+            generation_.fetch_add(1, std::memory_order_release);
         }
         start_.notify_all();
         part((unsigned)threads_.size());
-        std::unique_lock<std::mutex> lock(m_);
-        done_.wait(lock, [&] { return pending_ == 0; });
+        for (unsigned spins = 0; pending_.load(std::memory_order_acquire) != 0; ++spins)
+            if (spins > 4096) std::this_thread::yield();
     }
 
 private:
@@ -2125,28 +2133,85 @@ private:
     {
         unsigned long long seen = 0;
         for (;;) {
-            {
+            const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+            while (generation_.load(std::memory_order_acquire) == seen && std::chrono::steady_clock::now() < until) __builtin_ia32_pause();
+            if (generation_.load(std::memory_order_acquire) == seen) {
                 std::unique_lock<std::mutex> lock(m_);
-                start_.wait(lock, [&] { return generation_ != seen; });
-                seen = generation_;
-                if (stop_) return;
+                start_.wait(lock, [&] { return generation_.load(std::memory_order_acquire) != seen; });
             }
+            seen = generation_.load(std::memory_order_acquire);
+            if (stop_) return;
             part(i);
-            std::lock_guard<std::mutex> lock(m_);
-            if (--pending_ == 0) done_.notify_one();
+            pending_.fetch_sub(1, std::memory_order_release);
         }
     }
     std::vector<std::thread> threads_;
     std::mutex m_;
-    std::condition_variable start_, done_;
-    unsigned long long generation_ = 0;
-    unsigned pending_ = 0;
+    std::condition_variable start_;
+    std::atomic<unsigned long long> generation_{0};
+    std::atomic<unsigned> pending_{0};
     bool stop_ = false;
     char *dst_ = nullptr;
     const char *src_ = nullptr;
     size_t bytes_ = 0, each_ = 0;
 };
-constexpr size_t kBounceBytes = (size_t)8 << 20;          // pinned buffers the pool fills, two taking turns
+
+// The pinned pieces and the copy threads that large pageable transfers go through: one set for the process, made when
+// a transfer first wants it and given back with the last context.  A call holds it for the length of one transfer; a
+// second thread that wants it meanwhile takes the runtime's own pageable copy.
+// (2 MB pieces: the link's 55 GB/s needs about half a MB; a piece is also what nothing overlaps at either end.)
+constexpr size_t kPieceBytes = (size_t)2 << 20;
+constexpr uint32_t kPieces = 8;
+constexpr unsigned kCopyWorkers = 5;                      // and the caller (measured: 6 threads move 115 GB/s, 14 into fresh pages)
+struct HostStaging {
+    HostCopyPool pool{kCopyWorkers};
+    char *piece[kPieces] = {};
+    char *base = nullptr;
+};
+std::mutex g_staging_users_mutex, g_staging_mutex;        // the count of contexts; the set itself (held over a transfer)
+unsigned g_staging_users = 0;
+std::unique_ptr<HostStaging> g_staging;
+
+void staging_add_user()
+{
+    std::lock_guard<std::mutex> lock(g_staging_users_mutex);
+    ++g_staging_users;
+}
+
+void staging_drop_user()
+{
+    std::lock_guard<std::mutex> users(g_staging_users_mutex);
+    if (--g_staging_users) return;
+    std::lock_guard<std::mutex> lock(g_staging_mutex);
+    if (g_staging) (void)hipHostFree(g_staging->base);
+    g_staging.reset();
+}
+
+// The set, held by `lock` on return; null (and `lock` empty) when another thread has it or the host cannot give it.
+HostStaging *take_staging(std::unique_lock<std::mutex> &lock)
+{
+    lock = std::unique_lock<std::mutex>(g_staging_mutex, std::try_to_lock);
+    if (!lock.owns_lock()) return nullptr;
+    if (!g_staging) {
+        void *base = nullptr;
+        if (hipHostMalloc(&base, kPieces * kPieceBytes, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            lock.unlock();
+            return nullptr;
+        }
+        try {
+            g_staging.reset(new HostStaging);
+        } catch (...) {
+            (void)hipHostFree(base);
+            lock.unlock();
+            return nullptr;
+        }
+        g_staging->base = (char *)base;
+        for (uint32_t i = 0; i < kPieces; ++i) g_staging->piece[i] = g_staging->base + i * kPieceBytes;
+    }
+    return g_staging.get();
+}
+
 constexpr size_t kRotateLdsMax = 158 * 1024;
 enum : uint32_t { kStoreNone = 0, kStoreAll = 1, kStorePair = 2 };
 
@@ -2200,20 +2265,15 @@ struct pink_hip_ctx {
     float *st_img = nullptr, *st_heat = nullptr;
     uint32_t *st_best = nullptr, *st_bmu = nullptr;
     size_t st_images = 0;                  // capacity of the staging buffers, in images
-    char *st_pin = nullptr;                // kPinBytes in (as a whole, or as a ring of kPinSlots slots), kPinBytes out
-    hipEvent_t st_ev[8] = {};              // per slot: the copy out of it has run
-    uint32_t st_slot = 0;
-    bool st_ring_busy = false;             // a call returned with copies out of the ring still queued
+    char *st_pin = nullptr;                // kPinBytes in, kPinBytes out
     // per-image training calls that hand nothing back wait here until a launch group is full (or any other call comes)
     char *pend_pin[2] = {nullptr, nullptr};
-    hipEvent_t pend_ev[2] = {nullptr, nullptr};
+    hipEvent_t pend_ev[2] = {nullptr, nullptr}, pend_done = nullptr;     // the copy out of a buffer has run; the last group is trained
     uint32_t pend_count = 0, pend_cur = 0, pend_cap = 0;
     hipStream_t copy_stream = nullptr;     // host -> device copies of the next images while the kernels of the last run
     hipEvent_t copy_ev[2] = {};
-    // mappers, large pageable inputs: host threads fill two pinned buffers in turn, the copies to the device leave from those
-    std::unique_ptr<HostCopyPool> copy_pool;
-    char *bounce[2] = {nullptr, nullptr};
-    hipEvent_t bounce_ev[2] = {};
+    hipEvent_t piece_ev[kPieces] = {};     // large pageable transfers: the copy into or out of a pinned piece has run
+    bool staging_user = false;             // counted among the contexts that share the pinned pieces
     uint32_t *d_counts = nullptr;          // trainer: how often each neuron was the best match
     uint32_t *d_symoff = nullptr;          // [8][Epad] region positions under the 8 symmetries: packing fused into k_rotate
     bool fused_pack = false;
@@ -2248,6 +2308,8 @@ struct pink_hip_ctx {
     unsigned long long *d_slots = nullptr;
     uint32_t *d_resident_error = nullptr, *h_resident_error = nullptr;
     uint32_t exchange_tag = 1, spin_limit = 1u << 21;
+    struct ResidentGroup { const float *images; uint32_t count; uint32_t *bmu; };
+    std::vector<ResidentGroup> resident_queued;   // groups whose resident launches the host has not checked yet
     unsigned long long *d_src4 = nullptr;  // ... its per-element tables (see the kernel)
     uint32_t *d_kbyte = nullptr;
     uint32_t *d_grow = nullptr, *d_gvariant = nullptr;   // variant index -> row of the variant operand, and back
@@ -2822,12 +2884,19 @@ int run_train_small(pink_hip_ctx *ctx, uint32_t slot, uint32_t *dev_bmu_out)
     return launch_check(ctx, "k_train_small_u8");
 }
 
-// The first `images` images of the current group in one resident launch (small uint8 trainers).  `went_through`
-// false: a block gave up waiting for the others (the device was not free to hold all blocks at once); nothing of
-// the context has changed then, the context stops using this form, and the caller trains the group image by image.
-int run_train_small_resident(pink_hip_ctx *ctx, uint32_t images, uint32_t *dev_bmu, bool *went_through)
+// The two sets of buffers between which resident launches alternate.
+void swap_resident(pink_hip_ctx *ctx)
 {
-    *went_through = false;
+    std::swap(ctx->d_som, ctx->d_som_alt);
+    ctx->pa_cur ^= 1;
+    ctx->na_cur ^= 1;
+}
+
+// The first `images` images of the current group in one resident launch (small uint8 trainers), queued: whether every
+// block saw the others in time (they do unless the device was not free to hold all blocks at once) is for finish_resident
+// to see.  The buffers it writes are the current ones from here on.
+int run_train_small_resident(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, uint32_t *dev_bmu)
+{
     if (ctx->exchange_tag > 0xfffffff0u - images) {        // the tags wrap: back to 1, over slots that hold none
         HIP_TRY(ctx, hipMemsetAsync(ctx->d_slots, 0, kSlotWords * sizeof(unsigned long long), ctx->stream));
         ctx->exchange_tag = 1;
@@ -2840,6 +2909,7 @@ int run_train_small_resident(pink_hip_ctx *ctx, uint32_t images, uint32_t *dev_b
     a.bmu_out = dev_bmu;
     a.slots = ctx->d_slots;
     a.error = ctx->d_resident_error;
+    a.launch = (uint32_t)ctx->resident_queued.size() + 1;
     a.N = ctx->N; a.S = ctx->S; a.R = ctx->R; a.KS = ctx->gKS;
     a.nstored = std::min(2 * std::max(ctx->nrr, 1u), ctx->R);
     a.images = images; a.tag0 = ctx->exchange_tag; a.spin_limit = ctx->spin_limit;
@@ -2864,20 +2934,33 @@ int run_train_small_resident(pink_hip_ctx *ctx, uint32_t images, uint32_t *dev_b
 #undef LAUNCH_RESIDENT
         TRY(launch_check(ctx, "k_train_small_u8_resident"));
     }
-    HIP_TRY(ctx, hipMemcpyAsync(ctx->h_resident_error, ctx->d_resident_error, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    if (*ctx->h_resident_error) {
-        ctx->resident_train = false;
-        HIP_TRY(ctx, hipMemsetAsync(ctx->d_resident_error, 0, sizeof(uint32_t), ctx->stream));
-        HIP_TRY(ctx, hipMemsetAsync(ctx->d_slots, 0, kSlotWords * sizeof(unsigned long long), ctx->stream));
-        return PINK_HIP_OK;
-    }
-    std::swap(ctx->d_som, ctx->d_som_alt);
-    ctx->pa_cur ^= 1;
-    ctx->na_cur ^= 1;
-    hipLaunchKernelGGL(k_count_best_matches, dim3((images + 255) / 256), dim3(256), 0, ctx->stream, dev_bmu, images, ctx->d_counts);
+    hipLaunchKernelGGL(k_count_best_matches, dim3((images + 255) / 256), dim3(256), 0, ctx->stream, dev_bmu, images, ctx->d_counts,
+                       ctx->d_resident_error, ctx->h_resident_error);
     TRY(launch_check(ctx, "k_count_best_matches"));
-    *went_through = true;
+    ctx->resident_queued.push_back({dev_images, images, dev_bmu});
+    swap_resident(ctx);
+    return PINK_HIP_OK;
+}
+
+// Wait for the queued resident launches.  If one gave up, nothing after it has run: back to the buffers it started from,
+// its group and the later ones image by image, and the context stays with that form.
+int finish_resident(pink_hip_ctx *ctx)
+{
+    if (ctx->resident_queued.empty()) return PINK_HIP_OK;
+    std::vector<pink_hip_ctx::ResidentGroup> queued;
+    queued.swap(ctx->resident_queued);
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    const uint32_t failed = *ctx->h_resident_error;
+    if (!failed) return PINK_HIP_OK;
+    ctx->resident_train = false;
+    HIP_TRY(ctx, hipMemsetAsync(ctx->d_resident_error, 0, sizeof(uint32_t), ctx->stream));
+    HIP_TRY(ctx, hipMemsetAsync(ctx->d_slots, 0, kSlotWords * sizeof(unsigned long long), ctx->stream));
+    if ((queued.size() - (failed - 1)) & 1) swap_resident(ctx);
+    for (size_t g = failed - 1; g < queued.size(); ++g) {
+        TRY(run_rotate(ctx, queued[g].images, queued[g].count, kStorePair));
+        for (uint32_t b = 0; b < queued[g].count; ++b) TRY(run_train_small(ctx, b, queued[g].bmu + b));
+    }
     return PINK_HIP_OK;
 }
 
@@ -2909,14 +2992,10 @@ int free_all(pink_hip_ctx *ctx)
         if (ctx->pend_pin[i]) (void)hipHostFree(ctx->pend_pin[i]);
         if (ctx->pend_ev[i]) (void)hipEventDestroy(ctx->pend_ev[i]);
     }
-    for (hipEvent_t e : ctx->st_ev) if (e) (void)hipEventDestroy(e);
+    if (ctx->pend_done) (void)hipEventDestroy(ctx->pend_done);
     for (hipEvent_t e : ctx->copy_ev) if (e) (void)hipEventDestroy(e);
-    ctx->copy_pool.reset();
-    for (int i = 0; i < 2; ++i) {
-        if (ctx->bounce[i]) (void)hipHostFree(ctx->bounce[i]);
-        if (ctx->bounce_ev[i]) (void)hipEventDestroy(ctx->bounce_ev[i]);
-        ctx->bounce[i] = nullptr; ctx->bounce_ev[i] = nullptr;
-    }
+    for (hipEvent_t e : ctx->piece_ev) if (e) (void)hipEventDestroy(e);
+    if (ctx->staging_user) staging_drop_user();
     if (ctx->copy_stream) (void)hipStreamDestroy(ctx->copy_stream);
     if (ctx->d_counts) (void)hipFree(ctx->d_counts);
     for (void *p : {(void *)ctx->d_fPa, (void *)ctx->d_fPb, (void *)ctx->d_fna, (void *)ctx->d_fnb, (void *)ctx->d_fpart})
@@ -2948,6 +3027,8 @@ int init_ctx(pink_hip_ctx *ctx)
     const pink_hip_config &c = ctx->cfg;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     TRY(resolve_static_scratch(ctx));
+    staging_add_user();
+    ctx->staging_user = true;
     HIP_TRY(ctx, hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
 
     // Rotation tables: cos/sin of i * 2pi/num_rot in float, as the CPU evaluates them
@@ -3598,9 +3679,14 @@ void pink_hip_destroy(pink_hip_ctx *ctx)
 // launch group at a time: when the group is full, or when any other call on the context needs the state
 // they produce.  The order of the images and every result are those of training them call by call.
 int ensure_staging(pink_hip_ctx *ctx, size_t n);
-int flush_pending(pink_hip_ctx *ctx)
+static int copy_out(pink_hip_ctx *ctx, void *host, const void *dev, size_t bytes);
+static int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out);
+
+// The pending images go to the device and through training, queued.
+static int start_pending(pink_hip_ctx *ctx)
 {
-    if (!ctx || !ctx->pend_count) return PINK_HIP_OK;
+    TRY(finish_resident(ctx));                            // (may still need the staging buffer the images go to)
+    if (!ctx->pend_count) return PINK_HIP_OK;
     const uint32_t n = ctx->pend_count, cur = ctx->pend_cur;
     ctx->pend_count = 0;
     ctx->pend_cur ^= 1;
@@ -3609,7 +3695,17 @@ int flush_pending(pink_hip_ctx *ctx)
     HIP_TRY(ctx, hipMemcpyAsync(ctx->st_img, ctx->pend_pin[cur], (size_t)n * ctx->isz * sizeof(float), hipMemcpyHostToDevice,
                                 ctx->stream));
     HIP_TRY(ctx, hipEventRecord(ctx->pend_ev[cur], ctx->stream));
-    return pink_hip_train_device(ctx, ctx->st_img, n, ctx->st_bmu);
+    TRY(train_queued(ctx, ctx->st_img, n, ctx->st_bmu));
+    HIP_TRY(ctx, hipEventRecord(ctx->pend_done, ctx->stream));
+    return PINK_HIP_OK;
+}
+
+// What every other call on the context begins with: nothing pending, nothing unchecked.
+int flush_pending(pink_hip_ctx *ctx)
+{
+    if (!ctx) return PINK_HIP_OK;
+    TRY(start_pending(ctx));
+    return finish_resident(ctx);
 }
 
 int pink_hip_synchronize(pink_hip_ctx *ctx)
@@ -3638,10 +3734,7 @@ int pink_hip_get_som(pink_hip_ctx *ctx, float *host_som)
     if (!ctx || !host_som) return fail(ctx, PINK_HIP_EINVAL, "pink_hip_get_som: null argument");
     TRY(flush_pending(ctx));
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    HIP_TRY(ctx, hipMemcpyAsync(host_som, ctx->d_som, (size_t)ctx->N * ctx->S * sizeof(float), hipMemcpyDeviceToHost,
-                                ctx->stream));
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    return PINK_HIP_OK;
+    return copy_out(ctx, host_som, ctx->d_som, (size_t)ctx->N * ctx->S * sizeof(float));
 }
 
 int pink_hip_update_counts(pink_hip_ctx *ctx, uint32_t *host_counts_out)
@@ -3650,17 +3743,21 @@ int pink_hip_update_counts(pink_hip_ctx *ctx, uint32_t *host_counts_out)
     if (!ctx->trainer) return fail(ctx, PINK_HIP_ESTATE, "pink_hip_update_counts: context was created without update factors");
     TRY(flush_pending(ctx));
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    HIP_TRY(ctx, hipMemcpyAsync(host_counts_out, ctx->d_counts, (size_t)ctx->N * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    return PINK_HIP_OK;
+    return copy_out(ctx, host_counts_out, ctx->d_counts, (size_t)ctx->N * sizeof(uint32_t));
 }
 
 int pink_hip_train_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
 {
     if (!ctx || (!dev_images && n_images)) return fail(ctx, PINK_HIP_EINVAL, "pink_hip_train_device: null argument");
     if (!ctx->trainer) return fail(ctx, PINK_HIP_ESTATE, "pink_hip_train: context was created without update factors");
-    TRY(flush_pending(ctx));                              // (none while flush_pending itself calls this)
+    TRY(flush_pending(ctx));
     HIP_TRY(ctx, hipSetDevice(ctx->device));
+    TRY(train_queued(ctx, dev_images, n_images, dev_bmu_out));
+    return finish_resident(ctx);                          // (the images are the caller's again on return)
+}
+
+static int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
+{
     // The variants of an image and their packed distance operand do not depend on the SOM: they
     // are produced for a group of images per launch.  Distance and update stay strictly sequential.
     for (uint32_t done = 0; done < n_images; done += ctx->Bcap) {
@@ -3690,9 +3787,8 @@ int pink_hip_train_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n
             continue;
         }
         if (ctx->resident_train) {
-            bool went_through = false;
-            TRY(run_train_small_resident(ctx, B, dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group, &went_through));
-            if (went_through) continue;
+            TRY(run_train_small_resident(ctx, dev_images + (size_t)done * ctx->isz, B, dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group));
+            continue;
         }
         for (uint32_t b = 0; b < B; ++b) {
             if (ctx->small_train) {
@@ -3709,19 +3805,68 @@ int pink_hip_train_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n
 }
 
 constexpr size_t kPinBytes = (size_t)1 << 20;
-constexpr uint32_t kPinSlots = 8;
-constexpr size_t kSlotBytes = kPinBytes / kPinSlots;
+constexpr uint32_t kPendLook = 32;
+constexpr size_t kSlotBytes = kPinBytes / 8;              // a call's images join the pending launch group up to this size
+
+// The context's own pinned buffer for small transfers.
+static int ensure_pin(pink_hip_ctx *ctx)
+{
+    if (ctx->st_pin) return PINK_HIP_OK;
+    if (hipHostMalloc((void **)&ctx->st_pin, 2 * kPinBytes, hipHostMallocDefault) != hipSuccess) {
+        ctx->st_pin = nullptr;
+        return fail(ctx, PINK_HIP_ENOMEM, "pinned host allocation failed");
+    }
+    return PINK_HIP_OK;
+}
+
+static int ensure_piece_events(pink_hip_ctx *ctx)
+{
+    for (hipEvent_t &e : ctx->piece_ev)
+        if (!e) HIP_TRY(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return PINK_HIP_OK;
+}
+
+// Device -> pageable host memory behind everything queued on the context's stream; returns when it is there.  The
+// runtime's own pageable copy moves 18 GB/s; here the link's 55: small results through the context's pinned buffer,
+// larger ones through the shared pinned pieces, which host threads empty while the copies into the next ones run
+// (94 MB of weights 5.3 -> 1.9 ms).
+static int copy_out(pink_hip_ctx *ctx, void *host, const void *dev, size_t bytes)
+{
+    if (bytes <= kPinBytes) {
+        TRY(ensure_pin(ctx));
+        HIP_TRY(ctx, hipMemcpyAsync(ctx->st_pin + kPinBytes, dev, bytes, hipMemcpyDeviceToHost, ctx->stream));
+        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+        memcpy(host, ctx->st_pin + kPinBytes, bytes);
+        return PINK_HIP_OK;
+    }
+    std::unique_lock<std::mutex> lock;
+    HostStaging *st = take_staging(lock);
+    if (!st) {
+        HIP_TRY(ctx, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream));
+        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+        return PINK_HIP_OK;
+    }
+    TRY(ensure_piece_events(ctx));
+    const size_t pieces = (bytes + kPieceBytes - 1) / kPieceBytes;
+    size_t queued = 0;
+    for (size_t done = 0; done < pieces; ++done) {
+        for (; queued < pieces && queued < done + kPieces; ++queued) {
+            const size_t off = queued * kPieceBytes;
+            HIP_TRY(ctx, hipMemcpyAsync(st->piece[queued % kPieces], (const char *)dev + off, std::min(kPieceBytes, bytes - off),
+                                        hipMemcpyDeviceToHost, ctx->stream));
+            HIP_TRY(ctx, hipEventRecord(ctx->piece_ev[queued % kPieces], ctx->stream));
+        }
+        const size_t off = done * kPieceBytes;
+        HIP_TRY(ctx, hipEventSynchronize(ctx->piece_ev[done % kPieces]));
+        st->pool.copy((char *)host + off, st->piece[done % kPieces], std::min(kPieceBytes, bytes - off));
+    }
+    return PINK_HIP_OK;
+}
 
 // Staging for `n` images per chunk (grown on demand, freed with the context).
 int ensure_staging(pink_hip_ctx *ctx, size_t n)
 {
-    if (!ctx->st_pin) {
-        if (hipHostMalloc((void **)&ctx->st_pin, 2 * kPinBytes, hipHostMallocDefault) != hipSuccess) {
-            ctx->st_pin = nullptr;
-            return fail(ctx, PINK_HIP_ENOMEM, "pinned host allocation failed");
-        }
-        for (hipEvent_t &e : ctx->st_ev) HIP_TRY(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
+    TRY(ensure_pin(ctx));
     if (n <= ctx->st_images) return PINK_HIP_OK;
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu})
@@ -3743,11 +3888,6 @@ int ensure_staging(pink_hip_ctx *ctx, size_t n)
 hipError_t stage_in(pink_hip_ctx *ctx, void *dev, const void *host, size_t bytes)
 {
     if (bytes <= kPinBytes) {
-        if (ctx->st_ring_busy) {                           // queued calls may still read the buffer
-            const hipError_t e = hipStreamSynchronize(ctx->stream);
-            if (e != hipSuccess) return e;
-            ctx->st_ring_busy = false;
-        }
         memcpy(ctx->st_pin, host, bytes);
         return hipMemcpyAsync(dev, ctx->st_pin, bytes, hipMemcpyHostToDevice, ctx->stream);
     }
@@ -3773,7 +3913,6 @@ int staged_run(pink_hip_ctx *ctx, const float *host_images, uint32_t n, Run run)
     }
     // whatever still reads the staging buffer (queued per-image calls) finishes first
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    ctx->st_ring_busy = false;
     // (a trainer's kernels take long enough per image for 16 MB pieces to hide all copies but the first behind them:
     // cfg0 40 k -> 51 k images/s with pageable buffers; a mapper's launch groups want the larger pieces)
     // Nothing hides the copy of the first piece, so the pieces start at about 1 MB and double up to that size.
@@ -3785,55 +3924,35 @@ int staged_run(pink_hip_ctx *ctx, const float *host_images, uint32_t n, Run run)
     const uint32_t largest = whole_groups((size_t)(ctx->trainer ? 16 : 64) << 20);
     uint32_t piece = std::min(largest, std::max(whole_groups((size_t)1 << 20), std::min(ctx->Bcap, largest)));
     // A mapper's kernels are faster than the link, so its rate from host buffers is the rate of the copies, and a
-    // copy out of pageable memory is one host thread's work (about half of what the link takes): inputs of 32 MB and
-    // more go through two pinned buffers that four host threads fill side by side (cfg1 from pageable memory: 26 -> 42 GB/s,
-    // 1.6 M -> 2.56 M images/s).
-    // Set up all or nothing; a host that cannot give the threads or the pinned memory keeps the plain copies.
-    const bool pooled = !ctx->trainer && (size_t)n * img_bytes >= ((size_t)32 << 20);
-    if (pooled && !ctx->copy_pool) {
-        char *pin[2] = {nullptr, nullptr};
-        hipEvent_t ev[2] = {nullptr, nullptr};
-        bool ok = true;
-        for (int i = 0; i < 2 && ok; ++i)
-            ok = hipHostMalloc((void **)&pin[i], kBounceBytes, hipHostMallocDefault) == hipSuccess &&
-                 hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) == hipSuccess;
-        std::unique_ptr<HostCopyPool> pool;
-        if (ok) {
-            // (three workers and the caller; five or seven workers, buffers of 4 or 16 MB: the same 42 GB/s)
-            try { pool.reset(new HostCopyPool(3)); } catch (...) { ok = false; }
-        }
-        if (ok) {
-            ctx->copy_pool = std::move(pool);
-            for (int i = 0; i < 2; ++i) { ctx->bounce[i] = pin[i]; ctx->bounce_ev[i] = ev[i]; }
-        } else {
-            (void)hipGetLastError();
-            for (int i = 0; i < 2; ++i) {
-                if (ev[i]) (void)hipEventDestroy(ev[i]);
-                if (pin[i]) (void)hipHostFree(pin[i]);
-            }
-        }
-    }
-    uint32_t turn = 0, count = 0, bounce_turn = 0;
+    // copy out of pageable memory is one host thread's work (about half of what the link takes): its inputs go through
+    // the shared pinned pieces, which host threads fill side by side (cfg1 from pageable memory: 26 -> 42 GB/s,
+    // 1.6 M -> 2.56 M images/s).  Without those (another thread has them, the host refused them): the plain copies.
+    std::unique_lock<std::mutex> lock;
+    HostStaging *st = ctx->trainer ? nullptr : take_staging(lock);
+    if (st) TRY(ensure_piece_events(ctx));
+    uint32_t turn = 0, count = 0, slot = 0;
     for (uint32_t first = 0; first < n; first += count, turn ^= 1, piece = std::min(largest, 2 * piece)) {
         count = std::min(piece, n - first);
         float *dev = ctx->st_img + (size_t)first * ctx->isz;
-        if (pooled && ctx->copy_pool) {
+        if (st) {
             const char *src = (const char *)(host_images + (size_t)first * ctx->isz);
             const size_t bytes = (size_t)count * img_bytes;
-            for (size_t off = 0; off < bytes; off += kBounceBytes, bounce_turn ^= 1) {
-                const size_t len = std::min(kBounceBytes, bytes - off);
-                HIP_TRY(ctx, hipEventSynchronize(ctx->bounce_ev[bounce_turn]));       // its last copy to the device has run
-                ctx->copy_pool->copy(ctx->bounce[bounce_turn], src + off, len);
-                HIP_TRY(ctx, hipMemcpyAsync((char *)dev + off, ctx->bounce[bounce_turn], len, hipMemcpyHostToDevice, ctx->copy_stream));
-                HIP_TRY(ctx, hipEventRecord(ctx->bounce_ev[bounce_turn], ctx->copy_stream));
+            for (size_t off = 0; off < bytes; off += kPieceBytes, slot = (slot + 1) % kPieces) {
+                const size_t len = std::min(kPieceBytes, bytes - off);
+                HIP_TRY(ctx, hipEventSynchronize(ctx->piece_ev[slot]));               // its last copy to the device has run
+                st->pool.copy(st->piece[slot], src + off, len);
+                HIP_TRY(ctx, hipMemcpyAsync((char *)dev + off, st->piece[slot], len, hipMemcpyHostToDevice, ctx->copy_stream));
+                HIP_TRY(ctx, hipEventRecord(ctx->piece_ev[slot], ctx->copy_stream));
             }
         } else
-        HIP_TRY(ctx, hipMemcpyAsync(dev, host_images + (size_t)first * ctx->isz, count * img_bytes, hipMemcpyHostToDevice,
-                                    ctx->copy_stream));
+            HIP_TRY(ctx, hipMemcpyAsync(dev, host_images + (size_t)first * ctx->isz, count * img_bytes, hipMemcpyHostToDevice,
+                                        ctx->copy_stream));
         HIP_TRY(ctx, hipEventRecord(ctx->copy_ev[turn], ctx->copy_stream));
         HIP_TRY(ctx, hipStreamWaitEvent(ctx->stream, ctx->copy_ev[turn], 0));
         TRY(run(dev, first, count));
     }
+    // the pinned pieces are another call's as soon as this one lets go of them: their copies have to be through
+    if (st) HIP_TRY(ctx, hipStreamSynchronize(ctx->copy_stream));
     return PINK_HIP_OK;
 }
 }  // extern "C++"
@@ -3849,23 +3968,22 @@ int pink_hip_train(pink_hip_ctx *ctx, const float *host_images, uint32_t n_image
         // Nothing to hand back (the reference's operator() returns nothing either): the images join the
         // pending launch group in pinned memory and the call returns; see flush_pending.
         if (!ctx->pend_pin[0]) {
-            // both buffers and both events, or none of them: the context takes them only when all four exist
+            // all buffers and events, or none of them: the context takes them only when they exist
             char *pin[2] = {nullptr, nullptr};
-            hipEvent_t ev[2] = {nullptr, nullptr};
+            hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
             bool ok = true;
             for (int i = 0; i < 2 && ok; ++i)
-                ok = hipHostMalloc((void **)&pin[i], (size_t)ctx->Bcap * img_bytes, hipHostMallocDefault) == hipSuccess &&
-                     hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) == hipSuccess;
+                ok = hipHostMalloc((void **)&pin[i], (size_t)ctx->Bcap * img_bytes, hipHostMallocDefault) == hipSuccess;
+            for (int i = 0; i < 3 && ok; ++i) ok = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) == hipSuccess;
             if (!ok) {
                 (void)hipGetLastError();
-                for (int i = 0; i < 2; ++i) {
-                    if (ev[i]) (void)hipEventDestroy(ev[i]);
-                    if (pin[i]) (void)hipHostFree(pin[i]);
-                }
+                for (hipEvent_t e : ev) if (e) (void)hipEventDestroy(e);
+                for (char *q : pin) if (q) (void)hipHostFree(q);
                 return fail(ctx, PINK_HIP_ENOMEM, "pink_hip_train: pinned host buffers for queued images could not be set up");
             }
             ctx->pend_cap = ctx->Bcap;
             for (int i = 0; i < 2; ++i) { ctx->pend_pin[i] = pin[i]; ctx->pend_ev[i] = ev[i]; }
+            ctx->pend_done = ev[2];
         }
         for (uint32_t done = 0; done < n_images;) {
             const uint32_t take = std::min(n_images - done, ctx->pend_cap - ctx->pend_count);
@@ -3874,7 +3992,11 @@ int pink_hip_train(pink_hip_ctx *ctx, const float *host_images, uint32_t n_image
                    (size_t)take * img_bytes);
             ctx->pend_count += take;
             done += take;
-            if (ctx->pend_count == ctx->pend_cap) TRY(flush_pending(ctx));
+            // a full group goes; part of one goes too when the device has nothing to do (looked at every kPendLook images:
+            // the loop that brings the images one by one then runs beside the kernels, not before them)
+            if (ctx->pend_count == ctx->pend_cap ||
+                (ctx->pend_count % kPendLook < take && ctx->pend_count >= kPendLook && hipEventQuery(ctx->pend_done) == hipSuccess))
+                TRY(start_pending(ctx));
         }
         return PINK_HIP_OK;
     }
@@ -3885,15 +4007,11 @@ int pink_hip_train(pink_hip_ctx *ctx, const float *host_images, uint32_t n_image
     for (uint32_t done = 0; done < n_images; done += chunk) {
         const uint32_t n = std::min(chunk, n_images - done);
         TRY(staged_run(ctx, host_images + (size_t)done * ctx->isz, n, [&](const float *dev, uint32_t first, uint32_t count) {
-            return pink_hip_train_device(ctx, dev, count, ctx->st_bmu + first);
+            return train_queued(ctx, dev, count, ctx->st_bmu + first);
         }));
+        TRY(finish_resident(ctx));
         if (host_bmu_out) {
-            const size_t out_bytes = n * sizeof(uint32_t);
-            const bool small = out_bytes <= kPinBytes;
-            HIP_TRY(ctx, hipMemcpyAsync(small ? (void *)(ctx->st_pin + kPinBytes) : (void *)(host_bmu_out + done), ctx->st_bmu,
-                                        out_bytes, hipMemcpyDeviceToHost, ctx->stream));
-            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-            if (small) memcpy(host_bmu_out + done, ctx->st_pin + kPinBytes, out_bytes);
+            TRY(copy_out(ctx, host_bmu_out + done, ctx->st_bmu, n * sizeof(uint32_t)));
         } else {
             HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));      // the host images are the caller's again on return
         }
@@ -4016,23 +4134,24 @@ int pink_hip_map(pink_hip_ctx *ctx, const float *host_images, uint32_t n_images,
     TRY(ensure_staging(ctx, chunk));
     for (uint32_t done = 0; done < n_images; done += chunk) {
         const uint32_t n = std::min(chunk, n_images - done);
-        TRY(staged_run(ctx, host_images + (size_t)done * ctx->isz, n, [&](const float *dev, uint32_t first, uint32_t count) {
-            return pink_hip_map_device(ctx, dev, count, ctx->st_heat + (size_t)first * ctx->N, ctx->st_best + (size_t)first * ctx->N);
-        }));
         const size_t heat_bytes = (size_t)n * ctx->N * sizeof(float);       // the best rotations take as many bytes
+        // small results: the last kernel writes them into pinned host memory itself, no copies follow it
         const bool small = 2 * heat_bytes <= kPinBytes;
         char *pin_out = ctx->st_pin + kPinBytes;
+        float *heat = small ? (float *)pin_out : ctx->st_heat;
+        uint32_t *best = small ? (uint32_t *)(pin_out + heat_bytes) : ctx->st_best;
+        TRY(staged_run(ctx, host_images + (size_t)done * ctx->isz, n, [&](const float *dev, uint32_t first, uint32_t count) {
+            return pink_hip_map_device(ctx, dev, count, heat + (size_t)first * ctx->N, best + (size_t)first * ctx->N);
+        }));
         float *heat_dst = host_heatmap_out + (size_t)done * ctx->N;
         uint32_t *best_dst = host_best_rot_out ? host_best_rot_out + (size_t)done * ctx->N : nullptr;
-        HIP_TRY(ctx, hipMemcpyAsync(small ? (void *)pin_out : (void *)heat_dst, ctx->st_heat, heat_bytes, hipMemcpyDeviceToHost,
-                                    ctx->stream));
-        if (best_dst)
-            HIP_TRY(ctx, hipMemcpyAsync(small ? (void *)(pin_out + heat_bytes) : (void *)best_dst, ctx->st_best, heat_bytes,
-                                        hipMemcpyDeviceToHost, ctx->stream));
-        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
         if (small) {
-            memcpy(heat_dst, pin_out, heat_bytes);
-            if (best_dst) memcpy(best_dst, pin_out + heat_bytes, heat_bytes);
+            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+            memcpy(heat_dst, heat, heat_bytes);
+            if (best_dst) memcpy(best_dst, best, heat_bytes);
+        } else {
+            TRY(copy_out(ctx, heat_dst, heat, heat_bytes));
+            if (best_dst) TRY(copy_out(ctx, best_dst, best, heat_bytes));
         }
     }
     return PINK_HIP_OK;
