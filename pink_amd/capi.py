@@ -79,12 +79,13 @@ def lib():
         L.pink_hip_destroy.restype = None
         L.pink_hip_last_error.argtypes = [vp]
         L.pink_hip_last_error.restype = C.c_char_p
-        L.pink_hip_set_som.argtypes = [vp, f32p]
-        L.pink_hip_get_som.argtypes = [vp, f32p]
-        L.pink_hip_train.argtypes = [vp, f32p, u32, u32p]
-        L.pink_hip_update_counts.argtypes = [vp, u32p]
+        # (untyped pointers where arrays go in and out once per image: see _ptr)
+        L.pink_hip_set_som.argtypes = [vp, vp]
+        L.pink_hip_get_som.argtypes = [vp, vp]
+        L.pink_hip_train.argtypes = [vp, vp, u32, vp]
+        L.pink_hip_update_counts.argtypes = [vp, vp]
         L.pink_hip_train_device.argtypes = [vp, vp, u32, vp]
-        L.pink_hip_map.argtypes = [vp, f32p, u32, f32p, u32p]
+        L.pink_hip_map.argtypes = [vp, vp, u32, vp, vp]
         L.pink_hip_map_device.argtypes = [vp, vp, u32, vp, vp]
         L.pink_hip_map_device_static.argtypes = [vp, vp, u32, vp, vp]
         L.pink_hip_synchronize.argtypes = [vp]
@@ -113,6 +114,18 @@ def _f32(a):
 
 def _u32(a):
     return a.ctypes.data_as(C.POINTER(C.c_uint32))
+
+
+_Byte = C.c_char * 1
+
+
+def _ptr(a):
+    """The data of a contiguous array as an argument for an untyped pointer: a buffer view, a fifth of the time that
+    numpy's ctypes attribute takes (read-only and empty arrays go through that)."""
+    try:
+        return _Byte.from_buffer(a)
+    except (TypeError, ValueError):
+        return a.ctypes.data
 
 
 def device_info():
@@ -242,13 +255,13 @@ class Context:
     def set_som(self, som):
         som = np.ascontiguousarray(som, np.float32)
         assert som.size == self.N * self.S
-        self._check(self._L.pink_hip_set_som(self._h, _f32(som)))
+        self._check(self._L.pink_hip_set_som(self._h, _ptr(som)))
 
     def get_som(self, out=None):
         if out is None:
             out = np.empty((self.N, self.S), np.float32)
         assert out.dtype == np.float32 and out.flags.c_contiguous and out.size == self.N * self.S
-        self._check(self._L.pink_hip_get_som(self._h, _f32(out)))
+        self._check(self._L.pink_hip_get_som(self._h, _ptr(out)))
         return out
 
     def train(self, images, want_bmu=True):
@@ -259,16 +272,28 @@ class Context:
         n = images.size // self.image_size
         assert n * self.image_size == images.size
         if not want_bmu:
-            self._check(self._L.pink_hip_train(self._h, _f32(images), n, None))
+            self._check(self._L.pink_hip_train(self._h, _ptr(images), n, None))
             return None
         bmu = np.empty(n, np.uint32)
-        self._check(self._L.pink_hip_train(self._h, _f32(images), n, _u32(bmu)))
+        self._check(self._L.pink_hip_train(self._h, _ptr(images), n, _ptr(bmu)))
         return bmu
+
+    def train_image(self, image):
+        """train(image, want_bmu=False) for one contiguous float32 image of this context's size, unchecked."""
+        rc = self._L.pink_hip_train(self._h, _ptr(image), 1, None)
+        if rc:
+            self._check(rc)
+
+    def map_image(self, image, heat, best):
+        """map() for one contiguous float32 image of this context's size into arrays the caller keeps, unchecked."""
+        rc = self._L.pink_hip_map(self._h, _ptr(image), 1, _ptr(heat), _ptr(best))
+        if rc:
+            self._check(rc)
 
     def update_counts(self):
         """How often each neuron was the best match so far (the reference's update info)."""
         counts = np.empty(self.N, np.uint32)
-        self._check(self._L.pink_hip_update_counts(self._h, _u32(counts)))
+        self._check(self._L.pink_hip_update_counts(self._h, _ptr(counts)))
         return counts
 
     def train_device(self, dev_images_ptr, n, dev_bmu_ptr=None):
@@ -280,7 +305,7 @@ class Context:
         assert n * self.image_size == images.size
         heat = np.empty((n, self.N), np.float32)
         best = np.empty((n, self.N), np.uint32)
-        self._check(self._L.pink_hip_map(self._h, _f32(images), n, _f32(heat), _u32(best)))
+        self._check(self._L.pink_hip_map(self._h, _ptr(images), n, _ptr(heat), _ptr(best)))
         return heat, best
 
     def map_device(self, dev_images_ptr, n, dev_heat_ptr, dev_best_ptr=None):

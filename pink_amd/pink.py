@@ -91,7 +91,10 @@ def _as_float32_copy(buffer, what):
     a = np.asarray(buffer)
     if a.dtype != np.float32:
         raise TypeError("%s must be a float32 buffer" % what)     # py::arg().noconvert()
-    return np.array(a, dtype=np.float32, order="C", copy=True)     # the reference copies into a std::vector
+    return a.copy()                                                # the reference copies into a std::vector
+
+
+_DATA_NDIM = {"cartesian-1d": 1, "cartesian-2d": 2, "cartesian-3d": 3}
 
 
 class Data:
@@ -100,7 +103,7 @@ class Data:
     def __init__(self, buffer, data_type="float32", layout="cartesian-2d"):
         if data_type != "float32":
             raise exception(-1, "data-type not supported")
-        ndim = {"cartesian-1d": 1, "cartesian-2d": 2, "cartesian-3d": 3}.get(layout)
+        ndim = _DATA_NDIM.get(layout)
         if ndim is None:
             raise exception(-1, "layout " + layout + " is not supported")
         self._a = _as_float32_copy(buffer, "data")
@@ -204,6 +207,7 @@ class _Device:
         self.image_dim = None
         self.update_factors = update_factors
         self.counts_base = None
+        self.checked = None          # (shape, layout) of the last Data that for_images accepted for the current context
         # argument errors surface at construction, as in the reference; the image size is not known
         # yet and takes no part in these checks, so the neuron size stands in for it
         a = self.args
@@ -234,6 +238,7 @@ class _Device:
             self.ctx = self._context(image_dim)
             self.ctx.set_som(weights)
             self.image_dim = image_dim
+            self.checked = None
         return images.reshape(-1, channels, image_dim, image_dim)
 
 
@@ -272,8 +277,14 @@ class Trainer:
         """One image (Trainer.h:263-304).  Returns nothing, like the reference, and does not wait for
         the GPU: the image is copied, and images are trained in order a launch group at a time (when the group
         is full, or when update_som() or get_update_info() follows); those two wait for the result."""
-        images = self._dev.for_images(np.asarray(data)[None], getattr(data, "layout", "cartesian-2d"))
-        self._dev.ctx.train(images, want_bmu=False)
+        dev = self._dev
+        if type(data) is Data and dev.checked == (data._a.shape, data.layout):     # the loop's next image
+            dev.ctx.train_image(data._a)
+            return
+        images = dev.for_images(np.asarray(data)[None], getattr(data, "layout", "cartesian-2d"))
+        dev.ctx.train(images, want_bmu=False)
+        if type(data) is Data:
+            dev.checked = (data._a.shape, data.layout)
 
     def train(self, images, layout="cartesian-2d"):
         """Many images in order, one call: image k+1 sees the weights left by image k.  Returns the
@@ -284,7 +295,7 @@ class Trainer:
     def update_som(self):
         """Device weights -> the SOM object (Trainer.h:306-309)."""
         if self._dev.ctx is not None:
-            self._som._rows()[...] = self._dev.ctx.get_som()
+            self._dev.ctx.get_som(out=self._som._rows())
 
     @property
     def update_info(self):
@@ -308,11 +319,19 @@ class Mapper:
         self._dev = _Device(snapshot, number_of_rotations, use_flip, interpolation, use_gpu, euclidean_distance_dim,
                             euclidean_distance_shape, euclidean_distance_type, None)
         self.verbosity = verbosity
+        self._heat = np.empty(som.number_of_neurons, np.float32)       # one image's answer on its way into lists
+        self._best = np.empty(som.number_of_neurons, np.uint32)
 
     def __call__(self, data):
         """One image: (heatmap, best rotation per neuron) as two lists, like the bound
         std::tuple<std::vector<float>, std::vector<uint32_t>> (Mapper.h:181-208)."""
+        dev = self._dev
+        if type(data) is Data and dev.checked == (data._a.shape, data.layout):     # the loop's next image
+            dev.ctx.map_image(data._a, self._heat, self._best)
+            return self._heat.tolist(), self._best.tolist()
         heat, best = self.map(np.asarray(data)[None], getattr(data, "layout", "cartesian-2d"))
+        if type(data) is Data:
+            dev.checked = (data._a.shape, data.layout)
         return heat[0].tolist(), best[0].tolist()
 
     def map(self, images, layout="cartesian-2d"):
