@@ -2047,6 +2047,8 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
     if (tid == 0) a.na_next[n] = (long long)na;
 }
 
+#include "sym_train.inc"
+
 // m_update_info[bmu]++ for the images of a group (Trainer.h:302-303), behind a resident launch: nothing when that launch
 // or one before it gave up.  The error word goes to the host with it, which looks when it next waits for the stream.
 __global__ __launch_bounds__(256) void k_count_best_matches(const uint32_t *__restrict__ bmu, uint32_t images, uint32_t *__restrict__ counts,
@@ -2310,6 +2312,16 @@ struct pink_hip_ctx {
     uint32_t exchange_tag = 1, spin_limit = 1u << 21;
     struct ResidentGroup { const float *images; uint32_t count; uint32_t *bmu; };
     std::vector<ResidentGroup> resident_queued;   // groups whose resident launches the host has not checked yet
+    // integer trainers with the symmetries on the SOM side, resident over a launch group (k_train_sym_resident); the GEMM
+    // path's operands are then made when something else wants them
+    bool sym_train = false;
+    uint32_t sym_npb = 1, sym_nit = 0, sym_B = 0, sym_KS = 0, sym_RT = 0, sym_all = 0, sym_cells = 0, sym_outside = 0, sym_tag0 = 1;
+    size_t sym_lds = 0, sym_prep_lds = 0;
+    uint32_t *d_sym_upos = nullptr, *d_sym_outside = nullptr, *d_sym_best = nullptr;
+    uint4 *d_sym_elem = nullptr, *d_sym_at = nullptr;
+    v4i *d_sym_mask = nullptr, *d_sym_op = nullptr;
+    float *d_sym_x = nullptr;
+    long long *d_sym_norm = nullptr;
     unsigned long long *d_src4 = nullptr;  // ... its per-element tables (see the kernel)
     uint32_t *d_kbyte = nullptr;
     uint32_t *d_grow = nullptr, *d_gvariant = nullptr;   // variant index -> row of the variant operand, and back
@@ -2888,8 +2900,19 @@ int run_train_small(pink_hip_ctx *ctx, uint32_t slot, uint32_t *dev_bmu_out)
 void swap_resident(pink_hip_ctx *ctx)
 {
     std::swap(ctx->d_som, ctx->d_som_alt);
+    if (!ctx->small_train) return;
     ctx->pa_cur ^= 1;
     ctx->na_cur ^= 1;
+}
+
+int resident_launched(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, uint32_t *dev_bmu)
+{
+    hipLaunchKernelGGL(k_count_best_matches, dim3((images + 255) / 256), dim3(256), 0, ctx->stream, dev_bmu, images, ctx->d_counts,
+                       ctx->d_resident_error, ctx->h_resident_error);
+    TRY(launch_check(ctx, "k_count_best_matches"));
+    ctx->resident_queued.push_back({dev_images, images, dev_bmu});
+    swap_resident(ctx);
+    return PINK_HIP_OK;
 }
 
 // The first `images` images of the current group in one resident launch (small uint8 trainers), queued: whether every
@@ -2934,13 +2957,77 @@ int run_train_small_resident(pink_hip_ctx *ctx, const float *dev_images, uint32_
 #undef LAUNCH_RESIDENT
         TRY(launch_check(ctx, "k_train_small_u8_resident"));
     }
-    hipLaunchKernelGGL(k_count_best_matches, dim3((images + 255) / 256), dim3(256), 0, ctx->stream, dev_bmu, images, ctx->d_counts,
-                       ctx->d_resident_error, ctx->h_resident_error);
-    TRY(launch_check(ctx, "k_count_best_matches"));
-    ctx->resident_queued.push_back({dev_images, images, dev_bmu});
-    swap_resident(ctx);
-    return PINK_HIP_OK;
+    return resident_launched(ctx, dev_images, images, dev_bmu);
 }
+
+template <bool U16, int NPB>
+const void *sym_kernel_of(uint32_t cells)
+{
+    return cells <= 1 ? (const void *)k_train_sym_resident<U16, NPB, 1> : cells <= 2 ? (const void *)k_train_sym_resident<U16, NPB, 2>
+         : (const void *)k_train_sym_resident<U16, NPB, kSymMaxCells>;
+}
+
+template <bool U16>
+const void *sym_kernel_for(uint32_t npb, uint32_t cells)
+{
+    return npb == 1 ? sym_kernel_of<U16, 1>(cells) : npb == 2 ? sym_kernel_of<U16, 2>(cells) : sym_kernel_of<U16, 4>(cells);
+}
+
+const void *sym_kernel(const pink_hip_ctx *ctx)
+{
+    return ctx->cfg.ed_type == PINK_HIP_UINT16 ? sym_kernel_for<true>(ctx->sym_npb, ctx->sym_nit) : sym_kernel_for<false>(ctx->sym_npb, ctx->sym_nit);
+}
+
+const void *sym_prepare_kernel(const pink_hip_ctx *ctx)
+{
+    if (ctx->cfg.ed_type == PINK_HIP_UINT16)
+        return ctx->sym_prep_lds ? (const void *)k_sym_prepare<true, true> : (const void *)k_sym_prepare<true, false>;
+    return ctx->sym_prep_lds ? (const void *)k_sym_prepare<false, true> : (const void *)k_sym_prepare<false, false>;
+}
+
+// A launch group of an integer trainer with the symmetries on the SOM side: base rotations, the resident launch, the
+// elements outside the region.
+int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, uint32_t *dev_bmu)
+{
+    {
+        Timed t(ctx, kClsRotate);
+        SymPrep p{};
+        p.images = dev_images; p.cos_t = ctx->d_cos; p.sin_t = ctx->d_sin; p.upos = ctx->d_sym_upos; p.smask = ctx->d_sym_mask;
+        p.opnd = ctx->d_sym_op; p.xrows = ctx->d_sym_x; p.norm = ctx->d_sym_norm;
+        p.C = ctx->C; p.I = ctx->I; p.D = ctx->D; p.nrr = ctx->nrr_eff; p.RT = ctx->sym_RT; p.KS = ctx->sym_KS;
+        p.all_sym = ctx->sym_all;
+        // (an image in a large part of the LDS leaves room for few blocks on a CU: large ones then)
+        const uint32_t threads = ctx->sym_prep_lds > 40 * 1024 || images * ctx->sym_RT < (uint32_t)ctx->num_cu ? 1024 : 256;
+        void *args[] = {&p};
+        HIP_TRY(ctx, hipLaunchKernel(sym_prepare_kernel(ctx), dim3(ctx->sym_RT, images), dim3(threads), args, ctx->sym_prep_lds, ctx->stream));
+    }
+    {
+        Timed t(ctx, kClsUpdate);
+        SymTrain a{};
+        a.som = ctx->d_som; a.som_next = ctx->d_som_alt; a.opnd = ctx->d_sym_op; a.xrows = ctx->d_sym_x; a.norm = ctx->d_sym_norm;
+        a.factors_t = ctx->d_factors_t; a.cell_elem = ctx->d_sym_elem; a.cell_at = ctx->d_sym_at; a.best_variant = ctx->d_sym_best;
+        a.bmu_out = dev_bmu; a.slots = ctx->d_slots; a.error = ctx->d_resident_error;
+        a.launch = (uint32_t)ctx->resident_queued.size() + 1;
+        a.N = ctx->N; a.S = ctx->S; a.cells = ctx->sym_cells; a.KS = ctx->sym_KS; a.RT = ctx->sym_RT; a.nrr = ctx->nrr_eff;
+        a.num_rot = ctx->cfg.num_rot; a.use_flip = ctx->cfg.use_flip; a.images = images; a.tag0 = ctx->sym_tag0; a.spin_limit = ctx->spin_limit;
+        ctx->sym_tag0 = sym_tag(ctx->sym_tag0, images);
+        void *args[] = {&a};
+        HIP_TRY(ctx, hipLaunchKernel(sym_kernel(ctx), dim3((ctx->N + ctx->sym_npb - 1) / ctx->sym_npb), dim3(kSymThreads), args, ctx->sym_lds, ctx->stream));
+    }
+    if (ctx->sym_outside) {
+        Timed t(ctx, kClsUpdate);
+        SymOutside o{};
+        o.som = ctx->d_som; o.som_next = ctx->d_som_alt; o.images = dev_images; o.cos_t = ctx->d_cos; o.sin_t = ctx->d_sin;
+        o.factors = ctx->d_factors; o.best_variant = ctx->d_sym_best; o.bmu = dev_bmu; o.outside = ctx->d_sym_outside;
+        o.error = ctx->d_resident_error; o.count = ctx->sym_outside; o.N = ctx->N; o.S = ctx->S; o.C = ctx->C; o.I = ctx->I;
+        o.D = ctx->D; o.nrr = ctx->nrr_eff; o.num_rot = ctx->cfg.num_rot; o.images_n = images;
+        hipLaunchKernelGGL(k_sym_outside, dim3((ctx->sym_outside + 255) / 256, ctx->N), dim3(256), 0, ctx->stream, o);
+        TRY(launch_check(ctx, "k_sym_outside"));
+    }
+    return resident_launched(ctx, dev_images, images, dev_bmu);
+}
+
+int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out);
 
 // Wait for the queued resident launches.  If one gave up, nothing after it has run: back to the buffers it started from,
 // its group and the later ones image by image, and the context stays with that form.
@@ -2953,16 +3040,16 @@ int finish_resident(pink_hip_ctx *ctx)
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     const uint32_t failed = *ctx->h_resident_error;
     if (!failed) return PINK_HIP_OK;
-    ctx->resident_train = false;
-    HIP_TRY(ctx, hipMemsetAsync(ctx->d_resident_error, 0, sizeof(uint32_t), ctx->stream));
-    HIP_TRY(ctx, hipMemsetAsync(ctx->d_slots, 0, kSlotWords * sizeof(unsigned long long), ctx->stream));
     if ((queued.size() - (failed - 1)) & 1) swap_resident(ctx);
-    for (size_t g = failed - 1; g < queued.size(); ++g) {
-        TRY(run_rotate(ctx, queued[g].images, queued[g].count, kStorePair));
-        for (uint32_t b = 0; b < queued[g].count; ++b) TRY(run_train_small(ctx, b, queued[g].bmu + b));
-    }
+    if (ctx->sym_train) TRY(run_pack_som(ctx));            // the other path's operand of the SOM as it is now
+    ctx->resident_train = ctx->sym_train = false;
+    HIP_TRY(ctx, hipMemsetAsync(ctx->d_resident_error, 0, sizeof(uint32_t), ctx->stream));
+    for (size_t g = failed - 1; g < queued.size(); ++g) TRY(train_queued(ctx, queued[g].images, queued[g].count, queued[g].bmu));
     return PINK_HIP_OK;
 }
+
+// Images of a launch group.
+uint32_t train_group(const pink_hip_ctx *ctx) { return ctx->sym_train ? ctx->sym_B : ctx->Bcap; }
 
 int run_finalize(pink_hip_ctx *ctx, uint32_t B, float *dev_dist, long long *dev_ssd, uint32_t *dev_best, bool do_sqrt)
 {
@@ -2983,7 +3070,7 @@ int free_all(pink_hip_ctx *ctx)
     void *bufs[] = {ctx->d_som, ctx->d_rot, ctx->d_cos, ctx->d_sin, ctx->d_factors, ctx->d_factors_t, ctx->d_region, ctx->d_key,
                     ctx->d_somP, ctx->d_somP_alt, ctx->d_bmu_group, ctx->d_rotT, ctx->d_bmu_scratch, ctx->d_dist, ctx->d_ssd, ctx->d_best,
                     ctx->d_Pa, ctx->d_Pb, ctx->d_na, ctx->d_nb, ctx->d_poff, ctx->d_need, ctx->d_inv,
-                    ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_grow, ctx->d_gvariant, ctx->d_region4};
+                    ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu}) if (p) (void)hipFree(p);
     if (ctx->st_pin) (void)hipHostFree(ctx->st_pin);
@@ -3019,6 +3106,181 @@ int resolve_static_scratch(pink_hip_ctx *ctx)
         g_scratch_ptr[ctx->device] = (unsigned char *)p;
     }
     ctx->static_scratch = g_scratch_ptr[ctx->device];
+    return PINK_HIP_OK;
+}
+
+// PINK_HIP_RESIDENT_TRAINER=0: one launch per image and kernel from the start.
+bool resident_allowed()
+{
+    const char *off = getenv("PINK_HIP_RESIDENT_TRAINER");
+    return !off || atoi(off) != 0;
+}
+
+// What the blocks of a resident trainer exchange their words through, and the second weight array.
+int init_exchange(pink_hip_ctx *ctx, size_t slot_words)
+{
+    // (a test can make every wait give up at once, to see the group trained again image by image)
+    if (const char *limit = getenv("PINK_HIP_RESIDENT_SPIN_LIMIT")) ctx->spin_limit = (uint32_t)strtoul(limit, nullptr, 10);
+    // (... or start the tags of the exchange just below the value where they wrap, which 2^32 images take)
+    if (const char *tag = getenv("PINK_HIP_RESIDENT_FIRST_TAG")) ctx->exchange_tag = std::max(1u, (uint32_t)strtoul(tag, nullptr, 10));
+    TRY(dev_alloc(ctx, &ctx->d_som_alt, (size_t)ctx->N * ctx->S));
+    TRY(dev_alloc(ctx, &ctx->d_slots, slot_words));
+    HIP_TRY(ctx, hipMemset(ctx->d_slots, 0, slot_words * sizeof(unsigned long long)));
+    TRY(dev_alloc(ctx, &ctx->d_resident_error, 1));
+    HIP_TRY(ctx, hipMemset(ctx->d_resident_error, 0, sizeof(uint32_t)));
+    if (hipHostMalloc((void **)&ctx->h_resident_error, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+        ctx->h_resident_error = nullptr;
+        return fail(ctx, PINK_HIP_ENOMEM, "pinned host allocation failed");
+    }
+    return PINK_HIP_OK;
+}
+
+// Where element e of the region sits in the base rotation under symmetry sym = flip * 4 + quarter (see k_rotate).
+inline uint32_t symmetric_position(uint32_t off, uint32_t D, uint32_t sym)
+{
+    const uint32_t DD = D * D, ch = off / DD, x = (off % DD) / D, y = off % D, xs = (sym & 4) ? D - 1 - x : x;
+    switch (sym & 3) {
+    case 0: return ch * DD + xs * D + y;
+    case 1: return ch * DD + (D - 1 - y) * D + xs;
+    case 2: return ch * DD + (D - 1 - xs) * D + (D - 1 - y);
+    default: return ch * DD + y * D + (D - 1 - xs);
+    }
+}
+
+template <typename T>
+int upload(pink_hip_ctx *ctx, T **dev, const std::vector<T> &host)
+{
+    TRY(dev_alloc(ctx, dev, host.size()));
+    if (!host.empty()) HIP_TRY(ctx, hipMemcpy(*dev, host.data(), host.size() * sizeof(T), hipMemcpyHostToDevice));
+    return PINK_HIP_OK;
+}
+
+// Integer trainers whose neurons' eight symmetric operand rows fit the LDS of as many blocks as there are compute units:
+// the resident form with the symmetries on the SOM side.  (region: distinct elements, in the CPU's order.)
+int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
+{
+    const pink_hip_config &c = ctx->cfg;
+    const uint32_t D = ctx->D, DD = D * D;
+    if (!ctx->gemm || !ctx->fused_som || c.kernel_choice != PINK_HIP_KERNEL_AUTO || ctx->N > kSymMaxNeurons || D >= 4096 || ctx->C >= 256 ||
+        !resident_allowed())
+        return PINK_HIP_OK;
+    // Coordinates run to an even bound, the middle of an odd one twice (see sym_train.inc): place X of pixel x, and back.
+    const uint32_t odd = D & 1, mid = D / 2, Ds = D + odd, half = Ds / 2;
+    auto place = [&](uint32_t x) { return x + (odd && x > mid ? 1u : 0u); };
+    auto pixel = [&](uint32_t X) { return X - (odd && X > mid ? 1u : 0u); };
+    // cells of 2 x 2 places: id = (channel * half + X / 2) * half + Y / 2
+    auto cell_id = [&](uint32_t ch, uint32_t X, uint32_t Y) { return (ch * half + X / 2) * half + Y / 2; };
+    const uint32_t cells_all = ctx->C * half * half;
+    std::vector<uint4> elem_of(cells_all, make_uint4(~0u, ~0u, ~0u, ~0u));       // elements of the neuron per cell
+    std::vector<char> in_region(cells_all, 0), in_union(cells_all, 0);
+    for (uint32_t off : region) {
+        const uint32_t X = place((off % DD) / D), Y = place(off % D), id = cell_id(off / DD, X, Y);
+        (&elem_of[id].x)[(X & 1) * 2 + (Y & 1)] = off;
+        in_region[id] = 1;
+    }
+    auto moved = [&](uint32_t id, uint32_t sym) {           // where a cell goes under a symmetry (its first place decides)
+        const uint32_t ch = id / (half * half), off = ch * Ds * Ds + ((id / half) % half) * 2 * Ds + (id % half) * 2;
+        const uint32_t to = symmetric_position(off, Ds, sym);
+        return cell_id(ch, (to % (Ds * Ds)) / Ds, to % Ds);
+    };
+    auto valid = [&](uint32_t sym) { return (c.num_rot != 1 || (sym & 3) == 0) && (c.use_flip || sym < 4); };
+    for (uint32_t id = 0; id < cells_all; ++id)
+        for (uint32_t sym = 0; sym < 8; ++sym)
+            if (in_region[id] && valid(sym)) in_union[moved(id, sym)] = 1;
+    // the order of the cells, in the operand and over the threads: 4 x 4 of them at a time, so that the cells of a wave lie
+    // in a few lines of a row whichever symmetry reads it
+    auto listed = [&](const std::vector<char> &in) {
+        std::vector<uint32_t> ids;
+        for (uint32_t id = 0; id < cells_all; ++id) if (in[id]) ids.push_back(id);
+        auto key = [&](uint32_t id) {
+            const uint64_t ch = id / (half * half), x = (id / half) % half, y = id % half;
+            return (ch << 48) | ((x / 4) << 32) | ((y / 4) << 16) | ((x % 4) << 8) | (y % 4);
+        };
+        std::sort(ids.begin(), ids.end(), [&](uint32_t l, uint32_t r) { return key(l) < key(r); });
+        return ids;
+    };
+    const std::vector<uint32_t> cells = listed(in_region), all = listed(in_union);
+    ctx->sym_cells = (uint32_t)cells.size();
+    ctx->sym_RT = (ctx->nrr_eff + 15) / 16;
+    // every share of k a multiple of four k-steps
+    ctx->sym_KS = round_up(((uint32_t)all.size() * 4 + 63) / 64, 4 * sym_shares(ctx->sym_RT));
+    const uint32_t Kp = ctx->sym_KS * 64;
+    if (Kp > kSymMaxK) return PINK_HIP_OK;
+    const bool u16 = c.ed_type == PINK_HIP_UINT16;
+    // as few neurons per block as leave no more blocks than compute units: a block's part of an image shrinks with them
+    uint32_t npb = 1;
+    while (npb <= 4 && (ctx->N + npb - 1) / npb > (uint32_t)ctx->num_cu) npb *= 2;
+    if (npb > 4) return PINK_HIP_OK;
+    ctx->sym_npb = npb;
+    ctx->sym_nit = (npb * ctx->sym_cells + kSymLanes - 1) / kSymLanes;
+    ctx->sym_lds = sym_lds_bytes(npb, ctx->sym_KS, u16, ctx->N, ctx->sym_RT);
+    if (ctx->sym_nit > kSymMaxCells || ctx->sym_lds + 2048 > ctx->lds_max) return PINK_HIP_OK;
+    const size_t image_lds = (size_t)ctx->C * ctx->I * ctx->I * sizeof(float);
+    ctx->sym_prep_lds = image_lds <= 150 * 1024 ? image_lds : 0;
+
+    // position k of a row: element 2 r + c of cell k / 4
+    std::vector<uint32_t> rank(cells_all, 0), upos(Kp, ~0u);
+    for (uint32_t i = 0; i < all.size(); ++i) rank[all[i]] = i;
+    for (uint32_t i = 0; i < all.size(); ++i)
+        for (uint32_t b = 0; b < 4; ++b) {
+            const uint32_t ch = all[i] / (half * half), X = ((all[i] / half) % half) * 2 + (b >> 1), Y = (all[i] % half) * 2 + (b & 1);
+            upos[i * 4 + b] = (ch << 24) | (pixel(X) << 12) | pixel(Y);
+        }
+    std::vector<uint4> elem(cells.size()), at(cells.size());
+    std::vector<unsigned char> mask((size_t)8 * Kp, 0);
+    std::vector<std::vector<uint32_t>> seen(8);             // the pixels of P_s: the same for every s, or not
+    for (uint32_t i = 0; i < cells.size(); ++i) {
+        elem[i] = elem_of[cells[i]];
+        uint32_t a16[8];
+        for (uint32_t sym = 0; sym < 8; ++sym) {
+            const uint32_t to = valid(sym) ? rank[moved(cells[i], sym)] : 0u;
+            a16[sym] = sym_lds_address(to >> 2, sym) + (to & 3) * 4;
+            for (uint32_t b = 0; b < 4 && valid(sym); ++b)
+                if ((&elem[i].x)[b] != ~0u) {
+                    const uint32_t k = to * 4 + sym_cell_byte((int)sym, (int)b);
+                    mask[(size_t)sym * Kp + k] = 0xff;
+                    seen[sym].push_back(upos[k]);
+                }
+        }
+        at[i] = make_uint4(a16[0] | (a16[1] << 16), a16[2] | (a16[3] << 16), a16[4] | (a16[5] << 16), a16[6] | (a16[7] << 16));
+    }
+    ctx->sym_all = 1;
+    for (uint32_t sym = 0; sym < 8; ++sym) {
+        std::sort(seen[sym].begin(), seen[sym].end());
+        if (valid(sym) && seen[sym] != seen[0]) ctx->sym_all = 0;
+    }
+    std::vector<uint32_t> outside;
+    {
+        std::vector<char> inside(ctx->S, 0);
+        for (uint32_t off : region) inside[off] = 1;
+        for (uint32_t j = 0; j < ctx->S; ++j) if (!inside[j]) outside.push_back(j);
+        auto key = [&](uint32_t off) {
+            const uint64_t ch = off / DD, x = (off % DD) / D, y = off % D;
+            return (ch << 48) | ((x / 8) << 32) | ((y / 8) << 16) | ((x % 8) << 8) | (y % 8);
+        };
+        std::sort(outside.begin(), outside.end(), [&](uint32_t l, uint32_t r) { return key(l) < key(r); });
+    }
+    ctx->sym_outside = (uint32_t)outside.size();
+    TRY(upload(ctx, &ctx->d_sym_upos, upos));
+    TRY(upload(ctx, &ctx->d_sym_elem, elem));
+    TRY(upload(ctx, &ctx->d_sym_outside, outside));
+    TRY(upload(ctx, &ctx->d_sym_at, at));
+    TRY(upload(ctx, (unsigned char **)&ctx->d_sym_mask, mask));
+    // a group's operand and rows are written by one launch and read by the next: within the last-level cache
+    const size_t op_image = (size_t)(u16 ? 2 : 1) * ctx->sym_RT * ctx->sym_KS * 1024, x_image = (size_t)ctx->nrr_eff * Kp * sizeof(float);
+    size_t b = c.max_batch ? std::min<size_t>(c.max_batch, kSymGroupMax) : kSymGroupMax;
+    while (b > 8 && b * (op_image + x_image) > ((size_t)192 << 20)) --b;
+    ctx->sym_B = (uint32_t)b;
+    TRY(dev_alloc(ctx, &ctx->d_sym_op, b * op_image / 16));
+    TRY(dev_alloc(ctx, &ctx->d_sym_x, b * ctx->nrr_eff * Kp));
+    TRY(dev_alloc(ctx, &ctx->d_sym_norm, b * ctx->sym_RT * 16 * 8));
+    TRY(dev_alloc(ctx, &ctx->d_sym_best, b * ctx->N));
+    TRY(init_exchange(ctx, (size_t)2 * ctx->N * kSymStride));
+    ctx->sym_tag0 = (ctx->exchange_tag - 1) % 0xfffeu + 1;
+    ctx->sym_train = true;
+    // (limits are per kernel, not per context)
+    HIP_TRY(ctx, hipFuncSetAttribute(sym_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
+    if (ctx->sym_prep_lds) HIP_TRY(ctx, hipFuncSetAttribute(sym_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
     return PINK_HIP_OK;
 }
 
@@ -3479,27 +3741,15 @@ int init_ctx(pink_hip_ctx *ctx)
             HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_train_small_u8<4, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 32768));
             HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_train_small_u8<8, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 32768));
             // resident over a launch group: every block needs a compute unit of its own for the whole launch
-            ctx->resident_train = ctx->N <= (uint32_t)ctx->num_cu;
-            if (const char *off = getenv("PINK_HIP_RESIDENT_TRAINER")) ctx->resident_train = ctx->resident_train && atoi(off) != 0;
+            ctx->resident_train = ctx->N <= (uint32_t)ctx->num_cu && resident_allowed();
             if (ctx->resident_train) {
-                // (a test can make every wait give up at once, to see the group trained again image by image)
-                if (const char *limit = getenv("PINK_HIP_RESIDENT_SPIN_LIMIT")) ctx->spin_limit = (uint32_t)strtoul(limit, nullptr, 10);
-                // (... or start the tags of the exchange just below the value where they wrap, which 2^32 images take)
-                if (const char *tag = getenv("PINK_HIP_RESIDENT_FIRST_TAG")) ctx->exchange_tag = std::max(1u, (uint32_t)strtoul(tag, nullptr, 10));
-                TRY(dev_alloc(ctx, &ctx->d_som_alt, (size_t)ctx->N * ctx->S));
-                TRY(dev_alloc(ctx, &ctx->d_slots, (size_t)kSlotWords));
-                HIP_TRY(ctx, hipMemset(ctx->d_slots, 0, kSlotWords * sizeof(unsigned long long)));
-                TRY(dev_alloc(ctx, &ctx->d_resident_error, 1));
-                HIP_TRY(ctx, hipMemset(ctx->d_resident_error, 0, sizeof(uint32_t)));
-                if (hipHostMalloc((void **)&ctx->h_resident_error, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
-                    ctx->h_resident_error = nullptr;
-                    return fail(ctx, PINK_HIP_ENOMEM, "pinned host allocation failed");
-                }
+                TRY(init_exchange(ctx, kSlotWords));
                 HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_train_small_u8_resident<2, 4, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
                 HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_train_small_u8_resident<2, 4, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
                 HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_train_small_u8_resident<4, 8, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
             }
         }
+        if (one_to_one && !ctx->small_train) TRY(init_sym_train(ctx, region));
         // one launch per image where the float32 distance kernel runs in its one-wave-per-SIMD form (see k_train_f32_dpp;
         // up to 256 neurons: measured with 512 allowed, 17 x 17 and 18 x 18 neurons at 720 variants train no faster this
         // way than with an update launch of their own -- with three to four waves per SIMD the launch saved is paid in
@@ -3509,7 +3759,8 @@ int init_ctx(pink_hip_ctx *ctx)
         ctx->rows_f32_train = !ctx->fused_f32_train && c.ed_type == PINK_HIP_FLOAT && !ctx->f32gemm && ctx->d_somP && ctx->d_inv &&
                               B <= kReplayMax;
         if (ctx->fused_f32_train) TRY(dev_alloc(ctx, (uint32_t **)&ctx->d_somP_alt, (size_t)ctx->N * ctx->Epad + kDistOverrun));
-        if (ctx->fused_f32_train || ctx->rows_f32_train || ctx->resident_train) TRY(dev_alloc(ctx, &ctx->d_bmu_group, B));
+        if (ctx->fused_f32_train || ctx->rows_f32_train || ctx->resident_train || ctx->sym_train)
+            TRY(dev_alloc(ctx, &ctx->d_bmu_group, std::max<size_t>(B, ctx->sym_B)));
         TRY(dev_alloc(ctx, &ctx->d_factors, (size_t)ctx->N * ctx->N));
         HIP_TRY(ctx, hipMemcpy(ctx->d_factors, c.update_factors, (size_t)ctx->N * ctx->N * sizeof(float),
                                hipMemcpyHostToDevice));
@@ -3600,6 +3851,62 @@ int distance_group(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
     return PINK_HIP_OK;
 }
 
+// Training of images that are on the device, queued on the context's stream.
+int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
+{
+    if (ctx->sym_train) {
+        for (uint32_t done = 0; done < n_images; done += ctx->sym_B) {
+            const uint32_t B = std::min(ctx->sym_B, n_images - done);
+            TRY(run_sym_train(ctx, dev_images + (size_t)done * ctx->isz, B, dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group));
+        }
+        return PINK_HIP_OK;
+    }
+    // The variants of an image and their packed distance operand do not depend on the SOM: they
+    // are produced for a group of images per launch.  Distance and update stay strictly sequential.
+    for (uint32_t done = 0; done < n_images; done += ctx->Bcap) {
+        const uint32_t B = std::min(ctx->Bcap, n_images - done);
+        TRY(run_rotate(ctx, dev_images + (size_t)done * ctx->isz, B, ctx->pair_variants ? kStorePair : kStoreAll));
+        TRY(run_pack_rot(ctx, B));
+        if (ctx->fused_f32_train) {
+            // every launch but the first applies the update of the image before it; the last image's update and,
+            // ahead of it, all the others on the neurons' full images close the group
+            uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group;
+            {
+                // (per-kernel timing: one pair of events around the group's launches, which follow each other directly)
+                Timed t(ctx, kClsDist, B);
+                for (uint32_t b = 0; b < B; ++b) TRY(run_train_f32(ctx, b, b > 0, b > 0 ? bmu + b - 1 : nullptr));
+            }
+            if (B > 1) TRY(run_update_replay(ctx, B - 1, bmu));
+            TRY(run_update(ctx, B - 1, bmu + B - 1));
+            continue;
+        }
+        if (ctx->rows_f32_train) {
+            uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group;
+            for (uint32_t b = 0; b < B; ++b) {
+                TRY(run_dist(ctx, b, 1));
+                TRY(run_update_rows(ctx, b, bmu + b));
+            }
+            TRY(run_update_replay(ctx, B, bmu));
+            continue;
+        }
+        if (ctx->resident_train) {
+            TRY(run_train_small_resident(ctx, dev_images + (size_t)done * ctx->isz, B, dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group));
+            continue;
+        }
+        for (uint32_t b = 0; b < B; ++b) {
+            if (ctx->small_train) {
+                TRY(run_train_small(ctx, b, dev_bmu_out ? dev_bmu_out + done + b : ctx->d_bmu_scratch));
+                continue;
+            }
+            TRY(run_dist(ctx, b, 1));
+            TRY(run_update(ctx, b, dev_bmu_out ? dev_bmu_out + done + b : ctx->d_bmu_scratch));
+            if (!ctx->d_inv || (ctx->gemm && !ctx->fused_som)) TRY(run_pack_som(ctx));
+            else if (ctx->f32gemm) { Timed t(ctx, kClsPack); TRY(run_pack_frag_som(ctx)); }
+        }
+    }
+    return PINK_HIP_OK;
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------------
@@ -3680,7 +3987,6 @@ void pink_hip_destroy(pink_hip_ctx *ctx)
 // they produce.  The order of the images and every result are those of training them call by call.
 int ensure_staging(pink_hip_ctx *ctx, size_t n);
 static int copy_out(pink_hip_ctx *ctx, void *host, const void *dev, size_t bytes);
-static int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out);
 
 // The pending images go to the device and through training, queued.
 static int start_pending(pink_hip_ctx *ctx)
@@ -3754,54 +4060,6 @@ int pink_hip_train_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     TRY(train_queued(ctx, dev_images, n_images, dev_bmu_out));
     return finish_resident(ctx);                          // (the images are the caller's again on return)
-}
-
-static int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
-{
-    // The variants of an image and their packed distance operand do not depend on the SOM: they
-    // are produced for a group of images per launch.  Distance and update stay strictly sequential.
-    for (uint32_t done = 0; done < n_images; done += ctx->Bcap) {
-        const uint32_t B = std::min(ctx->Bcap, n_images - done);
-        TRY(run_rotate(ctx, dev_images + (size_t)done * ctx->isz, B, ctx->pair_variants ? kStorePair : kStoreAll));
-        TRY(run_pack_rot(ctx, B));
-        if (ctx->fused_f32_train) {
-            // every launch but the first applies the update of the image before it; the last image's update and,
-            // ahead of it, all the others on the neurons' full images close the group
-            uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group;
-            {
-                // (per-kernel timing: one pair of events around the group's launches, which follow each other directly)
-                Timed t(ctx, kClsDist, B);
-                for (uint32_t b = 0; b < B; ++b) TRY(run_train_f32(ctx, b, b > 0, b > 0 ? bmu + b - 1 : nullptr));
-            }
-            if (B > 1) TRY(run_update_replay(ctx, B - 1, bmu));
-            TRY(run_update(ctx, B - 1, bmu + B - 1));
-            continue;
-        }
-        if (ctx->rows_f32_train) {
-            uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group;
-            for (uint32_t b = 0; b < B; ++b) {
-                TRY(run_dist(ctx, b, 1));
-                TRY(run_update_rows(ctx, b, bmu + b));
-            }
-            TRY(run_update_replay(ctx, B, bmu));
-            continue;
-        }
-        if (ctx->resident_train) {
-            TRY(run_train_small_resident(ctx, dev_images + (size_t)done * ctx->isz, B, dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group));
-            continue;
-        }
-        for (uint32_t b = 0; b < B; ++b) {
-            if (ctx->small_train) {
-                TRY(run_train_small(ctx, b, dev_bmu_out ? dev_bmu_out + done + b : ctx->d_bmu_scratch));
-                continue;
-            }
-            TRY(run_dist(ctx, b, 1));
-            TRY(run_update(ctx, b, dev_bmu_out ? dev_bmu_out + done + b : ctx->d_bmu_scratch));
-            if (!ctx->d_inv || (ctx->gemm && !ctx->fused_som)) TRY(run_pack_som(ctx));
-            else if (ctx->f32gemm) { Timed t(ctx, kClsPack); TRY(run_pack_frag_som(ctx)); }
-        }
-    }
-    return PINK_HIP_OK;
 }
 
 constexpr size_t kPinBytes = (size_t)1 << 20;
@@ -3916,13 +4174,14 @@ int staged_run(pink_hip_ctx *ctx, const float *host_images, uint32_t n, Run run)
     // (a trainer's kernels take long enough per image for 16 MB pieces to hide all copies but the first behind them:
     // cfg0 40 k -> 51 k images/s with pageable buffers; a mapper's launch groups want the larger pieces)
     // Nothing hides the copy of the first piece, so the pieces start at about 1 MB and double up to that size.
+    const uint32_t group = train_group(ctx);
     const auto whole_groups = [&](size_t bytes) {
         uint32_t images = (uint32_t)std::max<size_t>(1, bytes / img_bytes);
-        if (images > ctx->Bcap) images -= images % ctx->Bcap;
+        if (images > group) images -= images % group;
         return images;
     };
     const uint32_t largest = whole_groups((size_t)(ctx->trainer ? 16 : 64) << 20);
-    uint32_t piece = std::min(largest, std::max(whole_groups((size_t)1 << 20), std::min(ctx->Bcap, largest)));
+    uint32_t piece = std::min(largest, std::max(whole_groups((size_t)1 << 20), std::min(group, largest)));
     // A mapper's kernels are faster than the link, so its rate from host buffers is the rate of the copies, and a
     // copy out of pageable memory is one host thread's work (about half of what the link takes): its inputs go through
     // the shared pinned pieces, which host threads fill side by side (cfg1 from pageable memory: 26 -> 42 GB/s,
@@ -3973,7 +4232,7 @@ int pink_hip_train(pink_hip_ctx *ctx, const float *host_images, uint32_t n_image
             hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
             bool ok = true;
             for (int i = 0; i < 2 && ok; ++i)
-                ok = hipHostMalloc((void **)&pin[i], (size_t)ctx->Bcap * img_bytes, hipHostMallocDefault) == hipSuccess;
+                ok = hipHostMalloc((void **)&pin[i], (size_t)train_group(ctx) * img_bytes, hipHostMallocDefault) == hipSuccess;
             for (int i = 0; i < 3 && ok; ++i) ok = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) == hipSuccess;
             if (!ok) {
                 (void)hipGetLastError();
@@ -3981,7 +4240,7 @@ int pink_hip_train(pink_hip_ctx *ctx, const float *host_images, uint32_t n_image
                 for (char *q : pin) if (q) (void)hipHostFree(q);
                 return fail(ctx, PINK_HIP_ENOMEM, "pink_hip_train: pinned host buffers for queued images could not be set up");
             }
-            ctx->pend_cap = ctx->Bcap;
+            ctx->pend_cap = train_group(ctx);
             for (int i = 0; i < 2; ++i) { ctx->pend_pin[i] = pin[i]; ctx->pend_ev[i] = ev[i]; }
             ctx->pend_done = ev[2];
         }
@@ -4186,7 +4445,8 @@ int pink_hip_distance(pink_hip_ctx *ctx, const float *host_image, float *host_di
     HIP_TRY(ctx, hipMalloc((void **)&d_img, (size_t)ctx->isz * sizeof(float)));
     hipError_t e = hipMemcpyAsync(d_img, host_image, (size_t)ctx->isz * sizeof(float), hipMemcpyHostToDevice, ctx->stream);
     int rc = PINK_HIP_OK;
-    if (e == hipSuccess) rc = distance_group(ctx, d_img, 1);
+    if (e == hipSuccess && ctx->sym_train) rc = run_pack_som(ctx);        // (its training does not keep this operand)
+    if (e == hipSuccess && rc == PINK_HIP_OK) rc = distance_group(ctx, d_img, 1);
     if (e == hipSuccess && rc == PINK_HIP_OK) rc = run_finalize(ctx, 1, ctx->d_dist, ctx->d_ssd, ctx->d_best, false);
     const size_t n = ctx->N;
     if (e == hipSuccess && rc == PINK_HIP_OK && host_dist_out)

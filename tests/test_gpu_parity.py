@@ -541,6 +541,57 @@ def test_small_uint8_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, ed, sha
         assert np.array_equal(bits(d1), bits(d2)) and np.array_equal(ssd1, ssd2) and np.array_equal(best1, best2)
 
 
+RESIDENT_SYMMETRIC_SHAPES = [
+    (3, 1, 9, 9, 1, False, 7, capi.QUADRATIC, capi.UINT8, 5),          # one variant
+    (1, 1, 16, 16, 4, True, 12, capi.QUADRATIC, capi.UINT16, 5),       # one neuron, one base rotation: k cut seven ways
+    (7, 1, 16, 16, 4, True, 11, capi.CIRCULAR, capi.UINT16, 6),        # symmetries that cover different elements
+    (9, 1, 20, 14, 68, True, 9, capi.QUADRATIC, capi.UINT16, 5),       # 17 base rotations: two tiles, k cut three ways
+    (6, 2, 18, 12, 132, True, 8, capi.QUADRATIC, capi.UINT8, 4),       # 33: three tiles; two channels
+    (5, 1, 24, 33, 200, False, 31, capi.CIRCULAR, capi.UINT8, 4),      # 50: four tiles
+    (4, 1, 14, 10, 456, True, 7, capi.QUADRATIC, capi.UINT16, 3),      # 114: eight tiles for seven waves
+    (3, 1, 60, 64, 40, True, 60, capi.QUADRATIC, capi.UINT8, 3),       # ten elements per thread
+    (2, 1, 100, 100, 24, True, 97, capi.QUADRATIC, capi.UINT16, 2),    # 24
+    (257, 1, 12, 8, 20, True, 6, capi.QUADRATIC, capi.UINT8, 4),       # two neurons per block, the last block with one
+    (260, 1, 40, 36, 12, True, 36, capi.QUADRATIC, capi.UINT16, 3),
+    (520, 1, 12, 10, 20, True, 8, capi.CIRCULAR, capi.UINT16, 3),      # four neurons per block
+    (601, 1, 30, 28, 8, True, 28, capi.QUADRATIC, capi.UINT8, 3),
+    (2, 1, 208, 40, 60, True, 20, capi.QUADRATIC, capi.UINT8, 2),      # an image larger than the LDS
+]
+
+
+@pytest.mark.parametrize("form", ["resident", "gives up", "tags wrap"])
+@pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,shape_,ed_type,n", RESIDENT_SYMMETRIC_SHAPES)
+def test_resident_symmetric_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, form):
+    """Integer trainers keep their neurons' eight symmetric operand rows on the device over a launch group (see
+    test_small_uint8_trainer_forms for the exchange between the blocks and what happens when one gives up)."""
+    say("resident symmetric trainer", form, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n)
+    if form == "gives up":
+        monkeypatch.setenv("PINK_HIP_RESIDENT_SPIN_LIMIT", "0")
+    if form == "tags wrap":
+        monkeypatch.setenv("PINK_HIP_RESIDENT_FIRST_TAG", str(0xfffe - n + 2))      # 16-bit tags: 0xfffe is the last
+    rng = np.random.default_rng(N * 5 + I + nrot)
+    som0 = rng.random((N, C_ * D * D), dtype=np.float32)
+    imgs = rng.random((n, C_, I, I), dtype=np.float32)
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 1.0, 0.5)
+    F[F < 0.01] = 0.0
+    s = O.shape(N, C_, I, D, nrot, flip, ed, shape_, ed_type)
+    want = som0.copy()
+    obmu = O.train(s, want, imgs, F)
+    for max_batch in (0, 2):
+        with capi.Context(N, C_, I, D, nrot, flip, ed, shape_, ed_type, F, max_batch=max_batch) as ctx:
+            ctx.set_som(som0)
+            bmu = np.concatenate([ctx.train(imgs[:1]), ctx.train(imgs[1:])])
+            som = ctx.get_som()
+            counts = ctx.update_counts()
+            d1, ssd1, best1 = ctx.distance(imgs[0])
+            ctx.set_som(som)
+            d2, ssd2, best2 = ctx.distance(imgs[0])
+        assert np.array_equal(bmu, obmu), max_batch
+        assert np.array_equal(bits(som), bits(want)), max_batch
+        assert np.array_equal(counts, np.bincount(obmu, minlength=N)), max_batch
+        assert np.array_equal(bits(d1), bits(d2)) and np.array_equal(ssd1, ssd2) and np.array_equal(best1, best2)
+
+
 @pytest.mark.parametrize("N,ed_type", [(9, capi.FLOAT), (9, capi.UINT8), (530, capi.UINT8)])
 def test_train_with_any_factor_matrix(N, ed_type):
     # the C interface takes any N x N matrix, not only the symmetric ones that a distance functor gives
