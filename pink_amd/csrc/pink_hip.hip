@@ -2097,7 +2097,7 @@ class HostCopyPool {
 public:
     explicit HostCopyPool(unsigned workers)
     {
-        for (unsigned i = 0; i < workers; ++i) threads_.emplace_back([this, i] { loop(i); });
+        for (unsigned i = 0; i < workers; ++i) threads_.emplace_back([this] { loop(); });
     }
     ~HostCopyPool()
     {
@@ -2111,27 +2111,37 @@ public:
     }
     void copy(char *dst, const char *src, size_t bytes)
     {
-        const size_t parts = threads_.size() + 1;
+        start(dst, src, bytes);
+        finish();
+    }
+    // The two halves of copy(): the caller may do something else while the workers begin.  finish() has to follow.
+    void start(char *dst, const char *src, size_t bytes)
+    {
         dst_ = dst; src_ = src; bytes_ = bytes;
-        each_ = ((bytes + parts - 1) / parts + 4095) & ~(size_t)4095;
+        next_.store(0, std::memory_order_relaxed);
         pending_.store((unsigned)threads_.size(), std::memory_order_relaxed);
         {
             std::lock_guard<std::mutex> lock(m_);
             generation_.fetch_add(1, std::memory_order_release);
         }
         start_.notify_all();
-        part((unsigned)threads_.size());
+    }
+    void finish()
+    {
+        take_parts();
         for (unsigned spins = 0; pending_.load(std::memory_order_acquire) != 0; ++spins)
             if (spins > 4096) std::this_thread::yield();
     }
 
 private:
-    void part(unsigned i) const
+    // (whoever is free takes the next part)
+    void take_parts()
     {
-        const size_t off = (size_t)i * each_;
-        if (off < bytes_) memcpy(dst_ + off, src_ + off, std::min(each_, bytes_ - off));
+        constexpr size_t kPart = 128 << 10;
+        for (size_t off; (off = next_.fetch_add(kPart, std::memory_order_relaxed)) < bytes_;)
+            memcpy(dst_ + off, src_ + off, std::min(kPart, bytes_ - off));
     }
-    void loop(unsigned i)
+    void loop()
     {
         unsigned long long seen = 0;
         for (;;) {
@@ -2143,7 +2153,7 @@ private:
             }
             seen = generation_.load(std::memory_order_acquire);
             if (stop_) return;
-            part(i);
+            take_parts();
             pending_.fetch_sub(1, std::memory_order_release);
         }
     }
@@ -2155,7 +2165,8 @@ private:
     bool stop_ = false;
     char *dst_ = nullptr;
     const char *src_ = nullptr;
-    size_t bytes_ = 0, each_ = 0;
+    size_t bytes_ = 0;
+    std::atomic<size_t> next_{0};
 };
 
 // The pinned pieces and the copy threads that large pageable transfers go through: one set for the process, made when
@@ -2163,7 +2174,7 @@ private:
 // second thread that wants it meanwhile takes the runtime's own pageable copy.
 // (2 MB pieces: the link's 55 GB/s needs about half a MB; a piece is also what nothing overlaps at either end.)
 constexpr size_t kPieceBytes = (size_t)2 << 20;
-constexpr uint32_t kPieces = 8;
+constexpr uint32_t kPieces = 16;
 constexpr unsigned kCopyWorkers = 5;                      // and the caller (measured: 6 threads move 115 GB/s, 14 into fresh pages)
 struct HostStaging {
     HostCopyPool pool{kCopyWorkers};
@@ -4189,20 +4200,32 @@ int staged_run(pink_hip_ctx *ctx, const float *host_images, uint32_t n, Run run)
     std::unique_lock<std::mutex> lock;
     HostStaging *st = ctx->trainer ? nullptr : take_staging(lock);
     if (st) TRY(ensure_piece_events(ctx));
+    // (between two copies the link rests for some microseconds: large transfers go in larger pieces)
+    const size_t all = (size_t)n * img_bytes;
+    const uint32_t slots = all >= ((size_t)128 << 20) ? kPieces / 4 : all >= ((size_t)32 << 20) ? kPieces / 2 : kPieces;
+    const size_t most = kPieces / slots * kPieceBytes;
     uint32_t turn = 0, count = 0, slot = 0;
     for (uint32_t first = 0; first < n; first += count, turn ^= 1, piece = std::min(largest, 2 * piece)) {
         count = std::min(piece, n - first);
         float *dev = ctx->st_img + (size_t)first * ctx->isz;
         if (st) {
+            // a pinned piece's copy to the device is queued (some ten microseconds of this thread's time) while the workers
+            // fill the next one
             const char *src = (const char *)(host_images + (size_t)first * ctx->isz);
             const size_t bytes = (size_t)count * img_bytes;
-            for (size_t off = 0; off < bytes; off += kPieceBytes, slot = (slot + 1) % kPieces) {
-                const size_t len = std::min(kPieceBytes, bytes - off);
+            const auto send = [&](uint32_t from, size_t off) {
+                const hipError_t e = hipMemcpyAsync((char *)dev + off, st->base + from * most, std::min(most, bytes - off), hipMemcpyHostToDevice, ctx->copy_stream);
+                return e != hipSuccess ? e : hipEventRecord(ctx->piece_ev[from], ctx->copy_stream);
+            };
+            hipError_t sent = hipSuccess;
+            for (size_t off = 0; off < bytes && sent == hipSuccess; off += most, slot = (slot + 1) % slots) {
                 HIP_TRY(ctx, hipEventSynchronize(ctx->piece_ev[slot]));               // its last copy to the device has run
-                st->pool.copy(st->piece[slot], src + off, len);
-                HIP_TRY(ctx, hipMemcpyAsync((char *)dev + off, st->piece[slot], len, hipMemcpyHostToDevice, ctx->copy_stream));
-                HIP_TRY(ctx, hipEventRecord(ctx->piece_ev[slot], ctx->copy_stream));
+                st->pool.start(st->base + slot * most, src + off, std::min(most, bytes - off));
+                if (off) sent = send((slot + slots - 1) % slots, off - most);
+                st->pool.finish();
             }
+            if (sent == hipSuccess) sent = send((slot + slots - 1) % slots, (bytes - 1) / most * most);
+            HIP_TRY(ctx, sent);
         } else
             HIP_TRY(ctx, hipMemcpyAsync(dev, host_images + (size_t)first * ctx->isz, count * img_bytes, hipMemcpyHostToDevice,
                                         ctx->copy_stream));
