@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <chrono>
 #include <cmath>
@@ -2048,6 +2049,7 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
 }
 
 #include "sym_train.inc"
+#include "orbit_gemm.inc"
 
 // m_update_info[bmu]++ for the images of a group (Trainer.h:302-303), behind a resident launch: nothing when that launch
 // or one before it gave up.  The error word goes to the host with it, which looks when it next waits for the stream.
@@ -2338,6 +2340,25 @@ struct pink_hip_ctx {
     uint32_t *d_grow = nullptr, *d_gvariant = nullptr;   // variant index -> row of the variant operand, and back
     long long *d_gna = nullptr, *d_gnb = nullptr;
 
+    // mappers whose symmetries sit on the SOM side, rows of many images in one product (orbit_gemm.inc)
+    bool orbit = false;
+    int orb_mode = 0;
+    uint32_t orb_KS = 0, orb_all = 0, orb_ns = 8, orb_valid = 0;
+    size_t orb_prep_lds = 0;
+    uint32_t orb_rl = 0, orb_bands = 0, orb_stride = 0, orb_batch = 0;
+    char *d_orb_tables = nullptr;          // ... the tables below that init_orbit makes on the host
+    uint32_t *d_orb_elem = nullptr, *d_orb_sel = nullptr, *d_orb_index = nullptr;
+    float2 *d_orb_frac = nullptr;
+    uint32_t *d_orb_slots = nullptr;
+    uint2 *d_orb_bands = nullptr;
+    uint4 *d_orb_where = nullptr;
+    float *d_orb_x = nullptr, *d_orb_values = nullptr;
+    int *d_orb_part = nullptr;
+    size_t orb_part_bytes = 0;
+    v4i *d_orb_mask = nullptr, *d_orb_som = nullptr, *d_orb_rows = nullptr;
+    long long *d_orb_na = nullptr, *d_orb_nb = nullptr;
+    float *d_orb_sa = nullptr, *d_orb_ea = nullptr, *d_orb_sb = nullptr, *d_orb_eb = nullptr, *d_orb_dump = nullptr;
+
     unsigned char *static_scratch = nullptr;   // this device's copy of the file-scope scratch array
 
     // float32 distances recast as a GEMM on the matrix cores (kernel_choice PINK_HIP_KERNEL_MFMA_F32 only)
@@ -2479,9 +2500,14 @@ int run_pack_frag_som(pink_hip_ctx *ctx)
     return launch_check(ctx, "k_pack_frag_f32");
 }
 
+int run_orbit_som(pink_hip_ctx *ctx);
+
 int run_pack_som(pink_hip_ctx *ctx)
 {
     Timed t(ctx, kClsPack);
+    if (ctx->orbit) {
+        return run_orbit_som(ctx);
+    }
     if (ctx->gemm) {
         if (ctx->cfg.ed_type == PINK_HIP_UINT16)
             hipLaunchKernelGGL(k_pack_planes<true>, dim3(ctx->N, 1), dim3(1024), 2 * ctx->gKS * 32, ctx->stream, ctx->d_som, ctx->d_region,
@@ -3081,7 +3107,9 @@ int free_all(pink_hip_ctx *ctx)
     void *bufs[] = {ctx->d_som, ctx->d_rot, ctx->d_cos, ctx->d_sin, ctx->d_factors, ctx->d_factors_t, ctx->d_region, ctx->d_key,
                     ctx->d_somP, ctx->d_somP_alt, ctx->d_bmu_group, ctx->d_rotT, ctx->d_bmu_scratch, ctx->d_dist, ctx->d_ssd, ctx->d_best,
                     ctx->d_Pa, ctx->d_Pb, ctx->d_na, ctx->d_nb, ctx->d_poff, ctx->d_need, ctx->d_inv,
-                    ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4};
+                    ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4,
+                    ctx->d_orb_tables, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
+                    ctx->d_orb_sa, ctx->d_orb_ea, ctx->d_orb_sb, ctx->d_orb_eb, ctx->d_orb_dump};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu}) if (p) (void)hipFree(p);
     if (ctx->st_pin) (void)hipHostFree(ctx->st_pin);
@@ -3157,6 +3185,28 @@ inline uint32_t symmetric_position(uint32_t off, uint32_t D, uint32_t sym)
     default: return ch * DD + y * D + (D - 1 - xs);
     }
 }
+
+// Tables that go to the device in one piece: add() says where each will be, commit() takes the memory and fills it in.
+struct Tables {
+    std::vector<char> bytes;
+    std::vector<std::pair<void **, size_t>> wanted;
+    template <typename T>
+    void add(T **dev, const void *host, size_t size)
+    {
+        bytes.resize((bytes.size() + 255) & ~(size_t)255);
+        wanted.push_back({(void **)dev, bytes.size()});
+        bytes.insert(bytes.end(), (const char *)host, (const char *)host + size);
+    }
+    template <typename T>
+    void add(T **dev, const std::vector<T> &host) { add(dev, host.data(), host.size() * sizeof(T)); }
+    int commit(pink_hip_ctx *ctx, char **base)
+    {
+        TRY(dev_alloc(ctx, base, bytes.size()));
+        HIP_TRY(ctx, hipMemcpy(*base, bytes.data(), bytes.size(), hipMemcpyHostToDevice));
+        for (const auto &w : wanted) *w.first = *base + w.second;
+        return PINK_HIP_OK;
+    }
+};
 
 template <typename T>
 int upload(pink_hip_ctx *ctx, T **dev, const std::vector<T> &host)
@@ -3239,7 +3289,9 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         }
     std::vector<uint4> elem(cells.size()), at(cells.size());
     std::vector<unsigned char> mask((size_t)8 * Kp, 0);
-    std::vector<std::vector<uint32_t>> seen(8);             // the pixels of P_s: the same for every s, or not
+    std::vector<char> inside(ctx->S, 0);
+    for (uint32_t off : region) inside[off] = 1;
+    ctx->sym_all = 1;                                       // the pixels of P_s are the same for every s, or not
     for (uint32_t i = 0; i < cells.size(); ++i) {
         elem[i] = elem_of[cells[i]];
         uint32_t a16[8];
@@ -3250,20 +3302,13 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
                 if ((&elem[i].x)[b] != ~0u) {
                     const uint32_t k = to * 4 + sym_cell_byte((int)sym, (int)b);
                     mask[(size_t)sym * Kp + k] = 0xff;
-                    seen[sym].push_back(upos[k]);
+                    if (!inside[(upos[k] >> 24) * DD + ((upos[k] >> 12) & 0xfffu) * D + (upos[k] & 0xfffu)]) ctx->sym_all = 0;
                 }
         }
         at[i] = make_uint4(a16[0] | (a16[1] << 16), a16[2] | (a16[3] << 16), a16[4] | (a16[5] << 16), a16[6] | (a16[7] << 16));
     }
-    ctx->sym_all = 1;
-    for (uint32_t sym = 0; sym < 8; ++sym) {
-        std::sort(seen[sym].begin(), seen[sym].end());
-        if (valid(sym) && seen[sym] != seen[0]) ctx->sym_all = 0;
-    }
     std::vector<uint32_t> outside;
     {
-        std::vector<char> inside(ctx->S, 0);
-        for (uint32_t off : region) inside[off] = 1;
         for (uint32_t j = 0; j < ctx->S; ++j) if (!inside[j]) outside.push_back(j);
         auto key = [&](uint32_t off) {
             const uint64_t ch = off / DD, x = (off % DD) / D, y = off % D;
@@ -3293,6 +3338,256 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     HIP_TRY(ctx, hipFuncSetAttribute(sym_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
     if (ctx->sym_prep_lds) HIP_TRY(ctx, hipFuncSetAttribute(sym_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
     return PINK_HIP_OK;
+}
+
+const void *orbit_prepare_kernel(const pink_hip_ctx *ctx)
+{
+    const bool tile = ctx->orb_prep_lds != 0;
+    switch (ctx->orb_mode) {
+    case ORB_U8: return tile ? (const void *)k_orbit_prepare<ORB_U8, true> : (const void *)k_orbit_prepare<ORB_U8, false>;
+    case ORB_U16: return tile ? (const void *)k_orbit_prepare<ORB_U16, true> : (const void *)k_orbit_prepare<ORB_U16, false>;
+    default: return tile ? (const void *)k_orbit_prepare<ORB_F32, true> : (const void *)k_orbit_prepare<ORB_F32, false>;
+    }
+}
+
+// The tables of the orbit order (see orbit_gemm.inc) and the SOM's operand.  (region: distinct elements, in the CPU's order.)
+int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
+{
+    const pink_hip_config &c = ctx->cfg;
+    const uint32_t D = ctx->D, DD = D * D, odd = D & 1, mid = D / 2, Ds = D + odd;
+    auto place = [&](uint32_t x) { return x + (odd && x > mid ? 1u : 0u); };
+    auto pixel = [&](uint32_t X) { return X - (odd && X > mid ? 1u : 0u); };
+    auto moved = [&](uint32_t at, uint32_t sym) {           // place ch * Ds * Ds + X * Ds + Y under a symmetry
+        int x, y;
+        orbit_apply((int)sym, (int)((at % (Ds * Ds)) / Ds), (int)(at % Ds), (int)Ds - 1, x, y);
+        return at / (Ds * Ds) * (Ds * Ds) + (uint32_t)x * Ds + (uint32_t)y;
+    };
+    ctx->orb_mode = c.ed_type == PINK_HIP_UINT8 ? ORB_U8 : c.ed_type == PINK_HIP_UINT16 ? ORB_U16 : ORB_F32;
+    ctx->orb_ns = c.use_flip ? 8 : 4;
+    ctx->orb_valid = (c.num_rot == 1 ? 0x11u : 0xffu) & (c.use_flip ? 0xffu : 0x0fu);
+    // the orbits of the region's places, in the order of their first places, 8 x 8 places at a time (neighbouring pieces of a
+    // row then read neighbouring pixels)
+    std::vector<uint32_t> orbit_of((size_t)ctx->C * Ds * Ds, ~0u), reps;
+    for (uint32_t off : region) {
+        const uint32_t at = off / DD * Ds * Ds + place((off % DD) / D) * Ds + place(off % D);
+        uint32_t first = at;
+        for (uint32_t sym = 1; sym < 8; ++sym) first = std::min(first, moved(at, sym));
+        if (orbit_of[first] == ~0u) { orbit_of[first] = 0; reps.push_back(first); }
+    }
+    uint32_t corner = Ds;                                   // (of the region: k_screen_exact's patches then are runs of orbits)
+    for (uint32_t off : region) corner = std::min({corner, place((off % DD) / D), place(off % D)});
+    auto key = [&](uint32_t at) {
+        const uint64_t ch = at / (Ds * Ds), x = (at % (Ds * Ds)) / Ds + 8 - corner % 8, y = at % Ds + 8 - corner % 8;
+        return (ch << 48) | ((x / 8) << 32) | ((y / 8) << 16) | ((x % 8) << 8) | (y % 8);
+    };
+    std::sort(reps.begin(), reps.end(), [&](uint32_t l, uint32_t r) { return key(l) < key(r); });
+    for (uint32_t o = 0; o < reps.size(); ++o)
+        for (uint32_t sym = 0; sym < 8; ++sym) orbit_of[moved(reps[o], sym)] = o;
+    ctx->orb_KS = round_up(((uint32_t)reps.size() * 8 + 31) / 32, ctx->orb_mode == ORB_U8 ? 4u : 2u);       // (k_orbit_gemm's KC)
+    const uint32_t Kp = ctx->orb_KS * 32;
+    if (ctx->orb_mode == ORB_F32 && Kp > 65536) return PINK_HIP_OK;      // (positions in a row are 16 bits there)
+    std::vector<uint32_t> upos(Kp, ~0u), elem(Kp, ~0u), sel(16);
+    std::vector<std::array<uint32_t, 8>> where(region.size());           // [element][symmetry]: slot-major position in a row
+    for (uint32_t o = 0; o < reps.size(); ++o)
+        for (uint32_t p = 0; p < 8; ++p) {
+            const uint32_t at = moved(reps[o], p);
+            upos[o * 8 + p] = (at / (Ds * Ds) << 24) | (pixel((at % (Ds * Ds)) / Ds) << 12) | pixel(at % Ds);
+        }
+    uint32_t moves[8][8];                                   // where a slot goes under a symmetry
+    for (uint32_t sym = 0; sym < 8; ++sym)
+        for (uint32_t to = 0; to < 8; ++to) moves[sym][orbit_source((int)sym, (int)to)] = to;
+    std::vector<char> in_region(ctx->S, 0);
+    for (uint32_t off : region) in_region[off] = 1;
+    ctx->orb_all = 1;
+    std::vector<unsigned char> mask((size_t)8 * Kp, 0);
+    for (uint32_t e = 0; e < region.size(); ++e) {
+        const uint32_t off = region[e], at = off / DD * Ds * Ds + place((off % DD) / D) * Ds + place(off % D), o = orbit_of[at];
+        uint32_t p = 0;
+        while (moved(reps[o], p) != at) ++p;
+        elem[o * 8 + p] = off;
+        for (uint32_t sym = 0; sym < 8; ++sym)
+            if ((ctx->orb_valid >> sym) & 1) {
+                const uint32_t k = o * 8 + moves[sym][p], pos = upos[k];
+                mask[(size_t)sym * Kp + k] = 0xff;
+                where[e][sym] = moves[sym][p] * (Kp / 8) + o;
+                if (!in_region[(pos >> 24) * DD + ((pos >> 12) & 0xfffu) * D + (pos & 0xfffu)]) ctx->orb_all = 0;
+            }
+    }
+    for (uint32_t s = 0; s < 8; ++s) { sel[2 * s] = orbit_selector((int)s, 0); sel[2 * s + 1] = orbit_selector((int)s, 1); }
+    Tables tables;
+    uint32_t *d_upos = nullptr;
+    tables.add(&ctx->d_orb_elem, elem);
+    tables.add(&d_upos, upos);
+    tables.add(&ctx->d_orb_sel, sel);
+    tables.add(&ctx->d_orb_mask, mask.data(), mask.size());
+    const uint32_t planes = ctx->orb_mode == ORB_U8 ? 1 : 2;
+    TRY(dev_alloc(ctx, &ctx->d_orb_som, (size_t)planes * ctx->N * Kp / 16));
+    TRY(dev_alloc(ctx, &ctx->d_orb_na, ctx->N));
+    TRY(dev_alloc(ctx, &ctx->d_orb_sa, ctx->N));
+    TRY(dev_alloc(ctx, &ctx->d_orb_ea, ctx->N));
+    if (ctx->orb_mode == ORB_F32) TRY(dev_alloc(ctx, &ctx->d_orb_values, (size_t)ctx->N * Kp));
+    const size_t image_lds = (size_t)ctx->C * orbit_tile(ctx->I) * sizeof(float);
+    ctx->orb_prep_lds = image_lds <= 120 * 1024 ? image_lds : 0;
+    if (ctx->orb_prep_lds)
+        HIP_TRY(ctx, hipFuncSetAttribute(orbit_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024));
+    // as many base rotations per wave as there are, up to 16; two where the image comes out of memory: a wave's pixels are
+    // neighbours then, and a call with one image has blocks for a part of the chip
+    ctx->orb_rl = 0;
+    while ((1u << ctx->orb_rl) < ctx->nrr_eff && ctx->orb_rl < (ctx->orb_prep_lds ? 4u : 1u)) ++ctx->orb_rl;
+    if (ctx->orb_mode == ORB_F32) {
+        // bands of eight region rows (of a channel), their elements in 8 x 8 patches
+        std::vector<uint32_t> slots;
+        std::vector<uint2> bands;
+        std::vector<std::array<uint32_t, 8>> slot_where;
+        uint32_t first = 0, longest = 0;
+        while (first < region.size()) {
+            const uint32_t row0 = region[first] / D;        // (rows of all channels counted through)
+            uint32_t end = first, lo = ~0u, hi = 0;
+            while (end < region.size() && region[end] / D < row0 + 8 && region[end] / DD == region[first] / DD) {
+                lo = std::min(lo, region[end] % D); hi = std::max(hi, region[end] % D); ++end;
+            }
+            bands.push_back(make_uint2((uint32_t)slots.size() / 64, end - first));
+            longest = std::max(longest, end - first);
+            const uint32_t patches = (hi - lo) / 8 + 1;
+            slots.resize(slots.size() + (size_t)patches * 64, ~0u);
+            slot_where.resize(slots.size());
+            for (uint32_t e = first; e < end; ++e) {
+                const uint32_t y = region[e] % D - lo, x = region[e] / D - row0, at = (bands.back().x + y / 8) * 64 + x * 8 + y % 8;
+                slots[at] = e - first;
+                slot_where[at] = where[e];
+            }
+            first = end;
+        }
+        ctx->orb_bands = (uint32_t)bands.size();
+        bands.push_back(make_uint2((uint32_t)slots.size() / 64, 0u));
+        std::vector<uint4> w16(slots.size());
+        for (size_t t = 0; t < slots.size(); ++t) {
+            const auto &w = slot_where[t];
+            w16[t] = make_uint4(w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16), w[6] | (w[7] << 16));
+        }
+        ctx->orb_stride = round_up(longest, 4) + 4;
+        ctx->orb_batch = std::min<uint32_t>(kScreenBatch, std::max<uint32_t>(1, kScreenLds / 4 / ctx->orb_stride));
+        tables.add(&ctx->d_orb_slots, slots);
+        tables.add(&ctx->d_orb_bands, bands);
+        tables.add(&ctx->d_orb_where, w16);
+    }
+    TRY(tables.commit(ctx, &ctx->d_orb_tables));
+    {
+        const uint32_t blocks = (ctx->nrr_eff + (1u << ctx->orb_rl) - 1) >> ctx->orb_rl, groups = orbit_piece_groups(Kp / 16, ctx->orb_rl);
+        const size_t entries = (size_t)blocks * groups * 1024;
+        TRY(dev_alloc(ctx, &ctx->d_orb_index, entries));
+        TRY(dev_alloc(ctx, &ctx->d_orb_frac, entries));
+        OrbitTable t{};
+        t.cos_t = ctx->d_cos; t.sin_t = ctx->d_sin; t.upos = d_upos; t.index = ctx->d_orb_index; t.frac = ctx->d_orb_frac;
+        t.stride = ctx->orb_prep_lds ? orbit_stride(ctx->I) : ctx->I;
+        t.channel = ctx->orb_prep_lds ? orbit_tile(ctx->I) : ctx->I * ctx->I;
+        t.I = ctx->I; t.D = D; t.nrr = ctx->nrr_eff; t.pieces = Kp / 16; t.rl = ctx->orb_rl;
+        hipLaunchKernelGGL(k_orbit_table, dim3((groups * 1024 + 255) / 256, blocks), dim3(256), 0, ctx->stream, t);
+        TRY(launch_check(ctx, "k_orbit_table"));
+    }
+    ctx->orbit = true;
+    return PINK_HIP_OK;
+}
+
+// Bytes of a launch group of B images: the row operand (whole tiles of 32 rows), norms, and float32's squared distances.
+size_t orbit_rows_bytes(const pink_hip_ctx *ctx, size_t B)
+{
+    return (size_t)(ctx->orb_mode == ORB_U8 ? 1 : 2) * ((B * ctx->nrr_eff + 31) / 32) * ctx->orb_KS * 1024;
+}
+
+size_t orbit_image_bytes(const pink_hip_ctx *ctx)
+{
+    return orbit_rows_bytes(ctx, 1) + (size_t)ctx->N * 24 +
+           ctx->nrr_eff * (64 + (is_int(ctx) ? (size_t)0 : 4 + 4 * (size_t)ctx->N * ctx->orb_ns + (size_t)ctx->orb_KS * 128));
+}
+
+// Float32 mappers: whether screening pays (see k_screen_exact).  What summing a neuron's every variant takes grows with their
+// number, what is left to sum exactly does not: break-even lies near 100 variants (20 variants of 768 elements 10 % slower
+// with it, 8 of 1369 half as fast, 360 of 121 1.5 times as fast, 720 of 1024 3.8 times).  And what an image leaves in
+// memory has to fit the scratch of pink_hip_map_device_static.
+bool orbit_screens(const pink_hip_ctx *ctx)
+{
+    return ctx->R >= 128 && (size_t)ctx->nrr_eff * ctx->N * 8 * 4 + (size_t)ctx->nrr_eff * ctx->E * 12 <= ((size_t)24 << 20);
+}
+
+int run_orbit_som(pink_hip_ctx *ctx)
+{
+    const uint32_t Kp = ctx->orb_KS * 32;
+    auto go = [&](auto mode) {
+        hipLaunchKernelGGL(k_orbit_som<decltype(mode)::value>, dim3(ctx->N), dim3(256), 0, ctx->stream, ctx->d_som, ctx->d_orb_elem,
+                           (int *)ctx->d_orb_som, ctx->d_orb_na, ctx->d_orb_sa, ctx->d_orb_ea, ctx->d_orb_values, ctx->S, Kp, (size_t)ctx->N * Kp);
+    };
+    if (ctx->orb_mode == ORB_U8) go(std::integral_constant<int, ORB_U8>{});
+    else if (ctx->orb_mode == ORB_U16) go(std::integral_constant<int, ORB_U16>{});
+    else go(std::integral_constant<int, ORB_F32>{});
+    return launch_check(ctx, "k_orbit_som");
+}
+
+template <int MODE, int WM, int WN, int KC, int PD, int MINB>
+void launch_orbit_gemm(pink_hip_ctx *ctx, OrbitGemm a)
+{
+    a.row_tiles = (a.M + 64 * WM - 1) / (64 * WM);
+    a.col_tiles = (a.N * a.ns + 64 * WN - 1) / (64 * WN);
+    const uint32_t tiles = a.row_tiles * a.col_tiles, steps = a.KS / KC;
+    // Few tiles: as many splits of k as fill the chip twice, of at least four steps; what they leave has to fit its buffer.
+    a.splits = 1;
+    a.part_cols = a.col_tiles * 64 * WN;
+    if (WM * WN == 1 && tiles < (uint32_t)ctx->num_cu) {
+        const size_t part = (size_t)(MODE == ORB_U8 ? 4 : 12) * a.M * a.part_cols;
+        a.splits = (uint32_t)std::min<size_t>({(size_t)(2 * ctx->num_cu / tiles), (size_t)steps / 4, (size_t)16, ctx->orb_part_bytes / part});
+        a.splits = std::max(1u, a.splits);
+    }
+    a.steps_per = (steps + a.splits - 1) / a.splits;
+    a.splits = (steps + a.steps_per - 1) / a.steps_per;
+    const uint32_t per = (tiles * a.splits + 7) / 8;
+    hipLaunchKernelGGL((k_orbit_gemm<MODE, WM, WN, KC, PD, MINB>), dim3(8 * per), dim3(256), orbit_gemm_lds(MODE, WM, WN, KC, a.ns, a.nrr), ctx->stream, a);
+    if (a.splits > 1)
+        hipLaunchKernelGGL(k_orbit_finish<MODE>, dim3((a.N * a.ns + 63) / 64, (a.M + 15) / 16), dim3(256), 0, ctx->stream, a);
+}
+
+// Keys of B images: rows, product and, for float32, the exact sums of what is left.
+int run_orbit(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
+{
+    const bool u8 = ctx->orb_mode == ORB_U8, f32 = ctx->orb_mode == ORB_F32;
+    const uint32_t M = B * ctx->nrr_eff;
+    const size_t rows_plane = (size_t)((M + 31) / 32) * ctx->orb_KS * 64;
+    {
+        Timed t(ctx, kClsRotate);
+        OrbitPrep p{};
+        p.images = dev_images; p.index = ctx->d_orb_index; p.frac = ctx->d_orb_frac; p.mask = ctx->d_orb_mask;
+        p.opnd = ctx->d_orb_rows; p.norm = ctx->d_orb_nb; p.key = f32 ? nullptr : ctx->d_key; p.scale = ctx->d_orb_sb; p.err = ctx->d_orb_eb;
+        p.xrows = ctx->d_orb_x; p.plane = rows_plane; p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.KS = ctx->orb_KS;
+        p.all_sym = ctx->orb_all; p.rl = ctx->orb_rl;
+        const dim3 grid(B, (ctx->nrr_eff + (1u << p.rl) - 1) >> p.rl);
+        const uint32_t threads = ctx->orb_prep_lds > 64 * 1024 || grid.x * grid.y < (uint32_t)ctx->num_cu ? 1024 : ctx->orb_prep_lds > 24 * 1024 ? 512 : 256;
+        void *args[] = {&p};
+        HIP_TRY(ctx, hipLaunchKernel(orbit_prepare_kernel(ctx), grid, dim3(threads), args, ctx->orb_prep_lds, ctx->stream));
+    }
+    Timed t(ctx, kClsDist);
+    OrbitGemm a{};
+    a.rows = ctx->d_orb_rows; a.som = ctx->d_orb_som; a.norm_rows = ctx->d_orb_nb; a.norm_som = ctx->d_orb_na; a.selectors = ctx->d_orb_sel;
+    a.key = ctx->d_key; a.dump = ctx->d_orb_dump; a.part = ctx->d_orb_part; a.scale_rows = ctx->d_orb_sb; a.scale_som = ctx->d_orb_sa;
+    a.rows_plane = rows_plane; a.som_plane = (size_t)ctx->N * ctx->orb_KS * 2;
+    a.M = M; a.N = ctx->N; a.KS = ctx->orb_KS; a.nrr = ctx->nrr_eff; a.num_rot = ctx->cfg.num_rot; a.ns = ctx->orb_ns; a.valid = ctx->orb_valid;
+    // 64 x 128 tiles (a wave 32 x 64) read the operands less often; 64 x 64 ones fill the chip with few rows, and with two
+    // planes and short rows more of their blocks hide each other's beginnings and ends
+    const size_t columns = (size_t)a.N * a.ns, tiles = (size_t)((M + 63) / 64) * ((columns + 127) / 128);
+    const bool small = tiles < (size_t)4 * ctx->num_cu || (!u8 && a.KS < 64);
+    switch (ctx->orb_mode) {
+    case ORB_U8: if (small) launch_orbit_gemm<ORB_U8, 1, 1, 4, 4, 4>(ctx, a); else launch_orbit_gemm<ORB_U8, 1, 2, 4, 1, 4>(ctx, a); break;
+    case ORB_U16: if (small) launch_orbit_gemm<ORB_U16, 1, 1, 2, 4, 3>(ctx, a); else launch_orbit_gemm<ORB_U16, 1, 2, 2, 1, 3>(ctx, a); break;
+    default: if (small) launch_orbit_gemm<ORB_F32, 1, 1, 2, 4, 3>(ctx, a); else launch_orbit_gemm<ORB_F32, 1, 2, 2, 1, 3>(ctx, a); break;
+    }
+    TRY(launch_check(ctx, "k_orbit_gemm"));
+    if (!f32) return PINK_HIP_OK;
+    ScreenExact x{};
+    x.dump = ctx->d_orb_dump; x.values = ctx->d_orb_values; x.xrows = ctx->d_orb_x; x.err_rows = ctx->d_orb_eb; x.err_som = ctx->d_orb_ea;
+    x.slots = ctx->d_orb_slots; x.bands = ctx->d_orb_bands; x.where = ctx->d_orb_where; x.key = ctx->d_key;
+    x.N = ctx->N; x.E = ctx->E; x.K = ctx->orb_KS * 32; x.nrr = ctx->nrr_eff; x.num_rot = ctx->cfg.num_rot;
+    x.ns = ctx->orb_ns; x.valid = ctx->orb_valid; x.band_count = ctx->orb_bands;
+    x.stride = ctx->orb_stride; x.batch = ctx->orb_batch;
+    hipLaunchKernelGGL(k_screen_exact, dim3((ctx->N * x.ns + 31) / 32, B), dim3(256), (size_t)x.batch * x.stride * sizeof(float), ctx->stream, x);
+    return launch_check(ctx, "k_screen_exact");
 }
 
 int init_ctx(pink_hip_ctx *ctx)
@@ -3501,6 +3796,19 @@ int init_ctx(pink_hip_ctx *ctx)
         }
     }
 
+    // Mappers: rows of many images against the SOM, symmetries on the SOM side (orbit_gemm.inc).
+    {
+        bool distinct = true;
+        std::vector<char> seen(ctx->S, 0);
+        for (uint32_t off : region) { if (seen[off]) distinct = false; seen[off] = 1; }
+        const bool fits = !ctx->trainer && distinct && c.kernel_choice == PINK_HIP_KERNEL_AUTO && ctx->D < 4095 && ctx->C < 256;
+        if (fits && (is_int(ctx) ? !ctx->mfma_sym : orbit_screens(ctx))) {
+            TRY(init_orbit(ctx, region));
+            if (ctx->orbit) ctx->mfma = false;
+            if (ctx->orbit && is_int(ctx)) ctx->gemm = true;
+        }
+    }
+
     // Float32 distances on the matrix cores: only on request.
     if (c.kernel_choice == PINK_HIP_KERNEL_MFMA_F32) {
         if (is_int(ctx)) return fail(ctx, PINK_HIP_EINVAL, "the float32 matrix-core distance kernel needs the float distance type");
@@ -3538,7 +3846,7 @@ int init_ctx(pink_hip_ctx *ctx)
     }
     // Operand packing inside the rotation kernel: float32 rows, or byte planes of single-channel
     // integer contexts, whenever the kernel keeps its base rotation in LDS.
-    ctx->fused_pack = !ctx->mfma && !ctx->mfma_sym && ctx->C < 256 && (size_t)ctx->D * ctx->Dp < ((size_t)1 << 24) &&
+    ctx->fused_pack = !ctx->mfma && !ctx->mfma_sym && !ctx->orbit && ctx->C < 256 && (size_t)ctx->D * ctx->Dp < ((size_t)1 << 24) &&
                       (ctx->gemm ? (ctx->C == 1 || ctx->rot_nch == ctx->C) : !is_int(ctx));
     // Neither the base rotation nor the image fits LDS: interpolating every packed element out of global
     // memory is slow, so the rotation kernel stores two symmetries and packing kernels of their own read
@@ -3559,7 +3867,7 @@ int init_ctx(pink_hip_ctx *ctx)
     // Float variants of a whole launch group: for the update kernel and for a separate packing kernel.
     // The other contexts keep room for one image (pink_hip_rotate).
     ctx->pair_variants = ctx->trainer && (ctx->fused_pack || ctx->pair_pack) && ctx->S < (1u << 24);   // (the update kernel's divisions)
-    const bool group_variants = ctx->trainer || !(ctx->mfma || ctx->mfma_sym || ctx->fused_pack);
+    const bool group_variants = ctx->trainer || !(ctx->mfma || ctx->mfma_sym || ctx->orbit || ctx->fused_pack);
 
     // Launch-group size: one image for a trainer; for a mapper as many as fit ~4 GiB.
     size_t per_image = ((size_t)ctx->R * ctx->S + (size_t)ctx->Epad * ctx->Rpad) * 4 + (size_t)ctx->N * 24;
@@ -3593,10 +3901,14 @@ int init_ctx(pink_hip_ctx *ctx)
         }
         ctx->Bcap = (uint32_t)b;
     } else {
-        size_t b = c.max_batch ? c.max_batch : ((ctx->mfma || ctx->mfma_sym) ? 2048 : 256);
+        size_t b = c.max_batch ? c.max_batch : ((ctx->mfma || ctx->mfma_sym || ctx->orbit) ? 2048 : 256);
         const size_t budget = (size_t)4 << 30;
+        if (ctx->orbit) per_image = orbit_image_bytes(ctx);
         while (b > 1 && b * per_image > budget) b >>= 1;
-        if (ctx->gemm && !c.max_batch) {
+        if (ctx->orbit && !c.max_batch) {
+            // the product reads a group's rows soon after they are written: within the last-level cache
+            while (b > 16 && b * per_image > ((size_t)240 << 20)) b -= std::max<size_t>(1, b / 16);
+        } else if (ctx->gemm && !c.max_batch) {
             // the GEMM reads a group's variant operand right after the rotation kernel wrote it: a group whose
             // operand stays within the 256 MB last-level cache maps faster than a larger one (measured: the
             // optimum is the largest power of two with at most ~190 MB, 128 images at 2048 uint8 elements)
@@ -3615,6 +3927,18 @@ int init_ctx(pink_hip_ctx *ctx)
         TRY(dev_alloc(ctx, &ctx->d_Pa, (size_t)ctx->slices * ctx->sym_tiles * ctx->KSs * 1024));
         TRY(dev_alloc(ctx, &ctx->d_na, (size_t)ctx->slices * ctx->sym_tiles * 32));
         TRY(dev_alloc(ctx, &ctx->d_Pb, B * ctx->RTP * pink_sym::unit_bytes(ctx->KSs)));
+    } else if (ctx->orbit) {
+        TRY(dev_alloc(ctx, (char **)&ctx->d_orb_rows, orbit_rows_bytes(ctx, B)));
+        TRY(dev_alloc(ctx, &ctx->d_orb_nb, B * ctx->nrr_eff * 8));
+        // (a launch with fewer 64 x 64 tiles than compute units, in at most 16 splits)
+        ctx->orb_part_bytes = std::min<size_t>((size_t)16 << 20, (size_t)2 * ctx->num_cu * 64 * 64 * (ctx->orb_mode == ORB_U8 ? 4 : 12));
+        TRY(dev_alloc(ctx, (char **)&ctx->d_orb_part, ctx->orb_part_bytes));
+        if (!is_int(ctx)) {
+            TRY(dev_alloc(ctx, &ctx->d_orb_sb, B));
+            TRY(dev_alloc(ctx, &ctx->d_orb_eb, B * ctx->nrr_eff));
+            TRY(dev_alloc(ctx, &ctx->d_orb_x, B * ctx->nrr_eff * ctx->orb_KS * 32));
+            TRY(dev_alloc(ctx, &ctx->d_orb_dump, B * ctx->nrr_eff * ctx->N * ctx->orb_ns));
+        }
     } else if (ctx->gemm) {
         const size_t planes = c.ed_type == PINK_HIP_UINT16 ? 2 : 1;
         const size_t a_vec = planes * (ctx->Np / 32) * ctx->gKS * 64, b_vec = planes * (ctx->Rp / 32) * ctx->gKS * 64;
@@ -3845,6 +4169,7 @@ int run_dist_sym(pink_hip_ctx *ctx, uint32_t B)
 
 int distance_group(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
 {
+    if (ctx->orbit) return run_orbit(ctx, dev_images, B);
     if (ctx->mfma_sym) {
         TRY(run_rotpack_sym(ctx, dev_images, B));
         TRY(run_dist_sym(ctx, B));
@@ -4308,8 +4633,11 @@ int pink_hip_map_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_i
         return fail(ctx, PINK_HIP_EINVAL, "pink_hip_map_device: null argument");
     if (ctx->trainer) return fail(ctx, PINK_HIP_ESTATE, "pink_hip_map_device: context was created with update factors (a trainer)");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    for (uint32_t done = 0; done < n_images; done += ctx->Bcap) {
-        const uint32_t B = std::min(ctx->Bcap, n_images - done);
+    // (orbit_gemm.inc's groups of the same size: a small last one would not fill the chip)
+    const uint32_t groups = (n_images + ctx->Bcap - 1) / ctx->Bcap;
+    const uint32_t each = ctx->orbit && groups ? (n_images + groups - 1) / groups : ctx->Bcap;
+    for (uint32_t done = 0; done < n_images; done += each) {
+        const uint32_t B = std::min(each, n_images - done);
         TRY(distance_group(ctx, dev_images + (size_t)done * ctx->isz, B));
         TRY(run_finalize(ctx, B, dev_heatmap_out + (size_t)done * ctx->N, nullptr,
                          dev_best_rot_out ? dev_best_rot_out + (size_t)done * ctx->N : nullptr, true));
@@ -4320,8 +4648,8 @@ int pink_hip_map_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_i
 // The per-group buffers of a mapping call, per image, in the order they are carved out of the static
 // scratch (every piece starts on a 256-byte boundary).
 struct StaticPieces {
-    size_t key = 0, Pb = 0, nb = 0, gPb = 0, gnb = 0, rot = 0, rotT = 0;
-    size_t per_image() const { return key + Pb + nb + gPb + gnb + rot + rotT; }
+    size_t key = 0, Pb = 0, nb = 0, gPb = 0, gnb = 0, rot = 0, rotT = 0, orows = 0, onb = 0, osb = 0, oeb = 0, odump = 0, ox = 0;
+    size_t per_image() const { return key + Pb + nb + gPb + gnb + rot + rotT + orows + onb + osb + oeb + odump + ox; }
 };
 
 static StaticPieces static_pieces(const pink_hip_ctx *ctx)
@@ -4329,6 +4657,17 @@ static StaticPieces static_pieces(const pink_hip_ctx *ctx)
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     StaticPieces p;
     p.key = up((size_t)ctx->N * sizeof(unsigned long long));
+    if (ctx->orbit) {
+        p.orows = up(orbit_rows_bytes(ctx, 1));
+        p.onb = up((size_t)ctx->nrr_eff * 64);
+        if (!is_int(ctx)) {
+            p.osb = up(sizeof(float));
+            p.oeb = up((size_t)ctx->nrr_eff * sizeof(float));
+            p.odump = up((size_t)ctx->nrr_eff * ctx->N * ctx->orb_ns * sizeof(float));
+            p.ox = up((size_t)ctx->nrr_eff * ctx->orb_KS * 32 * sizeof(float));
+        }
+        return p;
+    }
     if (ctx->mfma_sym) {
         p.Pb = up((size_t)ctx->RTP * pink_sym::unit_bytes(ctx->KSs));
     } else if (ctx->mfma) {
@@ -4380,7 +4719,9 @@ int pink_hip_map_device_static(pink_hip_ctx *ctx, const float *dev_images, uint3
     // the kernels take the scratch where they take the context's own buffers in pink_hip_map_device
     struct Saved {
         unsigned long long *key; signed char *Pb; int *nb; v4i *gPb; long long *gnb; float *rot; void *rotT;
-    } const saved{ctx->d_key, ctx->d_Pb, ctx->d_nb, ctx->d_gPb, ctx->d_gnb, ctx->d_rot, ctx->d_rotT};
+        v4i *orows; long long *onb; float *osb, *oeb, *odump, *ox;
+    } const saved{ctx->d_key, ctx->d_Pb, ctx->d_nb, ctx->d_gPb, ctx->d_gnb, ctx->d_rot, ctx->d_rotT,
+                  ctx->d_orb_rows, ctx->d_orb_nb, ctx->d_orb_sb, ctx->d_orb_eb, ctx->d_orb_dump, ctx->d_orb_x};
     unsigned char *at = ctx->static_scratch;
     auto carve = [&](size_t bytes_per_image) { unsigned char *p = at; at += (size_t)B * bytes_per_image; return p; };
     ctx->d_key = (unsigned long long *)carve(pc.key);
@@ -4390,6 +4731,12 @@ int pink_hip_map_device_static(pink_hip_ctx *ctx, const float *dev_images, uint3
     if (pc.gnb) ctx->d_gnb = (long long *)carve(pc.gnb);
     if (pc.rot) ctx->d_rot = (float *)carve(pc.rot);
     if (pc.rotT) ctx->d_rotT = carve(pc.rotT);
+    if (pc.orows) ctx->d_orb_rows = (v4i *)carve(pc.orows);
+    if (pc.onb) ctx->d_orb_nb = (long long *)carve(pc.onb);
+    if (pc.osb) ctx->d_orb_sb = (float *)carve(pc.osb);
+    if (pc.oeb) ctx->d_orb_eb = (float *)carve(pc.oeb);
+    if (pc.odump) ctx->d_orb_dump = (float *)carve(pc.odump);
+    if (pc.ox) ctx->d_orb_x = (float *)carve(pc.ox);
     int rc = PINK_HIP_OK;
     for (uint32_t done = 0; done < n_images && rc == PINK_HIP_OK; done += B) {
         const uint32_t b = std::min(B, n_images - done);
@@ -4400,6 +4747,8 @@ int pink_hip_map_device_static(pink_hip_ctx *ctx, const float *dev_images, uint3
     }
     ctx->d_key = saved.key; ctx->d_Pb = saved.Pb; ctx->d_nb = saved.nb; ctx->d_gPb = saved.gPb; ctx->d_gnb = saved.gnb;
     ctx->d_rot = saved.rot; ctx->d_rotT = saved.rotT;
+    ctx->d_orb_rows = saved.orows; ctx->d_orb_nb = saved.onb; ctx->d_orb_sb = saved.osb; ctx->d_orb_eb = saved.oeb; ctx->d_orb_dump = saved.odump;
+    ctx->d_orb_x = saved.ox;
     return rc;
 }
 

@@ -370,6 +370,52 @@ def test_map_uint8_kernels_over_shapes(N, C_, I, D, nrot, flip, ed, shape_, n):
     assert capi.KERNEL_MFMA_GEMM in ran and capi.KERNEL_MFMA_SYM in ran
 
 
+ORBIT_MAP_SHAPES = [
+    # N, C, I, D, num_rot, flip, ed, shape, type, images, data
+    (5, 1, 12, 9, 1, True, 7, capi.QUADRATIC, capi.UINT16, 3, "noise"),       # no quarter turns; an odd neuron
+    (70, 1, 60, 54, 4, True, 48, capi.QUADRATIC, capi.UINT8, 67, "noise"),    # one row per image: 32 images in a row tile
+    (9, 1, 61, 60, 12, False, 51, capi.QUADRATIC, capi.UINT8, 5, "noise"),    # four columns per neuron, unlike symmetries
+    (33, 2, 20, 14, 132, True, 10, capi.QUADRATIC, capi.UINT16, 9, "noise"),  # 33 rows per image: tiles of two images
+    (17, 1, 40, 57, 360, False, 41, capi.CIRCULAR, capi.UINT16, 4, "noise"),
+    (3, 1, 180, 254, 8, True, 181, capi.QUADRATIC, capi.UINT8, 1, "noise"),   # an image beyond the LDS, k in splits
+    (90, 1, 16, 12, 360, True, 8, capi.QUADRATIC, capi.UINT16, 300, "noise"), # the large tiles
+    (340, 1, 70, 64, 360, True, 60, capi.CIRCULAR, capi.UINT8, 4, "noise"),
+    (9, 1, 24, 18, 128, True, 13, capi.QUADRATIC, capi.FLOAT, 5, "noise"),    # 13 rows and columns: bands and patches cut short
+    (6, 3, 20, 15, 360, False, 9, capi.QUADRATIC, capi.FLOAT, 3, "noise"),
+    (37, 1, 30, 30, 456, True, 30, capi.CIRCULAR, capi.FLOAT, 6, "noise"),    # 114 rows: more than the kept ones
+    (13, 1, 150, 106, 72, True, 75, capi.CIRCULAR, capi.FLOAT, 2, "noise"),
+    (40, 1, 20, 14, 360, True, 10, capi.QUADRATIC, capi.FLOAT, 4, "flat"),    # every variant ties
+    (40, 1, 20, 14, 360, True, 10, capi.QUADRATIC, capi.FLOAT, 4, "mask"),    # values that rounding keeps, many ties
+    (12, 1, 20, 14, 360, True, 10, capi.QUADRATIC, capi.FLOAT, 4, "wide"),    # either sign, six orders of magnitude
+    (12, 1, 20, 14, 360, True, 10, capi.QUADRATIC, capi.FLOAT, 4, "tiny"),    # squares below the smallest normal number
+]
+
+
+@pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,shape_,ed_type,n,data", ORBIT_MAP_SHAPES)
+def test_map_with_orbit_rows(N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, data):
+    """Mappers whose rows are base rotations in the order of the symmetries' orbits; float32 distances are screened on rounded
+    values first, the variants that can be a neuron's closest are then summed exactly."""
+    say("orbit mapper", N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, data)
+    rng = np.random.default_rng(N * 7 + I + nrot)
+    imgs, som = rng.random((n, C_, I, I), dtype=np.float32), rng.random((N, C_ * D * D), dtype=np.float32)
+    if data == "flat":
+        imgs[:], som[:] = 0.25, 0.5
+    elif data == "mask":
+        imgs, som = (imgs < 0.1).astype(np.float32), (som < 0.1).astype(np.float32)
+    elif data == "wide":
+        imgs, som = ((imgs - 0.5) * 10.0 ** rng.integers(-3, 4, imgs.shape)).astype(np.float32), ((som - 0.5) * 300).astype(np.float32)
+    elif data == "tiny":
+        imgs, som = imgs * np.float32(1e-33), som * np.float32(1e-21)
+    s = O.shape(N, C_, I, D, nrot, flip, ed, shape_, ed_type)
+    want_heat, want_best = O.map_images(s, som, imgs)
+    with capi.Context(N, C_, I, D, nrot, flip, ed, shape_, ed_type) as ctx:
+        ctx.set_som(som)
+        heat, best = ctx.map(imgs)
+        one_heat, one_best = ctx.map(imgs[-1:])
+    assert np.array_equal(best, want_best) and np.array_equal(bits(heat), bits(want_heat))
+    assert np.array_equal(one_best, want_best[-1:]) and np.array_equal(bits(one_heat), bits(want_heat[-1:]))
+
+
 @pytest.mark.parametrize("ed_type", [capi.FLOAT, capi.UINT8, capi.UINT16])
 def test_equal_distances_go_to_the_first_variant(ed_type):
     """A constant image has 720 identical quantised variants: every kernel must report variant 0 for every neuron
