@@ -2352,6 +2352,11 @@ struct pink_hip_ctx {
     uint32_t *d_orb_slots = nullptr;
     uint2 *d_orb_bands = nullptr;
     uint4 *d_orb_where = nullptr;
+    unsigned char *d_orb_live = nullptr;
+    // ... and the trainers that keep their weights in that order: an image's rows start a tile of 32
+    bool orbit_train = false;
+    uint32_t orb_cur = 0, orb_pitch = 0, orb_outside = 0;      // the set of norms that belongs to the operand
+    uint32_t *d_orb_outside = nullptr, *d_orb_best = nullptr;
     float *d_orb_x = nullptr, *d_orb_values = nullptr;
     int *d_orb_part = nullptr;
     size_t orb_part_bytes = 0;
@@ -3108,7 +3113,7 @@ int free_all(pink_hip_ctx *ctx)
                     ctx->d_somP, ctx->d_somP_alt, ctx->d_bmu_group, ctx->d_rotT, ctx->d_bmu_scratch, ctx->d_dist, ctx->d_ssd, ctx->d_best,
                     ctx->d_Pa, ctx->d_Pb, ctx->d_na, ctx->d_nb, ctx->d_poff, ctx->d_need, ctx->d_inv,
                     ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4,
-                    ctx->d_orb_tables, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
+                    ctx->d_orb_tables, ctx->d_orb_outside, ctx->d_orb_best, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
                     ctx->d_orb_sa, ctx->d_orb_ea, ctx->d_orb_sb, ctx->d_orb_eb, ctx->d_orb_dump};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu}) if (p) (void)hipFree(p);
@@ -3216,6 +3221,22 @@ int upload(pink_hip_ctx *ctx, T **dev, const std::vector<T> &host)
     return PINK_HIP_OK;
 }
 
+// The elements of a neuron outside the region, in 8 x 8 patches (see k_sym_outside).
+std::vector<uint32_t> outside_elements(const pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
+{
+    const uint32_t D = ctx->D, DD = D * D;
+    std::vector<char> inside(ctx->S, 0);
+    for (uint32_t off : region) inside[off] = 1;
+    std::vector<uint32_t> outside;
+    for (uint32_t ch = 0; ch < ctx->C; ++ch)
+        for (uint32_t x0 = 0; x0 < D; x0 += 8)
+            for (uint32_t y0 = 0; y0 < D; y0 += 8)
+                for (uint32_t x = x0; x < std::min(x0 + 8, D); ++x)
+                    for (uint32_t y = y0; y < std::min(y0 + 8, D); ++y)
+                        if (const uint32_t j = ch * DD + x * D + y; !inside[j]) outside.push_back(j);
+    return outside;
+}
+
 // Integer trainers whose neurons' eight symmetric operand rows fit the LDS of as many blocks as there are compute units:
 // the resident form with the symmetries on the SOM side.  (region: distinct elements, in the CPU's order.)
 int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
@@ -3307,15 +3328,7 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         }
         at[i] = make_uint4(a16[0] | (a16[1] << 16), a16[2] | (a16[3] << 16), a16[4] | (a16[5] << 16), a16[6] | (a16[7] << 16));
     }
-    std::vector<uint32_t> outside;
-    {
-        for (uint32_t j = 0; j < ctx->S; ++j) if (!inside[j]) outside.push_back(j);
-        auto key = [&](uint32_t off) {
-            const uint64_t ch = off / DD, x = (off % DD) / D, y = off % D;
-            return (ch << 48) | ((x / 8) << 32) | ((y / 8) << 16) | ((x % 8) << 8) | (y % 8);
-        };
-        std::sort(outside.begin(), outside.end(), [&](uint32_t l, uint32_t r) { return key(l) < key(r); });
-    }
+    const std::vector<uint32_t> outside = outside_elements(ctx, region);
     ctx->sym_outside = (uint32_t)outside.size();
     TRY(upload(ctx, &ctx->d_sym_upos, upos));
     TRY(upload(ctx, &ctx->d_sym_elem, elem));
@@ -3340,13 +3353,19 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     return PINK_HIP_OK;
 }
 
+template <int MODE>
+const void *orbit_prepare_for(bool tile, bool x)
+{
+    if (MODE == ORB_F32 || x) return tile ? (const void *)k_orbit_prepare<MODE, true, true> : (const void *)k_orbit_prepare<MODE, false, true>;
+    return tile ? (const void *)k_orbit_prepare<MODE, true, MODE == ORB_F32> : (const void *)k_orbit_prepare<MODE, false, MODE == ORB_F32>;
+}
 const void *orbit_prepare_kernel(const pink_hip_ctx *ctx)
 {
     const bool tile = ctx->orb_prep_lds != 0;
     switch (ctx->orb_mode) {
-    case ORB_U8: return tile ? (const void *)k_orbit_prepare<ORB_U8, true> : (const void *)k_orbit_prepare<ORB_U8, false>;
-    case ORB_U16: return tile ? (const void *)k_orbit_prepare<ORB_U16, true> : (const void *)k_orbit_prepare<ORB_U16, false>;
-    default: return tile ? (const void *)k_orbit_prepare<ORB_F32, true> : (const void *)k_orbit_prepare<ORB_F32, false>;
+    case ORB_U8: return orbit_prepare_for<ORB_U8>(tile, ctx->trainer);
+    case ORB_U16: return orbit_prepare_for<ORB_U16>(tile, ctx->trainer);
+    default: return orbit_prepare_for<ORB_F32>(tile, true);
     }
 }
 
@@ -3413,27 +3432,31 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
                 if (!in_region[(pos >> 24) * DD + ((pos >> 12) & 0xfffu) * D + (pos & 0xfffu)]) ctx->orb_all = 0;
             }
     }
-    for (uint32_t s = 0; s < 8; ++s) { sel[2 * s] = orbit_selector((int)s, 0); sel[2 * s + 1] = orbit_selector((int)s, 1); }
     Tables tables;
     uint32_t *d_upos = nullptr;
+    std::vector<unsigned char> live(Kp / 8, 0);
+    for (uint32_t k = 0; k < Kp; ++k) if (elem[k] != ~0u) live[k / 8] |= (unsigned char)(1u << (k % 8));
+    tables.add(&ctx->d_orb_live, live);
+    for (uint32_t s = 0; s < 8; ++s) { sel[2 * s] = orbit_selector((int)s, 0); sel[2 * s + 1] = orbit_selector((int)s, 1); }
     tables.add(&ctx->d_orb_elem, elem);
     tables.add(&d_upos, upos);
     tables.add(&ctx->d_orb_sel, sel);
     tables.add(&ctx->d_orb_mask, mask.data(), mask.size());
     const uint32_t planes = ctx->orb_mode == ORB_U8 ? 1 : 2;
     TRY(dev_alloc(ctx, &ctx->d_orb_som, (size_t)planes * ctx->N * Kp / 16));
-    TRY(dev_alloc(ctx, &ctx->d_orb_na, ctx->N));
-    TRY(dev_alloc(ctx, &ctx->d_orb_sa, ctx->N));
-    TRY(dev_alloc(ctx, &ctx->d_orb_ea, ctx->N));
-    if (ctx->orb_mode == ORB_F32) TRY(dev_alloc(ctx, &ctx->d_orb_values, (size_t)ctx->N * Kp));
+    TRY(dev_alloc(ctx, &ctx->d_orb_na, 3 * (size_t)ctx->N));      // (a trainer's three sets take turns)
+    TRY(dev_alloc(ctx, &ctx->d_orb_sa, 3 * (size_t)ctx->N));
+    TRY(dev_alloc(ctx, &ctx->d_orb_ea, 3 * (size_t)ctx->N));
+    if (ctx->orb_mode == ORB_F32 || ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_values, (size_t)ctx->N * Kp));
     const size_t image_lds = (size_t)ctx->C * orbit_tile(ctx->I) * sizeof(float);
     ctx->orb_prep_lds = image_lds <= 120 * 1024 ? image_lds : 0;
     if (ctx->orb_prep_lds)
         HIP_TRY(ctx, hipFuncSetAttribute(orbit_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024));
-    // as many base rotations per wave as there are, up to 16; two where the image comes out of memory: a wave's pixels are
-    // neighbours then, and a call with one image has blocks for a part of the chip
+    // as many base rotations per wave as there are, up to 16; four for a trainer's few
+    // images of long rows, two where the image comes out of memory: a wave's pixels are neighbours then, and a call with one
+    // image has blocks for a part of the chip
     ctx->orb_rl = 0;
-    while ((1u << ctx->orb_rl) < ctx->nrr_eff && ctx->orb_rl < (ctx->orb_prep_lds ? 4u : 1u)) ++ctx->orb_rl;
+    while ((1u << ctx->orb_rl) < ctx->nrr_eff && ctx->orb_rl < (!ctx->orb_prep_lds ? 1u : ctx->trainer && Kp >= 4096 ? 2u : 4u)) ++ctx->orb_rl;
     if (ctx->orb_mode == ORB_F32) {
         // bands of eight region rows (of a channel), their elements in 8 x 8 patches
         std::vector<uint32_t> slots;
@@ -3485,20 +3508,23 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         hipLaunchKernelGGL(k_orbit_table, dim3((groups * 1024 + 255) / 256, blocks), dim3(256), 0, ctx->stream, t);
         TRY(launch_check(ctx, "k_orbit_table"));
     }
+    ctx->orb_pitch = ctx->trainer ? round_up(ctx->nrr_eff, 32) : ctx->nrr_eff;
     ctx->orbit = true;
+    ctx->orbit_train = ctx->trainer;
     return PINK_HIP_OK;
 }
 
 // Bytes of a launch group of B images: the row operand (whole tiles of 32 rows), norms, and float32's squared distances.
 size_t orbit_rows_bytes(const pink_hip_ctx *ctx, size_t B)
 {
-    return (size_t)(ctx->orb_mode == ORB_U8 ? 1 : 2) * ((B * ctx->nrr_eff + 31) / 32) * ctx->orb_KS * 1024;
+    return (size_t)(ctx->orb_mode == ORB_U8 ? 1 : 2) * ((B * ctx->orb_pitch + 31) / 32) * ctx->orb_KS * 1024;
 }
 
 size_t orbit_image_bytes(const pink_hip_ctx *ctx)
 {
     return orbit_rows_bytes(ctx, 1) + (size_t)ctx->N * 24 +
-           ctx->nrr_eff * (64 + (is_int(ctx) ? (size_t)0 : 4 + 4 * (size_t)ctx->N * ctx->orb_ns + (size_t)ctx->orb_KS * 128));
+           ctx->nrr_eff * (64 + (is_int(ctx) || ctx->trainer ? (size_t)0 : 4 + 4 * (size_t)ctx->N * ctx->orb_ns) +
+                           (is_int(ctx) && !ctx->trainer ? (size_t)0 : (size_t)ctx->orb_KS * 128));
 }
 
 // Float32 mappers: whether screening pays (see k_screen_exact).  What summing a neuron's every variant takes grows with their
@@ -3510,9 +3536,29 @@ bool orbit_screens(const pink_hip_ctx *ctx)
     return ctx->R >= 128 && (size_t)ctx->nrr_eff * ctx->N * 8 * 4 + (size_t)ctx->nrr_eff * ctx->E * 12 <= ((size_t)24 << 20);
 }
 
+// Trainers that keep their weights in the order of the orbits: integers where the resident form (init_sym_train) does not fit.
+bool orbit_trains(const pink_hip_ctx *ctx)
+{
+    if (!is_int(ctx)) return false;
+    // (below a dozen base rotations the product's tiles of 64 rows are mostly empty)
+    if (!ctx->gemm || ctx->E < 1024 || ctx->nrr_eff < 12 || !resident_allowed()) return false;
+    uint32_t npb = 1;
+    while (npb <= 4 && (ctx->N + npb - 1) / npb > (uint32_t)ctx->num_cu) npb *= 2;
+    const uint32_t RT = (ctx->nrr_eff + 15) / 16, KS = round_up((ctx->E + 63) / 64, 4 * sym_shares(RT));
+    const bool resident = ctx->N <= kSymMaxNeurons && KS * 64 <= kSymMaxK && npb <= 4 && npb * (ctx->E / 4) <= kSymMaxCells * kSymLanes &&
+                          sym_lds_bytes(npb, KS, ctx->cfg.ed_type == PINK_HIP_UINT16, ctx->N, RT) + 2048 <= ctx->lds_max;
+    return !resident;
+}
+
 int run_orbit_som(pink_hip_ctx *ctx)
 {
     const uint32_t Kp = ctx->orb_KS * 32;
+    // (the next set is the one that an update adds to)
+    ctx->orb_cur = 0;
+    if (ctx->orbit_train) {
+        HIP_TRY(ctx, hipMemsetAsync(ctx->d_orb_na, 0, 3 * (size_t)ctx->N * sizeof(long long), ctx->stream));
+        HIP_TRY(ctx, hipMemsetAsync(ctx->d_orb_ea, 0, 3 * (size_t)ctx->N * sizeof(float), ctx->stream));
+    }
     auto go = [&](auto mode) {
         hipLaunchKernelGGL(k_orbit_som<decltype(mode)::value>, dim3(ctx->N), dim3(256), 0, ctx->stream, ctx->d_som, ctx->d_orb_elem,
                            (int *)ctx->d_orb_som, ctx->d_orb_na, ctx->d_orb_sa, ctx->d_orb_ea, ctx->d_orb_values, ctx->S, Kp, (size_t)ctx->N * Kp);
@@ -3542,31 +3588,40 @@ void launch_orbit_gemm(pink_hip_ctx *ctx, OrbitGemm a)
     const uint32_t per = (tiles * a.splits + 7) / 8;
     hipLaunchKernelGGL((k_orbit_gemm<MODE, WM, WN, KC, PD, MINB>), dim3(8 * per), dim3(256), orbit_gemm_lds(MODE, WM, WN, KC, a.ns, a.nrr), ctx->stream, a);
     if (a.splits > 1)
-        hipLaunchKernelGGL(k_orbit_finish<MODE>, dim3((a.N * a.ns + 63) / 64, (a.M + 15) / 16), dim3(256), 0, ctx->stream, a);
+        hipLaunchKernelGGL(k_orbit_finish<MODE>, dim3((a.N * a.ns + 63) / 64, (a.M + 3) / 4), dim3(256), 0, ctx->stream, a);
 }
 
-// Keys of B images: rows, product and, for float32, the exact sums of what is left.
-int run_orbit(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
+// v4i between the planes of a group of B images' rows.
+size_t orbit_rows_plane(const pink_hip_ctx *ctx, uint32_t B) { return (size_t)((B * ctx->orb_pitch + 31) / 32) * ctx->orb_KS * 64; }
+
+// The rows of B images, and their keys reset.
+int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
+{
+    Timed t(ctx, kClsRotate);
+    OrbitPrep p{};
+    p.images = dev_images; p.index = ctx->d_orb_index; p.frac = ctx->d_orb_frac; p.mask = ctx->d_orb_mask;
+    p.opnd = ctx->d_orb_rows; p.norm = ctx->d_orb_nb; p.key = is_int(ctx) ? ctx->d_key : nullptr; p.scale = ctx->d_orb_sb; p.err = ctx->d_orb_eb;
+    p.xrows = ctx->d_orb_x; p.plane = orbit_rows_plane(ctx, B); p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.KS = ctx->orb_KS;
+    p.all_sym = ctx->orb_all; p.rl = ctx->orb_rl; p.pitch = ctx->orb_pitch;
+    const dim3 grid(B, (ctx->nrr_eff + (1u << p.rl) - 1) >> p.rl);
+    const uint32_t threads = ctx->orb_prep_lds > 64 * 1024 || grid.x * grid.y < (uint32_t)ctx->num_cu ? 1024 : ctx->orb_prep_lds > 24 * 1024 ? 512 : 256;
+    void *args[] = {&p};
+    HIP_TRY(ctx, hipLaunchKernel(orbit_prepare_kernel(ctx), grid, dim3(threads), args, ctx->orb_prep_lds, ctx->stream));
+    return PINK_HIP_OK;
+}
+
+// Keys of `B` images from image slot `slot` of a group of `of` images whose rows are there: the product and, for float32,
+// the exact sums of what is left.
+int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
 {
     const bool u8 = ctx->orb_mode == ORB_U8, f32 = ctx->orb_mode == ORB_F32;
     const uint32_t M = B * ctx->nrr_eff;
-    const size_t rows_plane = (size_t)((M + 31) / 32) * ctx->orb_KS * 64;
-    {
-        Timed t(ctx, kClsRotate);
-        OrbitPrep p{};
-        p.images = dev_images; p.index = ctx->d_orb_index; p.frac = ctx->d_orb_frac; p.mask = ctx->d_orb_mask;
-        p.opnd = ctx->d_orb_rows; p.norm = ctx->d_orb_nb; p.key = f32 ? nullptr : ctx->d_key; p.scale = ctx->d_orb_sb; p.err = ctx->d_orb_eb;
-        p.xrows = ctx->d_orb_x; p.plane = rows_plane; p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.KS = ctx->orb_KS;
-        p.all_sym = ctx->orb_all; p.rl = ctx->orb_rl;
-        const dim3 grid(B, (ctx->nrr_eff + (1u << p.rl) - 1) >> p.rl);
-        const uint32_t threads = ctx->orb_prep_lds > 64 * 1024 || grid.x * grid.y < (uint32_t)ctx->num_cu ? 1024 : ctx->orb_prep_lds > 24 * 1024 ? 512 : 256;
-        void *args[] = {&p};
-        HIP_TRY(ctx, hipLaunchKernel(orbit_prepare_kernel(ctx), grid, dim3(threads), args, ctx->orb_prep_lds, ctx->stream));
-    }
+    const size_t rows_plane = orbit_rows_plane(ctx, of), row = (size_t)slot * ctx->nrr_eff, set = (size_t)ctx->orb_cur * ctx->N;
+    unsigned long long *key = ctx->d_key + (size_t)slot * ctx->N;
     Timed t(ctx, kClsDist);
     OrbitGemm a{};
-    a.rows = ctx->d_orb_rows; a.som = ctx->d_orb_som; a.norm_rows = ctx->d_orb_nb; a.norm_som = ctx->d_orb_na; a.selectors = ctx->d_orb_sel;
-    a.key = ctx->d_key; a.dump = ctx->d_orb_dump; a.part = ctx->d_orb_part; a.scale_rows = ctx->d_orb_sb; a.scale_som = ctx->d_orb_sa;
+    a.rows = ctx->d_orb_rows + (size_t)slot * (ctx->orb_pitch / 32) * ctx->orb_KS * 64; a.som = ctx->d_orb_som; a.norm_rows = ctx->d_orb_nb + row * 8; a.norm_som = ctx->d_orb_na + set; a.selectors = ctx->d_orb_sel;
+    a.key = key; a.dump = ctx->d_orb_dump; a.part = ctx->d_orb_part; a.scale_rows = ctx->d_orb_sb ? ctx->d_orb_sb + slot : nullptr; a.scale_som = ctx->d_orb_sa + set;
     a.rows_plane = rows_plane; a.som_plane = (size_t)ctx->N * ctx->orb_KS * 2;
     a.M = M; a.N = ctx->N; a.KS = ctx->orb_KS; a.nrr = ctx->nrr_eff; a.num_rot = ctx->cfg.num_rot; a.ns = ctx->orb_ns; a.valid = ctx->orb_valid;
     // 64 x 128 tiles (a wave 32 x 64) read the operands less often; 64 x 64 ones fill the chip with few rows, and with two
@@ -3581,13 +3636,64 @@ int run_orbit(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
     TRY(launch_check(ctx, "k_orbit_gemm"));
     if (!f32) return PINK_HIP_OK;
     ScreenExact x{};
-    x.dump = ctx->d_orb_dump; x.values = ctx->d_orb_values; x.xrows = ctx->d_orb_x; x.err_rows = ctx->d_orb_eb; x.err_som = ctx->d_orb_ea;
-    x.slots = ctx->d_orb_slots; x.bands = ctx->d_orb_bands; x.where = ctx->d_orb_where; x.key = ctx->d_key;
+    x.dump = ctx->d_orb_dump; x.values = ctx->d_orb_values; x.xrows = ctx->d_orb_x + row * ctx->orb_KS * 32; x.err_rows = ctx->d_orb_eb + row; x.err_som = ctx->d_orb_ea + set; x.scale_som = ctx->d_orb_sa + set;
+    x.slots = ctx->d_orb_slots; x.bands = ctx->d_orb_bands; x.where = ctx->d_orb_where; x.key = key;
     x.N = ctx->N; x.E = ctx->E; x.K = ctx->orb_KS * 32; x.nrr = ctx->nrr_eff; x.num_rot = ctx->cfg.num_rot;
     x.ns = ctx->orb_ns; x.valid = ctx->orb_valid; x.band_count = ctx->orb_bands;
     x.stride = ctx->orb_stride; x.batch = ctx->orb_batch;
     hipLaunchKernelGGL(k_screen_exact, dim3((ctx->N * x.ns + 31) / 32, B), dim3(256), (size_t)x.batch * x.stride * sizeof(float), ctx->stream, x);
     return launch_check(ctx, "k_screen_exact");
+}
+
+int run_orbit(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
+{
+    TRY(run_orbit_rows(ctx, dev_images, B));
+    return run_orbit_keys(ctx, 0, B, B);
+}
+
+// Training: per image the keys and the update of the region's weights, per group the other weights (k_sym_outside), at the
+// end the region's weights back into the neurons.
+int run_orbit_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
+{
+    const uint32_t Kp = ctx->orb_KS * 32, K8 = Kp / 8;
+    // about eight blocks per compute unit; a block does whole neurons where there are many
+    const uint32_t parts = std::max(1u, std::min((K8 + 255) / 256, (8 * (uint32_t)ctx->num_cu + ctx->N - 1) / ctx->N));
+    for (uint32_t done = 0; done < n_images; done += ctx->Bcap) {
+        const uint32_t B = std::min(ctx->Bcap, n_images - done);
+        const float *images = dev_images + (size_t)done * ctx->isz;
+        uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group;
+        TRY(run_orbit_rows(ctx, images, B));
+        for (uint32_t b = 0; b < B; ++b) {
+            TRY(run_orbit_keys(ctx, b, 1, B));
+            Timed t(ctx, kClsUpdate);
+            OrbitUpdate u{};
+            u.values = ctx->d_orb_values; u.xrows = ctx->d_orb_x + (size_t)b * ctx->nrr_eff * Kp; u.factors_t = ctx->d_factors_t;
+            u.scale_rows = ctx->d_orb_sb + b; u.err_rows = ctx->d_orb_eb + (size_t)b * ctx->nrr_eff; u.live = ctx->d_orb_live; u.opnd = (uint2 *)ctx->d_orb_som;
+            u.key = ctx->d_key + (size_t)b * ctx->N; u.norm = ctx->d_orb_na; u.scale = ctx->d_orb_sa; u.err = ctx->d_orb_ea;
+            u.best_variant = ctx->d_orb_best + (size_t)b * ctx->N; u.bmu_out = bmu + b; u.counts = ctx->d_counts;
+            u.plane = (size_t)ctx->N * Kp; u.N = ctx->N; u.K8 = K8; u.nrr = ctx->nrr_eff; u.num_rot = ctx->cfg.num_rot; u.shift = ctx->shift; u.cur = ctx->orb_cur;
+            const dim3 grid(parts, ctx->N);
+            switch (ctx->orb_mode) {
+            case ORB_U8: hipLaunchKernelGGL(k_orbit_update<ORB_U8>, grid, dim3(256), 0, ctx->stream, u); break;
+            case ORB_U16: hipLaunchKernelGGL(k_orbit_update<ORB_U16>, grid, dim3(256), 0, ctx->stream, u); break;
+            default: hipLaunchKernelGGL(k_orbit_update<ORB_F32>, grid, dim3(256), 0, ctx->stream, u); break;
+            }
+            TRY(launch_check(ctx, "k_orbit_update"));
+            ctx->orb_cur = (ctx->orb_cur + 1) % 3;
+        }
+        if (ctx->orb_outside) {
+            Timed t(ctx, kClsUpdate);
+            SymOutside o{};
+            o.som = ctx->d_som; o.som_next = ctx->d_som; o.images = images; o.cos_t = ctx->d_cos; o.sin_t = ctx->d_sin;
+            o.factors = ctx->d_factors; o.best_variant = ctx->d_orb_best; o.bmu = bmu; o.outside = ctx->d_orb_outside;
+            o.count = ctx->orb_outside; o.N = ctx->N; o.S = ctx->S; o.C = ctx->C; o.I = ctx->I;
+            o.D = ctx->D; o.nrr = ctx->nrr_eff; o.num_rot = ctx->cfg.num_rot; o.images_n = B;
+            hipLaunchKernelGGL(k_sym_outside, dim3((ctx->orb_outside + 255) / 256, ctx->N), dim3(256), 0, ctx->stream, o);
+            TRY(launch_check(ctx, "k_sym_outside"));
+        }
+    }
+    hipLaunchKernelGGL(k_orbit_back, dim3((Kp + 255) / 256, ctx->N), dim3(256), 0, ctx->stream, ctx->d_orb_values, ctx->d_orb_elem, ctx->d_som, ctx->S, Kp);
+    return launch_check(ctx, "k_orbit_back");
 }
 
 int init_ctx(pink_hip_ctx *ctx)
@@ -3801,11 +3907,11 @@ int init_ctx(pink_hip_ctx *ctx)
         bool distinct = true;
         std::vector<char> seen(ctx->S, 0);
         for (uint32_t off : region) { if (seen[off]) distinct = false; seen[off] = 1; }
-        const bool fits = !ctx->trainer && distinct && c.kernel_choice == PINK_HIP_KERNEL_AUTO && ctx->D < 4095 && ctx->C < 256;
-        if (fits && (is_int(ctx) ? !ctx->mfma_sym : orbit_screens(ctx))) {
+        const bool fits = distinct && c.kernel_choice == PINK_HIP_KERNEL_AUTO && ctx->D < 4095 && ctx->C < 256;
+        if (fits && (ctx->trainer ? orbit_trains(ctx) : is_int(ctx) ? !ctx->mfma_sym : orbit_screens(ctx))) {
             TRY(init_orbit(ctx, region));
             if (ctx->orbit) ctx->mfma = false;
-            if (ctx->orbit && is_int(ctx)) ctx->gemm = true;
+            if (ctx->orbit && is_int(ctx)) ctx->gemm = true;               // (the matrix cores, for pink_hip_distance_kernel)
         }
     }
 
@@ -3851,7 +3957,7 @@ int init_ctx(pink_hip_ctx *ctx)
     // Neither the base rotation nor the image fits LDS: interpolating every packed element out of global
     // memory is slow, so the rotation kernel stores two symmetries and packing kernels of their own read
     // all eight out of those, with coalesced accesses
-    ctx->pair_pack = !ctx->use_lds && !ctx->image_lds && !ctx->mfma && !ctx->mfma_sym && ctx->S < (1u << 24);
+    ctx->pair_pack = !ctx->use_lds && !ctx->image_lds && !ctx->mfma && !ctx->mfma_sym && !ctx->orbit && ctx->S < (1u << 24);
     if (ctx->pair_pack) {
         ctx->fused_pack = false;
         const uint32_t D = ctx->D, DD = D * D;
@@ -3867,7 +3973,7 @@ int init_ctx(pink_hip_ctx *ctx)
     // Float variants of a whole launch group: for the update kernel and for a separate packing kernel.
     // The other contexts keep room for one image (pink_hip_rotate).
     ctx->pair_variants = ctx->trainer && (ctx->fused_pack || ctx->pair_pack) && ctx->S < (1u << 24);   // (the update kernel's divisions)
-    const bool group_variants = ctx->trainer || !(ctx->mfma || ctx->mfma_sym || ctx->orbit || ctx->fused_pack);
+    const bool group_variants = (ctx->trainer && !ctx->orbit) || !(ctx->mfma || ctx->mfma_sym || ctx->orbit || ctx->fused_pack);
 
     // Launch-group size: one image for a trainer; for a mapper as many as fit ~4 GiB.
     size_t per_image = ((size_t)ctx->R * ctx->S + (size_t)ctx->Epad * ctx->Rpad) * 4 + (size_t)ctx->N * 24;
@@ -3898,6 +4004,10 @@ int init_ctx(pink_hip_ctx *ctx)
             // the cache than the rotation kernel loses on smaller launches (hexagonal uint16 SOM: 30.6 us per image
             // with 16 images, 230 MB; 29.1-29.3 with 11 to 13; 29.7 with 8 to 10; 30.7 with 6)
             if (ctx->gemm) while (b > 8 && b * touched > ((size_t)192 << 20)) --b;
+        }
+        if (ctx->orbit) {
+            b = c.max_batch ? std::min<size_t>(c.max_batch, kSymGroupMax) : 64;
+            while (b > 4 && b * orbit_image_bytes(ctx) > ((size_t)192 << 20)) --b;
         }
         ctx->Bcap = (uint32_t)b;
     } else {
@@ -3936,8 +4046,14 @@ int init_ctx(pink_hip_ctx *ctx)
         if (!is_int(ctx)) {
             TRY(dev_alloc(ctx, &ctx->d_orb_sb, B));
             TRY(dev_alloc(ctx, &ctx->d_orb_eb, B * ctx->nrr_eff));
-            TRY(dev_alloc(ctx, &ctx->d_orb_x, B * ctx->nrr_eff * ctx->orb_KS * 32));
-            TRY(dev_alloc(ctx, &ctx->d_orb_dump, B * ctx->nrr_eff * ctx->N * ctx->orb_ns));
+            TRY(dev_alloc(ctx, &ctx->d_orb_dump, (ctx->trainer ? 1 : B) * ctx->nrr_eff * ctx->N * ctx->orb_ns));
+        }
+        if (!is_int(ctx) || ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_x, B * ctx->nrr_eff * ctx->orb_KS * 32));
+        if (ctx->trainer) {
+            TRY(dev_alloc(ctx, &ctx->d_orb_best, B * ctx->N));
+            const std::vector<uint32_t> outside = outside_elements(ctx, region);
+            ctx->orb_outside = (uint32_t)outside.size();
+            TRY(upload(ctx, &ctx->d_orb_outside, outside));
         }
     } else if (ctx->gemm) {
         const size_t planes = c.ed_type == PINK_HIP_UINT16 ? 2 : 1;
@@ -4037,7 +4153,7 @@ int init_ctx(pink_hip_ctx *ctx)
         if (one_to_one) {
             TRY(dev_alloc(ctx, &ctx->d_inv, inv.size()));
             HIP_TRY(ctx, hipMemcpy(ctx->d_inv, inv.data(), inv.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
-            ctx->fused_som = ctx->gemm;
+            ctx->fused_som = ctx->gemm && !ctx->orbit;
         }
         if (ctx->fused_som) {
             // where an element of a neuron lands inside the neuron's row of 32-row fragments of the SOM operand
@@ -4084,7 +4200,7 @@ int init_ctx(pink_hip_ctx *ctx)
                 HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_train_small_u8_resident<4, 8, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
             }
         }
-        if (one_to_one && !ctx->small_train) TRY(init_sym_train(ctx, region));
+        if (one_to_one && !ctx->small_train && !ctx->orbit_train) TRY(init_sym_train(ctx, region));
         // one launch per image where the float32 distance kernel runs in its one-wave-per-SIMD form (see k_train_f32_dpp;
         // up to 256 neurons: measured with 512 allowed, 17 x 17 and 18 x 18 neurons at 720 variants train no faster this
         // way than with an update launch of their own -- with three to four waves per SIMD the launch saved is paid in
@@ -4094,7 +4210,7 @@ int init_ctx(pink_hip_ctx *ctx)
         ctx->rows_f32_train = !ctx->fused_f32_train && c.ed_type == PINK_HIP_FLOAT && !ctx->f32gemm && ctx->d_somP && ctx->d_inv &&
                               B <= kReplayMax;
         if (ctx->fused_f32_train) TRY(dev_alloc(ctx, (uint32_t **)&ctx->d_somP_alt, (size_t)ctx->N * ctx->Epad + kDistOverrun));
-        if (ctx->fused_f32_train || ctx->rows_f32_train || ctx->resident_train || ctx->sym_train)
+        if (ctx->fused_f32_train || ctx->rows_f32_train || ctx->resident_train || ctx->sym_train || ctx->orbit_train)
             TRY(dev_alloc(ctx, &ctx->d_bmu_group, std::max<size_t>(B, ctx->sym_B)));
         TRY(dev_alloc(ctx, &ctx->d_factors, (size_t)ctx->N * ctx->N));
         HIP_TRY(ctx, hipMemcpy(ctx->d_factors, c.update_factors, (size_t)ctx->N * ctx->N * sizeof(float),
@@ -4190,6 +4306,7 @@ int distance_group(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
 // Training of images that are on the device, queued on the context's stream.
 int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
 {
+    if (ctx->orbit_train) return run_orbit_train(ctx, dev_images, n_images, dev_bmu_out);
     if (ctx->sym_train) {
         for (uint32_t done = 0; done < n_images; done += ctx->sym_B) {
             const uint32_t B = std::min(ctx->sym_B, n_images - done);

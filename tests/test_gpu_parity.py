@@ -638,6 +638,38 @@ def test_resident_symmetric_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, 
         assert np.array_equal(bits(d1), bits(d2)) and np.array_equal(ssd1, ssd2) and np.array_equal(best1, best2)
 
 
+ORBIT_TRAIN_SHAPES = [
+    (3, 1, 70, 99, 48, True, 95, capi.QUADRATIC, capi.UINT8, 5),       # 12 base rotations; an odd neuron
+    (5, 1, 60, 100, 180, False, 91, capi.QUADRATIC, capi.UINT16, 4),   # unlike symmetries, four columns per neuron
+    (4, 2, 64, 90, 132, True, 70, capi.QUADRATIC, capi.UINT8, 3),      # two channels
+    (1030, 1, 40, 36, 48, True, 33, capi.QUADRATIC, capi.UINT16, 3),   # more neurons than the resident form takes
+    (2, 1, 190, 120, 60, True, 110, capi.CIRCULAR, capi.UINT16, 3),    # an image beyond the LDS
+]
+
+
+@pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,shape_,ed_type,n", ORBIT_TRAIN_SHAPES)
+def test_trainer_with_weights_in_orbit_order(N, C_, I, D, nrot, flip, ed, shape_, ed_type, n):
+    """Integer trainers too large for the resident form: the region's weights stay in the order of the operand over a call."""
+    say("orbit trainer", N, C_, I, D, nrot, flip, ed, shape_, ed_type, n)
+    rng = np.random.default_rng(N + I + nrot)
+    som0, imgs = rng.random((N, C_ * D * D), dtype=np.float32), rng.random((n, C_, I, I), dtype=np.float32)
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 1.0, 0.5)
+    F[F < 0.01] = 0.0
+    s = O.shape(N, C_, I, D, nrot, flip, ed, shape_, ed_type)
+    want = som0.copy()
+    obmu = O.train(s, want, imgs, F)
+    for max_batch in (0, 2):
+        with capi.Context(N, C_, I, D, nrot, flip, ed, shape_, ed_type, F, max_batch=max_batch) as ctx:
+            ctx.set_som(som0)
+            bmu = np.concatenate([ctx.train(imgs[:1]), ctx.train(imgs[1:])])
+            som, counts = ctx.get_som(), ctx.update_counts()
+            d, ssd, best = ctx.distance(imgs[0])
+        assert np.array_equal(bmu, obmu) and np.array_equal(bits(som), bits(want)), max_batch
+        assert np.array_equal(counts, np.bincount(obmu, minlength=N)), max_batch
+        heat, rot = O.map_images(s, want, imgs[:1])
+        assert np.array_equal(best, rot[0]) and np.array_equal(bits(np.sqrt(d.astype(np.float64)).astype(np.float32)), bits(heat[0])), max_batch
+
+
 @pytest.mark.parametrize("N,ed_type", [(9, capi.FLOAT), (9, capi.UINT8), (530, capi.UINT8)])
 def test_train_with_any_factor_matrix(N, ed_type):
     # the C interface takes any N x N matrix, not only the symmetric ones that a distance functor gives
