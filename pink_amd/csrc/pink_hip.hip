@@ -2355,6 +2355,9 @@ struct pink_hip_ctx {
     unsigned char *d_orb_live = nullptr;
     // ... and the trainers that keep their weights in that order: an image's rows start a tile of 32
     bool orbit_train = false;
+    // ... and the float32 trainers that screen their distances: rows_f32_train's operands, the product's beside them
+    bool screen_train = false;
+    uint4 *d_orb_element = nullptr;
     uint32_t orb_cur = 0, orb_pitch = 0, orb_outside = 0;      // the set of norms that belongs to the operand
     uint32_t *d_orb_outside = nullptr, *d_orb_best = nullptr;
     float *d_orb_x = nullptr, *d_orb_values = nullptr;
@@ -2510,6 +2513,7 @@ int run_orbit_som(pink_hip_ctx *ctx);
 int run_pack_som(pink_hip_ctx *ctx)
 {
     Timed t(ctx, kClsPack);
+    if (ctx->screen_train) TRY(run_orbit_som(ctx));
     if (ctx->orbit) {
         return run_orbit_som(ctx);
     }
@@ -3445,9 +3449,9 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     const uint32_t planes = ctx->orb_mode == ORB_U8 ? 1 : 2;
     TRY(dev_alloc(ctx, &ctx->d_orb_som, (size_t)planes * ctx->N * Kp / 16));
     TRY(dev_alloc(ctx, &ctx->d_orb_na, 3 * (size_t)ctx->N));      // (a trainer's three sets take turns)
-    TRY(dev_alloc(ctx, &ctx->d_orb_sa, 3 * (size_t)ctx->N));
-    TRY(dev_alloc(ctx, &ctx->d_orb_ea, 3 * (size_t)ctx->N));
-    if (ctx->orb_mode == ORB_F32 || ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_values, (size_t)ctx->N * Kp));
+    TRY(dev_alloc(ctx, &ctx->d_orb_sa, ctx->N));
+    TRY(dev_alloc(ctx, &ctx->d_orb_ea, ctx->N));
+    if ((ctx->orb_mode == ORB_F32) != ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_values, (size_t)ctx->N * Kp));
     const size_t image_lds = (size_t)ctx->C * orbit_tile(ctx->I) * sizeof(float);
     ctx->orb_prep_lds = image_lds <= 120 * 1024 ? image_lds : 0;
     if (ctx->orb_prep_lds)
@@ -3457,7 +3461,11 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     // image has blocks for a part of the chip
     ctx->orb_rl = 0;
     while ((1u << ctx->orb_rl) < ctx->nrr_eff && ctx->orb_rl < (!ctx->orb_prep_lds ? 1u : ctx->trainer && Kp >= 4096 ? 2u : 4u)) ++ctx->orb_rl;
-    if (ctx->orb_mode == ORB_F32) {
+    if (ctx->orb_mode == ORB_F32 && ctx->trainer) {
+        std::vector<unsigned short> element(Kp, 0xffff);
+        for (uint32_t e = 0; e < region.size(); ++e) element[(where[e][0] % (Kp / 8)) * 8 + where[e][0] / (Kp / 8)] = (unsigned short)e;
+        tables.add(&ctx->d_orb_element, element.data(), element.size() * sizeof(element[0]));
+    } else if (ctx->orb_mode == ORB_F32) {
         // bands of eight region rows (of a channel), their elements in 8 x 8 patches
         std::vector<uint32_t> slots;
         std::vector<uint2> bands;
@@ -3509,8 +3517,9 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         TRY(launch_check(ctx, "k_orbit_table"));
     }
     ctx->orb_pitch = ctx->trainer ? round_up(ctx->nrr_eff, 32) : ctx->nrr_eff;
-    ctx->orbit = true;
-    ctx->orbit_train = ctx->trainer;
+    ctx->screen_train = ctx->trainer && ctx->orb_mode == ORB_F32;
+    ctx->orbit = !ctx->screen_train;
+    ctx->orbit_train = ctx->trainer && ctx->orbit;
     return PINK_HIP_OK;
 }
 
@@ -3536,10 +3545,16 @@ bool orbit_screens(const pink_hip_ctx *ctx)
     return ctx->R >= 128 && (size_t)ctx->nrr_eff * ctx->N * 8 * 4 + (size_t)ctx->nrr_eff * ctx->E * 12 <= ((size_t)24 << 20);
 }
 
-// Trainers that keep their weights in the order of the orbits: integers where the resident form (init_sym_train) does not fit.
+// Trainers that take the orbits' product: integers where the resident form (init_sym_train) does not fit, which keep their
+// weights in that order too; float32 where every variant's sum costs more than the product, the few sums that are left and
+// two launches more.  Those sums are a chain of E steps whatever the SOM's size, so there have to be two neurons per CU, and
+// (neurons x variants x elements, ratio of the times of an image): 0.3e9 0.66, 0.7e9 0.91, 0.84e9 1.01, 1.1e9 1.05, 1.3e9 1.19,
+// 2.2e9 1.85; 400 neurons, 2.9e9: 0.97.
 bool orbit_trains(const pink_hip_ctx *ctx)
 {
-    if (!is_int(ctx)) return false;
+    if (!is_int(ctx))
+        return ctx->R >= 128 && ctx->N >= 2 * (uint32_t)ctx->num_cu && (size_t)ctx->N * ctx->R * ctx->E >= 1000000000 &&
+               ctx->E < 65535 && (size_t)ctx->Epad * sizeof(float) + 1024 <= ctx->lds_max;
     // (below a dozen base rotations the product's tiles of 64 rows are mostly empty)
     if (!ctx->gemm || ctx->E < 1024 || ctx->nrr_eff < 12 || !resident_allowed()) return false;
     uint32_t npb = 1;
@@ -3555,10 +3570,7 @@ int run_orbit_som(pink_hip_ctx *ctx)
     const uint32_t Kp = ctx->orb_KS * 32;
     // (the next set is the one that an update adds to)
     ctx->orb_cur = 0;
-    if (ctx->orbit_train) {
-        HIP_TRY(ctx, hipMemsetAsync(ctx->d_orb_na, 0, 3 * (size_t)ctx->N * sizeof(long long), ctx->stream));
-        HIP_TRY(ctx, hipMemsetAsync(ctx->d_orb_ea, 0, 3 * (size_t)ctx->N * sizeof(float), ctx->stream));
-    }
+    if (ctx->orbit_train) HIP_TRY(ctx, hipMemsetAsync(ctx->d_orb_na, 0, 3 * (size_t)ctx->N * sizeof(long long), ctx->stream));
     auto go = [&](auto mode) {
         hipLaunchKernelGGL(k_orbit_som<decltype(mode)::value>, dim3(ctx->N), dim3(256), 0, ctx->stream, ctx->d_som, ctx->d_orb_elem,
                            (int *)ctx->d_orb_som, ctx->d_orb_na, ctx->d_orb_sa, ctx->d_orb_ea, ctx->d_orb_values, ctx->S, Kp, (size_t)ctx->N * Kp);
@@ -3621,7 +3633,7 @@ int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
     Timed t(ctx, kClsDist);
     OrbitGemm a{};
     a.rows = ctx->d_orb_rows + (size_t)slot * (ctx->orb_pitch / 32) * ctx->orb_KS * 64; a.som = ctx->d_orb_som; a.norm_rows = ctx->d_orb_nb + row * 8; a.norm_som = ctx->d_orb_na + set; a.selectors = ctx->d_orb_sel;
-    a.key = key; a.dump = ctx->d_orb_dump; a.part = ctx->d_orb_part; a.scale_rows = ctx->d_orb_sb ? ctx->d_orb_sb + slot : nullptr; a.scale_som = ctx->d_orb_sa + set;
+    a.key = key; a.dump = ctx->d_orb_dump; a.part = ctx->d_orb_part; a.scale_rows = ctx->d_orb_sb ? ctx->d_orb_sb + slot : nullptr; a.scale_som = ctx->d_orb_sa;
     a.rows_plane = rows_plane; a.som_plane = (size_t)ctx->N * ctx->orb_KS * 2;
     a.M = M; a.N = ctx->N; a.KS = ctx->orb_KS; a.nrr = ctx->nrr_eff; a.num_rot = ctx->cfg.num_rot; a.ns = ctx->orb_ns; a.valid = ctx->orb_valid;
     // 64 x 128 tiles (a wave 32 x 64) read the operands less often; 64 x 64 ones fill the chip with few rows, and with two
@@ -3635,8 +3647,17 @@ int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
     }
     TRY(launch_check(ctx, "k_orbit_gemm"));
     if (!f32) return PINK_HIP_OK;
+    if (ctx->screen_train) {
+        ScreenChain x{};
+        x.dump = ctx->d_orb_dump; x.som_rows = (const float *)ctx->d_somP; x.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad;
+        x.err_rows = ctx->d_orb_eb + row; x.err_som = ctx->d_orb_ea; x.scale_som = ctx->d_orb_sa; x.key = key;
+        x.N = ctx->N; x.E = ctx->E; x.Epad = ctx->Epad; x.K = ctx->orb_KS * 32; x.nrr = ctx->nrr_eff; x.num_rot = ctx->cfg.num_rot;
+        x.ns = ctx->orb_ns; x.valid = ctx->orb_valid;
+        hipLaunchKernelGGL(k_screen_chain, dim3((ctx->N + kChainNeurons - 1) / kChainNeurons), dim3(320), 0, ctx->stream, x);
+        return launch_check(ctx, "k_screen_chain");
+    }
     ScreenExact x{};
-    x.dump = ctx->d_orb_dump; x.values = ctx->d_orb_values; x.xrows = ctx->d_orb_x + row * ctx->orb_KS * 32; x.err_rows = ctx->d_orb_eb + row; x.err_som = ctx->d_orb_ea + set; x.scale_som = ctx->d_orb_sa + set;
+    x.dump = ctx->d_orb_dump; x.values = ctx->d_orb_values; x.xrows = ctx->d_orb_x + row * ctx->orb_KS * 32; x.err_rows = ctx->d_orb_eb + row; x.err_som = ctx->d_orb_ea; x.scale_som = ctx->d_orb_sa;
     x.slots = ctx->d_orb_slots; x.bands = ctx->d_orb_bands; x.where = ctx->d_orb_where; x.key = key;
     x.N = ctx->N; x.E = ctx->E; x.K = ctx->orb_KS * 32; x.nrr = ctx->nrr_eff; x.num_rot = ctx->cfg.num_rot;
     x.ns = ctx->orb_ns; x.valid = ctx->orb_valid; x.band_count = ctx->orb_bands;
@@ -3649,6 +3670,19 @@ int run_orbit(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
 {
     TRY(run_orbit_rows(ctx, dev_images, B));
     return run_orbit_keys(ctx, 0, B, B);
+}
+
+// The update of the image in slot `slot` of a float32 trainer that screens its distances.
+int run_screen_update(pink_hip_ctx *ctx, uint32_t slot, uint32_t *dev_bmu_out)
+{
+    Timed t(ctx, kClsUpdate);
+    ScreenUpdate u{};
+    u.som_rows = (float *)ctx->d_somP; u.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad; u.factors_t = ctx->d_factors_t;
+    u.scale_rows = ctx->d_orb_sb + slot; u.err_rows = ctx->d_orb_eb + (size_t)slot * ctx->nrr_eff; u.element = ctx->d_orb_element;
+    u.opnd = (uint2 *)ctx->d_orb_som; u.key = ctx->d_key + (size_t)slot * ctx->N; u.norm = ctx->d_orb_na; u.scale = ctx->d_orb_sa; u.err = ctx->d_orb_ea;
+    u.bmu_out = dev_bmu_out; u.counts = ctx->d_counts; u.plane = (size_t)ctx->N * ctx->orb_KS * 32; u.N = ctx->N; u.K8 = ctx->orb_KS * 4; u.Epad = ctx->Epad;
+    hipLaunchKernelGGL(k_screen_update, dim3(ctx->N), dim3(512), (size_t)ctx->Epad * sizeof(float), ctx->stream, u);
+    return launch_check(ctx, "k_screen_update");
 }
 
 // Training: per image the keys and the update of the region's weights, per group the other weights (k_sym_outside), at the
@@ -3668,16 +3702,13 @@ int run_orbit_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_image
             Timed t(ctx, kClsUpdate);
             OrbitUpdate u{};
             u.values = ctx->d_orb_values; u.xrows = ctx->d_orb_x + (size_t)b * ctx->nrr_eff * Kp; u.factors_t = ctx->d_factors_t;
-            u.scale_rows = ctx->d_orb_sb + b; u.err_rows = ctx->d_orb_eb + (size_t)b * ctx->nrr_eff; u.live = ctx->d_orb_live; u.opnd = (uint2 *)ctx->d_orb_som;
-            u.key = ctx->d_key + (size_t)b * ctx->N; u.norm = ctx->d_orb_na; u.scale = ctx->d_orb_sa; u.err = ctx->d_orb_ea;
+            u.live = ctx->d_orb_live; u.opnd = (uint2 *)ctx->d_orb_som;
+            u.key = ctx->d_key + (size_t)b * ctx->N; u.norm = ctx->d_orb_na;
             u.best_variant = ctx->d_orb_best + (size_t)b * ctx->N; u.bmu_out = bmu + b; u.counts = ctx->d_counts;
             u.plane = (size_t)ctx->N * Kp; u.N = ctx->N; u.K8 = K8; u.nrr = ctx->nrr_eff; u.num_rot = ctx->cfg.num_rot; u.shift = ctx->shift; u.cur = ctx->orb_cur;
             const dim3 grid(parts, ctx->N);
-            switch (ctx->orb_mode) {
-            case ORB_U8: hipLaunchKernelGGL(k_orbit_update<ORB_U8>, grid, dim3(256), 0, ctx->stream, u); break;
-            case ORB_U16: hipLaunchKernelGGL(k_orbit_update<ORB_U16>, grid, dim3(256), 0, ctx->stream, u); break;
-            default: hipLaunchKernelGGL(k_orbit_update<ORB_F32>, grid, dim3(256), 0, ctx->stream, u); break;
-            }
+            if (ctx->orb_mode == ORB_U8) hipLaunchKernelGGL(k_orbit_update<ORB_U8>, grid, dim3(256), 0, ctx->stream, u);
+            else hipLaunchKernelGGL(k_orbit_update<ORB_U16>, grid, dim3(256), 0, ctx->stream, u);
             TRY(launch_check(ctx, "k_orbit_update"));
             ctx->orb_cur = (ctx->orb_cur + 1) % 3;
         }
@@ -4046,7 +4077,7 @@ int init_ctx(pink_hip_ctx *ctx)
         if (!is_int(ctx)) {
             TRY(dev_alloc(ctx, &ctx->d_orb_sb, B));
             TRY(dev_alloc(ctx, &ctx->d_orb_eb, B * ctx->nrr_eff));
-            TRY(dev_alloc(ctx, &ctx->d_orb_dump, (ctx->trainer ? 1 : B) * ctx->nrr_eff * ctx->N * ctx->orb_ns));
+            TRY(dev_alloc(ctx, &ctx->d_orb_dump, B * ctx->nrr_eff * ctx->N * ctx->orb_ns));
         }
         if (!is_int(ctx) || ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_x, B * ctx->nrr_eff * ctx->orb_KS * 32));
         if (ctx->trainer) {
@@ -4209,6 +4240,17 @@ int init_ctx(pink_hip_ctx *ctx)
                                (size_t)(ctx->Rpad / kWave) * ((ctx->N + 3) / 4) <= (size_t)4 * ctx->num_cu;
         ctx->rows_f32_train = !ctx->fused_f32_train && c.ed_type == PINK_HIP_FLOAT && !ctx->f32gemm && ctx->d_somP && ctx->d_inv &&
                               B <= kReplayMax;
+        ctx->screen_train = ctx->screen_train && ctx->rows_f32_train;
+        if (ctx->screen_train) {
+            TRY(dev_alloc(ctx, (char **)&ctx->d_orb_rows, orbit_rows_bytes(ctx, B)));
+            TRY(dev_alloc(ctx, &ctx->d_orb_nb, B * ctx->nrr_eff * 8));
+            TRY(dev_alloc(ctx, &ctx->d_orb_sb, B));
+            TRY(dev_alloc(ctx, &ctx->d_orb_eb, B * ctx->nrr_eff));
+            TRY(dev_alloc(ctx, &ctx->d_orb_dump, (size_t)ctx->nrr_eff * ctx->N * ctx->orb_ns));
+            ctx->orb_part_bytes = (size_t)16 << 20;
+            TRY(dev_alloc(ctx, (char **)&ctx->d_orb_part, ctx->orb_part_bytes));
+            HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_screen_update, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 1024));
+        }
         if (ctx->fused_f32_train) TRY(dev_alloc(ctx, (uint32_t **)&ctx->d_somP_alt, (size_t)ctx->N * ctx->Epad + kDistOverrun));
         if (ctx->fused_f32_train || ctx->rows_f32_train || ctx->resident_train || ctx->sym_train || ctx->orbit_train)
             TRY(dev_alloc(ctx, &ctx->d_bmu_group, std::max<size_t>(B, ctx->sym_B)));
@@ -4334,8 +4376,14 @@ int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, 
             continue;
         }
         if (ctx->rows_f32_train) {
+            if (ctx->screen_train) TRY(run_orbit_rows(ctx, dev_images + (size_t)done * ctx->isz, B));
             uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group;
             for (uint32_t b = 0; b < B; ++b) {
+                if (ctx->screen_train) {
+                    TRY(run_orbit_keys(ctx, b, 1, B));
+                    TRY(run_screen_update(ctx, b, bmu + b));
+                    continue;
+                }
                 TRY(run_dist(ctx, b, 1));
                 TRY(run_update_rows(ctx, b, bmu + b));
             }

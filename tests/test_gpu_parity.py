@@ -670,6 +670,43 @@ def test_trainer_with_weights_in_orbit_order(N, C_, I, D, nrot, flip, ed, shape_
         assert np.array_equal(best, rot[0]) and np.array_equal(bits(np.sqrt(d.astype(np.float64)).astype(np.float32)), bits(heat[0])), max_batch
 
 
+SCREENED_TRAIN_SHAPES = [
+    (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 3, "blobs"),      # a block of two neurons at the end
+    (515, 2, 70, 60, 360, False, 53, capi.QUADRATIC, 3, "blobs"),      # four columns per neuron
+    (700, 1, 80, 70, 264, True, 61, capi.CIRCULAR, 3, "noise"),        # 66 base rotations: two lists
+    (640, 1, 90, 128, 128, True, 90, capi.QUADRATIC, 3, "zeros"),      # most variants alike: every candidate summed
+    (1200, 1, 64, 50, 180, True, 50, capi.QUADRATIC, 3, "nan"),
+]
+
+
+@pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,shape_,n,kind", SCREENED_TRAIN_SHAPES)
+def test_float_trainer_with_screened_distances(N, C_, I, D, nrot, flip, ed, shape_, n, kind):
+    """Large float32 trainers sum the variants that a product of rounded values leaves: the same bits as every variant summed."""
+    say("screened float trainer", N, C_, I, D, nrot, flip, ed, shape_, n, kind)
+    rng = np.random.default_rng(N + I)
+    som0, imgs = rng.random((N, C_ * D * D), dtype=np.float32), rng.random((n, C_, I, I), dtype=np.float32)
+    if kind == "blobs":
+        x = np.linspace(-1, 1, I, dtype=np.float32)
+        imgs = imgs * 0.1 + np.exp(-8 * (x[:, None] - imgs[:, :, :1, :1]) ** 2 - 20 * x[None, :] ** 2).astype(np.float32)
+    elif kind == "zeros":
+        imgs[imgs < 0.999] = 0.0
+    elif kind == "nan":
+        imgs[1, 0, I // 2, I // 2] = np.nan
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 1.0, 0.5)
+    F[F < 0.01] = 0.0
+    got = []
+    for kernel, max_batch in ((capi.KERNEL_VALU, 0), (capi.KERNEL_AUTO, 0), (capi.KERNEL_AUTO, 2)):
+        with capi.Context(N, C_, I, D, nrot, flip, ed, shape_, capi.FLOAT, F, kernel_choice=kernel, max_batch=max_batch) as ctx:
+            ctx.set_som(som0)
+            bmu = np.concatenate([ctx.train(imgs[:1]), ctx.train(imgs[1:])])
+            som = ctx.get_som()
+            d, ssd, best = ctx.distance(imgs[0])
+            got.append((bmu, np.isnan(som) if kind == "nan" else bits(som), ctx.update_counts(), bits(d), best))
+    for other in got[1:]:
+        for g, w in zip(other, got[0]):
+            assert np.array_equal(g, w)
+
+
 @pytest.mark.parametrize("N,ed_type", [(9, capi.FLOAT), (9, capi.UINT8), (530, capi.UINT8)])
 def test_train_with_any_factor_matrix(N, ed_type):
     # the C interface takes any N x N matrix, not only the symmetric ones that a distance functor gives
