@@ -3650,14 +3650,14 @@ int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
     if (ctx->screen_train) {
         ScreenChain x{};
         x.dump = ctx->d_orb_dump; x.som_rows = (const float *)ctx->d_somP; x.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad;
-        x.err_rows = ctx->d_orb_eb + row; x.err_som = ctx->d_orb_ea; x.scale_som = ctx->d_orb_sa; x.key = key;
-        x.N = ctx->N; x.E = ctx->E; x.Epad = ctx->Epad; x.K = ctx->orb_KS * 32; x.nrr = ctx->nrr_eff; x.num_rot = ctx->cfg.num_rot;
+        x.err_rows = ctx->d_orb_eb + row; x.err_som = ctx->d_orb_ea; x.key = key;
+        x.N = ctx->N; x.E = ctx->E; x.Epad = ctx->Epad; x.nrr = ctx->nrr_eff; x.num_rot = ctx->cfg.num_rot;
         x.ns = ctx->orb_ns; x.valid = ctx->orb_valid;
         hipLaunchKernelGGL(k_screen_chain, dim3((ctx->N + kChainNeurons - 1) / kChainNeurons), dim3(320), 0, ctx->stream, x);
         return launch_check(ctx, "k_screen_chain");
     }
     ScreenExact x{};
-    x.dump = ctx->d_orb_dump; x.values = ctx->d_orb_values; x.xrows = ctx->d_orb_x + row * ctx->orb_KS * 32; x.err_rows = ctx->d_orb_eb + row; x.err_som = ctx->d_orb_ea; x.scale_som = ctx->d_orb_sa;
+    x.dump = ctx->d_orb_dump; x.values = ctx->d_orb_values; x.xrows = ctx->d_orb_x + row * ctx->orb_KS * 32; x.err_rows = ctx->d_orb_eb + row; x.err_som = ctx->d_orb_ea;
     x.slots = ctx->d_orb_slots; x.bands = ctx->d_orb_bands; x.where = ctx->d_orb_where; x.key = key;
     x.N = ctx->N; x.E = ctx->E; x.K = ctx->orb_KS * 32; x.nrr = ctx->nrr_eff; x.num_rot = ctx->cfg.num_rot;
     x.ns = ctx->orb_ns; x.valid = ctx->orb_valid; x.band_count = ctx->orb_bands;
@@ -3678,7 +3678,7 @@ int run_screen_update(pink_hip_ctx *ctx, uint32_t slot, uint32_t *dev_bmu_out)
     Timed t(ctx, kClsUpdate);
     ScreenUpdate u{};
     u.som_rows = (float *)ctx->d_somP; u.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad; u.factors_t = ctx->d_factors_t;
-    u.scale_rows = ctx->d_orb_sb + slot; u.err_rows = ctx->d_orb_eb + (size_t)slot * ctx->nrr_eff; u.element = ctx->d_orb_element;
+    u.element = ctx->d_orb_element;
     u.opnd = (uint2 *)ctx->d_orb_som; u.key = ctx->d_key + (size_t)slot * ctx->N; u.norm = ctx->d_orb_na; u.scale = ctx->d_orb_sa; u.err = ctx->d_orb_ea;
     u.bmu_out = dev_bmu_out; u.counts = ctx->d_counts; u.plane = (size_t)ctx->N * ctx->orb_KS * 32; u.N = ctx->N; u.K8 = ctx->orb_KS * 4; u.Epad = ctx->Epad;
     hipLaunchKernelGGL(k_screen_update, dim3(ctx->N), dim3(512), (size_t)ctx->Epad * sizeof(float), ctx->stream, u);

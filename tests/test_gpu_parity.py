@@ -416,6 +416,29 @@ def test_map_with_orbit_rows(N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, da
     assert np.array_equal(one_best, want_best[-1:]) and np.array_equal(bits(one_heat), bits(want_heat[-1:]))
 
 
+def _nearly_round(rng, n, C_, I, scale):
+    """Images whose rotated copies differ by a thousandth: every variant's distance is close to every other's."""
+    x = np.linspace(-1, 1, I)
+    r2 = (x[:, None] ** 2 + x[None, :] ** 2) * rng.uniform(0.5, 3.0, (n, C_, 1, 1))
+    return (scale * (np.exp(-r2) + 1e-3 * rng.random((n, C_, I, I)))).astype(np.float32)
+
+
+@pytest.mark.parametrize("scale", [1e-20, 1e-19, 3e-19, 1e-18, 3e-18, 1e-15, 1.0, 1e15])
+def test_screening_keeps_the_closest_variant_at_every_scale(scale):
+    """The error of the rounded values is bounded by its measured size, whose squares are no float32 numbers any more where
+    the values (fluxes in physical units) are below about 1e-18."""
+    say("screening at scale", scale)
+    N, I, D, nrot, ed, n = 60, 16, 12, 360, 5, 400
+    rng = np.random.default_rng(17)
+    som = (scale * rng.random((N, D * D))).astype(np.float32)
+    imgs = _nearly_round(rng, n, 1, I, scale)
+    want_heat, want_best = O.map_images(O.shape(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT), som, imgs)
+    with capi.Context(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT) as ctx:
+        ctx.set_som(som)
+        heat, best = ctx.map(imgs)
+    assert np.array_equal(best, want_best) and np.array_equal(bits(heat), bits(want_heat))
+
+
 @pytest.mark.parametrize("ed_type", [capi.FLOAT, capi.UINT8, capi.UINT16])
 def test_equal_distances_go_to_the_first_variant(ed_type):
     """A constant image has 720 identical quantised variants: every kernel must report variant 0 for every neuron
@@ -676,12 +699,13 @@ SCREENED_TRAIN_SHAPES = [
     (700, 1, 80, 70, 264, True, 61, capi.CIRCULAR, 3, "noise"),        # 66 base rotations: two lists
     (640, 1, 90, 128, 128, True, 90, capi.QUADRATIC, 3, "zeros"),      # most variants alike: every candidate summed
     (1200, 1, 64, 50, 180, True, 50, capi.QUADRATIC, 3, "nan"),
+    (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 3, "flux"),       # every variant close, squares of errors no float32
 ]
 
 
 @pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,shape_,n,kind", SCREENED_TRAIN_SHAPES)
 def test_float_trainer_with_screened_distances(N, C_, I, D, nrot, flip, ed, shape_, n, kind):
-    """Large float32 trainers sum the variants that a product of rounded values leaves: the same bits as every variant summed."""
+    """Large float32 trainers sum the variants that a product of rounded values leaves: the oracle's bits, which sums them all."""
     say("screened float trainer", N, C_, I, D, nrot, flip, ed, shape_, n, kind)
     rng = np.random.default_rng(N + I)
     som0, imgs = rng.random((N, C_ * D * D), dtype=np.float32), rng.random((n, C_, I, I), dtype=np.float32)
@@ -692,19 +716,35 @@ def test_float_trainer_with_screened_distances(N, C_, I, D, nrot, flip, ed, shap
         imgs[imgs < 0.999] = 0.0
     elif kind == "nan":
         imgs[1, 0, I // 2, I // 2] = np.nan
+    elif kind == "flux":
+        imgs, som0 = _nearly_round(rng, n, C_, I, 5e-19), som0 * np.float32(5e-19)
     F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 1.0, 0.5)
     F[F < 0.01] = 0.0
-    got = []
-    for kernel, max_batch in ((capi.KERNEL_VALU, 0), (capi.KERNEL_AUTO, 0), (capi.KERNEL_AUTO, 2)):
-        with capi.Context(N, C_, I, D, nrot, flip, ed, shape_, capi.FLOAT, F, kernel_choice=kernel, max_batch=max_batch) as ctx:
+    s = O.shape(N, C_, I, D, nrot, flip, ed, shape_, capi.FLOAT)
+    want = som0.copy()
+    want_bmu = O.train(s, want, imgs, F)
+    want_d, want_best = O.map_images(s, want, imgs[:1])
+    if kind == "nan":       # (no order among such distances: the kernel that sums every variant is the measure)
+        with capi.Context(N, C_, I, D, nrot, flip, ed, shape_, capi.FLOAT, F, kernel_choice=capi.KERNEL_VALU) as ctx:
+            ctx.set_som(som0)
+            want_bmu = ctx.train(imgs)
+            want = ctx.get_som()
+            d, _, want_best = ctx.distance(imgs[0])
+            want_d, want_best = np.sqrt(d.astype(np.float64)).astype(np.float32)[None], want_best[None]
+    lost = np.isnan(want)
+    for max_batch in (0, 2):
+        with capi.Context(N, C_, I, D, nrot, flip, ed, shape_, capi.FLOAT, F, max_batch=max_batch) as ctx:
             ctx.set_som(som0)
             bmu = np.concatenate([ctx.train(imgs[:1]), ctx.train(imgs[1:])])
-            som = ctx.get_som()
-            d, ssd, best = ctx.distance(imgs[0])
-            got.append((bmu, np.isnan(som) if kind == "nan" else bits(som), ctx.update_counts(), bits(d), best))
-    for other in got[1:]:
-        for g, w in zip(other, got[0]):
-            assert np.array_equal(g, w)
+            som, counts = ctx.get_som(), ctx.update_counts()
+            d, _, best = ctx.distance(imgs[0])
+        assert lost.any() == (kind == "nan")
+        assert np.array_equal(bmu, want_bmu) and np.array_equal(counts, np.bincount(want_bmu, minlength=N)), max_batch
+        assert np.array_equal(np.isnan(som), lost) and np.array_equal(bits(som)[~lost], bits(want)[~lost]), max_batch
+        d = np.sqrt(d.astype(np.float64)).astype(np.float32)
+        known = ~np.isnan(want_d[0])
+        assert np.array_equal(np.isnan(d), ~known) and np.array_equal(bits(d)[known], bits(want_d[0])[known]), max_batch
+        assert np.array_equal(best[known], want_best[0][known]), max_batch
 
 
 @pytest.mark.parametrize("N,ed_type", [(9, capi.FLOAT), (9, capi.UINT8), (530, capi.UINT8)])
