@@ -922,25 +922,122 @@ __global__ __launch_bounds__(512) void k_train_f32_dpp(const float *__restrict__
 // but a full SIMD does.  Here a wave reads its neurons' elements with scalar loads (the neuron is the same
 // for all lanes) and `v_sub_f32 d, s, v` runs at the full rate; stages of 32 elements and few registers
 // let eight blocks share a CU.  Same chains, same order, same results.
-template <int TN, int KC, int MINB, int SW, bool NL>
-__global__ __launch_bounds__(256, MINB) void k_dist_f32_sg(const float *__restrict__ somP, const float *__restrict__ rotT,
-                                                           unsigned long long *__restrict__ key, uint32_t N, uint32_t Epad,
-                                                           uint32_t R, uint32_t Rpad, uint32_t lane_tiles, uint32_t scal_groups)
+// Rows on the lanes (64 per block, through LDS) and rows as scalar operands (TN per wave).  The lanes' rows come in by way of
+// a stager (request(set, c): chunk c of KC elements on its way into register set `set` of DEPTH; put(set, c): from there into
+// its LDS stage), which the first four waves of the block run.
+template <int KC, int DEPTH>
+struct RowStager {
+    static constexpr uint32_t kTPR = KC / 4, kStep = 256 / kTPR, kVec = KC / 16, kRow = KC + 4;
+    const float *from[kVec];
+    v4f *to;
+    v4f st[DEPTH][kVec];
+    // rows first, first + 1, ... of `rows` (loads are clamped to the last one of `count`)
+    __device__ __forceinline__ RowStager(const float *rows, uint32_t first, uint32_t count, uint32_t Epad, v4f *lds)
+    {
+        const uint32_t tid = threadIdx.x, row = tid / kTPR, col = (tid % kTPR) * 4;
+#pragma unroll
+        for (uint32_t i = 0; i < kVec; ++i) from[i] = rows + (size_t)min(first + row + kStep * i, count - 1) * Epad + col;
+        to = lds + (row * kRow + col) / 4;
+    }
+    __device__ __forceinline__ void request(int set, uint32_t c)
+    {
+#pragma unroll
+        for (uint32_t i = 0; i < kVec; ++i) st[set][i] = *(const v4f *)(from[i] + c * KC);
+    }
+    __device__ __forceinline__ void put(int set, uint32_t c)
+    {
+#pragma unroll
+        for (uint32_t i = 0; i < kVec; ++i) to[(c & 1) * (64 * kRow / 4) + i * (kStep * kRow / 4)] = st[set][i];
+    }
+};
+
+// acc[j] = the sum over a row's chunks of (scalar row j - lane's row)^2, in element order.
+template <int TN, int KC, int SW, int DEPTH, typename Stager, typename Row>
+__device__ __forceinline__ void sum_tile(float (&acc)[TN], Stager &stager, const v4f *lds, const Row *(&np)[TN], uint32_t Epad)
 {
     static_assert(KC == 64 || KC == 32, "stage width");
     static_assert(SW == 16 || SW == 8, "slab width");
     constexpr int ROW = KC + 4;
     constexpr int SLABS = KC / SW;
-    constexpr int VPT = KC / 16;
-    constexpr int TPR = KC / 4;
-    constexpr int RSTEP = 256 / TPR;
-    __shared__ v4f s_rot[2][64 * ROW / 4];
+    const uint32_t lane = threadIdx.x & 63, nchunks = Epad / KC;
+    const bool stages = threadIdx.x < 256;                // (whole waves)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[j] = 0.0f;
+    if (stages) {
+        stager.request(0, 0);
+        stager.put(0, 0);
+#pragma unroll
+        for (int u = 1; u <= DEPTH; ++u)
+            if ((uint32_t)u < nchunks) stager.request(u % DEPTH, u);
+    }
+    __syncthreads();
+
+    // Operands of a slab of SW elements wait in registers one slab ahead: the lane's SW rotation values
+    // (vector registers, from LDS) and the wave's TN x SW neuron values (scalar registers), in two sets
+    // that take turns.  Slab 0 of a chunk also moves the staged chunk c+1 into the other stage and requests
+    // chunk c+1+DEPTH; the barrier stands before the last slab: by then every wave holds all of chunk c in
+    // registers (its last slab prefetched) and has stored its part of chunk c+1, so the last slab may
+    // prefetch slab 0 of chunk c+1 and the next chunk (or the next tile's first) may overwrite this one's stage.
+    float bv[2][SW];
+    float an[2][TN][SW];
+    auto fetch = [&](int set, uint32_t c, int sl) {
+        const v4f *from = lds + (c & 1) * (64 * ROW / 4) + lane * (ROW / 4) + sl * (SW / 4);
+#pragma unroll
+        for (int q = 0; q < SW / 4; ++q) {
+            const v4f t4 = from[q];
+            bv[set][4 * q] = t4.x; bv[set][4 * q + 1] = t4.y; bv[set][4 * q + 2] = t4.z; bv[set][4 * q + 3] = t4.w;
+        }
+        const uint32_t k = min(c * KC + sl * SW, Epad - SW);     // (past the end: values nobody uses)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < SW; ++e) an[set][j][e] = np[j][k + e];
+    };
+    fetch(0, 0, 0);
+    for (uint32_t base = 0; base < nchunks; base += DEPTH)
+#pragma unroll
+    for (int turn = 0; turn < DEPTH; ++turn) {
+        const uint32_t c = base + turn;
+        if (DEPTH > 1 && c >= nchunks) break;
+#pragma unroll
+        for (int sl = 0; sl < SLABS; ++sl) {
+            const int set = sl & 1;
+            // this slab's operands were requested a slab ago; scalar loads return in any order, so the
+            // counter can only be waited down to zero: do it before the next requests join it
+            // (the builtin, not inline assembly: the compiler's own wait insertion must know of it, or it
+            // waits again at the first use, after the new requests; 0xc07f = lgkmcnt(0), the others untouched)
+            __builtin_amdgcn_s_waitcnt(0xc07f);
+            if (sl + 1 < SLABS) fetch(set ^ 1, c, sl + 1);
+            else fetch(set ^ 1, c + 1, 0);
+            if (sl == 0 && stages) {
+                if (c + 1 < nchunks) stager.put((turn + 1) % DEPTH, c + 1);
+                if (c + 1 + DEPTH < nchunks) stager.request((turn + 1) % DEPTH, c + 1 + DEPTH);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < SW; ++e)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const float d = __fsub_rn(an[set][j][e], bv[set][e]);
+                    acc[j] = __builtin_fmaf(d, d, acc[j]);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+            if (sl == SLABS - 2) __syncthreads();
+        }
+    }
+}
+
+template <int TN, int KC, int MINB, int SW, bool NL>
+__global__ __launch_bounds__(256, MINB) void k_dist_f32_sg(const float *__restrict__ somP, const float *__restrict__ rotT,
+                                                           unsigned long long *__restrict__ key, uint32_t N, uint32_t Epad,
+                                                           uint32_t R, uint32_t Rpad, uint32_t lane_tiles, uint32_t scal_groups)
+{
+    __shared__ v4f s_rot[2 * 64 * (KC + 4) / 4];
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t b = blockIdx.z;
-    // Rows on the lanes (64 per block, through LDS) and rows as scalar operands (TN per wave): rotations and
-    // neurons, or (NL) neurons and rotations -- whichever wastes fewer lanes on padding.  A chain is the same
-    // sequence of operations either way (the difference changes sign, its square does not).
+    // Rotations on the lanes and neurons as scalar operands, or (NL) the other way round -- whichever wastes fewer lanes on
+    // padding.  A chain is the same sequence of operations either way (the difference changes sign, its square does not).
     // Workgroups go to the 8 XCDs round-robin by linear id and each XCD has its own L2: XCD k takes the k-th run of
     // consecutive (lane tile, scalar group) pairs, lane tile slowest, so it streams a few lane tiles instead of all of them
     // (the grid is padded to a multiple of 8; the blocks beyond the last pair leave at once, whole)
@@ -957,82 +1054,8 @@ __global__ __launch_bounds__(256, MINB) void k_dist_f32_sg(const float *__restri
 #pragma unroll
     for (int j = 0; j < TN; ++j) np[j] = scalP + (size_t)min(s0 + j, scal_rows - 1) * Epad;
     float acc[TN];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[j] = 0.0f;
-
-    const uint32_t lrow = tid / TPR, lcol = (tid % TPR) * 4;
-    const float *lp[VPT];
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) lp[i] = laneP + (size_t)min(l0 + lrow + RSTEP * i, lane_rows - 1) * Epad + lcol;
-    const uint32_t lds_w = (lrow * ROW + lcol) / 4;
-    const uint32_t lds_wstep = RSTEP * ROW / 4;
-    const uint32_t nchunks = Epad / KC;
-    v4f st[VPT];
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) s_rot[0][lds_w + i * lds_wstep] = *(const v4f *)(lp[i]);
-    if (nchunks > 1) {
-#pragma unroll
-        for (int i = 0; i < VPT; ++i) st[i] = *(const v4f *)(lp[i] + KC);
-    }
-    __syncthreads();
-
-    // Operands of a slab of SW elements wait in registers one slab ahead: the lane's SW rotation values
-    // (vector registers, from LDS) and the wave's TN x SW neuron values (scalar registers), in two sets
-    // that take turns.  Slab 0 of a chunk also moves the staged chunk c+1 into the other stage and requests
-    // chunk c+2; the barrier stands before the last slab: by then every wave holds all of chunk c in
-    // registers (its last slab prefetched) and has stored its part of chunk c+1, so the last slab may
-    // prefetch slab 0 of chunk c+1 and the next chunk may overwrite this one's stage.
-    float bv[2][SW];
-    float an[2][TN][SW];
-    auto fetch = [&](int set, uint32_t c, int sl) {
-        const v4f *from = s_rot[c & 1] + lane * (ROW / 4) + sl * (SW / 4);
-#pragma unroll
-        for (int q = 0; q < SW / 4; ++q) {
-            const v4f t4 = from[q];
-            bv[set][4 * q] = t4.x; bv[set][4 * q + 1] = t4.y; bv[set][4 * q + 2] = t4.z; bv[set][4 * q + 3] = t4.w;
-        }
-        const uint32_t k = min(c * KC + sl * SW, Epad - SW);     // (past the end: values nobody uses)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int e = 0; e < SW; ++e) an[set][j][e] = np[j][k + e];
-    };
-    fetch(0, 0, 0);
-    for (uint32_t c = 0; c < nchunks; ++c) {
-#pragma unroll
-        for (int sl = 0; sl < SLABS; ++sl) {
-            const int set = sl & 1;
-            // this slab's operands were requested a slab ago; scalar loads return in any order, so the
-            // counter can only be waited down to zero: do it before the next requests join it
-            // (the builtin, not inline assembly: the compiler's own wait insertion must know of it, or it
-            // waits again at the first use, after the new requests; 0xc07f = lgkmcnt(0), the others untouched)
-            __builtin_amdgcn_s_waitcnt(0xc07f);
-            if (sl + 1 < SLABS) fetch(set ^ 1, c, sl + 1);
-            else fetch(set ^ 1, c + 1, 0);
-            if (sl == 0) {
-                if (c + 1 < nchunks) {
-                    v4f *nx = s_rot[(c + 1) & 1];
-#pragma unroll
-                    for (int i = 0; i < VPT; ++i) nx[lds_w + i * lds_wstep] = st[i];
-                }
-                if (c + 2 < nchunks) {
-                    const uint32_t k = (c + 2) * KC;
-#pragma unroll
-                    for (int i = 0; i < VPT; ++i) st[i] = *(const v4f *)(lp[i] + k);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int e = 0; e < SW; ++e)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const float d = NL ? __fsub_rn(bv[set][e], an[set][j][e]) : __fsub_rn(an[set][j][e], bv[set][e]);
-                    acc[j] = __builtin_fmaf(d, d, acc[j]);
-                }
-            __builtin_amdgcn_sched_barrier(0);
-            if (sl == SLABS - 2) __syncthreads();
-        }
-    }
+    RowStager<KC, 1> stager(laneP, l0, lane_rows, Epad, s_rot);
+    sum_tile<TN, KC, SW, 1>(acc, stager, s_rot, np, Epad);
 
     if constexpr (!NL) {
         const uint32_t r = l0 + lane;
@@ -2357,6 +2380,9 @@ struct pink_hip_ctx {
     bool orbit_train = false;
     // ... and the float32 trainers that screen their distances: rows_f32_train's operands, the product's beside them
     bool screen_train = false;
+    uint32_t screen_set = 0;               // the counts that the last image took
+    uint2 *d_screen_list = nullptr;
+    uint32_t *d_screen_wide = nullptr, *d_screen_counts = nullptr;
     uint4 *d_orb_element = nullptr;
     uint32_t orb_cur = 0, orb_pitch = 0, orb_outside = 0;      // the set of norms that belongs to the operand
     uint32_t *d_orb_outside = nullptr, *d_orb_best = nullptr;
@@ -3118,7 +3144,8 @@ int free_all(pink_hip_ctx *ctx)
                     ctx->d_Pa, ctx->d_Pb, ctx->d_na, ctx->d_nb, ctx->d_poff, ctx->d_need, ctx->d_inv,
                     ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4,
                     ctx->d_orb_tables, ctx->d_orb_outside, ctx->d_orb_best, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
-                    ctx->d_orb_sa, ctx->d_orb_ea, ctx->d_orb_sb, ctx->d_orb_eb, ctx->d_orb_dump};
+                    ctx->d_orb_sa, ctx->d_orb_ea, ctx->d_orb_sb, ctx->d_orb_eb, ctx->d_orb_dump,
+                    ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu}) if (p) (void)hipFree(p);
     if (ctx->st_pin) (void)hipHostFree(ctx->st_pin);
@@ -3636,6 +3663,7 @@ int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
     a.key = key; a.dump = ctx->d_orb_dump; a.part = ctx->d_orb_part; a.scale_rows = ctx->d_orb_sb ? ctx->d_orb_sb + slot : nullptr; a.scale_som = ctx->d_orb_sa;
     a.rows_plane = rows_plane; a.som_plane = (size_t)ctx->N * ctx->orb_KS * 2;
     a.M = M; a.N = ctx->N; a.KS = ctx->orb_KS; a.nrr = ctx->nrr_eff; a.num_rot = ctx->cfg.num_rot; a.ns = ctx->orb_ns; a.valid = ctx->orb_valid;
+    a.skip = ctx->d_screen_counts ? ctx->d_screen_counts + 2 * kCounts : nullptr;
     // 64 x 128 tiles (a wave 32 x 64) read the operands less often; 64 x 64 ones fill the chip with few rows, and with two
     // planes and short rows more of their blocks hide each other's beginnings and ends
     const size_t columns = (size_t)a.N * a.ns, tiles = (size_t)((M + 63) / 64) * ((columns + 127) / 128);
@@ -3648,13 +3676,26 @@ int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
     TRY(launch_check(ctx, "k_orbit_gemm"));
     if (!f32) return PINK_HIP_OK;
     if (ctx->screen_train) {
-        ScreenChain x{};
-        x.dump = ctx->d_orb_dump; x.som_rows = (const float *)ctx->d_somP; x.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad;
-        x.err_rows = ctx->d_orb_eb + row; x.err_som = ctx->d_orb_ea; x.key = key;
-        x.N = ctx->N; x.E = ctx->E; x.Epad = ctx->Epad; x.nrr = ctx->nrr_eff; x.num_rot = ctx->cfg.num_rot;
-        x.ns = ctx->orb_ns; x.valid = ctx->orb_valid;
-        hipLaunchKernelGGL(k_screen_chain, dim3((ctx->N + kChainNeurons - 1) / kChainNeurons), dim3(320), 0, ctx->stream, x);
-        return launch_check(ctx, "k_screen_chain");
+        ctx->screen_set ^= 1;
+        uint32_t *counts = ctx->d_screen_counts + kCounts * ctx->screen_set, *counts_next = ctx->d_screen_counts + kCounts * (ctx->screen_set ^ 1);
+        ScreenSelect l{};
+        l.dump = ctx->d_orb_dump; l.err_rows = ctx->d_orb_eb + row; l.err_som = ctx->d_orb_ea; l.key = key;
+        l.list = ctx->d_screen_list; l.wide = ctx->d_screen_wide; l.counts = counts; l.counts_next = counts_next;
+        l.some_list = ctx->d_screen_list + (size_t)ctx->N * kSelectFew; l.some = ctx->d_screen_wide + ctx->N;
+        l.skip = a.skip;
+        l.N = ctx->N; l.E = ctx->E; l.nrr = ctx->nrr_eff; l.num_rot = ctx->cfg.num_rot; l.ns = ctx->orb_ns; l.valid = ctx->orb_valid;
+        hipLaunchKernelGGL(k_screen_select, dim3((uint32_t)((columns + 63) / 64)), dim3(512), 0, ctx->stream, l);
+        TRY(launch_check(ctx, "k_screen_select"));
+        ScreenSums x{};
+        x.som_rows = (const float *)ctx->d_somP; x.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad;
+        x.list = l.list; x.some_list = l.some_list; x.wide = l.wide; x.some = l.some; x.counts = counts; x.key = key;
+        x.Epad = ctx->Epad; x.R = ctx->R; x.Rpad = ctx->Rpad;
+        x.wide_blocks = x.chain_blocks = 2 * (uint32_t)ctx->num_cu;        // (four blocks to a CU: all of them run at once)
+        hipLaunchKernelGGL(k_screen_sums, dim3(x.wide_blocks + x.chain_blocks), dim3(64 * kSumsWaves), 0, ctx->stream, x);
+        TRY(launch_check(ctx, "k_screen_sums"));
+        const uint32_t pairs = ctx->Rpad / kWave * ((ctx->N + 7) / 8);
+        hipLaunchKernelGGL(k_screen_many, dim3((pairs + 7) / 8 * 8), dim3(256), 0, ctx->stream, x);
+        return launch_check(ctx, "k_screen_many");
     }
     ScreenExact x{};
     x.dump = ctx->d_orb_dump; x.values = ctx->d_orb_values; x.xrows = ctx->d_orb_x + row * ctx->orb_KS * 32; x.err_rows = ctx->d_orb_eb + row; x.err_som = ctx->d_orb_ea;
@@ -3678,7 +3719,7 @@ int run_screen_update(pink_hip_ctx *ctx, uint32_t slot, uint32_t *dev_bmu_out)
     Timed t(ctx, kClsUpdate);
     ScreenUpdate u{};
     u.som_rows = (float *)ctx->d_somP; u.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad; u.factors_t = ctx->d_factors_t;
-    u.element = ctx->d_orb_element;
+    u.element = ctx->d_orb_element; u.listed = ctx->d_screen_counts + kCounts * ctx->screen_set; u.skip = ctx->d_screen_counts + 2 * kCounts;
     u.opnd = (uint2 *)ctx->d_orb_som; u.key = ctx->d_key + (size_t)slot * ctx->N; u.norm = ctx->d_orb_na; u.scale = ctx->d_orb_sa; u.err = ctx->d_orb_ea;
     u.bmu_out = dev_bmu_out; u.counts = ctx->d_counts; u.plane = (size_t)ctx->N * ctx->orb_KS * 32; u.N = ctx->N; u.K8 = ctx->orb_KS * 4; u.Epad = ctx->Epad;
     hipLaunchKernelGGL(k_screen_update, dim3(ctx->N), dim3(512), (size_t)ctx->Epad * sizeof(float), ctx->stream, u);
@@ -4247,6 +4288,9 @@ int init_ctx(pink_hip_ctx *ctx)
             TRY(dev_alloc(ctx, &ctx->d_orb_sb, B));
             TRY(dev_alloc(ctx, &ctx->d_orb_eb, B * ctx->nrr_eff));
             TRY(dev_alloc(ctx, &ctx->d_orb_dump, (size_t)ctx->nrr_eff * ctx->N * ctx->orb_ns));
+            TRY(dev_alloc(ctx, &ctx->d_screen_list, (size_t)ctx->N * (kSelectFew + kSelectSome)));
+            TRY(dev_alloc(ctx, &ctx->d_screen_wide, (size_t)2 * ctx->N));
+            TRY(upload(ctx, &ctx->d_screen_counts, std::vector<uint32_t>(2 * kCounts + 1, 0u)));       // (two sets, images to skip)
             ctx->orb_part_bytes = (size_t)16 << 20;
             TRY(dev_alloc(ctx, (char **)&ctx->d_orb_part, ctx->orb_part_bytes));
             HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_screen_update, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 1024));

@@ -416,11 +416,11 @@ def test_map_with_orbit_rows(N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, da
     assert np.array_equal(one_best, want_best[-1:]) and np.array_equal(bits(one_heat), bits(want_heat[-1:]))
 
 
-def _nearly_round(rng, n, C_, I, scale):
+def _nearly_round(rng, n, C_, I, scale, noise=1e-3):
     """Images whose rotated copies differ by a thousandth: every variant's distance is close to every other's."""
     x = np.linspace(-1, 1, I)
     r2 = (x[:, None] ** 2 + x[None, :] ** 2) * rng.uniform(0.5, 3.0, (n, C_, 1, 1))
-    return (scale * (np.exp(-r2) + 1e-3 * rng.random((n, C_, I, I)))).astype(np.float32)
+    return (scale * (np.exp(-r2) + noise * rng.random((n, C_, I, I)))).astype(np.float32)
 
 
 @pytest.mark.parametrize("scale", [1e-20, 1e-19, 3e-19, 1e-18, 3e-18, 1e-15, 1.0, 1e15])
@@ -697,7 +697,11 @@ SCREENED_TRAIN_SHAPES = [
     (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 3, "blobs"),      # a block of two neurons at the end
     (515, 2, 70, 60, 360, False, 53, capi.QUADRATIC, 3, "blobs"),      # four columns per neuron
     (700, 1, 80, 70, 264, True, 61, capi.CIRCULAR, 3, "noise"),        # 66 base rotations: two lists
-    (640, 1, 90, 128, 128, True, 90, capi.QUADRATIC, 3, "zeros"),      # most variants alike: every candidate summed
+    (640, 1, 90, 128, 128, True, 90, capi.QUADRATIC, 3, "zeros"),      # most variants alike: every variant of every neuron summed
+    (523, 1, 70, 60, 452, True, 49, capi.QUADRATIC, 3, "grown"),       # some neurons keep all variants; 113 base rotations
+    (517, 1, 70, 62, 360, True, 52, capi.QUADRATIC, 19, "flat"),      # ... image after image: no product for some of them, then again
+    (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 3, "close"),      # 18000 variants listed, more than one pass takes
+    (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 3, "closer"),     # 16300: one pass, in full batches
     (1200, 1, 64, 50, 180, True, 50, capi.QUADRATIC, 3, "nan"),
     (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 3, "flux"),       # every variant close, squares of errors no float32
 ]
@@ -714,12 +718,18 @@ def test_float_trainer_with_screened_distances(N, C_, I, D, nrot, flip, ed, shap
         imgs = imgs * 0.1 + np.exp(-8 * (x[:, None] - imgs[:, :, :1, :1]) ** 2 - 20 * x[None, :] ** 2).astype(np.float32)
     elif kind == "zeros":
         imgs[imgs < 0.999] = 0.0
+    elif kind == "flat":
+        imgs[:-1] = 0.25
+    elif kind == "grown":
+        som0[::9] *= 3000.0                                            # (far above the images: distances differ by less than they round)
     elif kind == "nan":
         imgs[1, 0, I // 2, I // 2] = np.nan
+    elif kind.startswith("close"):
+        imgs = _nearly_round(rng, n, C_, I, 1.0, 0.02 if kind == "close" else 0.03)
     elif kind == "flux":
         imgs, som0 = _nearly_round(rng, n, C_, I, 5e-19), som0 * np.float32(5e-19)
-    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 1.0, 0.5)
-    F[F < 0.01] = 0.0
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.MEXICAN_HAT if kind == "grown" else capi.GAUSSIAN, 1.0, 0.5)
+    F[np.abs(F) < 0.01] = 0.0
     s = O.shape(N, C_, I, D, nrot, flip, ed, shape_, capi.FLOAT)
     want = som0.copy()
     want_bmu = O.train(s, want, imgs, F)
