@@ -952,7 +952,7 @@ struct RowStager {
 };
 
 // acc[j] = the sum over a row's chunks of (scalar row j - lane's row)^2, in element order.
-template <int TN, int KC, int SW, int DEPTH, typename Stager, typename Row>
+template <int TN, int KC, int SW, int DEPTH, uint32_t STAGING = 256, typename Stager, typename Row>
 __device__ __forceinline__ void sum_tile(float (&acc)[TN], Stager &stager, const v4f *lds, const Row *(&np)[TN], uint32_t Epad)
 {
     static_assert(KC == 64 || KC == 32, "stage width");
@@ -960,7 +960,7 @@ __device__ __forceinline__ void sum_tile(float (&acc)[TN], Stager &stager, const
     constexpr int ROW = KC + 4;
     constexpr int SLABS = KC / SW;
     const uint32_t lane = threadIdx.x & 63, nchunks = Epad / KC;
-    const bool stages = threadIdx.x < 256;                // (whole waves)
+    const bool stages = threadIdx.x < STAGING;            // (whole waves)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[j] = 0.0f;
     if (stages) {
@@ -1024,6 +1024,22 @@ __device__ __forceinline__ void sum_tile(float (&acc)[TN], Stager &stager, const
             __builtin_amdgcn_sched_barrier(0);
             if (sl == SLABS - 2) __syncthreads();
         }
+    }
+}
+
+// ... the part of a wave without scalar rows in it.
+template <int DEPTH, typename Stager>
+__device__ __forceinline__ void sum_tile_staging_only(Stager &stager, uint32_t nchunks)
+{
+    static_assert(DEPTH == 1, "one register set");
+    stager.request(0, 0);
+    stager.put(0, 0);
+    if (nchunks > 1) stager.request(0, 1);
+    __syncthreads();
+    for (uint32_t c = 0; c < nchunks; ++c) {
+        if (c + 1 < nchunks) stager.put(0, c + 1);
+        if (c + 2 < nchunks) stager.request(0, c + 2);
+        __syncthreads();
     }
 }
 
@@ -2375,6 +2391,7 @@ struct pink_hip_ctx {
     uint32_t *d_orb_slots = nullptr;
     uint2 *d_orb_bands = nullptr;
     uint4 *d_orb_where = nullptr;
+    unsigned short *d_orb_place = nullptr;
     unsigned char *d_orb_live = nullptr;
     // ... and the trainers that keep their weights in that order: an image's rows start a tile of 32
     bool orbit_train = false;
@@ -2541,7 +2558,8 @@ int run_pack_som(pink_hip_ctx *ctx)
     Timed t(ctx, kClsPack);
     if (ctx->screen_train) TRY(run_orbit_som(ctx));
     if (ctx->orbit) {
-        return run_orbit_som(ctx);
+        TRY(run_orbit_som(ctx));
+        if (is_int(ctx)) return PINK_HIP_OK;              // (float32: the rows in the CPU's order too)
     }
     if (ctx->gemm) {
         if (ctx->cfg.ed_type == PINK_HIP_UINT16)
@@ -3528,6 +3546,9 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         tables.add(&ctx->d_orb_slots, slots);
         tables.add(&ctx->d_orb_bands, bands);
         tables.add(&ctx->d_orb_where, w16);
+        std::vector<unsigned short> place;
+        for (const auto &w : where) place.insert(place.end(), w.begin(), w.end());
+        tables.add(&ctx->d_orb_place, place);
     }
     TRY(tables.commit(ctx, &ctx->d_orb_tables));
     {
@@ -3642,6 +3663,7 @@ int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
     p.opnd = ctx->d_orb_rows; p.norm = ctx->d_orb_nb; p.key = is_int(ctx) ? ctx->d_key : nullptr; p.scale = ctx->d_orb_sb; p.err = ctx->d_orb_eb;
     p.xrows = ctx->d_orb_x; p.plane = orbit_rows_plane(ctx, B); p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.KS = ctx->orb_KS;
     p.all_sym = ctx->orb_all; p.rl = ctx->orb_rl; p.pitch = ctx->orb_pitch;
+    p.wide_count = ctx->orbit && !is_int(ctx) ? ctx->d_screen_counts : nullptr;
     const dim3 grid(B, (ctx->nrr_eff + (1u << p.rl) - 1) >> p.rl);
     const uint32_t threads = ctx->orb_prep_lds > 64 * 1024 || grid.x * grid.y < (uint32_t)ctx->num_cu ? 1024 : ctx->orb_prep_lds > 24 * 1024 ? 512 : 256;
     void *args[] = {&p};
@@ -3663,7 +3685,7 @@ int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
     a.key = key; a.dump = ctx->d_orb_dump; a.part = ctx->d_orb_part; a.scale_rows = ctx->d_orb_sb ? ctx->d_orb_sb + slot : nullptr; a.scale_som = ctx->d_orb_sa;
     a.rows_plane = rows_plane; a.som_plane = (size_t)ctx->N * ctx->orb_KS * 2;
     a.M = M; a.N = ctx->N; a.KS = ctx->orb_KS; a.nrr = ctx->nrr_eff; a.num_rot = ctx->cfg.num_rot; a.ns = ctx->orb_ns; a.valid = ctx->orb_valid;
-    a.skip = ctx->d_screen_counts ? ctx->d_screen_counts + 2 * kCounts : nullptr;
+    a.skip = ctx->screen_train ? ctx->d_screen_counts + 2 * kCounts : nullptr;
     // 64 x 128 tiles (a wave 32 x 64) read the operands less often; 64 x 64 ones fill the chip with few rows, and with two
     // planes and short rows more of their blocks hide each other's beginnings and ends
     const size_t columns = (size_t)a.N * a.ns, tiles = (size_t)((M + 63) / 64) * ((columns + 127) / 128);
@@ -3702,9 +3724,18 @@ int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
     x.slots = ctx->d_orb_slots; x.bands = ctx->d_orb_bands; x.where = ctx->d_orb_where; x.key = key;
     x.N = ctx->N; x.E = ctx->E; x.K = ctx->orb_KS * 32; x.nrr = ctx->nrr_eff; x.num_rot = ctx->cfg.num_rot;
     x.ns = ctx->orb_ns; x.valid = ctx->orb_valid; x.band_count = ctx->orb_bands;
-    x.stride = ctx->orb_stride; x.batch = ctx->orb_batch;
+    x.stride = ctx->orb_stride; x.batch = ctx->orb_batch; x.wide = ctx->d_screen_wide; x.wide_count = ctx->d_screen_counts;
     hipLaunchKernelGGL(k_screen_exact, dim3((ctx->N * x.ns + 31) / 32, B), dim3(256), (size_t)x.batch * x.stride * sizeof(float), ctx->stream, x);
-    return launch_check(ctx, "k_screen_exact");
+    TRY(launch_check(ctx, "k_screen_exact"));
+    ScreenWide w{};
+    w.som_rows = (const float *)ctx->d_somP; w.xrows = x.xrows; w.place = ctx->d_orb_place; w.wide = x.wide; w.wide_count = x.wide_count; w.key = key;
+    w.N = x.N; w.E = x.E; w.Epad = ctx->Epad; w.K = x.K; w.nrr = x.nrr; w.num_rot = x.num_rot; w.images = B;
+    // (a block to a CU, two of them are no faster; fewer where even every neuron listed makes less work)
+    const size_t most = (size_t)B * ((w.nrr + 64 / x.ns - 1) / (64 / x.ns)) * ((w.N + 63) / 64);
+    const dim3 grid((uint32_t)std::min<size_t>((most + 7) / 8 * 8, (size_t)ctx->num_cu / 8 * 8));
+    if (x.ns == 8) hipLaunchKernelGGL(k_screen_wide<8>, grid, dim3(kWideThreads), 0, ctx->stream, w);
+    else hipLaunchKernelGGL(k_screen_wide<4>, grid, dim3(kWideThreads), 0, ctx->stream, w);
+    return launch_check(ctx, "k_screen_wide");
 }
 
 int run_orbit(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
@@ -4119,6 +4150,9 @@ int init_ctx(pink_hip_ctx *ctx)
             TRY(dev_alloc(ctx, &ctx->d_orb_sb, B));
             TRY(dev_alloc(ctx, &ctx->d_orb_eb, B * ctx->nrr_eff));
             TRY(dev_alloc(ctx, &ctx->d_orb_dump, B * ctx->nrr_eff * ctx->N * ctx->orb_ns));
+            TRY(dev_alloc(ctx, &ctx->d_screen_wide, B * ctx->N));
+            TRY(dev_alloc(ctx, &ctx->d_screen_counts, B));
+            TRY(dev_alloc(ctx, (uint32_t **)&ctx->d_somP, (size_t)ctx->N * ctx->Epad + kDistOverrun));
         }
         if (!is_int(ctx) || ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_x, B * ctx->nrr_eff * ctx->orb_KS * 32));
         if (ctx->trainer) {
