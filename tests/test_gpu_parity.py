@@ -386,6 +386,9 @@ ORBIT_MAP_SHAPES = [
     (13, 1, 150, 106, 72, True, 75, capi.CIRCULAR, capi.FLOAT, 2, "noise"),
     (40, 1, 20, 14, 360, True, 10, capi.QUADRATIC, capi.FLOAT, 4, "flat"),    # every variant ties
     (40, 1, 20, 14, 360, True, 10, capi.QUADRATIC, capi.FLOAT, 4, "mask"),    # values that rounding keeps, many ties
+    (5, 1, 12, 8, 128, True, 5, capi.QUADRATIC, capi.FLOAT, 1500, "thirds"),  # more images than are counted at a time
+    (70, 1, 30, 24, 360, False, 17, capi.QUADRATIC, capi.FLOAT, 60, "thirds"),  # two runs of 64 neurons, four columns per neuron
+    (40, 1, 20, 14, 360, True, 10, capi.QUADRATIC, capi.FLOAT, 150, "grown"),  # some neurons of an image keep every variant
     (12, 1, 20, 14, 360, True, 10, capi.QUADRATIC, capi.FLOAT, 4, "wide"),    # either sign, six orders of magnitude
     (12, 1, 20, 14, 360, True, 10, capi.QUADRATIC, capi.FLOAT, 4, "tiny"),    # squares below the smallest normal number
 ]
@@ -400,6 +403,10 @@ def test_map_with_orbit_rows(N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, da
     imgs, som = rng.random((n, C_, I, I), dtype=np.float32), rng.random((N, C_ * D * D), dtype=np.float32)
     if data == "flat":
         imgs[:], som[:] = 0.25, 0.5
+    elif data == "thirds":
+        imgs[::3] = 0.25
+    elif data == "grown":
+        som[::7] *= 3000.0
     elif data == "mask":
         imgs, som = (imgs < 0.1).astype(np.float32), (som < 0.1).astype(np.float32)
     elif data == "wide":
