@@ -2384,6 +2384,7 @@ struct pink_hip_ctx {
     int orb_mode = 0;
     uint32_t orb_KS = 0, orb_all = 0, orb_ns = 8, orb_valid = 0;
     size_t orb_prep_lds = 0;
+    uint32_t sum_images = 0;               // float32: launches of at most so many images sum every variant (summed_images)
     uint32_t orb_rl = 0, orb_bands = 0, orb_stride = 0, orb_batch = 0;
     char *d_orb_tables = nullptr;          // ... the tables below that init_orbit makes on the host
     uint32_t *d_orb_elem = nullptr, *d_orb_sel = nullptr, *d_orb_index = nullptr;
@@ -3584,13 +3585,28 @@ size_t orbit_image_bytes(const pink_hip_ctx *ctx)
                            (is_int(ctx) && !ctx->trainer ? (size_t)0 : (size_t)ctx->orb_KS * 128));
 }
 
-// Float32 mappers: whether screening pays (see k_screen_exact).  What summing a neuron's every variant takes grows with their
+// Float32 mappers: whether a full launch group of images is screened (see k_screen_exact; few images are summed all the same,
+// summed_images).  What summing a neuron's every variant takes grows with their
 // number, what is left to sum exactly does not: break-even lies near 100 variants (20 variants of 768 elements 10 % slower
 // with it, 8 of 1369 half as fast, 360 of 121 1.5 times as fast, 720 of 1024 3.8 times).  And what an image leaves in
 // memory has to fit the scratch of pink_hip_map_device_static.
 bool orbit_screens(const pink_hip_ctx *ctx)
 {
     return ctx->R >= 128 && (size_t)ctx->nrr_eff * ctx->N * 8 * 4 + (size_t)ctx->nrr_eff * ctx->E * 12 <= ((size_t)24 << 20);
+}
+
+// ... and the images of a launch up to which such a mapper sums every variant after all.  Screening launches three kernels more, and
+// the few sums that it leaves are one chain of E steps after all else: 9 + 0.021 E us.  The sums cost 29 ns per 10^6 neuron x
+// variant x element and the rotated variants 1.7 us per 10^6 variant x element more than screening them does.  Both fitted to
+// 9 to 1600 neurons, 128 to 720 variants, 400 to 4096 elements, 1 to 256 images; (summed / screened us) at 1024 elements, 720
+// variants: 9 neurons 16 images 60 / 66, 64 images 115 / 87; 100 neurons 1 image 35 / 62, 8 images 70 / 74, 16 images 105 / 78;
+// 1600 neurons 1 image 83 / 75.  A GiB at most for their rows.
+uint32_t summed_images(const pink_hip_ctx *ctx)
+{
+    const double variants = (double)ctx->R * ctx->E;
+    const double images = (9.0 + 0.021 * ctx->E) / (variants * (2.9e-8 * ctx->N + 1.7e-6));
+    const size_t row_bytes = (size_t)ctx->Epad * ctx->Rpad * 4 + (ctx->fused_pack ? 0 : (size_t)ctx->R * ctx->S * 4);
+    return (uint32_t)std::min({images, (double)ctx->Bcap, (double)((size_t)1 << 30) / (double)row_bytes});
 }
 
 // Trainers that take the orbits' product: integers where the resident form (init_sym_train) does not fit, which keep their
@@ -4055,12 +4071,13 @@ int init_ctx(pink_hip_ctx *ctx)
     }
     // Operand packing inside the rotation kernel: float32 rows, or byte planes of single-channel
     // integer contexts, whenever the kernel keeps its base rotation in LDS.
-    ctx->fused_pack = !ctx->mfma && !ctx->mfma_sym && !ctx->orbit && ctx->C < 256 && (size_t)ctx->D * ctx->Dp < ((size_t)1 << 24) &&
+    const bool orbit_only = ctx->orbit && is_int(ctx);     // (a float32 mapper sums calls with few images, summed_images)
+    ctx->fused_pack = !ctx->mfma && !ctx->mfma_sym && !orbit_only && ctx->C < 256 && (size_t)ctx->D * ctx->Dp < ((size_t)1 << 24) &&
                       (ctx->gemm ? (ctx->C == 1 || ctx->rot_nch == ctx->C) : !is_int(ctx));
     // Neither the base rotation nor the image fits LDS: interpolating every packed element out of global
     // memory is slow, so the rotation kernel stores two symmetries and packing kernels of their own read
     // all eight out of those, with coalesced accesses
-    ctx->pair_pack = !ctx->use_lds && !ctx->image_lds && !ctx->mfma && !ctx->mfma_sym && !ctx->orbit && ctx->S < (1u << 24);
+    ctx->pair_pack = !ctx->use_lds && !ctx->image_lds && !ctx->mfma && !ctx->mfma_sym && !orbit_only && ctx->S < (1u << 24);
     if (ctx->pair_pack) {
         ctx->fused_pack = false;
         const uint32_t D = ctx->D, DD = D * D;
@@ -4131,10 +4148,11 @@ int init_ctx(pink_hip_ctx *ctx)
         ctx->Bcap = (uint32_t)b;
     }
     const size_t B = ctx->Bcap;
+    if (ctx->orbit && !is_int(ctx)) ctx->sum_images = summed_images(ctx);
 
     TRY(dev_alloc(ctx, &ctx->d_som, (size_t)ctx->N * ctx->S));
     HIP_TRY(ctx, hipMemset(ctx->d_som, 0, (size_t)ctx->N * ctx->S * sizeof(float)));
-    TRY(dev_alloc(ctx, &ctx->d_rot, (group_variants ? B : 1) * ctx->R * ctx->S));
+    TRY(dev_alloc(ctx, &ctx->d_rot, std::max<size_t>(group_variants ? B : 1, ctx->fused_pack ? 0 : ctx->sum_images) * ctx->R * ctx->S));
     TRY(dev_alloc(ctx, &ctx->d_key, B * ctx->N));
     if (ctx->mfma_sym) {
         TRY(dev_alloc(ctx, &ctx->d_Pa, (size_t)ctx->slices * ctx->sym_tiles * ctx->KSs * 1024));
@@ -4153,6 +4171,9 @@ int init_ctx(pink_hip_ctx *ctx)
             TRY(dev_alloc(ctx, &ctx->d_screen_wide, B * ctx->N));
             TRY(dev_alloc(ctx, &ctx->d_screen_counts, B));
             TRY(dev_alloc(ctx, (uint32_t **)&ctx->d_somP, (size_t)ctx->N * ctx->Epad + kDistOverrun));
+            const size_t rows = (size_t)std::max(1u, ctx->sum_images) * ctx->Epad * ctx->Rpad;       // (pink_hip_rotate takes one image)
+            TRY(dev_alloc(ctx, (uint32_t **)&ctx->d_rotT, rows + kDistOverrun));
+            HIP_TRY(ctx, hipMemset(ctx->d_rotT, 0, rows * sizeof(uint32_t)));
         }
         if (!is_int(ctx) || ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_x, B * ctx->nrr_eff * ctx->orb_KS * 32));
         if (ctx->trainer) {
@@ -4403,9 +4424,9 @@ int run_dist_sym(pink_hip_ctx *ctx, uint32_t B)
     return PINK_HIP_OK;
 }
 
-int distance_group(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
+int distance_group(pink_hip_ctx *ctx, const float *dev_images, uint32_t B, bool summed)
 {
-    if (ctx->orbit) return run_orbit(ctx, dev_images, B);
+    if (ctx->orbit && !summed) return run_orbit(ctx, dev_images, B);
     if (ctx->mfma_sym) {
         TRY(run_rotpack_sym(ctx, dev_images, B));
         TRY(run_dist_sym(ctx, B));
@@ -4422,6 +4443,8 @@ int distance_group(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
     TRY(run_dist(ctx, 0, B));
     return PINK_HIP_OK;
 }
+
+int distance_group(pink_hip_ctx *ctx, const float *dev_images, uint32_t B) { return distance_group(ctx, dev_images, B, B <= ctx->sum_images); }
 
 // Training of images that are on the device, queued on the context's stream.
 int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
@@ -4895,12 +4918,12 @@ struct StaticPieces {
     size_t per_image() const { return key + Pb + nb + gPb + gnb + rot + rotT + orows + onb + osb + oeb + odump + ox; }
 };
 
-static StaticPieces static_pieces(const pink_hip_ctx *ctx)
+static StaticPieces static_pieces(const pink_hip_ctx *ctx, bool summed)
 {
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     StaticPieces p;
     p.key = up((size_t)ctx->N * sizeof(unsigned long long));
-    if (ctx->orbit) {
+    if (ctx->orbit && !summed) {
         p.orows = up(orbit_rows_bytes(ctx, 1));
         p.onb = up((size_t)ctx->nrr_eff * 64);
         if (!is_int(ctx)) {
@@ -4940,8 +4963,8 @@ int pink_hip_map_device_static(pink_hip_ctx *ctx, const float *dev_images, uint3
     if (ctx->profiling)
         return fail(ctx, PINK_HIP_ESTATE, "pink_hip_map_device_static: per-kernel timing creates events; switch it off");
     if (!ctx->static_scratch) return fail(ctx, PINK_HIP_ESTATE, "pink_hip_map_device_static: no static scratch on this device");
-    const StaticPieces pc = static_pieces(ctx);
-    const size_t per_image = pc.per_image();
+    StaticPieces pc = static_pieces(ctx, false);
+    size_t per_image = pc.per_image();
     // (the float distance kernel of small problems reads up to kDistOverrun floats past the last row of its
     // operand, the piece carved last)
     const size_t capacity = PINK_HIP_STATIC_SCRATCH_BYTES - kDistOverrun * sizeof(float);
@@ -4950,6 +4973,10 @@ int pink_hip_map_device_static(pink_hip_ctx *ctx, const float *dev_images, uint3
                                           " bytes of scratch, the static scratch holds " + std::to_string(capacity));
     if (n_images == 0) return PINK_HIP_OK;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
+    // (few images of a float32 mapper: every variant summed where the scratch holds their rows)
+    const StaticPieces sums = static_pieces(ctx, true);
+    const bool summed = n_images <= ctx->sum_images && (size_t)n_images * sums.per_image() <= capacity;
+    if (summed) { pc = sums; per_image = pc.per_image(); }
     const uint32_t B = (uint32_t)std::min<size_t>({(size_t)ctx->Bcap, capacity / per_image, (size_t)n_images});
 
     // the scratch keeps what the last call (of any context on this GPU) left: rows beyond the last variant
@@ -4983,7 +5010,7 @@ int pink_hip_map_device_static(pink_hip_ctx *ctx, const float *dev_images, uint3
     int rc = PINK_HIP_OK;
     for (uint32_t done = 0; done < n_images && rc == PINK_HIP_OK; done += B) {
         const uint32_t b = std::min(B, n_images - done);
-        rc = distance_group(ctx, dev_images + (size_t)done * ctx->isz, b);
+        rc = distance_group(ctx, dev_images + (size_t)done * ctx->isz, b, summed);
         if (rc == PINK_HIP_OK)
             rc = run_finalize(ctx, b, dev_heatmap_out + (size_t)done * ctx->N, nullptr,
                               dev_best_rot_out ? dev_best_rot_out + (size_t)done * ctx->N : nullptr, true);

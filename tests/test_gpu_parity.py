@@ -397,7 +397,8 @@ ORBIT_MAP_SHAPES = [
 @pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,shape_,ed_type,n,data", ORBIT_MAP_SHAPES)
 def test_map_with_orbit_rows(N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, data):
     """Mappers whose rows are base rotations in the order of the symmetries' orbits; float32 distances are screened on rounded
-    values first, the variants that can be a neuron's closest are then summed exactly."""
+    values first, the variants that can be a neuron's closest are then summed exactly.  A call with few float32 images sums every
+    variant instead: the images come often enough here that the call screens them, and a single one that is summed."""
     say("orbit mapper", N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, data)
     rng = np.random.default_rng(N * 7 + I + nrot)
     imgs, som = rng.random((n, C_, I, I), dtype=np.float32), rng.random((N, C_ * D * D), dtype=np.float32)
@@ -417,9 +418,15 @@ def test_map_with_orbit_rows(N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, da
     want_heat, want_best = O.map_images(s, som, imgs)
     with capi.Context(N, C_, I, D, nrot, flip, ed, shape_, ed_type) as ctx:
         ctx.set_som(som)
-        heat, best = ctx.map(imgs)
+        times = 1
+        if ed_type == capi.FLOAT:
+            variant_elements = nrot * (2 if flip else 1) * ctx.region_size
+            times += int((9.0 + 0.021 * ctx.region_size) / (1.7e-6 * variant_elements)) // n
+        heat, best = ctx.map(np.tile(imgs, (times, 1, 1, 1)))
         one_heat, one_best = ctx.map(imgs[-1:])
-    assert np.array_equal(best, want_best) and np.array_equal(bits(heat), bits(want_heat))
+    for t in range(times):
+        part = slice(t * n, (t + 1) * n)
+        assert np.array_equal(best[part], want_best) and np.array_equal(bits(heat[part]), bits(want_heat)), t
     assert np.array_equal(one_best, want_best[-1:]) and np.array_equal(bits(one_heat), bits(want_heat[-1:]))
 
 

@@ -73,6 +73,8 @@ SHAPES = [
     (70, 1, 40, 29, 16, True, 21, capi.CIRCULAR, capi.UINT16, capi.KERNEL_AUTO, 19),         # GEMM, two byte planes
     (9, 2, 17, 24, 8, True, 13, capi.QUADRATIC, capi.UINT8, capi.KERNEL_VALU, 11),           # float variants + a packing kernel
     (50, 1, 64, 44, 360, True, 32, capi.QUADRATIC, capi.FLOAT, capi.KERNEL_AUTO, 13),        # float32 rows out of the rotation kernel
+    (50, 1, 64, 44, 360, True, 32, capi.QUADRATIC, capi.FLOAT, capi.KERNEL_AUTO, 61),        # ... so many images that distances are screened
+    (8, 1, 290, 205, 128, True, 21, capi.QUADRATIC, capi.FLOAT, capi.KERNEL_AUTO, 3),        # few images, neurons beyond the LDS
     (5, 1, 290, 205, 8, True, 40, capi.CIRCULAR, capi.FLOAT, capi.KERNEL_AUTO, 3),           # nothing in LDS: two stored symmetries + packing kernels
 ]
 
