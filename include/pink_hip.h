@@ -146,15 +146,20 @@ int pink_hip_train(pink_hip_ctx *ctx, const float *host_images, uint32_t n_image
  * best match, over all images this context has trained, counted on the device. */
 int pink_hip_update_counts(pink_hip_ctx *ctx, uint32_t *host_counts_out);
 /* Same with the images already on the device and the BMUs left on the device;
- * asynchronous on the context's stream (see pink_hip_synchronize).  A small uint8 trainer
- * (at most 64 neurons, 32 variants, 2048 elements per neuron) trains a launch group of up
- * to 256 images in ONE launch whose blocks stay on the device and exchange one word per
- * image; the host waits for the call's launches and learns from them whether every block saw
- * the others in time (they do unless other work keeps the device's compute units busy for
- * seconds).  If not, the launches behind the one that gave up changed nothing, their groups are trained again with
- * one launch per image, and the context stays with that form.  The environment variable
- * PINK_HIP_RESIDENT_TRAINER=0, read when a context is created, selects the one launch per
- * image from the start. */
+ * asynchronous on the context's stream (see pink_hip_synchronize), but for the first kind of
+ * trainer below.  Integer trainers train a launch group of images in ONE launch whose blocks stay
+ * on the device and exchange one word per image, every wait bounded: they need all their blocks
+ * on the device at once, which other work there may keep from them.
+ *   - uint8, at most 64 neurons, 32 variants, 2048 elements per neuron, groups of up to 256
+ *     images: the host waits for the call's launches and learns from them whether a block gave
+ *     up waiting.  Then the launches behind it have changed nothing, their groups are trained
+ *     again with one launch per image, and the context stays with that form.
+ *   - uint8 and uint16, up to 1024 neurons whose operand fits the compute units' LDS: queued.  A
+ *     launch behind each does its group over, without that need, if a block gave up; the calls
+ *     that follow take a launch per image and kernel for some 256 images (four times as many
+ *     each time it happens), then the resident form is tried again.
+ * The environment variable PINK_HIP_RESIDENT_TRAINER=0, read when a context is created, selects
+ * the other forms from the start. */
 int pink_hip_train_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out);
 
 /* Mapper<...,true>::operator()(Data const&) (Mapper.h:181-208) for n_images images:

@@ -2091,13 +2091,19 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
 #include "orbit_gemm.inc"
 
 // m_update_info[bmu]++ for the images of a group (Trainer.h:302-303), behind a resident launch: nothing when that launch
-// or one before it gave up.  The error word goes to the host with it, which looks when it next waits for the stream.
+// or one before it gave up and nobody rescued it.  The error word goes to the host with it, which looks when it next comes by.
+// rescue: k_sym_rescue's ticket and, behind it, its counts per image, for the next one.
 __global__ __launch_bounds__(256) void k_count_best_matches(const uint32_t *__restrict__ bmu, uint32_t images, uint32_t *__restrict__ counts,
-                                                            const uint32_t *__restrict__ error, uint32_t *__restrict__ host_error)
+                                                            const uint32_t *__restrict__ error, uint32_t *__restrict__ host_error,
+                                                            uint32_t *__restrict__ rescue)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, e = *error;
     if (t == 0) *host_error = e;
-    if (t < images && e == 0) atomicAdd(&counts[bmu[t]], 1u);
+    if (t < images && (e == 0 || rescue)) atomicAdd(&counts[bmu[t]], 1u);
+    if (rescue && e) {
+        if (t < images) rescue[1 + t] = 0;
+        if (t == 0) rescue[0] = 0;
+    }
 }
 
 // Decode keys: distance (optionally square-rooted for the mapper, Mapper.h:206), exact
@@ -2366,7 +2372,11 @@ struct pink_hip_ctx {
     std::vector<ResidentGroup> resident_queued;   // groups whose resident launches the host has not checked yet
     // integer trainers with the symmetries on the SOM side, resident over a launch group (k_train_sym_resident); the GEMM
     // path's operands are then made when something else wants them
-    bool sym_train = false;
+    bool sym_form = false, sym_train = false;              // the context can; it does at present
+    uint32_t sym_launch = 0, sym_seen = 0;                 // the last resident launch queued; the last one before the slots were cleared
+    uint64_t sym_pause = 0, sym_pause_next = 256;          // images to train the other way after a launch gave up; ... the next time
+    uint32_t *d_sym_rescue = nullptr;
+    unsigned long long *d_sym_keys = nullptr;
     uint32_t sym_npb = 1, sym_nit = 0, sym_B = 0, sym_KS = 0, sym_RT = 0, sym_all = 0, sym_cells = 0, sym_outside = 0, sym_tag0 = 1;
     size_t sym_lds = 0, sym_prep_lds = 0;
     uint32_t *d_sym_upos = nullptr, *d_sym_outside = nullptr, *d_sym_best = nullptr;
@@ -2998,10 +3008,11 @@ void swap_resident(pink_hip_ctx *ctx)
 
 int resident_launched(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, uint32_t *dev_bmu)
 {
+    const bool rescued = ctx->sym_train;
     hipLaunchKernelGGL(k_count_best_matches, dim3((images + 255) / 256), dim3(256), 0, ctx->stream, dev_bmu, images, ctx->d_counts,
-                       ctx->d_resident_error, ctx->h_resident_error);
+                       ctx->d_resident_error, ctx->h_resident_error, rescued ? ctx->d_sym_rescue : nullptr);
     TRY(launch_check(ctx, "k_count_best_matches"));
-    ctx->resident_queued.push_back({dev_images, images, dev_bmu});
+    if (!rescued) ctx->resident_queued.push_back({dev_images, images, dev_bmu});
     swap_resident(ctx);
     return PINK_HIP_OK;
 }
@@ -3094,23 +3105,30 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
     }
     {
         Timed t(ctx, kClsUpdate);
-        SymTrain a{};
+        SymRescue rescue{};
+        SymTrain &a = rescue.t;
         a.som = ctx->d_som; a.som_next = ctx->d_som_alt; a.opnd = ctx->d_sym_op; a.xrows = ctx->d_sym_x; a.norm = ctx->d_sym_norm;
         a.factors_t = ctx->d_factors_t; a.cell_elem = ctx->d_sym_elem; a.cell_at = ctx->d_sym_at; a.best_variant = ctx->d_sym_best;
         a.bmu_out = dev_bmu; a.slots = ctx->d_slots; a.error = ctx->d_resident_error;
-        a.launch = (uint32_t)ctx->resident_queued.size() + 1;
+        a.launch = ++ctx->sym_launch;
         a.N = ctx->N; a.S = ctx->S; a.cells = ctx->sym_cells; a.KS = ctx->sym_KS; a.RT = ctx->sym_RT; a.nrr = ctx->nrr_eff;
         a.num_rot = ctx->cfg.num_rot; a.use_flip = ctx->cfg.use_flip; a.images = images; a.tag0 = ctx->sym_tag0; a.spin_limit = ctx->spin_limit;
         ctx->sym_tag0 = sym_tag(ctx->sym_tag0, images);
         void *args[] = {&a};
         HIP_TRY(ctx, hipLaunchKernel(sym_kernel(ctx), dim3((ctx->N + ctx->sym_npb - 1) / ctx->sym_npb), dim3(kSymThreads), args, ctx->sym_lds, ctx->stream));
+        rescue.keys = ctx->d_sym_keys; rescue.ticket = ctx->d_sym_rescue; rescue.done = ctx->d_sym_rescue + 1;
+        const dim3 grid(std::min(ctx->N, 2 * (uint32_t)ctx->num_cu));
+        const size_t lds = (size_t)ctx->sym_cells * sizeof(uint2);
+        if (ctx->cfg.ed_type == PINK_HIP_UINT16) hipLaunchKernelGGL(k_sym_rescue<true>, grid, dim3(512), lds, ctx->stream, rescue);
+        else hipLaunchKernelGGL(k_sym_rescue<false>, grid, dim3(512), lds, ctx->stream, rescue);
+        TRY(launch_check(ctx, "k_sym_rescue"));
     }
     if (ctx->sym_outside) {
         Timed t(ctx, kClsUpdate);
         SymOutside o{};
         o.som = ctx->d_som; o.som_next = ctx->d_som_alt; o.images = dev_images; o.cos_t = ctx->d_cos; o.sin_t = ctx->d_sin;
         o.factors = ctx->d_factors; o.best_variant = ctx->d_sym_best; o.bmu = dev_bmu; o.outside = ctx->d_sym_outside;
-        o.error = ctx->d_resident_error; o.count = ctx->sym_outside; o.N = ctx->N; o.S = ctx->S; o.C = ctx->C; o.I = ctx->I;
+        o.count = ctx->sym_outside; o.N = ctx->N; o.S = ctx->S; o.C = ctx->C; o.I = ctx->I;
         o.D = ctx->D; o.nrr = ctx->nrr_eff; o.num_rot = ctx->cfg.num_rot; o.images_n = images;
         hipLaunchKernelGGL(k_sym_outside, dim3((ctx->sym_outside + 255) / 256, ctx->N), dim3(256), 0, ctx->stream, o);
         TRY(launch_check(ctx, "k_sym_outside"));
@@ -3120,8 +3138,8 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
 
 int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out);
 
-// Wait for the queued resident launches.  If one gave up, nothing after it has run: back to the buffers it started from,
-// its group and the later ones image by image, and the context stays with that form.
+// Wait for the queued resident launches of a small uint8 trainer.  If one gave up, nothing after it has run: back to the buffers it
+// started from, its group and the later ones image by image, and the context stays with that form.
 int finish_resident(pink_hip_ctx *ctx)
 {
     if (ctx->resident_queued.empty()) return PINK_HIP_OK;
@@ -3132,10 +3150,34 @@ int finish_resident(pink_hip_ctx *ctx)
     const uint32_t failed = *ctx->h_resident_error;
     if (!failed) return PINK_HIP_OK;
     if ((queued.size() - (failed - 1)) & 1) swap_resident(ctx);
-    if (ctx->sym_train) TRY(run_pack_som(ctx));            // the other path's operand of the SOM as it is now
-    ctx->resident_train = ctx->sym_train = false;
+    ctx->resident_train = false;
     HIP_TRY(ctx, hipMemsetAsync(ctx->d_resident_error, 0, sizeof(uint32_t), ctx->stream));
     for (size_t g = failed - 1; g < queued.size(); ++g) TRY(train_queued(ctx, queued[g].images, queued[g].count, queued[g].bmu));
+    return PINK_HIP_OK;
+}
+
+// Whether an integer trainer that can be resident is: after a launch gave up (k_sym_rescue has done its group and those queued
+// behind it) the next images go through the other form, then it is tried again.  The host's copy of the error word says so some
+// time after; a launch that failed before the slots were cleared is not counted twice.
+int choose_sym_form(pink_hip_ctx *ctx, uint32_t n_images)
+{
+    if (!ctx->sym_form) return PINK_HIP_OK;
+    const uint32_t failed = *(const volatile uint32_t *)ctx->h_resident_error;
+    if (ctx->sym_train && failed && (int32_t)(failed - ctx->sym_seen) > 0) {
+        ctx->sym_seen = ctx->sym_launch;
+        const size_t slots = (size_t)ctx->N * kSymStride;              // (16-byte words of both sets)
+        hipLaunchKernelGGL(k_fill_zero, dim3((uint32_t)((slots + 255) / 256)), dim3(256), 0, ctx->stream, (v4i *)ctx->d_slots, slots);
+        hipLaunchKernelGGL(k_fill_zero, dim3(1), dim3(256), 0, ctx->stream, (v4i *)ctx->d_resident_error, (size_t)1);
+        TRY(launch_check(ctx, "k_fill_zero"));
+        TRY(run_pack_som(ctx));                            // the other form's operand of the SOM as it is now
+        ctx->sym_train = false;
+        ctx->sym_pause = ctx->sym_pause_next;
+        ctx->sym_pause_next = std::min<uint64_t>(4 * ctx->sym_pause_next, 1u << 20);
+    }
+    if (!ctx->sym_train) {
+        if (ctx->sym_pause == 0) ctx->sym_train = true;
+        else ctx->sym_pause -= std::min<uint64_t>(ctx->sym_pause, n_images);
+    }
     return PINK_HIP_OK;
 }
 
@@ -3164,7 +3206,7 @@ int free_all(pink_hip_ctx *ctx)
                     ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4,
                     ctx->d_orb_tables, ctx->d_orb_outside, ctx->d_orb_best, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
                     ctx->d_orb_sa, ctx->d_orb_ea, ctx->d_orb_sb, ctx->d_orb_eb, ctx->d_orb_dump,
-                    ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts};
+                    ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts, ctx->d_sym_keys, ctx->d_sym_rescue};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu}) if (p) (void)hipFree(p);
     if (ctx->st_pin) (void)hipHostFree(ctx->st_pin);
@@ -3220,12 +3262,13 @@ int init_exchange(pink_hip_ctx *ctx, size_t slot_words)
     TRY(dev_alloc(ctx, &ctx->d_som_alt, (size_t)ctx->N * ctx->S));
     TRY(dev_alloc(ctx, &ctx->d_slots, slot_words));
     HIP_TRY(ctx, hipMemset(ctx->d_slots, 0, slot_words * sizeof(unsigned long long)));
-    TRY(dev_alloc(ctx, &ctx->d_resident_error, 1));
-    HIP_TRY(ctx, hipMemset(ctx->d_resident_error, 0, sizeof(uint32_t)));
+    TRY(dev_alloc(ctx, &ctx->d_resident_error, 4));
+    HIP_TRY(ctx, hipMemset(ctx->d_resident_error, 0, 4 * sizeof(uint32_t)));
     if (hipHostMalloc((void **)&ctx->h_resident_error, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
         ctx->h_resident_error = nullptr;
         return fail(ctx, PINK_HIP_ENOMEM, "pinned host allocation failed");
     }
+    *ctx->h_resident_error = 0;
     return PINK_HIP_OK;
 }
 
@@ -3396,7 +3439,10 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     TRY(dev_alloc(ctx, &ctx->d_sym_best, b * ctx->N));
     TRY(init_exchange(ctx, (size_t)2 * ctx->N * kSymStride));
     ctx->sym_tag0 = (ctx->exchange_tag - 1) % 0xfffeu + 1;
-    ctx->sym_train = true;
+    TRY(dev_alloc(ctx, &ctx->d_sym_keys, b * ctx->N));
+    TRY(dev_alloc(ctx, &ctx->d_sym_rescue, b + 1));
+    HIP_TRY(ctx, hipMemset(ctx->d_sym_rescue, 0, (b + 1) * sizeof(uint32_t)));
+    ctx->sym_form = ctx->sym_train = true;
     // (limits are per kernel, not per context)
     HIP_TRY(ctx, hipFuncSetAttribute(sym_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
     if (ctx->sym_prep_lds) HIP_TRY(ctx, hipFuncSetAttribute(sym_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
@@ -4450,6 +4496,7 @@ int distance_group(pink_hip_ctx *ctx, const float *dev_images, uint32_t B) { ret
 int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
 {
     if (ctx->orbit_train) return run_orbit_train(ctx, dev_images, n_images, dev_bmu_out);
+    TRY(choose_sym_form(ctx, n_images));
     if (ctx->sym_train) {
         for (uint32_t done = 0; done < n_images; done += ctx->sym_B) {
             const uint32_t B = std::min(ctx->sym_B, n_images - done);

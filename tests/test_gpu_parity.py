@@ -646,7 +646,8 @@ RESIDENT_SYMMETRIC_SHAPES = [
 @pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,shape_,ed_type,n", RESIDENT_SYMMETRIC_SHAPES)
 def test_resident_symmetric_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, form):
     """Integer trainers keep their neurons' eight symmetric operand rows on the device over a launch group (see
-    test_small_uint8_trainer_forms for the exchange between the blocks and what happens when one gives up)."""
+    test_small_uint8_trainer_forms for the exchange between the blocks).  What a launch that gives up leaves undone, and the groups
+    queued behind it, the launch that follows it trains; the next call takes the other form."""
     say("resident symmetric trainer", form, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n)
     if form == "gives up":
         monkeypatch.setenv("PINK_HIP_RESIDENT_SPIN_LIMIT", "0")
@@ -660,10 +661,12 @@ def test_resident_symmetric_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, 
     s = O.shape(N, C_, I, D, nrot, flip, ed, shape_, ed_type)
     want = som0.copy()
     obmu = O.train(s, want, imgs, F)
-    for max_batch in (0, 2):
+    for max_batch, first in ((0, 1), (2, 1), (1, n)):
         with capi.Context(N, C_, I, D, nrot, flip, ed, shape_, ed_type, F, max_batch=max_batch) as ctx:
             ctx.set_som(som0)
-            bmu = np.concatenate([ctx.train(imgs[:1]), ctx.train(imgs[1:])])
+            bmu = ctx.train(imgs[:first])
+            if first < n:
+                bmu = np.concatenate([bmu, ctx.train(imgs[first:])])
             som = ctx.get_som()
             counts = ctx.update_counts()
             d1, ssd1, best1 = ctx.distance(imgs[0])
@@ -673,6 +676,46 @@ def test_resident_symmetric_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, 
         assert np.array_equal(bits(som), bits(want)), max_batch
         assert np.array_equal(counts, np.bincount(obmu, minlength=N)), max_batch
         assert np.array_equal(bits(d1), bits(d2)) and np.array_equal(ssd1, ssd2) and np.array_equal(best1, best2)
+
+
+def test_resident_symmetric_trainer_tries_again(monkeypatch):
+    """After a launch that gave up, the trainer takes the other form for some 256 images and is then resident again."""
+    monkeypatch.setenv("PINK_HIP_RESIDENT_SPIN_LIMIT", "0")
+    N, C_, I, D, nrot, ed, ed_type = 6, 2, 18, 12, 132, 8, capi.UINT8
+    rng = np.random.default_rng(8)
+    som0 = rng.random((N, C_ * D * D), dtype=np.float32)
+    imgs = rng.random((320, C_, I, I), dtype=np.float32)
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 1.0, 0.5)
+    want = som0.copy()
+    obmu = O.train(O.shape(N, C_, I, D, nrot, True, ed, capi.QUADRATIC, ed_type), want, imgs, F)
+    with capi.Context(N, C_, I, D, nrot, True, ed, capi.QUADRATIC, ed_type, F) as ctx:
+        ctx.set_som(som0)
+        # gives up; the other form, for as many images as the pause lasts; resident and gives up; the other form
+        bmu = np.concatenate([ctx.train(imgs[a:b]) for a, b in ((0, 5), (5, 265), (265, 270), (270, 320))])
+        som, counts = ctx.get_som(), ctx.update_counts()
+    assert np.array_equal(bmu, obmu) and np.array_equal(bits(som), bits(want)) and np.array_equal(counts, np.bincount(obmu, minlength=N))
+
+
+def test_resident_symmetric_training_is_queued():
+    """pink_hip_train_device returns while the device still trains (uint8, the command line's sizes for 64-pixel images)."""
+    import time
+    from test_zz_no_alloc import Hip
+    N, I, D, ed, n = 100, 64, 91, 45, 3000
+    F = capi.make_update_factors(capi.CARTESIAN, [10, 10], capi.GAUSSIAN, 1.1, 0.2)
+    hip = Hip()
+    imgs, bmu = hip.upload(np.random.default_rng(4).random((n, 1, I, I), dtype=np.float32)), hip.alloc(4 * n)
+    with capi.Context(N, 1, I, D, 360, True, ed, capi.QUADRATIC, capi.UINT8, F) as ctx:
+        ctx.set_som(np.zeros((N, D * D), np.float32))
+        ctx.train_device(imgs, 100, bmu)
+        ctx.synchronize()
+        start = time.perf_counter()
+        ctx.train_device(imgs, n, bmu)
+        queued = time.perf_counter() - start
+        ctx.synchronize()
+        whole = time.perf_counter() - start
+    hip.release()
+    say("queued after", queued, "of", whole)
+    assert queued < 0.5 * whole
 
 
 ORBIT_TRAIN_SHAPES = [
