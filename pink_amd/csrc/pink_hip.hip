@@ -41,6 +41,7 @@
 
 #include "mfma_u8_sym.h"
 #include "pink_hip.h"
+#include "resident_use.h"
 
 // Scratch of pink_hip_map_device_static, the entry point for callers that cannot allocate: the
 // per-group buffers of a mapping call (argmin keys, the packed variant operand, variant norms, float
@@ -2272,6 +2273,18 @@ HostStaging *take_staging(std::unique_lock<std::mutex> &lock)
     return g_staging.get();
 }
 
+// Resident launches in flight, per device: their blocks wait for each other, so launches of several contexts that only fit the
+// device in part would stop each other until their polls run out (seconds).  A launch is queued behind as many of the others as
+// it takes for all blocks that may run at once to have a place (resident_waits); each context has one launch running at a time
+// (its stream).  Other processes on the device are not seen: what they keep apart gives up and is done over.
+struct ResidentUse : ResidentShape {
+    const void *owner;
+    hipEvent_t done;            // recorded behind the owner's last launch
+};
+constexpr int kMaxDevices = 64;
+std::mutex g_resident_mutex;
+std::vector<ResidentUse> g_resident[kMaxDevices];         // in the order of the launches
+
 constexpr size_t kRotateLdsMax = 158 * 1024;
 enum : uint32_t { kStoreNone = 0, kStoreAll = 1, kStorePair = 2 };
 
@@ -2368,6 +2381,8 @@ struct pink_hip_ctx {
     unsigned long long *d_slots = nullptr;
     uint32_t *d_resident_error = nullptr, *h_resident_error = nullptr;
     uint32_t exchange_tag = 1, spin_limit = 1u << 21;
+    uint32_t resident_per_unit = 1;        // blocks of its resident kernel that a compute unit holds
+    hipEvent_t resident_done = nullptr;
     struct ResidentGroup { const float *images; uint32_t count; uint32_t *bmu; };
     std::vector<ResidentGroup> resident_queued;   // groups whose resident launches the host has not checked yet
     // integer trainers with the symmetries on the SOM side, resident over a launch group (k_train_sym_resident); the GEMM
@@ -2997,6 +3012,23 @@ int run_train_small(pink_hip_ctx *ctx, uint32_t slot, uint32_t *dev_bmu_out)
     return launch_check(ctx, "k_train_small_u8");
 }
 
+// A resident launch of `blocks`, behind what it has to be behind (see ResidentUse).
+template <typename Launch>
+int launch_resident(pink_hip_ctx *ctx, uint32_t blocks, Launch launch)
+{
+    std::lock_guard<std::mutex> lock(g_resident_mutex);
+    std::vector<ResidentUse> &uses = g_resident[ctx->device];
+    uses.erase(std::remove_if(uses.begin(), uses.end(), [&](const ResidentUse &u) { return u.owner == ctx || hipEventQuery(u.done) == hipSuccess; }), uses.end());
+    (void)hipGetLastError();                              // (a launch that still runs is no error)
+    const ResidentShape mine{blocks, ctx->resident_per_unit};
+    const size_t waits = resident_waits(uses, uses.size(), mine, (uint32_t)ctx->num_cu);
+    for (size_t i = 0; i < waits; ++i) HIP_TRY(ctx, hipStreamWaitEvent(ctx->stream, uses[i].done, 0));
+    TRY(launch());
+    HIP_TRY(ctx, hipEventRecord(ctx->resident_done, ctx->stream));
+    uses.push_back({mine, ctx, ctx->resident_done});
+    return PINK_HIP_OK;
+}
+
 // The two sets of buffers between which resident launches alternate.
 void swap_resident(pink_hip_ctx *ctx)
 {
@@ -3015,6 +3047,14 @@ int resident_launched(pink_hip_ctx *ctx, const float *dev_images, uint32_t image
     if (!rescued) ctx->resident_queued.push_back({dev_images, images, dev_bmu});
     swap_resident(ctx);
     return PINK_HIP_OK;
+}
+
+// (elements of a neuron per thread, k-steps per wave in one batch, variant elements per thread in registers)
+decltype(&k_train_small_u8_resident<2, 4, 4>) small_resident_kernel(const pink_hip_ctx *ctx)
+{
+    const uint32_t nstored = std::min(2 * std::max(ctx->nrr, 1u), ctx->R);
+    if (ctx->S <= 1024 && (size_t)nstored * ctx->S <= 4 * kResidentThreads) return k_train_small_u8_resident<2, 4, 4>;
+    return ctx->S <= 1024 ? k_train_small_u8_resident<2, 4, 8> : k_train_small_u8_resident<4, 8, 8>;
 }
 
 // The first `images` images of the current group in one resident launch (small uint8 trainers), queued: whether every
@@ -3048,16 +3088,11 @@ int run_train_small_resident(pink_hip_ctx *ctx, const float *dev_images, uint32_
     const size_t lds = (size_t)2 * a.nstored * ctx->S * sizeof(float);
     {
         Timed t(ctx, kClsUpdate);
-#define LAUNCH_RESIDENT(...)                                                                                          \
-    hipLaunchKernelGGL((k_train_small_u8_resident<__VA_ARGS__>), dim3(ctx->N), dim3(kResidentThreads), lds, ctx->stream, ctx->d_som, \
-                       ctx->d_som_alt, ctx->d_rot, pa, pa_next, ctx->d_gPb, ctx->d_factors, ctx->d_src4, ctx->d_kbyte, a)
-        // (elements of a neuron per thread, k-steps per wave in one batch, variant elements per thread in registers)
-        const bool few_variant_elements = (size_t)a.nstored * ctx->S <= 4 * kResidentThreads;
-        if (ctx->S <= 1024 && few_variant_elements) LAUNCH_RESIDENT(2, 4, 4);
-        else if (ctx->S <= 1024) LAUNCH_RESIDENT(2, 4, 8);
-        else LAUNCH_RESIDENT(4, 8, 8);
-#undef LAUNCH_RESIDENT
-        TRY(launch_check(ctx, "k_train_small_u8_resident"));
+        TRY(launch_resident(ctx, ctx->N, [&] {
+            hipLaunchKernelGGL(small_resident_kernel(ctx), dim3(ctx->N), dim3(kResidentThreads), lds, ctx->stream, ctx->d_som,
+                               ctx->d_som_alt, ctx->d_rot, pa, pa_next, ctx->d_gPb, ctx->d_factors, ctx->d_src4, ctx->d_kbyte, a);
+            return launch_check(ctx, "k_train_small_u8_resident");
+        }));
     }
     return resident_launched(ctx, dev_images, images, dev_bmu);
 }
@@ -3115,7 +3150,11 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         a.num_rot = ctx->cfg.num_rot; a.use_flip = ctx->cfg.use_flip; a.images = images; a.tag0 = ctx->sym_tag0; a.spin_limit = ctx->spin_limit;
         ctx->sym_tag0 = sym_tag(ctx->sym_tag0, images);
         void *args[] = {&a};
-        HIP_TRY(ctx, hipLaunchKernel(sym_kernel(ctx), dim3((ctx->N + ctx->sym_npb - 1) / ctx->sym_npb), dim3(kSymThreads), args, ctx->sym_lds, ctx->stream));
+        const uint32_t blocks = (ctx->N + ctx->sym_npb - 1) / ctx->sym_npb;
+        TRY(launch_resident(ctx, blocks, [&] {
+            HIP_TRY(ctx, hipLaunchKernel(sym_kernel(ctx), dim3(blocks), dim3(kSymThreads), args, ctx->sym_lds, ctx->stream));
+            return (int)PINK_HIP_OK;
+        }));
         rescue.keys = ctx->d_sym_keys; rescue.ticket = ctx->d_sym_rescue; rescue.done = ctx->d_sym_rescue + 1;
         const dim3 grid(std::min(ctx->N, 2 * (uint32_t)ctx->num_cu));
         const size_t lds = (size_t)ctx->sym_cells * sizeof(uint2);
@@ -3219,6 +3258,14 @@ int free_all(pink_hip_ctx *ctx)
     for (hipEvent_t e : ctx->copy_ev) if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : ctx->piece_ev) if (e) (void)hipEventDestroy(e);
     if (ctx->staging_user) staging_drop_user();
+    if (ctx->resident_done) {
+        {
+            std::lock_guard<std::mutex> lock(g_resident_mutex);
+            std::vector<ResidentUse> &uses = g_resident[ctx->device];
+            uses.erase(std::remove_if(uses.begin(), uses.end(), [&](const ResidentUse &u) { return u.owner == ctx; }), uses.end());
+        }
+        (void)hipEventDestroy(ctx->resident_done);
+    }
     if (ctx->copy_stream) (void)hipStreamDestroy(ctx->copy_stream);
     if (ctx->d_counts) (void)hipFree(ctx->d_counts);
     for (void *p : {(void *)ctx->d_fPa, (void *)ctx->d_fPb, (void *)ctx->d_fna, (void *)ctx->d_fnb, (void *)ctx->d_fpart})
@@ -3228,7 +3275,6 @@ int free_all(pink_hip_ctx *ctx)
 }
 
 // The address of the file-scope scratch array on the current device, asked for once per device.
-constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mutex;
 unsigned char *g_scratch_ptr[kMaxDevices] = {};
 
@@ -3253,8 +3299,12 @@ bool resident_allowed()
 }
 
 // What the blocks of a resident trainer exchange their words through, and the second weight array.
-int init_exchange(pink_hip_ctx *ctx, size_t slot_words)
+int init_exchange(pink_hip_ctx *ctx, size_t slot_words, const void *kernel, uint32_t threads, size_t lds)
 {
+    int per_unit = 0;
+    HIP_TRY(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_unit, kernel, (int)threads, lds));
+    ctx->resident_per_unit = (uint32_t)std::max(1, per_unit);
+    HIP_TRY(ctx, hipEventCreateWithFlags(&ctx->resident_done, hipEventDisableTiming));
     // (a test can make every wait give up at once, to see the group trained again image by image)
     if (const char *limit = getenv("PINK_HIP_RESIDENT_SPIN_LIMIT")) ctx->spin_limit = (uint32_t)strtoul(limit, nullptr, 10);
     // (... or start the tags of the exchange just below the value where they wrap, which 2^32 images take)
@@ -3437,15 +3487,15 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     TRY(dev_alloc(ctx, &ctx->d_sym_x, b * ctx->nrr_eff * Kp));
     TRY(dev_alloc(ctx, &ctx->d_sym_norm, b * ctx->sym_RT * 16 * 8));
     TRY(dev_alloc(ctx, &ctx->d_sym_best, b * ctx->N));
-    TRY(init_exchange(ctx, (size_t)2 * ctx->N * kSymStride));
+    // (limits are per kernel, not per context)
+    HIP_TRY(ctx, hipFuncSetAttribute(sym_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
+    if (ctx->sym_prep_lds) HIP_TRY(ctx, hipFuncSetAttribute(sym_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
+    TRY(init_exchange(ctx, (size_t)2 * ctx->N * kSymStride, sym_kernel(ctx), kSymThreads, ctx->sym_lds));
     ctx->sym_tag0 = (ctx->exchange_tag - 1) % 0xfffeu + 1;
     TRY(dev_alloc(ctx, &ctx->d_sym_keys, b * ctx->N));
     TRY(dev_alloc(ctx, &ctx->d_sym_rescue, b + 1));
     HIP_TRY(ctx, hipMemset(ctx->d_sym_rescue, 0, (b + 1) * sizeof(uint32_t)));
     ctx->sym_form = ctx->sym_train = true;
-    // (limits are per kernel, not per context)
-    HIP_TRY(ctx, hipFuncSetAttribute(sym_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
-    if (ctx->sym_prep_lds) HIP_TRY(ctx, hipFuncSetAttribute(sym_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
     return PINK_HIP_OK;
 }
 
@@ -4367,10 +4417,8 @@ int init_ctx(pink_hip_ctx *ctx)
             // resident over a launch group: every block needs a compute unit of its own for the whole launch
             ctx->resident_train = ctx->N <= (uint32_t)ctx->num_cu && resident_allowed();
             if (ctx->resident_train) {
-                TRY(init_exchange(ctx, kSlotWords));
-                HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_train_small_u8_resident<2, 4, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
-                HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_train_small_u8_resident<2, 4, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
-                HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_train_small_u8_resident<4, 8, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
+                HIP_TRY(ctx, hipFuncSetAttribute((const void *)small_resident_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
+                TRY(init_exchange(ctx, kSlotWords, (const void *)small_resident_kernel(ctx), kResidentThreads, (size_t)2 * nstored * ctx->S * sizeof(float)));
             }
         }
         if (one_to_one && !ctx->small_train && !ctx->orbit_train) TRY(init_sym_train(ctx, region));

@@ -5,8 +5,10 @@
 // Usage: test_host args   -> argument validation only (no device needed)
 //        test_host gpu    -> everything
 #define PINK_HIP_STANDALONE
+#include "../../pink_amd/csrc/resident_use.h"
 #include "pink_hip_som.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -118,10 +120,38 @@ static void test_mapper()
     }
 }
 
+// Resident launches that may run at once have a place for every block, and none waits without need.
+static void test_resident_rule()
+{
+    auto fits = [](std::vector<ResidentShape> const& v, size_t first, ResidentShape mine, uint32_t units) {
+        uint32_t smallest = mine.per_unit, blocks = mine.blocks;
+        for (size_t i = first; i < v.size(); ++i) { blocks += v[i].blocks; smallest = std::min(smallest, v[i].per_unit); }
+        return blocks <= units * smallest;
+    };
+    using V = std::vector<ResidentShape>;
+    EXPECT(resident_waits(V{}, 0, {256, 1}, 256) == 0);
+    EXPECT(resident_waits(V{{166, 1}}, 1, {166, 1}, 256) == 1);
+    EXPECT(resident_waits(V{{100, 1}}, 1, {100, 1}, 256) == 0);
+    EXPECT(resident_waits(V(7, {64, 2}), 7, {64, 2}, 256) == 0);      // eight small trainers, two blocks a unit
+    EXPECT(resident_waits(V(8, {64, 2}), 8, {64, 2}, 256) == 1);
+    EXPECT(resident_waits(V{{64, 2}, {200, 1}}, 2, {64, 2}, 256) == 2);
+    uint32_t state = 1;
+    auto draw = [&](uint32_t n) { state = state * 1664525u + 1013904223u; return (state >> 8) % n; };
+    for (int round = 0; round < 2000; ++round) {
+        V in_flight(draw(9));
+        for (auto& s : in_flight) s = {1 + draw(256), 1 + draw(4)};
+        ResidentShape const mine{1 + draw(256), 1 + draw(4)};
+        size_t const waits = resident_waits(in_flight, in_flight.size(), mine, 256);
+        EXPECT(waits <= in_flight.size() and fits(in_flight, waits, mine, 256));
+        EXPECT(waits == 0 or not fits(in_flight, waits - 1, mine, 256));
+    }
+}
+
 int main(int argc, char** argv)
 {
     bool const gpu = argc > 1 and std::strcmp(argv[1], "gpu") == 0;
     test_arguments();
+    test_resident_rule();
     if (gpu) {
         test_trainer();
         test_mapper();

@@ -696,6 +696,33 @@ def test_resident_symmetric_trainer_tries_again(monkeypatch):
     assert np.array_equal(bmu, obmu) and np.array_equal(bits(som), bits(want)) and np.array_equal(counts, np.bincount(obmu, minlength=N))
 
 
+def test_resident_trainers_side_by_side():
+    """Resident trainers whose blocks do not fit the device together, a thread each: their launches take turns."""
+    import threading
+    N, I, D, nrot, ed, n, ed_type = 200, 40, 32, 36, 32, 90, capi.UINT16          # (200 of 256 compute units, twice)
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 1.0, 0.5)
+    work, got = [], {}
+    for k in range(3):
+        rng = np.random.default_rng(k)
+        som0, imgs = rng.random((N, D * D), dtype=np.float32), rng.random((n, 1, I, I), dtype=np.float32)
+        want = som0.copy()
+        work.append((som0, imgs, want, O.train(O.shape(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, ed_type), want, imgs, F)))
+
+    def train(k):
+        som0, imgs = work[k][:2]
+        with capi.Context(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, ed_type, F, max_batch=6) as ctx:
+            ctx.set_som(som0)
+            got[k] = (np.concatenate([ctx.train(imgs[i:i + 30]) for i in range(0, n, 30)]), ctx.get_som())
+
+    threads = [threading.Thread(target=train, args=(k,)) for k in range(len(work))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k, (_, _, want, bmu) in enumerate(work):
+        assert np.array_equal(got[k][0], bmu) and np.array_equal(bits(got[k][1]), bits(want)), k
+
+
 def test_resident_symmetric_training_is_queued():
     """pink_hip_train_device returns while the device still trains (uint8, the command line's sizes for 64-pixel images)."""
     import time
