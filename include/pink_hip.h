@@ -165,9 +165,9 @@ int pink_hip_train_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n
 /* Mapper<...,true>::operator()(Data const&) (Mapper.h:181-208) for n_images images:
  * heatmap_out[i*N + n] = sqrt(min over rotations of the distance), already square-rooted
  * (Mapper.h:206); best_rot_out[i*N + n] = index of that rotation (may be NULL).
- * A call that moves more than 1 MB of images or results (here and in pink_hip_get_som) shares 16 MB of pinned memory and
- * five helper threads with the other contexts of the process; they exist from the first such call until the last context
- * is destroyed. */
+ * A call that moves more than 1 MB of images or results (here and in pink_hip_get_som) takes 32 MB of pinned memory and
+ * five helper threads for its length; calls of up to four threads at once each have theirs, which all contexts of the
+ * process share from the first such call until the last context is destroyed. */
 int pink_hip_map(pink_hip_ctx *ctx, const float *host_images, uint32_t n_images,
                  float *host_heatmap_out, uint32_t *host_best_rot_out);
 int pink_hip_map_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images,

@@ -2217,61 +2217,78 @@ private:
     std::atomic<size_t> next_{0};
 };
 
-// The pinned pieces and the copy threads that large pageable transfers go through: one set for the process, made when
-// a transfer first wants it and given back with the last context.  A call holds it for the length of one transfer; a
-// second thread that wants it meanwhile takes the runtime's own pageable copy.
+// The pinned pieces and the copy threads that large pageable transfers go through: sets that the contexts of the process share, a
+// call holding one for the length of one transfer.  A set is made when a transfer finds none free, up to kStagingSets, and all are
+// given back with the last context.  A call beyond those takes the runtime's own pageable copy: the link is full by then.
 // (2 MB pieces: the link's 55 GB/s needs about half a MB; a piece is also what nothing overlaps at either end.)
 constexpr size_t kPieceBytes = (size_t)2 << 20;
 constexpr uint32_t kPieces = 16;
 constexpr unsigned kCopyWorkers = 5;                      // and the caller (measured: 6 threads move 115 GB/s, 14 into fresh pages)
+constexpr size_t kStagingSets = 4;
 struct HostStaging {
     HostCopyPool pool{kCopyWorkers};
     char *piece[kPieces] = {};
     char *base = nullptr;
+    bool taken = false;
 };
-std::mutex g_staging_users_mutex, g_staging_mutex;        // the count of contexts; the set itself (held over a transfer)
-unsigned g_staging_users = 0;
-std::unique_ptr<HostStaging> g_staging;
+std::mutex g_staging_mutex;
+unsigned g_staging_users = 0;                             // contexts
+std::vector<std::unique_ptr<HostStaging>> g_staging;
 
 void staging_add_user()
 {
-    std::lock_guard<std::mutex> lock(g_staging_users_mutex);
+    std::lock_guard<std::mutex> lock(g_staging_mutex);
     ++g_staging_users;
 }
 
 void staging_drop_user()
 {
-    std::lock_guard<std::mutex> users(g_staging_users_mutex);
-    if (--g_staging_users) return;
     std::lock_guard<std::mutex> lock(g_staging_mutex);
-    if (g_staging) (void)hipHostFree(g_staging->base);
-    g_staging.reset();
+    if (--g_staging_users) return;
+    for (auto &set : g_staging) (void)hipHostFree(set->base);          // (nobody holds one without a context)
+    g_staging.clear();
 }
 
-// The set, held by `lock` on return; null (and `lock` empty) when another thread has it or the host cannot give it.
-HostStaging *take_staging(std::unique_lock<std::mutex> &lock)
-{
-    lock = std::unique_lock<std::mutex>(g_staging_mutex, std::try_to_lock);
-    if (!lock.owns_lock()) return nullptr;
-    if (!g_staging) {
+// A set for one transfer; get() is null when there is none to be had.
+class StagingLease {
+public:
+    StagingLease() = default;
+    StagingLease(const StagingLease &) = delete;
+    StagingLease &operator=(const StagingLease &) = delete;
+    ~StagingLease()
+    {
+        if (!set_) return;
+        std::lock_guard<std::mutex> lock(g_staging_mutex);
+        set_->taken = false;
+    }
+    HostStaging *take()
+    {
+        std::lock_guard<std::mutex> lock(g_staging_mutex);
+        for (auto &set : g_staging)
+            if (!set->taken) { set_ = set.get(); set_->taken = true; return set_; }
+        if (g_staging.size() >= kStagingSets) return nullptr;
         void *base = nullptr;
         if (hipHostMalloc(&base, kPieces * kPieceBytes, hipHostMallocPortable) != hipSuccess) {
             (void)hipGetLastError();
-            lock.unlock();
             return nullptr;
         }
         try {
-            g_staging.reset(new HostStaging);
+            g_staging.reserve(kStagingSets);
+            g_staging.emplace_back(new HostStaging);
         } catch (...) {
             (void)hipHostFree(base);
-            lock.unlock();
             return nullptr;
         }
-        g_staging->base = (char *)base;
-        for (uint32_t i = 0; i < kPieces; ++i) g_staging->piece[i] = g_staging->base + i * kPieceBytes;
+        set_ = g_staging.back().get();
+        set_->base = (char *)base;
+        for (uint32_t i = 0; i < kPieces; ++i) set_->piece[i] = set_->base + i * kPieceBytes;
+        set_->taken = true;
+        return set_;
     }
-    return g_staging.get();
-}
+
+private:
+    HostStaging *set_ = nullptr;
+};
 
 // Resident launches in flight, per device: their blocks wait for each other, so launches of several contexts that only fit the
 // device in part would stop each other until their polls run out (seconds).  A launch is queued behind as many of the others as
@@ -4794,8 +4811,8 @@ static int copy_out(pink_hip_ctx *ctx, void *host, const void *dev, size_t bytes
         memcpy(host, ctx->st_pin + kPinBytes, bytes);
         return PINK_HIP_OK;
     }
-    std::unique_lock<std::mutex> lock;
-    HostStaging *st = take_staging(lock);
+    StagingLease lease;
+    HostStaging *st = lease.take();
     if (!st) {
         HIP_TRY(ctx, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream));
         HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
@@ -4882,9 +4899,9 @@ int staged_run(pink_hip_ctx *ctx, const float *host_images, uint32_t n, Run run)
     // A mapper's kernels are faster than the link, so its rate from host buffers is the rate of the copies, and a
     // copy out of pageable memory is one host thread's work (about half of what the link takes): its inputs go through
     // the shared pinned pieces, which host threads fill side by side (cfg1 from pageable memory: 26 -> 42 GB/s,
-    // 1.6 M -> 2.56 M images/s).  Without those (another thread has them, the host refused them): the plain copies.
-    std::unique_lock<std::mutex> lock;
-    HostStaging *st = ctx->trainer ? nullptr : take_staging(lock);
+    // 1.6 M -> 2.56 M images/s).  Without those (four other calls have them, the host refused them): the plain copies.
+    StagingLease lease;
+    HostStaging *st = ctx->trainer ? nullptr : lease.take();
     if (st) TRY(ensure_piece_events(ctx));
     // (between two copies the link rests for some microseconds: large transfers go in larger pieces)
     const size_t all = (size_t)n * img_bytes;

@@ -976,6 +976,44 @@ def test_host_buffers_in_pieces_match_smaller_calls():
     assert np.array_equal(results[0][2], np.bincount(results[0][0], minlength=tiny["N"]))
 
 
+def test_large_transfers_of_several_threads_at_once():
+    """Six threads, each with its own mapper or trainer and host buffers of some MB: four have pinned pieces, the others none."""
+    import threading
+    N, D, n = 36, 64, 700
+    rng = np.random.default_rng(12)
+    som = rng.random((300, D * D), dtype=np.float32)
+    imgs = [rng.random((n, 1, D, D), dtype=np.float32) for _ in range(6)]
+    start, bad = threading.Barrier(6), []
+
+    def work(k):
+        trainer = k % 3 == 2                              # (a trainer's large transfer is its SOM)
+        size = 300 if trainer else N
+        factors = capi.make_update_factors(capi.CARTESIAN, [size], capi.GAUSSIAN, 1.0, 0.3) if trainer else None
+        with capi.Context(size, 1, D, D, 4, True, 20, capi.QUADRATIC, capi.UINT8, factors) as ctx:
+            ctx.set_som(som[:size])
+            if trainer:
+                ctx.train(imgs[k][:20])
+                want = ctx.get_som()
+                start.wait()
+                got = [ctx.get_som() for _ in range(20)]
+                bad.extend(k for g in got if not np.array_equal(bits(g), bits(want)))
+            else:
+                pieces = [ctx.map(imgs[k][i:i + 50]) for i in range(0, n, 50)]        # (below 1 MB a piece)
+                want = [np.concatenate(p) for p in zip(*pieces)]
+                start.wait()
+                for _ in range(8):
+                    heat, best = ctx.map(imgs[k])
+                    if not (np.array_equal(bits(heat), bits(want[0])) and np.array_equal(best, want[1])):
+                        bad.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
 def test_empty_inputs_are_no_ops():
     w = synthetic.WORKLOADS["cfg4"]
     som = synthetic.initial_som(w)
