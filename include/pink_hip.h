@@ -155,9 +155,10 @@ int pink_hip_update_counts(pink_hip_ctx *ctx, uint32_t *host_counts_out);
  *     up waiting.  Then the launches behind it have changed nothing, their groups are trained
  *     again with one launch per image, and the context stays with that form.
  *   - uint8 and uint16, up to 1024 neurons whose operand fits the compute units' LDS: queued.  A
- *     launch behind each does its group over, without that need, if a block gave up; the calls
- *     that follow take a launch per image and kernel for some 256 images (four times as many
- *     each time it happens), then the resident form is tried again.
+ *     launch behind each does its group over, without that need, if a block gave up (some fifty
+ *     times as long), and later groups of the call try again.  The calls that follow take a
+ *     launch per image and kernel for some 256 images (four times as many each time it
+ *     happens), then the resident form.
  * The environment variable PINK_HIP_RESIDENT_TRAINER=0, read when a context is created, selects
  * the other forms from the start. */
 int pink_hip_train_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out);

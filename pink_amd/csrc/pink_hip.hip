@@ -2093,17 +2093,26 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
 
 // m_update_info[bmu]++ for the images of a group (Trainer.h:302-303), behind a resident launch: nothing when that launch
 // or one before it gave up and nobody rescued it.  The error word goes to the host with it, which looks when it next comes by.
-// rescue: k_sym_rescue's ticket and, behind it, its counts per image, for the next one.
+// Behind k_sym_rescue (one block, `rescue` its ticket and counts per image): what it and the next launch need is made ready again,
+// and how many groups are left to it before a resident launch is tried once more: one after a failure, twice as many after
+// each that follows without a success between (error: the launch that failed, groups left, groups next time).
 __global__ __launch_bounds__(256) void k_count_best_matches(const uint32_t *__restrict__ bmu, uint32_t images, uint32_t *__restrict__ counts,
-                                                            const uint32_t *__restrict__ error, uint32_t *__restrict__ host_error,
-                                                            uint32_t *__restrict__ rescue)
+                                                            uint32_t *__restrict__ error, uint32_t *__restrict__ host_error,
+                                                            uint32_t *__restrict__ rescue, unsigned long long *__restrict__ slots, uint32_t slot_words)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, e = *error;
     if (t == 0) *host_error = e;
     if (t < images && (e == 0 || rescue)) atomicAdd(&counts[bmu[t]], 1u);
-    if (rescue && e) {
-        if (t < images) rescue[1 + t] = 0;
-        if (t == 0) rescue[0] = 0;
+    if (!rescue) return;
+    __syncthreads();
+    if (e) {
+        for (uint32_t i = t; i <= images; i += 256) rescue[i] = 0;
+        for (uint32_t i = t; i < slot_words; i += 256) slots[i] = 0;
+    }
+    if (t == 0) {
+        if (!e) error[2] = 0;
+        else if (error[1]) { if (--error[1] == 0) error[0] = 0; }
+        else error[1] = error[2] = error[2] ? min(2 * error[2], 64u) : 1u;
     }
 }
 
@@ -3059,7 +3068,8 @@ int resident_launched(pink_hip_ctx *ctx, const float *dev_images, uint32_t image
 {
     const bool rescued = ctx->sym_train;
     hipLaunchKernelGGL(k_count_best_matches, dim3((images + 255) / 256), dim3(256), 0, ctx->stream, dev_bmu, images, ctx->d_counts,
-                       ctx->d_resident_error, ctx->h_resident_error, rescued ? ctx->d_sym_rescue : nullptr);
+                       ctx->d_resident_error, ctx->h_resident_error, rescued ? ctx->d_sym_rescue : nullptr, ctx->d_slots,
+                       rescued ? 2 * ctx->N * kSymStride : 0u);
     TRY(launch_check(ctx, "k_count_best_matches"));
     if (!rescued) ctx->resident_queued.push_back({dev_images, images, dev_bmu});
     swap_resident(ctx);
@@ -3174,9 +3184,9 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         }));
         rescue.keys = ctx->d_sym_keys; rescue.ticket = ctx->d_sym_rescue; rescue.done = ctx->d_sym_rescue + 1;
         const dim3 grid(std::min(ctx->N, 2 * (uint32_t)ctx->num_cu));
-        const size_t lds = (size_t)ctx->sym_cells * sizeof(uint2);
-        if (ctx->cfg.ed_type == PINK_HIP_UINT16) hipLaunchKernelGGL(k_sym_rescue<true>, grid, dim3(512), lds, ctx->stream, rescue);
-        else hipLaunchKernelGGL(k_sym_rescue<false>, grid, dim3(512), lds, ctx->stream, rescue);
+        const size_t lds = (size_t)ctx->sym_cells * (sizeof(uint2) + 1);
+        if (ctx->cfg.ed_type == PINK_HIP_UINT16) hipLaunchKernelGGL(k_sym_rescue<true>, grid, dim3(kRescueThreads), lds, ctx->stream, rescue);
+        else hipLaunchKernelGGL(k_sym_rescue<false>, grid, dim3(kRescueThreads), lds, ctx->stream, rescue);
         TRY(launch_check(ctx, "k_sym_rescue"));
     }
     if (ctx->sym_outside) {
