@@ -51,11 +51,13 @@ COUNTER_TRAFFIC_PER_IMAGE = {
     ("cfg0", "update"): ((28.133e6 + 0.774e6 + 1.706e6 + 1.184e6) / 48, "profiles/cfg0_train_f32_counters.txt"),   # per group of 48
     ("cfg1", "rotate"): ((96.042e6 + 207.618e6) / 2048, "profiles/cfg1_map_u8_counters.txt"),
     ("cfg1", "distance"): ((214.632e6 + 1.639e6) / 2048, "profiles/cfg1_map_u8_counters.txt"),
-    ("cfg2", "distance"): (32.971e6 + 0.069e6, "profiles/cfg2_train_u16_counters.txt"),
-    ("cfg2", "update"): (28.845e6 + 17.831e6, "profiles/cfg2_train_u16_counters.txt"),
-    ("cfg3", "distance"): (252.417e6 + 0.576e6, "profiles/cfg3_train_f32_3ch_counters.txt"),
+    # the resident launch of 64 images and the one that brings the elements outside the region up to date
+    ("cfg2", "update"): ((819.878e6 + 7.440e6 + 206.588e6 + 12.635e6) / 64, "profiles/cfg2_train_u16_counters.txt"),
+    # the product, its sums over splits, the selection, the exact sums of variants and of neurons
+    ("cfg3", "distance"): (33.222e6 + 13.824e6 + 13.959e6 + 2.304e6 + 2.477e6 + 0.117e6 + 145.810e6 + 1.165e6 + 11.708e6 + 0.006e6,
+                           "profiles/cfg3_train_f32_3ch_counters.txt"),
     # the operand rows per image and a sixteenth of the launch that brings the neurons' full images up to date
-    ("cfg3", "update"): (73.894e6 + 47.153e6 + (323.973e6 + 95.049e6) / 16, "profiles/cfg3_train_f32_3ch_counters.txt"),
+    ("cfg3", "update"): (70.644e6 + 71.889e6 + (396.569e6 + 94.937e6) / 16, "profiles/cfg3_train_f32_3ch_counters.txt"),
     ("cfg4", "update"): ((85.604e6 + 0.835e6) / 256, "profiles/cfg4_train_u8_counters.txt"),     # the resident launch of 256 images
 }
 
@@ -102,13 +104,31 @@ def algorithmic_per_image(w, E, path):
     }
 
 
-def distance_path_name(w, path, times):
+def screened(w, times, images):
+    """Whether a float32 trainer screened its distances in this run: it then rotates every group of images twice (variants, and the
+    product's rows); its update launches are one per image and one per group."""
+    groups = times["update"][0] - images
+    return w.ed_type == 0 and w.mode == "train" and groups > 0 and times["rotate"][0] == 2 * groups
+
+
+def small_resident(w):
+    return w.ed_type == 2 and w.som_size <= 64 and w.R <= 32
+
+
+def distance_path_name(w, path, times, images):
     """The kernel that computed the distances in this run, by the library's path and what was launched."""
     from pink_amd import capi
+    if screened(w, times, images):
+        return ("int8 MFMA product of 16-bit values for every (neuron, variant) pair, then float32 sums in the CPU's order of the "
+                "variants that can be a neuron's closest")
     if w.ed_type == capi.FLOAT and path != capi.KERNEL_MFMA_F32:
         if w.mode == "train" and 0 < times["update"][0] < times["distance"][0]:
             return "float32 vector ALU, one (neuron, variant) pair per lane, DPP broadcast; the launch also applies the update of the image before"
         return "float32 vector ALU, one (neuron, variant) pair per lane"
+    if w.mode == "train" and path == capi.KERNEL_MFMA_GEMM and times["distance"][0] == 0 and not small_resident(w):
+        return ("int8 MFMA inside the resident launch of an integer trainer (one launch per group of images: distances with the "
+                "symmetries on the SOM side, best match, update; one to four neurons per block, a 64-bit word per neuron and image "
+                "exchanged through memory)")
     if w.mode == "train" and path == capi.KERNEL_MFMA_GEMM and times["distance"][0] == 0:
         return ("int8 MFMA inside the resident launch of a small uint8 trainer (one launch per group of images: distances, "
                 "best match, update; one block per neuron, a 64-bit word per block and image exchanged through memory)")
@@ -274,6 +294,12 @@ def run_workload(name, steps, warmup, n_images, kernel, cpu_budget_s, host_inclu
         achieved = alg["distance"]["ops"] * per_s / 1e12
         notes = ("float32 MFMA recast |a|^2 + |b|^2 - 2 a.b, requested with --kernel mfma_f32: not the CPU's summation "
                  "order (distances to a relative tolerance only); never the default")
+    elif dominant == "distance" and screened(w, times, prof_images):
+        bound, unit, peak = "mfma", "TOP/s", MFMA_INT8_PEAK_TOPS
+        achieved = alg["distance"]["ops"] * per_s / 1e12
+        notes = ("every pair's operations priced at the int8 peak, though two of the class's launches do them: four byte-plane products "
+                 "per pair element, counted once; the rest of its time goes to the float32 sums of the variants left, a serial chain per "
+                 "variant, and to the neurons that keep all of theirs")
     elif dominant == "distance" and w.ed_type == capi.FLOAT:
         # direct float32 form on the vector ALU: subtract + fma per pair element, counted as 2 ops
         bound, unit, peak = "valu", "TFLOP/s", FP32_PEAK_TFLOPS
@@ -302,7 +328,12 @@ def run_workload(name, steps, warmup, n_images, kernel, cpu_budget_s, host_inclu
         if dominant == "rotate" and path != capi.KERNEL_VALU:
             notes = ("vector-ALU bound (exact bilinear arithmetic per operand byte), far from HBM: "
                      "algorithmic bytes = image read + packed operand written")
-        if dominant == "update" and times["distance"][0] == 0:
+        if dominant == "update" and times["distance"][0] == 0 and not small_resident(w):
+            notes = ("distances, best match and update of a whole group of images in one resident launch (class 'update', with the "
+                     "elements outside the region, one more launch per group): an image's base rotations are pulled through every "
+                     "compute unit from the L2s, the blocks exchange a 64-bit word per neuron, every block repeats the search; "
+                     "bound by that chain, not by HBM: no roofline claimed")
+        elif dominant == "update" and times["distance"][0] == 0:
             notes = ("a small uint8 trainer: distances, best match and update of a whole group of images in one resident "
                      "launch (class 'update'), one block per neuron; per image the blocks exchange one 64-bit word each "
                      "through memory (store, then polls: about 0.9 us) around about 1 us of lone-wave instruction issue; "
@@ -318,7 +349,7 @@ def run_workload(name, steps, warmup, n_images, kernel, cpu_budget_s, host_inclu
         "share_of_kernel_time": round(ms / total_ms, 4),
         "kernel_ms": {k: round(v[1], 4) for k, v in times.items()},
         "kernel_us_per_image": {k: round(v[1] * 1e3 / prof_images, 4) for k, v in times.items()},
-        "distance_path": distance_path_name(w, path, times),
+        "distance_path": distance_path_name(w, path, times, prof_images),
     }
     if second_peak:
         roofline["measured_ceiling"] = {"what": second_peak[0], "peak": second_peak[1], "unit": unit,

@@ -2305,7 +2305,8 @@ private:
 // (its stream).  Other processes on the device are not seen: what they keep apart gives up and is done over.
 struct ResidentUse : ResidentShape {
     const void *owner;
-    hipEvent_t done;            // recorded behind the owner's last launch
+    hipStream_t stream;
+    hipEvent_t done;            // for who waits: recorded behind what stands in the stream then
 };
 constexpr int kMaxDevices = 64;
 std::mutex g_resident_mutex;
@@ -3044,14 +3045,18 @@ int launch_resident(pink_hip_ctx *ctx, uint32_t blocks, Launch launch)
 {
     std::lock_guard<std::mutex> lock(g_resident_mutex);
     std::vector<ResidentUse> &uses = g_resident[ctx->device];
-    uses.erase(std::remove_if(uses.begin(), uses.end(), [&](const ResidentUse &u) { return u.owner == ctx || hipEventQuery(u.done) == hipSuccess; }), uses.end());
-    (void)hipGetLastError();                              // (a launch that still runs is no error)
+    uses.erase(std::remove_if(uses.begin(), uses.end(), [&](const ResidentUse &u) { return u.owner == ctx || hipStreamQuery(u.stream) == hipSuccess; }), uses.end());
     const ResidentShape mine{blocks, ctx->resident_per_unit};
-    const size_t waits = resident_waits(uses, uses.size(), mine, (uint32_t)ctx->num_cu);
-    for (size_t i = 0; i < waits; ++i) HIP_TRY(ctx, hipStreamWaitEvent(ctx->stream, uses[i].done, 0));
+    if (!uses.empty()) {
+        (void)hipGetLastError();                          // (a stream that still runs is no error)
+        const size_t waits = resident_waits(uses, uses.size(), mine, (uint32_t)ctx->num_cu);
+        for (size_t i = 0; i < waits; ++i) {
+            HIP_TRY(ctx, hipEventRecord(uses[i].done, uses[i].stream));
+            HIP_TRY(ctx, hipStreamWaitEvent(ctx->stream, uses[i].done, 0));
+        }
+    }
     TRY(launch());
-    HIP_TRY(ctx, hipEventRecord(ctx->resident_done, ctx->stream));
-    uses.push_back({mine, ctx, ctx->resident_done});
+    uses.push_back({mine, ctx, ctx->stream, ctx->resident_done});
     return PINK_HIP_OK;
 }
 
