@@ -3739,9 +3739,10 @@ uint32_t summed_images(const pink_hip_ctx *ctx)
 
 // Trainers that take the orbits' product: integers where the resident form (init_sym_train) does not fit, which keep their
 // weights in that order too; float32 where every variant's sum costs more than the product, the few sums that are left and
-// two launches more.  Those sums are a chain of E steps whatever the SOM's size, so there have to be two neurons per CU, and
-// (neurons x variants x elements, ratio of the times of an image): 0.3e9 0.66, 0.7e9 0.91, 0.84e9 1.01, 1.1e9 1.05, 1.3e9 1.19,
-// 2.2e9 1.85; 400 neurons, 2.9e9: 0.97.
+// three launches more.  Those sums are a chain of E steps whatever the SOM's size, so there have to be two neurons per CU, and
+// (neurons x variants x elements, summed / screened time of an image; the lower half with the sums in lists of three neurons):
+// 0.3e9 0.66, 0.7e9 0.91, 0.84e9 1.01, 400 neurons, 2.9e9 0.97; 1.01e9 1.20, 1.06e9 1.10, 1.11e9 1.34, 1.31e9 1.37, 2.23e9 2.2,
+// 4.3e9 2.0.
 bool orbit_trains(const pink_hip_ctx *ctx)
 {
     if (!is_int(ctx))
@@ -3773,8 +3774,9 @@ int run_orbit_som(pink_hip_ctx *ctx)
     return launch_check(ctx, "k_orbit_som");
 }
 
+// (finish: whether the sums of splits, if there are any, become keys or distances here)
 template <int MODE, int WM, int WN, int KC, int PD, int MINB>
-void launch_orbit_gemm(pink_hip_ctx *ctx, OrbitGemm a)
+void launch_orbit_gemm(pink_hip_ctx *ctx, OrbitGemm &a, bool finish)
 {
     a.row_tiles = (a.M + 64 * WM - 1) / (64 * WM);
     a.col_tiles = (a.N * a.ns + 64 * WN - 1) / (64 * WN);
@@ -3791,7 +3793,7 @@ void launch_orbit_gemm(pink_hip_ctx *ctx, OrbitGemm a)
     a.splits = (steps + a.steps_per - 1) / a.steps_per;
     const uint32_t per = (tiles * a.splits + 7) / 8;
     hipLaunchKernelGGL((k_orbit_gemm<MODE, WM, WN, KC, PD, MINB>), dim3(8 * per), dim3(256), orbit_gemm_lds(MODE, WM, WN, KC, a.ns, a.nrr), ctx->stream, a);
-    if (a.splits > 1)
+    if (a.splits > 1 && finish)
         hipLaunchKernelGGL(k_orbit_finish<MODE>, dim3((a.N * a.ns + 63) / 64, (a.M + 3) / 4), dim3(256), 0, ctx->stream, a);
 }
 
@@ -3834,10 +3836,11 @@ int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
     // planes and short rows more of their blocks hide each other's beginnings and ends
     const size_t columns = (size_t)a.N * a.ns, tiles = (size_t)((M + 63) / 64) * ((columns + 127) / 128);
     const bool small = tiles < (size_t)4 * ctx->num_cu || (!u8 && a.KS < 64);
+    const bool finish = !ctx->screen_train || a.nrr > kSelectRows;         // (k_screen_select does it)
     switch (ctx->orb_mode) {
-    case ORB_U8: if (small) launch_orbit_gemm<ORB_U8, 1, 1, 4, 4, 4>(ctx, a); else launch_orbit_gemm<ORB_U8, 1, 2, 4, 1, 4>(ctx, a); break;
-    case ORB_U16: if (small) launch_orbit_gemm<ORB_U16, 1, 1, 2, 4, 3>(ctx, a); else launch_orbit_gemm<ORB_U16, 1, 2, 2, 1, 3>(ctx, a); break;
-    default: if (small) launch_orbit_gemm<ORB_F32, 1, 1, 2, 4, 3>(ctx, a); else launch_orbit_gemm<ORB_F32, 1, 2, 2, 1, 3>(ctx, a); break;
+    case ORB_U8: if (small) launch_orbit_gemm<ORB_U8, 1, 1, 4, 4, 4>(ctx, a, finish); else launch_orbit_gemm<ORB_U8, 1, 2, 4, 1, 4>(ctx, a, finish); break;
+    case ORB_U16: if (small) launch_orbit_gemm<ORB_U16, 1, 1, 2, 4, 3>(ctx, a, finish); else launch_orbit_gemm<ORB_U16, 1, 2, 2, 1, 3>(ctx, a, finish); break;
+    default: if (small) launch_orbit_gemm<ORB_F32, 1, 1, 2, 4, 3>(ctx, a, finish); else launch_orbit_gemm<ORB_F32, 1, 2, 2, 1, 3>(ctx, a, finish); break;
     }
     TRY(launch_check(ctx, "k_orbit_gemm"));
     if (!f32) return PINK_HIP_OK;
@@ -3850,7 +3853,9 @@ int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
         l.some_list = ctx->d_screen_list + (size_t)ctx->N * kSelectFew; l.some = ctx->d_screen_wide + ctx->N;
         l.skip = a.skip;
         l.N = ctx->N; l.E = ctx->E; l.nrr = ctx->nrr_eff; l.num_rot = ctx->cfg.num_rot; l.ns = ctx->orb_ns; l.valid = ctx->orb_valid;
-        hipLaunchKernelGGL(k_screen_select, dim3((uint32_t)((columns + 63) / 64)), dim3(512), 0, ctx->stream, l);
+        const dim3 blocks((uint32_t)((columns + 63) / 64));
+        if (a.splits > 1 && !finish) hipLaunchKernelGGL(k_screen_select<true>, blocks, dim3(64 * kSelectWaves), 0, ctx->stream, l, a);
+        else hipLaunchKernelGGL(k_screen_select<false>, blocks, dim3(64 * kSelectWaves), 0, ctx->stream, l, a);
         TRY(launch_check(ctx, "k_screen_select"));
         ScreenSums x{};
         x.som_rows = (const float *)ctx->d_somP; x.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad;
@@ -3859,6 +3864,7 @@ int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
         x.wide_blocks = x.chain_blocks = 2 * (uint32_t)ctx->num_cu;        // (four blocks to a CU: all of them run at once)
         hipLaunchKernelGGL(k_screen_sums, dim3(x.wide_blocks + x.chain_blocks), dim3(64 * kSumsWaves), 0, ctx->stream, x);
         TRY(launch_check(ctx, "k_screen_sums"));
+        if (screen_items(ctx->N, ctx->R) <= 2 * x.wide_blocks) return PINK_HIP_OK;
         const uint32_t pairs = ctx->Rpad / kWave * ((ctx->N + 7) / 8);
         hipLaunchKernelGGL(k_screen_many, dim3((pairs + 7) / 8 * 8), dim3(256), 0, ctx->stream, x);
         return launch_check(ctx, "k_screen_many");
