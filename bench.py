@@ -53,11 +53,11 @@ COUNTER_TRAFFIC_PER_IMAGE = {
     ("cfg1", "distance"): ((214.632e6 + 1.639e6) / 2048, "profiles/cfg1_map_u8_counters.txt"),
     # the resident launch of 64 images and the one that brings the elements outside the region up to date
     ("cfg2", "update"): ((819.878e6 + 7.440e6 + 206.588e6 + 12.635e6) / 64, "profiles/cfg2_train_u16_counters.txt"),
-    # the product, its sums over splits, the selection, the exact sums of variants and of neurons
-    ("cfg3", "distance"): (33.222e6 + 13.824e6 + 13.959e6 + 2.304e6 + 2.477e6 + 0.117e6 + 145.810e6 + 1.165e6 + 11.708e6 + 0.006e6,
+    # the product, the selection, the exact sums of variants and of neurons
+    ("cfg3", "distance"): (33.229e6 + 13.824e6 + 14.031e6 + 0.118e6 + 156.047e6 + 1.316e6 + 1.424e6 + 0.001e6,
                            "profiles/cfg3_train_f32_3ch_counters.txt"),
     # the operand rows per image and a sixteenth of the launch that brings the neurons' full images up to date
-    ("cfg3", "update"): (70.644e6 + 71.889e6 + (396.569e6 + 94.937e6) / 16, "profiles/cfg3_train_f32_3ch_counters.txt"),
+    ("cfg3", "update"): (70.642e6 + 71.889e6 + (396.602e6 + 94.939e6) / 16, "profiles/cfg3_train_f32_3ch_counters.txt"),
     ("cfg4", "update"): ((85.604e6 + 0.835e6) / 256, "profiles/cfg4_train_u8_counters.txt"),     # the resident launch of 256 images
 }
 

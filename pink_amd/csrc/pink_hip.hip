@@ -3740,8 +3740,8 @@ uint32_t summed_images(const pink_hip_ctx *ctx)
 // Trainers that take the orbits' product: integers where the resident form (init_sym_train) does not fit, which keep their
 // weights in that order too; float32 where every variant's sum costs more than the product, the few sums that are left and
 // three launches more.  Those sums are a chain of E steps whatever the SOM's size, so there have to be two neurons per CU, and
-// (neurons x variants x elements, summed / screened time of an image; the lower half with the sums in lists of three neurons):
-// 0.3e9 0.66, 0.7e9 0.91, 0.84e9 1.01, 400 neurons, 2.9e9 0.97; 1.01e9 1.20, 1.06e9 1.10, 1.11e9 1.34, 1.31e9 1.37, 2.23e9 2.2,
+// (neurons x variants x elements, summed / screened time of an image; the first four with the sums in lists of three neurons each):
+// 0.3e9 0.66, 0.7e9 0.91, 0.84e9 1.01, 400 neurons of 2.9e9 0.97; 1.01e9 1.20, 1.06e9 1.10, 1.11e9 1.34, 1.31e9 1.37, 2.23e9 2.2,
 // 4.3e9 2.0.
 bool orbit_trains(const pink_hip_ctx *ctx)
 {
