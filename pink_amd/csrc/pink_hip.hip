@@ -1596,16 +1596,29 @@ template <int EPT>       // elements per thread, 256 apart
 __global__ __launch_bounds__(256) void k_update_replay(float *__restrict__ som, const float *__restrict__ rot,
                                                        const unsigned long long *__restrict__ key, const float *__restrict__ factors,
                                                        const uint32_t *__restrict__ bmu, uint32_t images, uint32_t N, uint32_t S,
-                                                       uint32_t R, uint32_t shift, VariantPair vp)
+                                                       uint32_t R, uint32_t shift, VariantPair vp, const float *__restrict__ moves)
 {
     __shared__ float s_f[kReplayMax];
     __shared__ uint32_t s_row[kReplayMax];   // stored row of the group's variants * 4 + how it is read
+    __shared__ uint32_t s_moved[4];
     // (neurons vary fastest over the grid: the blocks that run side by side then read the same stretch of elements of
     // whatever variants their neurons were closest to -- a few MB that stay in L2 -- and not whole variants)
     // (several elements per thread: what an image costs the thread beside its elements -- its row, how it is read, its
     // factor, out of LDS -- is paid once for all of them)
     const uint32_t n = blockIdx.x, j = blockIdx.y * (256 * EPT) + threadIdx.x;
-    if (threadIdx.x < images) {
+    // (the images that move the neuron, in order: the closest variant of another may not be known)
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const float mine = threadIdx.x >= images ? 0.0f : moves ? moves[(size_t)threadIdx.x * N + n] : factors[(size_t)bmu[threadIdx.x] * N + n];
+    const unsigned long long moved = __ballot(mine != 0.0f);
+    if (lane == 0) s_moved[wave] = (uint32_t)__popcll(moved);
+    __syncthreads();
+    uint32_t at = (uint32_t)__popcll(moved & ((1ull << lane) - 1)), count = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < 4; ++w) {
+        at += w < wave ? s_moved[w] : 0u;
+        count += s_moved[w];
+    }
+    if (mine != 0.0f) {
         const uint32_t i = threadIdx.x;
         const uint32_t r = (uint32_t)(key[(size_t)i * N + n] & ((1ull << shift) - 1ull));
         uint32_t row = r, which = 0;
@@ -1616,10 +1629,11 @@ __global__ __launch_bounds__(256) void k_update_replay(float *__restrict__ som, 
             row = (q & 1) * vp.nrr + b;
             which = 2 * (fl ^ (q >> 1)) + (q >> 1);
         }
-        s_f[i] = factors[(size_t)bmu[i] * N + n];
-        s_row[i] = (i * R + row) * 4 + which;
+        s_f[at] = mine;
+        s_row[at] = (i * R + row) * 4 + which;
     }
     __syncthreads();
+    if (count == 0) return;
     if (j >= S) return;
     uint32_t jj[EPT];
 #pragma unroll
@@ -1639,13 +1653,13 @@ __global__ __launch_bounds__(256) void k_update_replay(float *__restrict__ som, 
     float w[EPT];
 #pragma unroll
     for (int e = 0; e < EPT; ++e) w[e] = som[(size_t)n * S + jj[e]];
-    for (uint32_t i0 = 0; i0 < images; i0 += 8) {
+    for (uint32_t i0 = 0; i0 < count; i0 += 8) {
         float x[8][EPT], f[8];
 #pragma unroll
         for (uint32_t u = 0; u < 8; ++u) {
-            const uint32_t i = min(i0 + u, images - 1);
+            const uint32_t i = min(i0 + u, count - 1);
             const uint32_t rw = s_row[i], which = rw & 3;
-            f[u] = i0 + u < images ? s_f[i] : 0.0f;
+            f[u] = i0 + u < count ? s_f[i] : 0.0f;
             const float *row = rot + (size_t)(rw >> 2) * S;
 #pragma unroll
             for (int e = 0; e < EPT; ++e)
@@ -2088,6 +2102,7 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
     if (tid == 0) a.na_next[n] = (long long)na;
 }
 
+#include "ordered_sum.inc"
 #include "sym_train.inc"
 #include "orbit_gemm.inc"
 
@@ -2452,7 +2467,11 @@ struct pink_hip_ctx {
     bool screen_train = false;
     uint32_t screen_set = 0;               // the counts that the last image took
     uint2 *d_screen_list = nullptr;
-    uint32_t *d_screen_wide = nullptr, *d_screen_counts = nullptr;
+    uint32_t *d_screen_wide = nullptr, *d_screen_counts = nullptr, *d_screen_choice = nullptr;
+    float2 *d_screen_bound = nullptr;
+    float *d_screen_moves = nullptr;       // [image][N]
+    float2 *d_screen_range = nullptr;      // (WeightRange)
+    uint32_t *d_screen_negative = nullptr;
     uint4 *d_orb_element = nullptr;
     uint32_t orb_cur = 0, orb_pitch = 0, orb_outside = 0;      // the set of norms that belongs to the operand
     uint32_t *d_orb_outside = nullptr, *d_orb_best = nullptr;
@@ -2605,11 +2624,15 @@ int run_pack_frag_som(pink_hip_ctx *ctx)
 }
 
 int run_orbit_som(pink_hip_ctx *ctx);
+int run_screen_range(pink_hip_ctx *ctx);
 
 int run_pack_som(pink_hip_ctx *ctx)
 {
     Timed t(ctx, kClsPack);
-    if (ctx->screen_train) TRY(run_orbit_som(ctx));
+    if (ctx->screen_train) {
+        TRY(run_orbit_som(ctx));
+        TRY(run_screen_range(ctx));
+    }
     if (ctx->orbit) {
         TRY(run_orbit_som(ctx));
         if (is_int(ctx)) return PINK_HIP_OK;              // (float32: the rows in the CPU's order too)
@@ -2997,7 +3020,8 @@ int run_update_replay(pink_hip_ctx *ctx, uint32_t images, const uint32_t *dev_bm
 #define LAUNCH_REPLAY(EPT_)                                                                                                   \
     hipLaunchKernelGGL(k_update_replay<EPT_>, dim3(ctx->N, (ctx->S + 256 * EPT_ - 1) / (256 * EPT_)), dim3(256), 0, ctx->stream, \
                        ctx->d_som, ctx->d_rot + (size_t)first * ctx->R * ctx->S, ctx->d_key + (size_t)first * ctx->N,            \
-                       ctx->d_factors, dev_bmu + first, count, ctx->N, ctx->S, ctx->R, ctx->shift, vp)
+                       ctx->d_factors, dev_bmu + first, count, ctx->N, ctx->S, ctx->R, ctx->shift, vp,                                            \
+                       ctx->screen_train ? ctx->d_screen_moves + (size_t)first * ctx->N : nullptr)
         // (large SOMs: several elements per thread -- 1600 neurons of 3 x 70 x 70: 13.6 us per image with one, 10.2 with
         // two, 9.0 with four; small ones need the blocks -- 100 neurons of 45 x 45: 0.42, 0.46)
         const size_t weights = (size_t)ctx->N * ctx->S;
@@ -3277,7 +3301,7 @@ int free_all(pink_hip_ctx *ctx)
                     ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4,
                     ctx->d_orb_tables, ctx->d_orb_outside, ctx->d_orb_best, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
                     ctx->d_orb_sa, ctx->d_orb_ea, ctx->d_orb_sb, ctx->d_orb_eb, ctx->d_orb_dump,
-                    ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts, ctx->d_sym_keys, ctx->d_sym_rescue};
+                    ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts, ctx->d_screen_choice, ctx->d_screen_bound, ctx->d_screen_moves, ctx->d_screen_range, ctx->d_screen_negative, ctx->d_sym_keys, ctx->d_sym_rescue};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu}) if (p) (void)hipFree(p);
     if (ctx->st_pin) (void)hipHostFree(ctx->st_pin);
@@ -3774,6 +3798,13 @@ int run_orbit_som(pink_hip_ctx *ctx)
     return launch_check(ctx, "k_orbit_som");
 }
 
+// (float32 trainers) what is known of the weights, from all of them.
+int run_screen_range(pink_hip_ctx *ctx)
+{
+    hipLaunchKernelGGL(k_screen_range, dim3(ctx->N), dim3(256), 0, ctx->stream, ctx->d_som, (WeightRange *)ctx->d_screen_range, ctx->S);
+    return launch_check(ctx, "k_screen_range");
+}
+
 // (finish: whether the sums of splits, if there are any, become keys or distances here)
 template <int MODE, int WM, int WN, int KC, int PD, int MINB>
 void launch_orbit_gemm(pink_hip_ctx *ctx, OrbitGemm &a, bool finish)
@@ -3800,6 +3831,9 @@ void launch_orbit_gemm(pink_hip_ctx *ctx, OrbitGemm &a, bool finish)
 // v4i between the planes of a group of B images' rows.
 size_t orbit_rows_plane(const pink_hip_ctx *ctx, uint32_t B) { return (size_t)((B * ctx->orb_pitch + 31) / 32) * ctx->orb_KS * 64; }
 
+// Variants of a neuron that k_screen_select lists one by one; with more of them the neuron is summed whole.
+uint32_t screen_keep(uint32_t R) { return std::max(16u, R / 4); }
+
 // The rows of B images, and their keys reset.
 int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
 {
@@ -3810,6 +3844,7 @@ int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
     p.xrows = ctx->d_orb_x; p.plane = orbit_rows_plane(ctx, B); p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.KS = ctx->orb_KS;
     p.all_sym = ctx->orb_all; p.rl = ctx->orb_rl; p.pitch = ctx->orb_pitch;
     p.wide_count = ctx->orbit && !is_int(ctx) ? ctx->d_screen_counts : nullptr;
+    p.negative = ctx->d_screen_negative;
     const dim3 grid(B, (ctx->nrr_eff + (1u << p.rl) - 1) >> p.rl);
     const uint32_t threads = ctx->orb_prep_lds > 64 * 1024 || grid.x * grid.y < (uint32_t)ctx->num_cu ? 1024 : ctx->orb_prep_lds > 24 * 1024 ? 512 : 256;
     void *args[] = {&p};
@@ -3850,8 +3885,7 @@ int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
         ScreenSelect l{};
         l.dump = ctx->d_orb_dump; l.err_rows = ctx->d_orb_eb + row; l.err_som = ctx->d_orb_ea; l.key = key;
         l.list = ctx->d_screen_list; l.wide = ctx->d_screen_wide; l.counts = counts; l.counts_next = counts_next;
-        l.some_list = ctx->d_screen_list + (size_t)ctx->N * kSelectFew; l.some = ctx->d_screen_wide + ctx->N;
-        l.skip = a.skip;
+        l.skip = a.skip; l.bound = ctx->d_screen_bound; l.keep = screen_keep(ctx->R);
         l.N = ctx->N; l.E = ctx->E; l.nrr = ctx->nrr_eff; l.num_rot = ctx->cfg.num_rot; l.ns = ctx->orb_ns; l.valid = ctx->orb_valid;
         const dim3 blocks((uint32_t)((columns + 63) / 64));
         if (a.splits > 1 && !finish) hipLaunchKernelGGL(k_screen_select<true>, blocks, dim3(64 * kSelectWaves), 0, ctx->stream, l, a);
@@ -3859,10 +3893,15 @@ int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
         TRY(launch_check(ctx, "k_screen_select"));
         ScreenSums x{};
         x.som_rows = (const float *)ctx->d_somP; x.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad;
-        x.list = l.list; x.some_list = l.some_list; x.wide = l.wide; x.some = l.some; x.counts = counts; x.key = key;
-        x.Epad = ctx->Epad; x.R = ctx->R; x.Rpad = ctx->Rpad;
-        x.wide_blocks = x.chain_blocks = 2 * (uint32_t)ctx->num_cu;        // (four blocks to a CU: all of them run at once)
-        hipLaunchKernelGGL(k_screen_sums, dim3(x.wide_blocks + x.chain_blocks), dim3(64 * kSumsWaves), 0, ctx->stream, x);
+        x.list = l.list; x.wide = l.wide; x.counts = counts; x.key = key; x.bound = l.bound; x.factors = ctx->d_factors;
+        x.moves = ctx->d_screen_moves + (size_t)slot * ctx->N; x.choice = ctx->d_screen_choice;
+        x.range = (const WeightRange *)ctx->d_screen_range; x.scale_rows = a.scale_rows;
+        x.N = ctx->N; x.Epad = ctx->Epad; x.R = ctx->R; x.Rpad = ctx->Rpad;
+        x.wide_blocks = x.pair_blocks = 2 * (uint32_t)ctx->num_cu;
+        const dim3 sums(x.wide_blocks + x.pair_blocks);
+        if (ctx->Epad <= 512) hipLaunchKernelGGL(k_screen_sums<8>, sums, dim3(64 * kSumsWaves), 0, ctx->stream, x);
+        else if (ctx->Epad <= 1024) hipLaunchKernelGGL(k_screen_sums<16>, sums, dim3(64 * kSumsWaves), 0, ctx->stream, x);
+        else hipLaunchKernelGGL(k_screen_sums<32>, sums, dim3(64 * kSumsWaves), 0, ctx->stream, x);
         TRY(launch_check(ctx, "k_screen_sums"));
         if (screen_items(ctx->N, ctx->R) <= 2 * x.wide_blocks) return PINK_HIP_OK;
         const uint32_t pairs = ctx->Rpad / kWave * ((ctx->N + 7) / 8);
@@ -3902,6 +3941,8 @@ int run_screen_update(pink_hip_ctx *ctx, uint32_t slot, uint32_t *dev_bmu_out)
     u.som_rows = (float *)ctx->d_somP; u.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad; u.factors_t = ctx->d_factors_t;
     u.element = ctx->d_orb_element; u.listed = ctx->d_screen_counts + kCounts * ctx->screen_set; u.skip = ctx->d_screen_counts + 2 * kCounts;
     u.opnd = (uint2 *)ctx->d_orb_som; u.key = ctx->d_key + (size_t)slot * ctx->N; u.norm = ctx->d_orb_na; u.scale = ctx->d_orb_sa; u.err = ctx->d_orb_ea;
+    u.bound = ctx->d_screen_bound; u.moves = ctx->d_screen_moves + (size_t)slot * ctx->N; u.choice = ctx->d_screen_choice;
+    u.range = (WeightRange *)ctx->d_screen_range; u.scale_rows = ctx->d_orb_sb + slot; u.negative = ctx->d_screen_negative + slot;
     u.bmu_out = dev_bmu_out; u.counts = ctx->d_counts; u.plane = (size_t)ctx->N * ctx->orb_KS * 32; u.N = ctx->N; u.K8 = ctx->orb_KS * 4; u.Epad = ctx->Epad;
     hipLaunchKernelGGL(k_screen_update, dim3(ctx->N), dim3(512), (size_t)ctx->Epad * sizeof(float), ctx->stream, u);
     return launch_check(ctx, "k_screen_update");
@@ -4475,8 +4516,13 @@ int init_ctx(pink_hip_ctx *ctx)
             TRY(dev_alloc(ctx, &ctx->d_orb_sb, B));
             TRY(dev_alloc(ctx, &ctx->d_orb_eb, B * ctx->nrr_eff));
             TRY(dev_alloc(ctx, &ctx->d_orb_dump, (size_t)ctx->nrr_eff * ctx->N * ctx->orb_ns));
-            TRY(dev_alloc(ctx, &ctx->d_screen_list, (size_t)ctx->N * (kSelectFew + kSelectSome)));
-            TRY(dev_alloc(ctx, &ctx->d_screen_wide, (size_t)2 * ctx->N));
+            TRY(dev_alloc(ctx, &ctx->d_screen_list, (size_t)ctx->N * screen_keep(ctx->R)));
+            TRY(dev_alloc(ctx, &ctx->d_screen_wide, ctx->N));
+            TRY(dev_alloc(ctx, &ctx->d_screen_bound, ctx->N));
+            TRY(dev_alloc(ctx, &ctx->d_screen_moves, B * ctx->N));
+            TRY(dev_alloc(ctx, &ctx->d_screen_range, ctx->N));
+            TRY(dev_alloc(ctx, &ctx->d_screen_negative, B));
+            TRY(dev_alloc(ctx, &ctx->d_screen_choice, 2));
             TRY(upload(ctx, &ctx->d_screen_counts, std::vector<uint32_t>(2 * kCounts + 1, 0u)));       // (two sets, images to skip)
             ctx->orb_part_bytes = (size_t)16 << 20;
             TRY(dev_alloc(ctx, (char **)&ctx->d_orb_part, ctx->orb_part_bytes));
@@ -4622,6 +4668,7 @@ int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, 
                 TRY(run_update_rows(ctx, b, bmu + b));
             }
             TRY(run_update_replay(ctx, B, bmu));
+            if (ctx->screen_train) TRY(run_screen_range(ctx));
             continue;
         }
         if (ctx->resident_train) {

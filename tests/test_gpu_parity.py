@@ -784,10 +784,14 @@ SCREENED_TRAIN_SHAPES = [
     (640, 1, 90, 128, 128, True, 90, capi.QUADRATIC, 3, "zeros"),      # most variants alike: every variant of every neuron summed
     (523, 1, 70, 60, 452, True, 49, capi.QUADRATIC, 3, "grown"),       # some neurons keep all variants; 113 base rotations
     (517, 1, 70, 62, 360, True, 52, capi.QUADRATIC, 19, "flat"),      # ... image after image: no product for some of them, then again
-    (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 3, "close"),      # 18000 variants listed, more than one pass takes
-    (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 3, "closer"),     # 16300: one pass, in full batches
+    (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 3, "close"),      # 18000 variants listed
+    (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 3, "closer"),     # 16300
     (1200, 1, 64, 50, 180, True, 50, capi.QUADRATIC, 3, "nan"),
     (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 3, "flux"),       # every variant close, squares of errors no float32
+    (3100, 1, 40, 30, 360, True, 22, capi.QUADRATIC, 3, "steps"),      # sums that meet ties; runs of 8
+    (900, 1, 60, 56, 360, True, 45, capi.QUADRATIC, 3, "steps"),       # ... of 32
+    (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 5, "tail"),       # factors down to nothing: which neurons do they move?
+    (1000, 1, 60, 44, 360, True, 43, capi.CIRCULAR, 5, "tail"),
 ]
 
 
@@ -795,6 +799,7 @@ SCREENED_TRAIN_SHAPES = [
 def test_float_trainer_with_screened_distances(N, C_, I, D, nrot, flip, ed, shape_, n, kind):
     """Large float32 trainers sum the variants that a product of rounded values leaves: the oracle's bits, which sums them all."""
     say("screened float trainer", N, C_, I, D, nrot, flip, ed, shape_, n, kind)
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.MEXICAN_HAT if kind == "grown" else capi.GAUSSIAN, 1.0, 0.5)
     rng = np.random.default_rng(N + I)
     som0, imgs = rng.random((N, C_ * D * D), dtype=np.float32), rng.random((n, C_, I, I), dtype=np.float32)
     if kind == "blobs":
@@ -810,10 +815,25 @@ def test_float_trainer_with_screened_distances(N, C_, I, D, nrot, flip, ed, shap
         imgs[1, 0, I // 2, I // 2] = np.nan
     elif kind.startswith("close"):
         imgs = _nearly_round(rng, n, C_, I, 1.0, 0.02 if kind == "close" else 0.03)
+    elif kind == "steps":
+        # few bits in every value: images alike under the symmetries but for a few pixels, neurons a multiple of 2^-10 beside them
+        half = np.rint(imgs * 4) / 4
+        imgs = half + half[:, :, ::-1] + half[:, :, :, ::-1] + half[:, :, ::-1, ::-1]
+        imgs = (imgs + imgs.transpose(0, 1, 3, 2)).astype(np.float32)
+        imgs[:, :, I // 3, I // 2] += np.float32(2.0 ** -9)
+        m = (I - D) // 2
+        som0 = (imgs[0, :, m:m + D, m:m + D].reshape(1, -1) + np.rint((som0 - 0.5) * 2048) / 1024).astype(np.float32)
+    elif kind == "tail":
+        F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 90.0, 0.5) ** np.float32(1.7)
+        F[:, ::5] *= np.float32(1e-8)
+        som0[1::4] += np.float32(0.5)                                  # (no small weights)
+        som0[2::4, ::D] *= np.float32(1e-12)
+        som0[3::4, 7] = 0.0
+        imgs[3] -= np.float32(0.25)
     elif kind == "flux":
         imgs, som0 = _nearly_round(rng, n, C_, I, 5e-19), som0 * np.float32(5e-19)
-    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.MEXICAN_HAT if kind == "grown" else capi.GAUSSIAN, 1.0, 0.5)
-    F[np.abs(F) < 0.01] = 0.0
+    if kind != "tail":
+        F[np.abs(F) < 0.01] = 0.0
     s = O.shape(N, C_, I, D, nrot, flip, ed, shape_, capi.FLOAT)
     want = som0.copy()
     want_bmu = O.train(s, want, imgs, F)
