@@ -2105,6 +2105,7 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
 #include "ordered_sum.inc"
 #include "sym_train.inc"
 #include "orbit_gemm.inc"
+#include "coef_gemm.inc"
 
 // m_update_info[bmu]++ for the images of a group (Trainer.h:302-303), behind a resident launch: nothing when that launch
 // or one before it gave up and nobody rescued it.  The error word goes to the host with it, which looks when it next comes by.
@@ -2452,14 +2453,18 @@ struct pink_hip_ctx {
     uint32_t orb_KS = 0, orb_all = 0, orb_ns = 8, orb_valid = 0;
     size_t orb_prep_lds = 0;
     uint32_t sum_images = 0;               // float32: launches of at most so many images sum every variant (summed_images)
-    uint32_t orb_rl = 0, orb_bands = 0, orb_stride = 0, orb_batch = 0;
+    uint32_t orb_rl = 0, orb_Ox = 0;       // (float32) orbits, a multiple of 16
     char *d_orb_tables = nullptr;          // ... the tables below that init_orbit makes on the host
     uint32_t *d_orb_elem = nullptr, *d_orb_sel = nullptr, *d_orb_index = nullptr;
     float2 *d_orb_frac = nullptr;
-    uint32_t *d_orb_slots = nullptr;
-    uint2 *d_orb_bands = nullptr;
-    uint4 *d_orb_where = nullptr;
     unsigned short *d_orb_place = nullptr;
+    float *d_coef_weight = nullptr;        // (float32, coef_gemm.inc)
+    unsigned char *d_coef_outside = nullptr;
+    uint2 *d_coef_beside = nullptr;
+    unsigned short *d_coef_to = nullptr;
+    uint32_t coef_beside = 0;
+    void *d_coef_neuron = nullptr, *d_coef_image = nullptr, *d_coef_row = nullptr;
+    uint32_t *d_coef_words = nullptr, *d_coef_upper = nullptr;
     unsigned char *d_orb_live = nullptr;
     // ... and the trainers that keep their weights in that order: an image's rows start a tile of 32
     bool orbit_train = false;
@@ -2471,7 +2476,6 @@ struct pink_hip_ctx {
     float2 *d_screen_bound = nullptr;
     float *d_screen_moves = nullptr;       // [image][N]
     float2 *d_screen_range = nullptr;      // (WeightRange)
-    uint32_t *d_screen_negative = nullptr;
     uint4 *d_orb_element = nullptr;
     uint32_t orb_cur = 0, orb_pitch = 0, orb_outside = 0;      // the set of norms that belongs to the operand
     uint32_t *d_orb_outside = nullptr, *d_orb_best = nullptr;
@@ -2480,7 +2484,6 @@ struct pink_hip_ctx {
     size_t orb_part_bytes = 0;
     v4i *d_orb_mask = nullptr, *d_orb_som = nullptr, *d_orb_rows = nullptr;
     long long *d_orb_na = nullptr, *d_orb_nb = nullptr;
-    float *d_orb_sa = nullptr, *d_orb_ea = nullptr, *d_orb_sb = nullptr, *d_orb_eb = nullptr, *d_orb_dump = nullptr;
 
     unsigned char *static_scratch = nullptr;   // this device's copy of the file-scope scratch array
 
@@ -3300,8 +3303,7 @@ int free_all(pink_hip_ctx *ctx)
                     ctx->d_Pa, ctx->d_Pb, ctx->d_na, ctx->d_nb, ctx->d_poff, ctx->d_need, ctx->d_inv,
                     ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4,
                     ctx->d_orb_tables, ctx->d_orb_outside, ctx->d_orb_best, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
-                    ctx->d_orb_sa, ctx->d_orb_ea, ctx->d_orb_sb, ctx->d_orb_eb, ctx->d_orb_dump,
-                    ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts, ctx->d_screen_choice, ctx->d_screen_bound, ctx->d_screen_moves, ctx->d_screen_range, ctx->d_screen_negative, ctx->d_sym_keys, ctx->d_sym_rescue};
+                    ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts, ctx->d_screen_choice, ctx->d_screen_bound, ctx->d_screen_moves, ctx->d_screen_range, ctx->d_coef_neuron, ctx->d_coef_image, ctx->d_coef_row, ctx->d_coef_words, ctx->d_coef_upper, ctx->d_sym_keys, ctx->d_sym_rescue};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu}) if (p) (void)hipFree(p);
     if (ctx->st_pin) (void)hipHostFree(ctx->st_pin);
@@ -3558,8 +3560,8 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
 template <int MODE>
 const void *orbit_prepare_for(bool tile, bool x)
 {
-    if (MODE == ORB_F32 || x) return tile ? (const void *)k_orbit_prepare<MODE, true, true> : (const void *)k_orbit_prepare<MODE, false, true>;
-    return tile ? (const void *)k_orbit_prepare<MODE, true, MODE == ORB_F32> : (const void *)k_orbit_prepare<MODE, false, MODE == ORB_F32>;
+    if (x) return tile ? (const void *)k_orbit_prepare<MODE, true, true> : (const void *)k_orbit_prepare<MODE, false, true>;
+    return tile ? (const void *)k_orbit_prepare<MODE, true, false> : (const void *)k_orbit_prepare<MODE, false, false>;
 }
 const void *orbit_prepare_kernel(const pink_hip_ctx *ctx)
 {
@@ -3567,7 +3569,9 @@ const void *orbit_prepare_kernel(const pink_hip_ctx *ctx)
     switch (ctx->orb_mode) {
     case ORB_U8: return orbit_prepare_for<ORB_U8>(tile, ctx->trainer);
     case ORB_U16: return orbit_prepare_for<ORB_U16>(tile, ctx->trainer);
-    default: return orbit_prepare_for<ORB_F32>(tile, true);
+    default:
+        if (ctx->trainer) return tile ? (const void *)k_coef_prepare<true, false> : (const void *)k_coef_prepare<false, false>;
+        return tile ? (const void *)k_coef_prepare<true, true> : (const void *)k_coef_prepare<false, true>;
     }
 }
 
@@ -3595,7 +3599,7 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         for (uint32_t sym = 1; sym < 8; ++sym) first = std::min(first, moved(at, sym));
         if (orbit_of[first] == ~0u) { orbit_of[first] = 0; reps.push_back(first); }
     }
-    uint32_t corner = Ds;                                   // (of the region: k_screen_exact's patches then are runs of orbits)
+    uint32_t corner = Ds;                                   // (of the region)
     for (uint32_t off : region) corner = std::min({corner, place((off % DD) / D), place(off % D)});
     auto key = [&](uint32_t at) {
         const uint64_t ch = at / (Ds * Ds), x = (at % (Ds * Ds)) / Ds + 8 - corner % 8, y = at % Ds + 8 - corner % 8;
@@ -3604,9 +3608,11 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     std::sort(reps.begin(), reps.end(), [&](uint32_t l, uint32_t r) { return key(l) < key(r); });
     for (uint32_t o = 0; o < reps.size(); ++o)
         for (uint32_t sym = 0; sym < 8; ++sym) orbit_of[moved(reps[o], sym)] = o;
-    ctx->orb_KS = round_up(((uint32_t)reps.size() * 8 + 31) / 32, ctx->orb_mode == ORB_U8 ? 4u : 2u);       // (k_orbit_gemm's KC)
+    const bool f32 = ctx->orb_mode == ORB_F32;
+    ctx->orb_KS = round_up(((uint32_t)reps.size() * 8 + 31) / 32, f32 ? 16u : ctx->orb_mode == ORB_U8 ? 4u : 2u);       // (k_coef_gemm's steps, k_orbit_gemm's KC)
     const uint32_t Kp = ctx->orb_KS * 32;
-    if (ctx->orb_mode == ORB_F32 && Kp > 65536) return PINK_HIP_OK;      // (positions in a row are 16 bits there)
+    ctx->orb_Ox = round_up((uint32_t)reps.size(), 16);
+    if (f32 && Kp > 65536) return PINK_HIP_OK;      // (positions in a row are 16 bits there)
     std::vector<uint32_t> upos(Kp, ~0u), elem(Kp, ~0u), sel(16);
     std::vector<std::array<uint32_t, 8>> where(region.size());           // [element][symmetry]: slot-major position in a row
     for (uint32_t o = 0; o < reps.size(); ++o)
@@ -3617,8 +3623,8 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     uint32_t moves[8][8];                                   // where a slot goes under a symmetry
     for (uint32_t sym = 0; sym < 8; ++sym)
         for (uint32_t to = 0; to < 8; ++to) moves[sym][orbit_source((int)sym, (int)to)] = to;
-    std::vector<char> in_region(ctx->S, 0);
-    for (uint32_t off : region) in_region[off] = 1;
+    std::vector<uint32_t> in_region(ctx->S, 0);             // (place in the CPU's order + 1)
+    for (uint32_t e = 0; e < region.size(); ++e) in_region[region[e]] = e + 1;
     ctx->orb_all = 1;
     std::vector<unsigned char> mask((size_t)8 * Kp, 0);
     for (uint32_t e = 0; e < region.size(); ++e) {
@@ -3630,12 +3636,41 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
             if ((ctx->orb_valid >> sym) & 1) {
                 const uint32_t k = o * 8 + moves[sym][p], pos = upos[k];
                 mask[(size_t)sym * Kp + k] = 0xff;
-                where[e][sym] = moves[sym][p] * (Kp / 8) + o;
+                where[e][sym] = moves[sym][p] * (f32 ? ctx->orb_Ox : Kp / 8) + o;
                 if (!in_region[(pos >> 24) * DD + ((pos >> 12) & 0xfffu) * D + (pos & 0xfffu)]) ctx->orb_all = 0;
             }
     }
     Tables tables;
     uint32_t *d_upos = nullptr;
+    std::vector<float> weight;
+    std::vector<unsigned char> outside;
+    std::vector<uint2> beside;
+    if (f32) {
+        // an element is in every slot of its orbit whose place is its own (on an axis or a diagonal two of them, in the
+        // centre eight), divided by the root of their number
+        auto pixel_of = [&](uint32_t pos) { return (pos >> 24) * DD + ((pos >> 12) & 0xfffu) * D + (pos & 0xfffu); };
+        weight.assign(Kp / 8, 0.0f);
+        outside.assign(Kp, 0);
+        for (uint32_t o = 0; o < reps.size(); ++o) {
+            uint32_t same = 0;
+            for (uint32_t p = 0; p < 8; ++p) {
+                same += upos[o * 8 + p] == upos[o * 8];
+                const uint32_t off = pixel_of(upos[o * 8 + p]);
+                elem[o * 8 + p] = in_region[off] ? off : ~0u;
+            }
+            weight[o] = 1.0f / sqrtf((float)same);
+            // under symmetry s the region is where the slots go that hold its elements
+            for (uint32_t p = 0; p < 8; ++p) outside[o * 8 + p] = (unsigned char)ctx->orb_valid;
+            for (uint32_t sym = 0; sym < 8; ++sym)
+                for (uint32_t p = 0; p < 8; ++p)
+                    if (elem[o * 8 + p] != ~0u) outside[o * 8 + moves[sym][p]] &= (unsigned char)~(1u << sym);
+            const float square = 1.0f / (float)same;
+            uint32_t bits = 0;
+            memcpy(&bits, &square, 4);
+            for (uint32_t p = 0; p < 8; ++p)
+                if (outside[o * 8 + p]) beside.push_back(make_uint2(((p * ctx->orb_Ox + o) << 8) | outside[o * 8 + p], bits));
+        }
+    }
     std::vector<unsigned char> live(Kp / 8, 0);
     for (uint32_t k = 0; k < Kp; ++k) if (elem[k] != ~0u) live[k / 8] |= (unsigned char)(1u << (k % 8));
     tables.add(&ctx->d_orb_live, live);
@@ -3646,10 +3681,9 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     tables.add(&ctx->d_orb_mask, mask.data(), mask.size());
     const uint32_t planes = ctx->orb_mode == ORB_U8 ? 1 : 2;
     TRY(dev_alloc(ctx, &ctx->d_orb_som, (size_t)planes * ctx->N * Kp / 16));
-    TRY(dev_alloc(ctx, &ctx->d_orb_na, 3 * (size_t)ctx->N));      // (a trainer's three sets take turns)
-    TRY(dev_alloc(ctx, &ctx->d_orb_sa, ctx->N));
-    TRY(dev_alloc(ctx, &ctx->d_orb_ea, ctx->N));
-    if ((ctx->orb_mode == ORB_F32) != ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_values, (size_t)ctx->N * Kp));
+    if (f32) TRY(dev_alloc(ctx, (CoefNeuron **)&ctx->d_coef_neuron, ctx->N));
+    else TRY(dev_alloc(ctx, &ctx->d_orb_na, 3 * (size_t)ctx->N));        // (a trainer's three sets take turns)
+    if (!f32 && ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_values, (size_t)ctx->N * Kp));
     const size_t image_lds = (size_t)ctx->C * orbit_tile(ctx->I) * sizeof(float);
     ctx->orb_prep_lds = image_lds <= 120 * 1024 ? image_lds : 0;
     if (ctx->orb_prep_lds)
@@ -3659,54 +3693,37 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     // image has blocks for a part of the chip
     ctx->orb_rl = 0;
     while ((1u << ctx->orb_rl) < ctx->nrr_eff && ctx->orb_rl < (!ctx->orb_prep_lds ? 1u : ctx->trainer && Kp >= 4096 ? 2u : 4u)) ++ctx->orb_rl;
-    if (ctx->orb_mode == ORB_F32 && ctx->trainer) {
-        std::vector<unsigned short> element(Kp, 0xffff);
-        for (uint32_t e = 0; e < region.size(); ++e) element[(where[e][0] % (Kp / 8)) * 8 + where[e][0] / (Kp / 8)] = (unsigned short)e;
-        tables.add(&ctx->d_orb_element, element.data(), element.size() * sizeof(element[0]));
-    } else if (ctx->orb_mode == ORB_F32) {
-        // bands of eight region rows (of a channel), their elements in 8 x 8 patches
-        std::vector<uint32_t> slots;
-        std::vector<uint2> bands;
-        std::vector<std::array<uint32_t, 8>> slot_where;
-        uint32_t first = 0, longest = 0;
-        while (first < region.size()) {
-            const uint32_t row0 = region[first] / D;        // (rows of all channels counted through)
-            uint32_t end = first, lo = ~0u, hi = 0;
-            while (end < region.size() && region[end] / D < row0 + 8 && region[end] / DD == region[first] / DD) {
-                lo = std::min(lo, region[end] % D); hi = std::max(hi, region[end] % D); ++end;
+    if (f32) {
+        tables.add(&ctx->d_coef_weight, weight);
+        if (ctx->trainer) {
+            tables.add(&ctx->d_coef_outside, outside);
+            std::vector<unsigned short> element(Kp, 0xffff);
+            for (uint32_t k = 0; k < Kp; ++k) if (elem[k] != ~0u) element[k] = (unsigned short)(in_region[elem[k]] - 1);
+            tables.add(&ctx->d_orb_element, element.data(), element.size() * sizeof(element[0]));
+        } else {
+            std::vector<unsigned short> places;
+            for (uint32_t sym = 0; sym < 8; ++sym)
+                for (const auto &w : where) places.push_back((unsigned short)w[sym]);
+            tables.add(&ctx->d_orb_place, places);
+            // where k_coef_pairs puts a row's values: an element's run, or a place behind all of them
+            const uint32_t K = ctx->orb_Ox * 8, none = pair_row(ctx->E);
+            if (none < 65536) {
+                std::vector<unsigned short> to((size_t)8 * K, (unsigned short)none);
+                for (uint32_t e = 0; e < region.size(); ++e)
+                    for (uint32_t sym = 0; sym < 8; ++sym)
+                        if ((ctx->orb_valid >> sym) & 1) to[(size_t)sym * K + where[e][sym]] = (unsigned short)pair_place(e, pair_run(ctx->E));
+                tables.add(&ctx->d_coef_to, to);
+                HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_coef_pairs<true, 16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
             }
-            bands.push_back(make_uint2((uint32_t)slots.size() / 64, end - first));
-            longest = std::max(longest, end - first);
-            const uint32_t patches = (hi - lo) / 8 + 1;
-            slots.resize(slots.size() + (size_t)patches * 64, ~0u);
-            slot_where.resize(slots.size());
-            for (uint32_t e = first; e < end; ++e) {
-                const uint32_t y = region[e] % D - lo, x = region[e] / D - row0, at = (bands.back().x + y / 8) * 64 + x * 8 + y % 8;
-                slots[at] = e - first;
-                slot_where[at] = where[e];
-            }
-            first = end;
+            if (!ctx->orb_all) { tables.add(&ctx->d_coef_beside, beside); ctx->coef_beside = (uint32_t)beside.size(); }
+            HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_coef_map, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kMapSteps * 16 * kCoefStride * 16)));
         }
-        ctx->orb_bands = (uint32_t)bands.size();
-        bands.push_back(make_uint2((uint32_t)slots.size() / 64, 0u));
-        std::vector<uint4> w16(slots.size());
-        for (size_t t = 0; t < slots.size(); ++t) {
-            const auto &w = slot_where[t];
-            w16[t] = make_uint4(w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16), w[6] | (w[7] << 16));
-        }
-        ctx->orb_stride = round_up(longest, 4) + 4;
-        ctx->orb_batch = std::min<uint32_t>(kScreenBatch, std::max<uint32_t>(1, kScreenLds / 4 / ctx->orb_stride));
-        tables.add(&ctx->d_orb_slots, slots);
-        tables.add(&ctx->d_orb_bands, bands);
-        tables.add(&ctx->d_orb_where, w16);
-        std::vector<unsigned short> place;
-        for (const auto &w : where) place.insert(place.end(), w.begin(), w.end());
-        tables.add(&ctx->d_orb_place, place);
     }
     TRY(tables.commit(ctx, &ctx->d_orb_tables));
     {
         const uint32_t blocks = (ctx->nrr_eff + (1u << ctx->orb_rl) - 1) >> ctx->orb_rl, groups = orbit_piece_groups(Kp / 16, ctx->orb_rl);
-        const size_t entries = (size_t)blocks * groups * 1024;
+        const uint32_t tiles = (ctx->nrr_eff + 15) / 16;
+        const size_t entries = f32 ? (size_t)tiles * Kp * 16 : (size_t)blocks * groups * 1024;
         TRY(dev_alloc(ctx, &ctx->d_orb_index, entries));
         TRY(dev_alloc(ctx, &ctx->d_orb_frac, entries));
         OrbitTable t{};
@@ -3714,27 +3731,29 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         t.stride = ctx->orb_prep_lds ? orbit_stride(ctx->I) : ctx->I;
         t.channel = ctx->orb_prep_lds ? orbit_tile(ctx->I) : ctx->I * ctx->I;
         t.I = ctx->I; t.D = D; t.nrr = ctx->nrr_eff; t.pieces = Kp / 16; t.rl = ctx->orb_rl;
-        hipLaunchKernelGGL(k_orbit_table, dim3((groups * 1024 + 255) / 256, blocks), dim3(256), 0, ctx->stream, t);
+        if (f32) hipLaunchKernelGGL(k_coef_table, dim3((uint32_t)(entries / 256)), dim3(256), 0, ctx->stream, t, Kp / 512);
+        else hipLaunchKernelGGL(k_orbit_table, dim3((groups * 1024 + 255) / 256, blocks), dim3(256), 0, ctx->stream, t);
         TRY(launch_check(ctx, "k_orbit_table"));
     }
-    ctx->orb_pitch = ctx->trainer ? round_up(ctx->nrr_eff, 32) : ctx->nrr_eff;
-    ctx->screen_train = ctx->trainer && ctx->orb_mode == ORB_F32;
+    ctx->orb_pitch = ctx->trainer ? round_up(ctx->nrr_eff, f32 ? 16 : 32) : ctx->nrr_eff;
+    ctx->screen_train = ctx->trainer && f32;
     ctx->orbit = !ctx->screen_train;
     ctx->orbit_train = ctx->trainer && ctx->orbit;
     return PINK_HIP_OK;
 }
 
-// Bytes of a launch group of B images: the row operand (whole tiles of 32 rows), norms, and float32's squared distances.
+// Bytes of a launch group of B images: the row operand (whole tiles of 32 rows; float32: of 16), norms, a float32 mapper's words.
 size_t orbit_rows_bytes(const pink_hip_ctx *ctx, size_t B)
 {
+    if (ctx->orb_mode == ORB_F32) return (B * ctx->orb_pitch + 15) / 16 * ctx->orb_KS * 1024;
     return (size_t)(ctx->orb_mode == ORB_U8 ? 1 : 2) * ((B * ctx->orb_pitch + 31) / 32) * ctx->orb_KS * 1024;
 }
 
 size_t orbit_image_bytes(const pink_hip_ctx *ctx)
 {
     return orbit_rows_bytes(ctx, 1) + (size_t)ctx->N * 24 +
-           ctx->nrr_eff * (64 + (is_int(ctx) || ctx->trainer ? (size_t)0 : 4 + 4 * (size_t)ctx->N * ctx->orb_ns) +
-                           (is_int(ctx) && !ctx->trainer ? (size_t)0 : (size_t)ctx->orb_KS * 128));
+           ctx->nrr_eff * (64 + (is_int(ctx) || ctx->trainer ? (size_t)0 : 4 * (size_t)ctx->N) +
+                           (is_int(ctx) && !ctx->trainer ? (size_t)0 : is_int(ctx) ? (size_t)ctx->orb_KS * 128 : (size_t)ctx->orb_Ox * 32));
 }
 
 // Float32 mappers: whether a full launch group of images is screened (see k_screen_exact; few images are summed all the same,
@@ -3761,6 +3780,9 @@ uint32_t summed_images(const pink_hip_ctx *ctx)
     return (uint32_t)std::min({images, (double)ctx->Bcap, (double)((size_t)1 << 30) / (double)row_bytes});
 }
 
+// (the neuron's row and its operand; an odd square's orbits are up to a quarter of its elements where these are few)
+size_t screen_update_lds(uint32_t Epad, uint32_t Op) { return (size_t)Epad * sizeof(float) + (size_t)Op * 16; }
+
 // Trainers that take the orbits' product: integers where the resident form (init_sym_train) does not fit, which keep their
 // weights in that order too; float32 where every variant's sum costs more than the product, the few sums that are left and
 // three launches more.  Those sums are a chain of E steps whatever the SOM's size, so there have to be two neurons per CU, and
@@ -3771,7 +3793,7 @@ bool orbit_trains(const pink_hip_ctx *ctx)
 {
     if (!is_int(ctx))
         return ctx->R >= 128 && ctx->N >= 2 * (uint32_t)ctx->num_cu && (size_t)ctx->N * ctx->R * ctx->E >= 1000000000 &&
-               ctx->E < 65535 && (size_t)ctx->Epad * sizeof(float) + 1024 <= ctx->lds_max;
+               ctx->E < 65535 && screen_update_lds(ctx->Epad, ctx->Epad / 4 + 64) + 1024 <= ctx->lds_max;
     // (below a dozen base rotations the product's tiles of 64 rows are mostly empty)
     if (!ctx->gemm || ctx->E < 1024 || ctx->nrr_eff < 12 || !resident_allowed()) return false;
     uint32_t npb = 1;
@@ -3785,16 +3807,20 @@ bool orbit_trains(const pink_hip_ctx *ctx)
 int run_orbit_som(pink_hip_ctx *ctx)
 {
     const uint32_t Kp = ctx->orb_KS * 32;
+    if (ctx->orb_mode == ORB_F32) {
+        CoefSom a{ctx->d_som, ctx->d_orb_elem, ctx->d_coef_weight, (uint32_t *)ctx->d_orb_som, (CoefNeuron *)ctx->d_coef_neuron, ctx->S, Kp / 8};
+        hipLaunchKernelGGL(k_coef_som, dim3(ctx->N), dim3(256), 0, ctx->stream, a);
+        return launch_check(ctx, "k_coef_som");
+    }
     // (the next set is the one that an update adds to)
     ctx->orb_cur = 0;
     if (ctx->orbit_train) HIP_TRY(ctx, hipMemsetAsync(ctx->d_orb_na, 0, 3 * (size_t)ctx->N * sizeof(long long), ctx->stream));
     auto go = [&](auto mode) {
         hipLaunchKernelGGL(k_orbit_som<decltype(mode)::value>, dim3(ctx->N), dim3(256), 0, ctx->stream, ctx->d_som, ctx->d_orb_elem,
-                           (int *)ctx->d_orb_som, ctx->d_orb_na, ctx->d_orb_sa, ctx->d_orb_ea, ctx->d_orb_values, ctx->S, Kp, (size_t)ctx->N * Kp);
+                           (int *)ctx->d_orb_som, ctx->d_orb_na, ctx->d_orb_values, ctx->S, Kp, (size_t)ctx->N * Kp);
     };
     if (ctx->orb_mode == ORB_U8) go(std::integral_constant<int, ORB_U8>{});
-    else if (ctx->orb_mode == ORB_U16) go(std::integral_constant<int, ORB_U16>{});
-    else go(std::integral_constant<int, ORB_F32>{});
+    else go(std::integral_constant<int, ORB_U16>{});
     return launch_check(ctx, "k_orbit_som");
 }
 
@@ -3805,9 +3831,8 @@ int run_screen_range(pink_hip_ctx *ctx)
     return launch_check(ctx, "k_screen_range");
 }
 
-// (finish: whether the sums of splits, if there are any, become keys or distances here)
 template <int MODE, int WM, int WN, int KC, int PD, int MINB>
-void launch_orbit_gemm(pink_hip_ctx *ctx, OrbitGemm &a, bool finish)
+void launch_orbit_gemm(pink_hip_ctx *ctx, OrbitGemm &a)
 {
     a.row_tiles = (a.M + 64 * WM - 1) / (64 * WM);
     a.col_tiles = (a.N * a.ns + 64 * WN - 1) / (64 * WN);
@@ -3824,7 +3849,7 @@ void launch_orbit_gemm(pink_hip_ctx *ctx, OrbitGemm &a, bool finish)
     a.splits = (steps + a.steps_per - 1) / a.steps_per;
     const uint32_t per = (tiles * a.splits + 7) / 8;
     hipLaunchKernelGGL((k_orbit_gemm<MODE, WM, WN, KC, PD, MINB>), dim3(8 * per), dim3(256), orbit_gemm_lds(MODE, WM, WN, KC, a.ns, a.nrr), ctx->stream, a);
-    if (a.splits > 1 && finish)
+    if (a.splits > 1)
         hipLaunchKernelGGL(k_orbit_finish<MODE>, dim3((a.N * a.ns + 63) / 64, (a.M + 3) / 4), dim3(256), 0, ctx->stream, a);
 }
 
@@ -3838,13 +3863,33 @@ uint32_t screen_keep(uint32_t R) { return std::max(16u, R / 4); }
 int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
 {
     Timed t(ctx, kClsRotate);
+    if (ctx->orb_mode == ORB_F32) {
+        CoefPrep p{};
+        p.images = dev_images; p.index = ctx->d_orb_index; p.frac = ctx->d_orb_frac; p.weight = ctx->d_coef_weight; p.outside = ctx->d_coef_outside;
+        p.opnd = (uint32_t *)ctx->d_orb_rows; p.row = (CoefRow *)ctx->d_coef_row; p.image = (CoefImage *)ctx->d_coef_image; p.xrows = ctx->d_orb_x;
+        if (!ctx->trainer) { p.wide_count = ctx->d_screen_counts + 1; p.list_count = ctx->d_screen_counts; p.upper = ctx->d_coef_upper; }
+        p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.Op = ctx->orb_KS * 4; p.Ox = ctx->orb_Ox; p.all_sym = ctx->orb_all; p.pitch = ctx->orb_pitch;
+        // Large images: a block has a CU to itself and takes all its waves.  Others: four waves, so that blocks that load, work and store share a
+        // CU, and as many tiles as leave a dozen waves per CU (an image is loaded once for them).
+        const bool large = ctx->orb_prep_lds > 50 * 1024 || !ctx->orb_prep_lds;
+        const uint32_t tiles = (ctx->nrr_eff + 15) / 16, quarters = p.Ox / 16;
+        p.tiles = std::min({tiles, kPrepareTiles, std::max(1u, (uint32_t)((size_t)B * tiles / (3 * (size_t)ctx->num_cu)))});
+        if (large) p.tiles = std::min(p.tiles, (2 * coef_prepare_waves(true) + quarters - 1) / quarters);
+        const uint32_t waves = std::min(large || B * tiles < 2 * (uint32_t)ctx->num_cu ? coef_prepare_waves(ctx->orb_prep_lds != 0) : 4u, quarters * p.tiles);
+        void *args[] = {&p};
+        HIP_TRY(ctx, hipLaunchKernel(orbit_prepare_kernel(ctx), dim3(B, (tiles + p.tiles - 1) / p.tiles), dim3(64 * waves), args, ctx->orb_prep_lds, ctx->stream));
+        if (ctx->coef_beside) {
+            const CoefBeside e{ctx->d_orb_x, ctx->d_coef_beside, p.row, ctx->coef_beside, B * ctx->nrr_eff, p.Ox * 8};
+            hipLaunchKernelGGL(k_coef_beside, dim3((e.rows + 3) / 4), dim3(256), 0, ctx->stream, e);
+            TRY(launch_check(ctx, "k_coef_beside"));
+        }
+        return PINK_HIP_OK;
+    }
     OrbitPrep p{};
     p.images = dev_images; p.index = ctx->d_orb_index; p.frac = ctx->d_orb_frac; p.mask = ctx->d_orb_mask;
-    p.opnd = ctx->d_orb_rows; p.norm = ctx->d_orb_nb; p.key = is_int(ctx) ? ctx->d_key : nullptr; p.scale = ctx->d_orb_sb; p.err = ctx->d_orb_eb;
+    p.opnd = ctx->d_orb_rows; p.norm = ctx->d_orb_nb; p.key = ctx->d_key;
     p.xrows = ctx->d_orb_x; p.plane = orbit_rows_plane(ctx, B); p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.KS = ctx->orb_KS;
     p.all_sym = ctx->orb_all; p.rl = ctx->orb_rl; p.pitch = ctx->orb_pitch;
-    p.wide_count = ctx->orbit && !is_int(ctx) ? ctx->d_screen_counts : nullptr;
-    p.negative = ctx->d_screen_negative;
     const dim3 grid(B, (ctx->nrr_eff + (1u << p.rl) - 1) >> p.rl);
     const uint32_t threads = ctx->orb_prep_lds > 64 * 1024 || grid.x * grid.y < (uint32_t)ctx->num_cu ? 1024 : ctx->orb_prep_lds > 24 * 1024 ? 512 : 256;
     void *args[] = {&p};
@@ -3852,85 +3897,143 @@ int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
     return PINK_HIP_OK;
 }
 
-// Keys of `B` images from image slot `slot` of a group of `of` images whose rows are there: the product and, for float32,
-// the exact sums of what is left.
+// How a float32 product is cut into splits: as many as fill the chip twice, of at least two steps, as far as the buffer goes.
+void coef_splits(const pink_hip_ctx *ctx, CoefGemm &a)
+{
+    const size_t blocks = (size_t)a.row_tiles * a.col_tiles, part = (size_t)a.M * a.N * 8 * sizeof(float);
+    const uint32_t splits = (uint32_t)std::min<size_t>({std::max<size_t>(1, 2 * (size_t)ctx->num_cu / blocks), std::max(1u, a.steps / 2), std::max<size_t>(1, ctx->orb_part_bytes / part)});
+    a.steps_per = (a.steps + splits - 1) / splits;
+    a.splits = (a.steps + a.steps_per - 1) / a.steps_per;
+}
+CoefGemm coef_gemm_args(const pink_hip_ctx *ctx, uint32_t slot, uint32_t B)
+{
+    CoefGemm a{};
+    a.M = B * ctx->nrr_eff; a.N = ctx->N; a.E = ctx->E; a.steps = ctx->orb_KS / 16; a.nrr = ctx->nrr_eff; a.valid = ctx->orb_valid; a.all_sym = ctx->orb_all;
+    a.rows = ctx->d_orb_rows + (size_t)slot * (ctx->orb_pitch / 16) * a.steps * 1024; a.som = ctx->d_orb_som;
+    a.row = (const CoefRow *)ctx->d_coef_row + (size_t)slot * a.nrr; a.neuron = (const CoefNeuron *)ctx->d_coef_neuron;
+    a.image = (const CoefImage *)ctx->d_coef_image + slot; a.words = ctx->d_coef_words; a.upper = ctx->d_coef_upper; a.part = (float *)ctx->d_orb_part;
+    a.row_tiles = (a.M + 63) / 64;
+    a.col_tiles = (a.N + 15) / 16;
+    return a;
+}
+template <bool PARTS>
+void launch_coef_gemm(pink_hip_ctx *ctx, CoefGemm &a)
+{
+    const uint32_t per = (a.row_tiles * a.col_tiles * (PARTS ? a.splits : 1) + 7) / 8;
+    hipLaunchKernelGGL(k_coef_gemm<PARTS>, dim3(8 * per), dim3(256), 0, ctx->stream, a);
+}
+void launch_coef_map(pink_hip_ctx *ctx, CoefGemm &a)
+{
+    // two blocks to a CU
+    const uint32_t chunks = std::min((a.row_tiles + 7) / 8, std::max(1u, 2 * (uint32_t)ctx->num_cu / 8 / a.col_tiles)) * 8;
+    hipLaunchKernelGGL(k_coef_map, dim3(chunks * a.col_tiles), dim3(256), a.steps * 16 * kCoefStride * 16, ctx->stream, a);
+}
+
+// A float32 mapper's keys, its images' rows there: the product's words, the variants that they leave, their sums.
+int run_coef_keys(pink_hip_ctx *ctx, uint32_t B)
+{
+    Timed t(ctx, kClsDist);
+    CoefGemm a = coef_gemm_args(ctx, 0, B);
+    const uint32_t cu = (uint32_t)ctx->num_cu;
+    if (a.row_tiles * a.col_tiles < cu && a.steps > 2) {
+        coef_splits(ctx, a);
+        launch_coef_gemm<true>(ctx, a);
+        hipLaunchKernelGGL(k_coef_finish, dim3((a.M * a.N + 255) / 256), dim3(256), 0, ctx->stream, a);
+    } else if (a.steps <= kMapSteps) launch_coef_map(ctx, a);
+    else launch_coef_gemm<false>(ctx, a);
+    TRY(launch_check(ctx, "k_coef_gemm"));
+    CoefPick q{};
+    q.words = a.words; q.upper = a.upper; q.key = ctx->d_key; q.list = ctx->d_screen_list; q.list_count = ctx->d_screen_counts;
+    q.wide = ctx->d_screen_wide; q.wide_count = ctx->d_screen_counts + 1; q.N = a.N; q.nrr = a.nrr; q.total = B * a.N;
+    hipLaunchKernelGGL(k_coef_pick, dim3((q.total + 63) / 64), dim3(256), 0, ctx->stream, q);
+    TRY(launch_check(ctx, "k_coef_pick"));
+    CoefPairs x{};
+    x.som_rows = (const float *)ctx->d_somP; x.xrows = ctx->d_orb_x; x.place = ctx->d_orb_place; x.list = q.list; x.list_count = q.list_count; x.key = q.key;
+    x.N = a.N; x.E = a.E; x.Epad = ctx->Epad; x.K = ctx->orb_Ox * 8; x.nrr = a.nrr; x.num_rot = ctx->cfg.num_rot;
+    // a row in LDS where eight waves of a CU have room for theirs
+    const uint32_t row = pair_row(x.E) + 4;
+    const bool whole = ctx->d_coef_to && row * 4 * 8 <= ctx->lds_max;
+    x.lds = whole ? row : 64 * (16 + 4);
+    x.to = ctx->d_coef_to;
+    const uint32_t lds = x.lds * 4 * kPairWaves;
+    const dim3 pairs(std::min((q.total + 1) / 2, std::min(8u, (uint32_t)(ctx->lds_max / lds)) * cu));
+    if (!whole) hipLaunchKernelGGL((k_coef_pairs<false, 16>), pairs, dim3(64 * kPairWaves), lds, ctx->stream, x);
+    else if (pair_run(x.E) == 4) hipLaunchKernelGGL((k_coef_pairs<true, 4>), pairs, dim3(64 * kPairWaves), lds, ctx->stream, x);
+    else if (pair_run(x.E) == 8) hipLaunchKernelGGL((k_coef_pairs<true, 8>), pairs, dim3(64 * kPairWaves), lds, ctx->stream, x);
+    else hipLaunchKernelGGL((k_coef_pairs<true, 16>), pairs, dim3(64 * kPairWaves), lds, ctx->stream, x);
+    TRY(launch_check(ctx, "k_coef_pairs"));
+    ScreenWide w{};
+    w.som_rows = x.som_rows; w.xrows = x.xrows; w.place = ctx->d_orb_place; w.wide = q.wide; w.wide_count = q.wide_count; w.key = q.key;
+    w.N = x.N; w.E = x.E; w.Epad = ctx->Epad; w.K = x.K; w.nrr = x.nrr; w.num_rot = x.num_rot; w.images = B;
+    // (a block to a CU, two of them are no faster; fewer where even every neuron listed makes less work)
+    const size_t most = (size_t)B * ((w.nrr + 64 / ctx->orb_ns - 1) / (64 / ctx->orb_ns)) * ((w.N + 63) / 64);
+    const dim3 grid((uint32_t)std::min<size_t>((most + 7) / 8 * 8, (size_t)cu / 8 * 8));
+    if (ctx->orb_ns == 8) hipLaunchKernelGGL(k_screen_wide<8>, grid, dim3(kWideThreads), 0, ctx->stream, w);
+    else hipLaunchKernelGGL(k_screen_wide<4>, grid, dim3(kWideThreads), 0, ctx->stream, w);
+    return launch_check(ctx, "k_screen_wide");
+}
+
+// A float32 trainer's closest variants for the image in slot `slot`, as far as the update needs them.
+int run_screen_keys(pink_hip_ctx *ctx, uint32_t slot)
+{
+    Timed t(ctx, kClsDist);
+    CoefGemm a = coef_gemm_args(ctx, slot, 1);
+    a.skip = ctx->d_screen_counts + 2 * kCounts;
+    coef_splits(ctx, a);
+    launch_coef_gemm<true>(ctx, a);
+    TRY(launch_check(ctx, "k_coef_gemm"));
+    ctx->screen_set ^= 1;
+    uint32_t *counts = ctx->d_screen_counts + kCounts * ctx->screen_set, *counts_next = ctx->d_screen_counts + kCounts * (ctx->screen_set ^ 1);
+    ScreenSelect l{};
+    l.g = a; l.key = ctx->d_key + (size_t)slot * ctx->N; l.bound = ctx->d_screen_bound;
+    l.list = ctx->d_screen_list; l.wide = ctx->d_screen_wide; l.counts = counts; l.counts_next = counts_next;
+    l.num_rot = ctx->cfg.num_rot; l.keep = screen_keep(ctx->R);
+    hipLaunchKernelGGL(k_screen_select, dim3((ctx->N + 15) / 16), dim3(64 * kSelectWaves), 0, ctx->stream, l);
+    TRY(launch_check(ctx, "k_screen_select"));
+    ScreenSums x{};
+    x.som_rows = (const float *)ctx->d_somP; x.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad;
+    x.list = l.list; x.wide = l.wide; x.counts = counts; x.key = l.key; x.bound = l.bound; x.factors = ctx->d_factors;
+    x.moves = ctx->d_screen_moves + (size_t)slot * ctx->N; x.choice = ctx->d_screen_choice;
+    x.range = (const WeightRange *)ctx->d_screen_range; x.image = a.image;
+    x.N = ctx->N; x.Epad = ctx->Epad; x.R = ctx->R; x.Rpad = ctx->Rpad;
+    x.wide_blocks = x.pair_blocks = 2 * (uint32_t)ctx->num_cu;
+    const dim3 sums(x.wide_blocks + x.pair_blocks);
+    if (ctx->Epad <= 512) hipLaunchKernelGGL(k_screen_sums<8>, sums, dim3(64 * kSumsWaves), 0, ctx->stream, x);
+    else if (ctx->Epad <= 1024) hipLaunchKernelGGL(k_screen_sums<16>, sums, dim3(64 * kSumsWaves), 0, ctx->stream, x);
+    else hipLaunchKernelGGL(k_screen_sums<32>, sums, dim3(64 * kSumsWaves), 0, ctx->stream, x);
+    TRY(launch_check(ctx, "k_screen_sums"));
+    if (screen_items(ctx->N, ctx->R) <= 2 * x.wide_blocks) return PINK_HIP_OK;
+    const uint32_t many = ctx->Rpad / kWave * ((ctx->N + 7) / 8);
+    hipLaunchKernelGGL(k_screen_many, dim3((many + 7) / 8 * 8), dim3(256), 0, ctx->stream, x);
+    return launch_check(ctx, "k_screen_many");
+}
+
+// Keys of `B` images from image slot `slot` of a group of `of` images whose rows are there (integers).
 int run_orbit_keys(pink_hip_ctx *ctx, uint32_t slot, uint32_t B, uint32_t of)
 {
-    const bool u8 = ctx->orb_mode == ORB_U8, f32 = ctx->orb_mode == ORB_F32;
+    const bool u8 = ctx->orb_mode == ORB_U8;
     const uint32_t M = B * ctx->nrr_eff;
     const size_t rows_plane = orbit_rows_plane(ctx, of), row = (size_t)slot * ctx->nrr_eff, set = (size_t)ctx->orb_cur * ctx->N;
     unsigned long long *key = ctx->d_key + (size_t)slot * ctx->N;
     Timed t(ctx, kClsDist);
     OrbitGemm a{};
     a.rows = ctx->d_orb_rows + (size_t)slot * (ctx->orb_pitch / 32) * ctx->orb_KS * 64; a.som = ctx->d_orb_som; a.norm_rows = ctx->d_orb_nb + row * 8; a.norm_som = ctx->d_orb_na + set; a.selectors = ctx->d_orb_sel;
-    a.key = key; a.dump = ctx->d_orb_dump; a.part = ctx->d_orb_part; a.scale_rows = ctx->d_orb_sb ? ctx->d_orb_sb + slot : nullptr; a.scale_som = ctx->d_orb_sa;
+    a.key = key; a.part = ctx->d_orb_part;
     a.rows_plane = rows_plane; a.som_plane = (size_t)ctx->N * ctx->orb_KS * 2;
     a.M = M; a.N = ctx->N; a.KS = ctx->orb_KS; a.nrr = ctx->nrr_eff; a.num_rot = ctx->cfg.num_rot; a.ns = ctx->orb_ns; a.valid = ctx->orb_valid;
-    a.skip = ctx->screen_train ? ctx->d_screen_counts + 2 * kCounts : nullptr;
     // 64 x 128 tiles (a wave 32 x 64) read the operands less often; 64 x 64 ones fill the chip with few rows, and with two
     // planes and short rows more of their blocks hide each other's beginnings and ends
     const size_t columns = (size_t)a.N * a.ns, tiles = (size_t)((M + 63) / 64) * ((columns + 127) / 128);
     const bool small = tiles < (size_t)4 * ctx->num_cu || (!u8 && a.KS < 64);
-    const bool finish = !ctx->screen_train || a.nrr > kSelectRows;         // (k_screen_select does it)
-    switch (ctx->orb_mode) {
-    case ORB_U8: if (small) launch_orbit_gemm<ORB_U8, 1, 1, 4, 4, 4>(ctx, a, finish); else launch_orbit_gemm<ORB_U8, 1, 2, 4, 1, 4>(ctx, a, finish); break;
-    case ORB_U16: if (small) launch_orbit_gemm<ORB_U16, 1, 1, 2, 4, 3>(ctx, a, finish); else launch_orbit_gemm<ORB_U16, 1, 2, 2, 1, 3>(ctx, a, finish); break;
-    default: if (small) launch_orbit_gemm<ORB_F32, 1, 1, 2, 4, 3>(ctx, a, finish); else launch_orbit_gemm<ORB_F32, 1, 2, 2, 1, 3>(ctx, a, finish); break;
-    }
-    TRY(launch_check(ctx, "k_orbit_gemm"));
-    if (!f32) return PINK_HIP_OK;
-    if (ctx->screen_train) {
-        ctx->screen_set ^= 1;
-        uint32_t *counts = ctx->d_screen_counts + kCounts * ctx->screen_set, *counts_next = ctx->d_screen_counts + kCounts * (ctx->screen_set ^ 1);
-        ScreenSelect l{};
-        l.dump = ctx->d_orb_dump; l.err_rows = ctx->d_orb_eb + row; l.err_som = ctx->d_orb_ea; l.key = key;
-        l.list = ctx->d_screen_list; l.wide = ctx->d_screen_wide; l.counts = counts; l.counts_next = counts_next;
-        l.skip = a.skip; l.bound = ctx->d_screen_bound; l.keep = screen_keep(ctx->R);
-        l.N = ctx->N; l.E = ctx->E; l.nrr = ctx->nrr_eff; l.num_rot = ctx->cfg.num_rot; l.ns = ctx->orb_ns; l.valid = ctx->orb_valid;
-        const dim3 blocks((uint32_t)((columns + 63) / 64));
-        if (a.splits > 1 && !finish) hipLaunchKernelGGL(k_screen_select<true>, blocks, dim3(64 * kSelectWaves), 0, ctx->stream, l, a);
-        else hipLaunchKernelGGL(k_screen_select<false>, blocks, dim3(64 * kSelectWaves), 0, ctx->stream, l, a);
-        TRY(launch_check(ctx, "k_screen_select"));
-        ScreenSums x{};
-        x.som_rows = (const float *)ctx->d_somP; x.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad;
-        x.list = l.list; x.wide = l.wide; x.counts = counts; x.key = key; x.bound = l.bound; x.factors = ctx->d_factors;
-        x.moves = ctx->d_screen_moves + (size_t)slot * ctx->N; x.choice = ctx->d_screen_choice;
-        x.range = (const WeightRange *)ctx->d_screen_range; x.scale_rows = a.scale_rows;
-        x.N = ctx->N; x.Epad = ctx->Epad; x.R = ctx->R; x.Rpad = ctx->Rpad;
-        x.wide_blocks = x.pair_blocks = 2 * (uint32_t)ctx->num_cu;
-        const dim3 sums(x.wide_blocks + x.pair_blocks);
-        if (ctx->Epad <= 512) hipLaunchKernelGGL(k_screen_sums<8>, sums, dim3(64 * kSumsWaves), 0, ctx->stream, x);
-        else if (ctx->Epad <= 1024) hipLaunchKernelGGL(k_screen_sums<16>, sums, dim3(64 * kSumsWaves), 0, ctx->stream, x);
-        else hipLaunchKernelGGL(k_screen_sums<32>, sums, dim3(64 * kSumsWaves), 0, ctx->stream, x);
-        TRY(launch_check(ctx, "k_screen_sums"));
-        if (screen_items(ctx->N, ctx->R) <= 2 * x.wide_blocks) return PINK_HIP_OK;
-        const uint32_t pairs = ctx->Rpad / kWave * ((ctx->N + 7) / 8);
-        hipLaunchKernelGGL(k_screen_many, dim3((pairs + 7) / 8 * 8), dim3(256), 0, ctx->stream, x);
-        return launch_check(ctx, "k_screen_many");
-    }
-    ScreenExact x{};
-    x.dump = ctx->d_orb_dump; x.values = ctx->d_orb_values; x.xrows = ctx->d_orb_x + row * ctx->orb_KS * 32; x.err_rows = ctx->d_orb_eb + row; x.err_som = ctx->d_orb_ea;
-    x.slots = ctx->d_orb_slots; x.bands = ctx->d_orb_bands; x.where = ctx->d_orb_where; x.key = key;
-    x.N = ctx->N; x.E = ctx->E; x.K = ctx->orb_KS * 32; x.nrr = ctx->nrr_eff; x.num_rot = ctx->cfg.num_rot;
-    x.ns = ctx->orb_ns; x.valid = ctx->orb_valid; x.band_count = ctx->orb_bands;
-    x.stride = ctx->orb_stride; x.batch = ctx->orb_batch; x.wide = ctx->d_screen_wide; x.wide_count = ctx->d_screen_counts;
-    hipLaunchKernelGGL(k_screen_exact, dim3((ctx->N * x.ns + 31) / 32, B), dim3(256), (size_t)x.batch * x.stride * sizeof(float), ctx->stream, x);
-    TRY(launch_check(ctx, "k_screen_exact"));
-    ScreenWide w{};
-    w.som_rows = (const float *)ctx->d_somP; w.xrows = x.xrows; w.place = ctx->d_orb_place; w.wide = x.wide; w.wide_count = x.wide_count; w.key = key;
-    w.N = x.N; w.E = x.E; w.Epad = ctx->Epad; w.K = x.K; w.nrr = x.nrr; w.num_rot = x.num_rot; w.images = B;
-    // (a block to a CU, two of them are no faster; fewer where even every neuron listed makes less work)
-    const size_t most = (size_t)B * ((w.nrr + 64 / x.ns - 1) / (64 / x.ns)) * ((w.N + 63) / 64);
-    const dim3 grid((uint32_t)std::min<size_t>((most + 7) / 8 * 8, (size_t)ctx->num_cu / 8 * 8));
-    if (x.ns == 8) hipLaunchKernelGGL(k_screen_wide<8>, grid, dim3(kWideThreads), 0, ctx->stream, w);
-    else hipLaunchKernelGGL(k_screen_wide<4>, grid, dim3(kWideThreads), 0, ctx->stream, w);
-    return launch_check(ctx, "k_screen_wide");
+    if (u8) { if (small) launch_orbit_gemm<ORB_U8, 1, 1, 4, 4, 4>(ctx, a); else launch_orbit_gemm<ORB_U8, 1, 2, 4, 1, 4>(ctx, a); }
+    else { if (small) launch_orbit_gemm<ORB_U16, 1, 1, 2, 4, 3>(ctx, a); else launch_orbit_gemm<ORB_U16, 1, 2, 2, 1, 3>(ctx, a); }
+    return launch_check(ctx, "k_orbit_gemm");
 }
 
 int run_orbit(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
 {
     TRY(run_orbit_rows(ctx, dev_images, B));
-    return run_orbit_keys(ctx, 0, B, B);
+    return ctx->orb_mode == ORB_F32 ? run_coef_keys(ctx, B) : run_orbit_keys(ctx, 0, B, B);
 }
 
 // The update of the image in slot `slot` of a float32 trainer that screens its distances.
@@ -3939,12 +4042,12 @@ int run_screen_update(pink_hip_ctx *ctx, uint32_t slot, uint32_t *dev_bmu_out)
     Timed t(ctx, kClsUpdate);
     ScreenUpdate u{};
     u.som_rows = (float *)ctx->d_somP; u.rows = (const float *)ctx->d_rotT + (size_t)slot * ctx->Epad * ctx->Rpad; u.factors_t = ctx->d_factors_t;
-    u.element = ctx->d_orb_element; u.listed = ctx->d_screen_counts + kCounts * ctx->screen_set; u.skip = ctx->d_screen_counts + 2 * kCounts;
-    u.opnd = (uint2 *)ctx->d_orb_som; u.key = ctx->d_key + (size_t)slot * ctx->N; u.norm = ctx->d_orb_na; u.scale = ctx->d_orb_sa; u.err = ctx->d_orb_ea;
+    u.element = ctx->d_orb_element; u.weight = ctx->d_coef_weight; u.listed = ctx->d_screen_counts + kCounts * ctx->screen_set; u.skip = ctx->d_screen_counts + 2 * kCounts;
+    u.opnd = ctx->d_orb_som; u.neuron = (CoefNeuron *)ctx->d_coef_neuron; u.key = ctx->d_key + (size_t)slot * ctx->N;
     u.bound = ctx->d_screen_bound; u.moves = ctx->d_screen_moves + (size_t)slot * ctx->N; u.choice = ctx->d_screen_choice;
-    u.range = (WeightRange *)ctx->d_screen_range; u.scale_rows = ctx->d_orb_sb + slot; u.negative = ctx->d_screen_negative + slot;
-    u.bmu_out = dev_bmu_out; u.counts = ctx->d_counts; u.plane = (size_t)ctx->N * ctx->orb_KS * 32; u.N = ctx->N; u.K8 = ctx->orb_KS * 4; u.Epad = ctx->Epad;
-    hipLaunchKernelGGL(k_screen_update, dim3(ctx->N), dim3(512), (size_t)ctx->Epad * sizeof(float), ctx->stream, u);
+    u.range = (WeightRange *)ctx->d_screen_range; u.image = (const CoefImage *)ctx->d_coef_image + slot;
+    u.bmu_out = dev_bmu_out; u.counts = ctx->d_counts; u.N = ctx->N; u.Op = ctx->orb_KS * 4; u.Epad = ctx->Epad;
+    hipLaunchKernelGGL(k_screen_update, dim3(ctx->N), dim3(512), screen_update_lds(ctx->Epad, u.Op), ctx->stream, u);
     return launch_check(ctx, "k_screen_update");
 }
 
@@ -4335,22 +4438,26 @@ int init_ctx(pink_hip_ctx *ctx)
         TRY(dev_alloc(ctx, &ctx->d_Pb, B * ctx->RTP * pink_sym::unit_bytes(ctx->KSs)));
     } else if (ctx->orbit) {
         TRY(dev_alloc(ctx, (char **)&ctx->d_orb_rows, orbit_rows_bytes(ctx, B)));
-        TRY(dev_alloc(ctx, &ctx->d_orb_nb, B * ctx->nrr_eff * 8));
+        if (is_int(ctx)) TRY(dev_alloc(ctx, &ctx->d_orb_nb, B * ctx->nrr_eff * 8));
+        else TRY(dev_alloc(ctx, (CoefRow **)&ctx->d_coef_row, B * ctx->nrr_eff));
         // (a launch with fewer 64 x 64 tiles than compute units, in at most 16 splits)
         ctx->orb_part_bytes = std::min<size_t>((size_t)16 << 20, (size_t)2 * ctx->num_cu * 64 * 64 * (ctx->orb_mode == ORB_U8 ? 4 : 12));
+        if (!is_int(ctx)) ctx->orb_part_bytes = (size_t)64 * 16 * 2 * ctx->num_cu * 32;        // (fewer 64 x 16 tiles than compute units, twice as many splits)
         TRY(dev_alloc(ctx, (char **)&ctx->d_orb_part, ctx->orb_part_bytes));
         if (!is_int(ctx)) {
-            TRY(dev_alloc(ctx, &ctx->d_orb_sb, B));
-            TRY(dev_alloc(ctx, &ctx->d_orb_eb, B * ctx->nrr_eff));
-            TRY(dev_alloc(ctx, &ctx->d_orb_dump, B * ctx->nrr_eff * ctx->N * ctx->orb_ns));
+            TRY(dev_alloc(ctx, (CoefImage **)&ctx->d_coef_image, B));
+            TRY(dev_alloc(ctx, &ctx->d_coef_words, B * ctx->nrr_eff * ctx->N));
+            TRY(dev_alloc(ctx, &ctx->d_coef_upper, B * ctx->N));
+            TRY(dev_alloc(ctx, &ctx->d_screen_list, B * ctx->N * kPairKeep));
             TRY(dev_alloc(ctx, &ctx->d_screen_wide, B * ctx->N));
-            TRY(dev_alloc(ctx, &ctx->d_screen_counts, B));
+            TRY(dev_alloc(ctx, &ctx->d_screen_counts, B + 1));
             TRY(dev_alloc(ctx, (uint32_t **)&ctx->d_somP, (size_t)ctx->N * ctx->Epad + kDistOverrun));
             const size_t rows = (size_t)std::max(1u, ctx->sum_images) * ctx->Epad * ctx->Rpad;       // (pink_hip_rotate takes one image)
             TRY(dev_alloc(ctx, (uint32_t **)&ctx->d_rotT, rows + kDistOverrun));
             HIP_TRY(ctx, hipMemset(ctx->d_rotT, 0, rows * sizeof(uint32_t)));
         }
-        if (!is_int(ctx) || ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_x, B * ctx->nrr_eff * ctx->orb_KS * 32));
+        if (!is_int(ctx)) TRY(dev_alloc(ctx, &ctx->d_orb_x, B * ctx->nrr_eff * ctx->orb_Ox * 8));
+        else if (ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_x, B * ctx->nrr_eff * ctx->orb_KS * 32));
         if (ctx->trainer) {
             TRY(dev_alloc(ctx, &ctx->d_orb_best, B * ctx->N));
             const std::vector<uint32_t> outside = outside_elements(ctx, region);
@@ -4512,19 +4619,16 @@ int init_ctx(pink_hip_ctx *ctx)
         ctx->screen_train = ctx->screen_train && ctx->rows_f32_train;
         if (ctx->screen_train) {
             TRY(dev_alloc(ctx, (char **)&ctx->d_orb_rows, orbit_rows_bytes(ctx, B)));
-            TRY(dev_alloc(ctx, &ctx->d_orb_nb, B * ctx->nrr_eff * 8));
-            TRY(dev_alloc(ctx, &ctx->d_orb_sb, B));
-            TRY(dev_alloc(ctx, &ctx->d_orb_eb, B * ctx->nrr_eff));
-            TRY(dev_alloc(ctx, &ctx->d_orb_dump, (size_t)ctx->nrr_eff * ctx->N * ctx->orb_ns));
+            TRY(dev_alloc(ctx, (CoefRow **)&ctx->d_coef_row, B * ctx->nrr_eff));
+            TRY(dev_alloc(ctx, (CoefImage **)&ctx->d_coef_image, B));
             TRY(dev_alloc(ctx, &ctx->d_screen_list, (size_t)ctx->N * screen_keep(ctx->R)));
             TRY(dev_alloc(ctx, &ctx->d_screen_wide, ctx->N));
             TRY(dev_alloc(ctx, &ctx->d_screen_bound, ctx->N));
             TRY(dev_alloc(ctx, &ctx->d_screen_moves, B * ctx->N));
             TRY(dev_alloc(ctx, &ctx->d_screen_range, ctx->N));
-            TRY(dev_alloc(ctx, &ctx->d_screen_negative, B));
             TRY(dev_alloc(ctx, &ctx->d_screen_choice, 2));
             TRY(upload(ctx, &ctx->d_screen_counts, std::vector<uint32_t>(2 * kCounts + 1, 0u)));       // (two sets, images to skip)
-            ctx->orb_part_bytes = (size_t)16 << 20;
+            ctx->orb_part_bytes = std::max((size_t)24 << 20, (size_t)ctx->nrr_eff * ctx->N * 32);
             TRY(dev_alloc(ctx, (char **)&ctx->d_orb_part, ctx->orb_part_bytes));
             HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_screen_update, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 1024));
         }
@@ -4660,7 +4764,7 @@ int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, 
             uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group;
             for (uint32_t b = 0; b < B; ++b) {
                 if (ctx->screen_train) {
-                    TRY(run_orbit_keys(ctx, b, 1, B));
+                    TRY(run_screen_keys(ctx, b));
                     TRY(run_screen_update(ctx, b, bmu + b));
                     continue;
                 }
@@ -5094,8 +5198,8 @@ int pink_hip_map_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_i
 // The per-group buffers of a mapping call, per image, in the order they are carved out of the static
 // scratch (every piece starts on a 256-byte boundary).
 struct StaticPieces {
-    size_t key = 0, Pb = 0, nb = 0, gPb = 0, gnb = 0, rot = 0, rotT = 0, orows = 0, onb = 0, osb = 0, oeb = 0, odump = 0, ox = 0;
-    size_t per_image() const { return key + Pb + nb + gPb + gnb + rot + rotT + orows + onb + osb + oeb + odump + ox; }
+    size_t key = 0, Pb = 0, nb = 0, gPb = 0, gnb = 0, rot = 0, rotT = 0, orows = 0, onb = 0, oimage = 0, orow = 0, owords = 0, ox = 0;
+    size_t per_image() const { return key + Pb + nb + gPb + gnb + rot + rotT + orows + onb + oimage + orow + owords + ox; }
 };
 
 static StaticPieces static_pieces(const pink_hip_ctx *ctx, bool summed)
@@ -5105,12 +5209,12 @@ static StaticPieces static_pieces(const pink_hip_ctx *ctx, bool summed)
     p.key = up((size_t)ctx->N * sizeof(unsigned long long));
     if (ctx->orbit && !summed) {
         p.orows = up(orbit_rows_bytes(ctx, 1));
-        p.onb = up((size_t)ctx->nrr_eff * 64);
-        if (!is_int(ctx)) {
-            p.osb = up(sizeof(float));
-            p.oeb = up((size_t)ctx->nrr_eff * sizeof(float));
-            p.odump = up((size_t)ctx->nrr_eff * ctx->N * ctx->orb_ns * sizeof(float));
-            p.ox = up((size_t)ctx->nrr_eff * ctx->orb_KS * 32 * sizeof(float));
+        if (is_int(ctx)) p.onb = up((size_t)ctx->nrr_eff * 64);
+        else {
+            p.oimage = up(sizeof(CoefImage));
+            p.orow = up((size_t)ctx->nrr_eff * sizeof(CoefRow));
+            p.owords = up((size_t)ctx->nrr_eff * ctx->N * sizeof(uint32_t));
+            p.ox = up((size_t)ctx->nrr_eff * ctx->orb_Ox * 8 * sizeof(float));
         }
         return p;
     }
@@ -5169,9 +5273,9 @@ int pink_hip_map_device_static(pink_hip_ctx *ctx, const float *dev_images, uint3
     // the kernels take the scratch where they take the context's own buffers in pink_hip_map_device
     struct Saved {
         unsigned long long *key; signed char *Pb; int *nb; v4i *gPb; long long *gnb; float *rot; void *rotT;
-        v4i *orows; long long *onb; float *osb, *oeb, *odump, *ox;
+        v4i *orows; long long *onb; void *oimage, *orow; uint32_t *owords; float *ox;
     } const saved{ctx->d_key, ctx->d_Pb, ctx->d_nb, ctx->d_gPb, ctx->d_gnb, ctx->d_rot, ctx->d_rotT,
-                  ctx->d_orb_rows, ctx->d_orb_nb, ctx->d_orb_sb, ctx->d_orb_eb, ctx->d_orb_dump, ctx->d_orb_x};
+                  ctx->d_orb_rows, ctx->d_orb_nb, ctx->d_coef_image, ctx->d_coef_row, ctx->d_coef_words, ctx->d_orb_x};
     unsigned char *at = ctx->static_scratch;
     auto carve = [&](size_t bytes_per_image) { unsigned char *p = at; at += (size_t)B * bytes_per_image; return p; };
     ctx->d_key = (unsigned long long *)carve(pc.key);
@@ -5183,9 +5287,9 @@ int pink_hip_map_device_static(pink_hip_ctx *ctx, const float *dev_images, uint3
     if (pc.rotT) ctx->d_rotT = carve(pc.rotT);
     if (pc.orows) ctx->d_orb_rows = (v4i *)carve(pc.orows);
     if (pc.onb) ctx->d_orb_nb = (long long *)carve(pc.onb);
-    if (pc.osb) ctx->d_orb_sb = (float *)carve(pc.osb);
-    if (pc.oeb) ctx->d_orb_eb = (float *)carve(pc.oeb);
-    if (pc.odump) ctx->d_orb_dump = (float *)carve(pc.odump);
+    if (pc.oimage) ctx->d_coef_image = carve(pc.oimage);
+    if (pc.orow) ctx->d_coef_row = carve(pc.orow);
+    if (pc.owords) ctx->d_coef_words = (uint32_t *)carve(pc.owords);
     if (pc.ox) ctx->d_orb_x = (float *)carve(pc.ox);
     int rc = PINK_HIP_OK;
     for (uint32_t done = 0; done < n_images && rc == PINK_HIP_OK; done += B) {
@@ -5197,7 +5301,7 @@ int pink_hip_map_device_static(pink_hip_ctx *ctx, const float *dev_images, uint3
     }
     ctx->d_key = saved.key; ctx->d_Pb = saved.Pb; ctx->d_nb = saved.nb; ctx->d_gPb = saved.gPb; ctx->d_gnb = saved.gnb;
     ctx->d_rot = saved.rot; ctx->d_rotT = saved.rotT;
-    ctx->d_orb_rows = saved.orows; ctx->d_orb_nb = saved.onb; ctx->d_orb_sb = saved.osb; ctx->d_orb_eb = saved.oeb; ctx->d_orb_dump = saved.odump;
+    ctx->d_orb_rows = saved.orows; ctx->d_orb_nb = saved.onb; ctx->d_coef_image = saved.oimage; ctx->d_coef_row = saved.orow; ctx->d_coef_words = saved.owords;
     ctx->d_orb_x = saved.ox;
     return rc;
 }
