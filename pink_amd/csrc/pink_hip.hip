@@ -3780,20 +3780,21 @@ uint32_t summed_images(const pink_hip_ctx *ctx)
     return (uint32_t)std::min({images, (double)ctx->Bcap, (double)((size_t)1 << 30) / (double)row_bytes});
 }
 
-// (the neuron's row and its operand; an odd square's orbits are up to a quarter of its elements where these are few)
-size_t screen_update_lds(uint32_t Epad, uint32_t Op) { return (size_t)Epad * sizeof(float) + (size_t)Op * 16; }
-
 // Trainers that take the orbits' product: integers where the resident form (init_sym_train) does not fit, which keep their
-// weights in that order too; float32 where every variant's sum costs more than the product, the few sums that are left and
-// three launches more.  Those sums are a chain of E steps whatever the SOM's size, so there have to be two neurons per CU, and
-// (neurons x variants x elements, summed / screened time of an image; the first four with the sums in lists of three neurons each):
-// 0.3e9 0.66, 0.7e9 0.91, 0.84e9 1.01, 400 neurons of 2.9e9 0.97; 1.01e9 1.20, 1.06e9 1.10, 1.11e9 1.34, 1.31e9 1.37, 2.23e9 2.2,
-// 4.3e9 2.0.
+// weights in that order too; float32 where every variant's sum costs more than the product and the sums that it leaves.
+// Summing all: a chain of E steps and, with more neurons than fill the chip, its share of the vector ALUs, E (0.0095 + 4.6e-8 N R) us
+// per image; screening: five dependent launches and what grows with the elements, 22 + 0.0035 E.  (summed / screened
+// us at N R E: 9 720 2304 25 / 30, 9 720 4096 42 / 35, 9 720 16384 167 / 77, 100 720 2304 31 / 31, 100 720 4096 50 / 38, 256 720 1024
+// 25 / 27, 256 720 4096 80 / 41, 484 720 1024 34 / 30, 900 720 576 32 / 30, 1600 720 576 45 / 31, 1600 720 4096 255 / 58, 9 80 8100 72 / 28,
+// 900 80 8100 88 / 39.)  Very long rows leave many variants in question, whose rows come from memory again and again: 100 720 16384
+// 193 / 111, 49 720 29241 315 / 204, but 256 720 16384 297 / 325, 256 720 28900 544 / 719.
 bool orbit_trains(const pink_hip_ctx *ctx)
 {
-    if (!is_int(ctx))
-        return ctx->R >= 128 && ctx->N >= 2 * (uint32_t)ctx->num_cu && (size_t)ctx->N * ctx->R * ctx->E >= 1000000000 &&
-               ctx->E < 65535 && screen_update_lds(ctx->Epad, ctx->Epad / 4 + 64) + 1024 <= ctx->lds_max;
+    if (!is_int(ctx)) {
+        const double E = ctx->E, NR = (double)ctx->N * ctx->R;
+        return ctx->R >= 8 && E * (0.006 + 4.6e-8 * NR) >= 22.0 && (E <= 12000 || NR * E <= 1.7e9) && ctx->E < 65535 &&
+               (size_t)ctx->Epad * sizeof(float) + 1024 <= ctx->lds_max;
+    }
     // (below a dozen base rotations the product's tiles of 64 rows are mostly empty)
     if (!ctx->gemm || ctx->E < 1024 || ctx->nrr_eff < 12 || !resident_allowed()) return false;
     uint32_t npb = 1;
@@ -3857,7 +3858,9 @@ void launch_orbit_gemm(pink_hip_ctx *ctx, OrbitGemm &a)
 size_t orbit_rows_plane(const pink_hip_ctx *ctx, uint32_t B) { return (size_t)((B * ctx->orb_pitch + 31) / 32) * ctx->orb_KS * 64; }
 
 // Variants of a neuron that k_screen_select lists one by one; with more of them the neuron is summed whole.
-uint32_t screen_keep(uint32_t R) { return std::max(16u, R / 4); }
+// (a variant's sum takes what five variants of a whole neuron do, but no other waits for it; half of the variants, a quarter, us per
+// image: 256 neurons, 720 variants of 8100 elements 60, 87, 900 neurons 85, 118)
+uint32_t screen_keep(uint32_t R) { return std::max(8u, R / 2); }
 
 // The rows of B images, and their keys reset.
 int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
@@ -4047,7 +4050,9 @@ int run_screen_update(pink_hip_ctx *ctx, uint32_t slot, uint32_t *dev_bmu_out)
     u.bound = ctx->d_screen_bound; u.moves = ctx->d_screen_moves + (size_t)slot * ctx->N; u.choice = ctx->d_screen_choice;
     u.range = (WeightRange *)ctx->d_screen_range; u.image = (const CoefImage *)ctx->d_coef_image + slot;
     u.bmu_out = dev_bmu_out; u.counts = ctx->d_counts; u.N = ctx->N; u.Op = ctx->orb_KS * 4; u.Epad = ctx->Epad;
-    hipLaunchKernelGGL(k_screen_update, dim3(ctx->N), dim3(512), screen_update_lds(ctx->Epad, u.Op), ctx->stream, u);
+    const size_t row = (size_t)ctx->Epad * sizeof(float), both = row + (size_t)u.Op * 16;
+    if (both + 1024 <= ctx->lds_max) hipLaunchKernelGGL(k_screen_update<true>, dim3(ctx->N), dim3(512), both, ctx->stream, u);
+    else hipLaunchKernelGGL(k_screen_update<false>, dim3(ctx->N), dim3(512), row, ctx->stream, u);
     return launch_check(ctx, "k_screen_update");
 }
 
@@ -4612,7 +4617,8 @@ int init_ctx(pink_hip_ctx *ctx)
         // up to 256 neurons: measured with 512 allowed, 17 x 17 and 18 x 18 neurons at 720 variants train no faster this
         // way than with an update launch of their own -- with three to four waves per SIMD the launch saved is paid in
         // instructions)
-        ctx->fused_f32_train = c.ed_type == PINK_HIP_FLOAT && !ctx->f32gemm && ctx->d_somP && ctx->d_inv && ctx->N <= 256 &&
+        ctx->screen_train = ctx->screen_train && !ctx->f32gemm && ctx->d_somP && ctx->d_inv && B <= kReplayMax;
+        ctx->fused_f32_train = !ctx->screen_train && c.ed_type == PINK_HIP_FLOAT && !ctx->f32gemm && ctx->d_somP && ctx->d_inv && ctx->N <= 256 &&
                                (size_t)(ctx->Rpad / kWave) * ((ctx->N + 3) / 4) <= (size_t)4 * ctx->num_cu;
         ctx->rows_f32_train = !ctx->fused_f32_train && c.ed_type == PINK_HIP_FLOAT && !ctx->f32gemm && ctx->d_somP && ctx->d_inv &&
                               B <= kReplayMax;
@@ -4630,7 +4636,8 @@ int init_ctx(pink_hip_ctx *ctx)
             TRY(upload(ctx, &ctx->d_screen_counts, std::vector<uint32_t>(2 * kCounts + 1, 0u)));       // (two sets, images to skip)
             ctx->orb_part_bytes = std::max((size_t)24 << 20, (size_t)ctx->nrr_eff * ctx->N * 32);
             TRY(dev_alloc(ctx, (char **)&ctx->d_orb_part, ctx->orb_part_bytes));
-            HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_screen_update, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 1024));
+            HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_screen_update<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 1024));
+            HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_screen_update<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 1024));
         }
         if (ctx->fused_f32_train) TRY(dev_alloc(ctx, (uint32_t **)&ctx->d_somP_alt, (size_t)ctx->N * ctx->Epad + kDistOverrun));
         if (ctx->fused_f32_train || ctx->rows_f32_train || ctx->resident_train || ctx->sym_train || ctx->orbit_train)

@@ -792,6 +792,10 @@ SCREENED_TRAIN_SHAPES = [
     (900, 1, 60, 56, 360, True, 45, capi.QUADRATIC, 3, "steps"),       # ... of 32
     (1037, 1, 60, 44, 360, True, 37, capi.QUADRATIC, 5, "tail"),       # factors down to nothing: which neurons do they move?
     (1000, 1, 60, 44, 360, True, 43, capi.CIRCULAR, 5, "tail"),
+    (9, 1, 100, 96, 360, True, 91, capi.QUADRATIC, 3, "blobs"),        # few neurons, long rows
+    (49, 1, 180, 176, 128, True, 171, capi.QUADRATIC, 2, "noise"),     # ... longer than the LDS holds beside their operand
+    (30, 2, 80, 80, 4, True, 73, capi.CIRCULAR, 3, "steps"),           # the symmetries only
+    (100, 1, 64, 60, 100, False, 60, capi.QUADRATIC, 5, "tail"),
 ]
 
 
