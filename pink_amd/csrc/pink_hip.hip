@@ -2106,6 +2106,7 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
 #include "sym_train.inc"
 #include "orbit_gemm.inc"
 #include "coef_gemm.inc"
+#include "f32_train.inc"
 
 // m_update_info[bmu]++ for the images of a group (Trainer.h:302-303), behind a resident launch: nothing when that launch
 // or one before it gave up and nobody rescued it.  The error word goes to the host with it, which looks when it next comes by.
@@ -2432,6 +2433,16 @@ struct pink_hip_ctx {
     // path's operands are then made when something else wants them
     bool sym_form = false, sym_train = false;              // the context can; it does at present
     uint32_t sym_launch = 0, sym_seen = 0;                 // the last resident launch queued; the last one before the slots were cleared
+    bool sym_f32 = false;                                  // float32 (f32_train.inc)
+    uint32_t sym_row = 0, sym_sum_waves = 0;
+    float *d_sym_err = nullptr;
+    float2 *d_sym_image = nullptr;
+    uint2 *d_sym_run = nullptr;
+    unsigned short *d_sym_to = nullptr;
+    uint32_t *d_sym_from = nullptr;
+    float *d_sym_turned = nullptr;
+    uint2 *d_sym_state = nullptr;
+    bool sym_proven = false;                                // a resident launch has gone through since one gave up (float32)
     uint64_t sym_pause = 0, sym_pause_next = 256;          // images to train the other way after a launch gave up; ... the next time
     uint32_t *d_sym_rescue = nullptr;
     unsigned long long *d_sym_keys = nullptr;
@@ -3169,17 +3180,29 @@ const void *sym_kernel_for(uint32_t npb, uint32_t cells)
     return npb == 1 ? sym_kernel_of<U16, 1>(cells) : npb == 2 ? sym_kernel_of<U16, 2>(cells) : sym_kernel_of<U16, 4>(cells);
 }
 
+template <int NPB>
+const void *f32_kernel_of(uint32_t cells)
+{
+    return cells <= 1 ? (const void *)k_train_f32_resident<NPB, 1> : cells <= 2 ? (const void *)k_train_f32_resident<NPB, 2>
+         : (const void *)k_train_f32_resident<NPB, kSymMaxCells>;
+}
+
 const void *sym_kernel(const pink_hip_ctx *ctx)
 {
+    if (ctx->sym_f32) return ctx->sym_npb == 1 ? f32_kernel_of<1>(ctx->sym_nit) : ctx->sym_npb == 2 ? f32_kernel_of<2>(ctx->sym_nit) : f32_kernel_of<4>(ctx->sym_nit);
     return ctx->cfg.ed_type == PINK_HIP_UINT16 ? sym_kernel_for<true>(ctx->sym_npb, ctx->sym_nit) : sym_kernel_for<false>(ctx->sym_npb, ctx->sym_nit);
 }
 
 const void *sym_prepare_kernel(const pink_hip_ctx *ctx)
 {
+    if (ctx->sym_f32) return ctx->sym_prep_lds ? (const void *)k_f32_prepare<true> : (const void *)k_f32_prepare<false>;
     if (ctx->cfg.ed_type == PINK_HIP_UINT16)
         return ctx->sym_prep_lds ? (const void *)k_sym_prepare<true, true> : (const void *)k_sym_prepare<true, false>;
     return ctx->sym_prep_lds ? (const void *)k_sym_prepare<false, true> : (const void *)k_sym_prepare<false, false>;
 }
+
+// Items of k_f32_rescue per image and neuron: as many as find a compute unit.
+uint32_t f32_rescue_parts(const pink_hip_ctx *ctx) { return std::max(1u, (uint32_t)ctx->num_cu / ctx->N); }
 
 // A launch group of an integer trainer with the symmetries on the SOM side: base rotations, the resident launch, the
 // elements outside the region.
@@ -3194,10 +3217,45 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         p.all_sym = ctx->sym_all;
         // (an image in a large part of the LDS leaves room for few blocks on a CU: large ones then)
         const uint32_t threads = ctx->sym_prep_lds > 40 * 1024 || images * ctx->sym_RT < (uint32_t)ctx->num_cu ? 1024 : 256;
-        void *args[] = {&p};
+        F32Prep pf{p.images, p.cos_t, p.sin_t, p.upos, p.smask, p.opnd, p.xrows, ctx->d_sym_err, (double *)ctx->d_sym_norm, ctx->d_sym_image, ctx->d_sym_state,
+                   p.C, p.I, p.D, p.nrr, p.RT, p.KS, p.all_sym};
+        void *args[] = {ctx->sym_f32 ? (void *)&pf : (void *)&p};
         HIP_TRY(ctx, hipLaunchKernel(sym_prepare_kernel(ctx), dim3(ctx->sym_RT, images), dim3(threads), args, ctx->sym_prep_lds, ctx->stream));
     }
-    {
+    const uint32_t blocks = (ctx->N + ctx->sym_npb - 1) / ctx->sym_npb;
+    auto resident = [&](void *arg) {
+        return launch_resident(ctx, blocks, [&] {
+            void *args[] = {arg};
+            HIP_TRY(ctx, hipLaunchKernel(sym_kernel(ctx), dim3(blocks), dim3(kSymThreads), args, ctx->sym_lds, ctx->stream));
+            return (int)PINK_HIP_OK;
+        });
+    };
+    const dim3 rescuers(std::min(ctx->N, 2 * (uint32_t)ctx->num_cu));
+    if (ctx->sym_f32) {
+        F32Rescue rescue{};
+        F32Train &a = rescue.t;
+        a.som = ctx->d_som; a.som_next = ctx->d_som_alt; a.opnd = ctx->d_sym_op; a.xrows = ctx->d_sym_x; a.norm = (const double *)ctx->d_sym_norm;
+        a.err = ctx->d_sym_err; a.image = ctx->d_sym_image;
+        a.factors_t = ctx->d_factors_t; a.cell_elem = ctx->d_sym_elem; a.cell_at = ctx->d_sym_at; a.cell_run = ctx->d_sym_run; a.to = ctx->d_sym_to;
+        a.state = ctx->d_sym_state;
+        a.best_variant = ctx->d_sym_best; a.bmu_out = dev_bmu; a.slots = ctx->d_slots; a.error = ctx->d_resident_error;
+        a.launch = ++ctx->sym_launch;
+        a.N = ctx->N; a.S = ctx->S; a.E = ctx->E; a.cells = ctx->sym_cells; a.KS = ctx->sym_KS; a.RT = ctx->sym_RT; a.nrr = ctx->nrr_eff;
+        a.num_rot = ctx->cfg.num_rot; a.use_flip = ctx->cfg.use_flip; a.images = images; a.tag0 = ctx->sym_tag0; a.spin_limit = ctx->spin_limit;
+        a.row = ctx->sym_row; a.sum_waves = ctx->sym_sum_waves;
+        ctx->sym_tag0 = sym_tag(ctx->sym_tag0, images);
+        {
+            // (per-kernel timing: the images' distances, one pair of events around them as in the form with a launch per image)
+            Timed t(ctx, kClsDist, images);
+            TRY(resident(&a));
+        }
+        Timed t(ctx, kClsUpdate);
+        rescue.keys = ctx->d_sym_keys; rescue.ticket = ctx->d_sym_rescue; rescue.done = ctx->d_sym_rescue + 1;
+        rescue.som = ctx->d_som; rescue.from = ctx->d_sym_from; rescue.x_turned = ctx->d_sym_turned;
+        rescue.parts = f32_rescue_parts(ctx);
+        hipLaunchKernelGGL(k_f32_rescue, dim3(std::max(ctx->N, (uint32_t)ctx->num_cu)), dim3(kRescueThreads), (a.row + 4) * sizeof(float), ctx->stream, rescue);
+        TRY(launch_check(ctx, "k_f32_rescue"));
+    } else {
         Timed t(ctx, kClsUpdate);
         SymRescue rescue{};
         SymTrain &a = rescue.t;
@@ -3208,17 +3266,11 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         a.N = ctx->N; a.S = ctx->S; a.cells = ctx->sym_cells; a.KS = ctx->sym_KS; a.RT = ctx->sym_RT; a.nrr = ctx->nrr_eff;
         a.num_rot = ctx->cfg.num_rot; a.use_flip = ctx->cfg.use_flip; a.images = images; a.tag0 = ctx->sym_tag0; a.spin_limit = ctx->spin_limit;
         ctx->sym_tag0 = sym_tag(ctx->sym_tag0, images);
-        void *args[] = {&a};
-        const uint32_t blocks = (ctx->N + ctx->sym_npb - 1) / ctx->sym_npb;
-        TRY(launch_resident(ctx, blocks, [&] {
-            HIP_TRY(ctx, hipLaunchKernel(sym_kernel(ctx), dim3(blocks), dim3(kSymThreads), args, ctx->sym_lds, ctx->stream));
-            return (int)PINK_HIP_OK;
-        }));
+        TRY(resident(&a));
         rescue.keys = ctx->d_sym_keys; rescue.ticket = ctx->d_sym_rescue; rescue.done = ctx->d_sym_rescue + 1;
-        const dim3 grid(std::min(ctx->N, 2 * (uint32_t)ctx->num_cu));
         const size_t lds = (size_t)ctx->sym_cells * (sizeof(uint2) + 1);
-        if (ctx->cfg.ed_type == PINK_HIP_UINT16) hipLaunchKernelGGL(k_sym_rescue<true>, grid, dim3(kRescueThreads), lds, ctx->stream, rescue);
-        else hipLaunchKernelGGL(k_sym_rescue<false>, grid, dim3(kRescueThreads), lds, ctx->stream, rescue);
+        if (ctx->cfg.ed_type == PINK_HIP_UINT16) hipLaunchKernelGGL(k_sym_rescue<true>, rescuers, dim3(kRescueThreads), lds, ctx->stream, rescue);
+        else hipLaunchKernelGGL(k_sym_rescue<false>, rescuers, dim3(kRescueThreads), lds, ctx->stream, rescue);
         TRY(launch_check(ctx, "k_sym_rescue"));
     }
     if (ctx->sym_outside) {
@@ -3268,7 +3320,7 @@ int choose_sym_form(pink_hip_ctx *ctx, uint32_t n_images)
         hipLaunchKernelGGL(k_fill_zero, dim3(1), dim3(256), 0, ctx->stream, (v4i *)ctx->d_resident_error, (size_t)1);
         TRY(launch_check(ctx, "k_fill_zero"));
         TRY(run_pack_som(ctx));                            // the other form's operand of the SOM as it is now
-        ctx->sym_train = false;
+        ctx->sym_train = ctx->sym_proven = false;
         ctx->sym_pause = ctx->sym_pause_next;
         ctx->sym_pause_next = std::min<uint64_t>(4 * ctx->sym_pause_next, 1u << 20);
     }
@@ -3303,7 +3355,7 @@ int free_all(pink_hip_ctx *ctx)
                     ctx->d_Pa, ctx->d_Pb, ctx->d_na, ctx->d_nb, ctx->d_poff, ctx->d_need, ctx->d_inv,
                     ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4,
                     ctx->d_orb_tables, ctx->d_orb_outside, ctx->d_orb_best, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
-                    ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts, ctx->d_screen_choice, ctx->d_screen_bound, ctx->d_screen_moves, ctx->d_screen_range, ctx->d_coef_neuron, ctx->d_coef_image, ctx->d_coef_row, ctx->d_coef_words, ctx->d_coef_upper, ctx->d_sym_keys, ctx->d_sym_rescue};
+                    ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts, ctx->d_screen_choice, ctx->d_screen_bound, ctx->d_screen_moves, ctx->d_screen_range, ctx->d_coef_neuron, ctx->d_coef_image, ctx->d_coef_row, ctx->d_coef_words, ctx->d_coef_upper, ctx->d_sym_keys, ctx->d_sym_rescue, ctx->d_sym_err, ctx->d_sym_image, ctx->d_sym_run, ctx->d_sym_to, ctx->d_sym_from, ctx->d_sym_turned, ctx->d_sym_state};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu}) if (p) (void)hipFree(p);
     if (ctx->st_pin) (void)hipHostFree(ctx->st_pin);
@@ -3444,7 +3496,8 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
 {
     const pink_hip_config &c = ctx->cfg;
     const uint32_t D = ctx->D, DD = D * D;
-    if (!ctx->gemm || !ctx->fused_som || c.kernel_choice != PINK_HIP_KERNEL_AUTO || ctx->N > kSymMaxNeurons || D >= 4096 || ctx->C >= 256 ||
+    const bool f32 = c.ed_type == PINK_HIP_FLOAT;
+    if ((f32 ? !ctx->d_inv : !ctx->gemm || !ctx->fused_som) || c.kernel_choice != PINK_HIP_KERNEL_AUTO || ctx->N > kSymMaxNeurons || D >= 4096 || ctx->C >= 256 ||
         !resident_allowed())
         return PINK_HIP_OK;
     // Coordinates run to an even bound, the middle of an odd one twice (see sym_train.inc): place X of pixel x, and back.
@@ -3488,15 +3541,27 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     // every share of k a multiple of four k-steps
     ctx->sym_KS = round_up(((uint32_t)all.size() * 4 + 63) / 64, 4 * sym_shares(ctx->sym_RT));
     const uint32_t Kp = ctx->sym_KS * 64;
-    if (Kp > kSymMaxK) return PINK_HIP_OK;
-    const bool u16 = c.ed_type == PINK_HIP_UINT16;
+    if (Kp > kSymMaxK || (f32 && ctx->sym_RT > kSymWorkers)) return PINK_HIP_OK;
+    const bool u16 = c.ed_type != PINK_HIP_UINT8;           // (two planes)
     // as few neurons per block as leave no more blocks than compute units: a block's part of an image shrinks with them
     uint32_t npb = 1;
     while (npb <= 4 && (ctx->N + npb - 1) / npb > (uint32_t)ctx->num_cu) npb *= 2;
+    // Float32, us an image (fields of spots, 720 variants; launch per image | resident): the exchange between the blocks, 4 us, is what
+    // short regions spend.  N 9: E 256 6.4 | 7.1, 576 9.1 | 7.7, 1936 22 | 13; N 100: 144 7.0 | 6.7, 1936 27 | 13; N 256: 144
+    // 9.1 | 7.2; N 484: 64 9.4 | 7.9; four neurons to a block, N 1024: 144 15 | 14, 576 28 | 21.
+    if (f32 && ctx->E < 400 && (npb > 2 || (uint64_t)ctx->N * ctx->E < 30000)) return PINK_HIP_OK;
     if (npb > 4) return PINK_HIP_OK;
     ctx->sym_npb = npb;
     ctx->sym_nit = (npb * ctx->sym_cells + kSymLanes - 1) / kSymLanes;
-    ctx->sym_lds = sym_lds_bytes(npb, ctx->sym_KS, u16, ctx->N, ctx->sym_RT);
+    ctx->sym_lds = f32 ? f32_lds_bytes(npb, ctx->sym_KS, ctx->N, ctx->sym_RT, ctx->E) : sym_lds_bytes(npb, ctx->sym_KS, u16, ctx->N, ctx->sym_RT);
+    if (f32) {
+        // the rest of the LDS for the rows of waves that sum, two of them at least
+        ctx->sym_row = f32_row(ctx->E);
+        const size_t row = (size_t)(ctx->sym_row + 4) * sizeof(float);
+        if (ctx->sym_lds + 2 * row + 4096 > ctx->lds_max || ctx->sym_row >= 65536) return PINK_HIP_OK;
+        ctx->sym_sum_waves = (uint32_t)std::min<size_t>(kSymWorkers, (ctx->lds_max - 4096 - ctx->sym_lds) / row);
+        ctx->sym_lds += ctx->sym_sum_waves * row;
+    }
     if (ctx->sym_nit > kSymMaxCells || ctx->sym_lds + 2048 > ctx->lds_max) return PINK_HIP_OK;
     const size_t image_lds = (size_t)ctx->C * ctx->I * ctx->I * sizeof(float);
     ctx->sym_prep_lds = image_lds <= 150 * 1024 ? image_lds : 0;
@@ -3529,6 +3594,32 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         }
         at[i] = make_uint4(a16[0] | (a16[1] << 16), a16[2] | (a16[3] << 16), a16[4] | (a16[5] << 16), a16[6] | (a16[7] << 16));
     }
+    if (f32) {
+        // where the elements' runs are: of a cell, and of a base rotation's values under a symmetry
+        std::vector<uint32_t> order(ctx->S, ~0u);
+        for (uint32_t e = 0; e < region.size(); ++e) order[region[e]] = e;
+        std::vector<uint2> run(cells.size());
+        std::vector<unsigned short> to((size_t)8 * Kp, (unsigned short)ctx->sym_row);
+        const uint32_t E32 = round_up(ctx->E, kF32Ahead);
+        std::vector<uint32_t> from((size_t)8 * E32, 0);
+        for (uint32_t i = 0; i < cells.size(); ++i) {
+            uint32_t place4[4];
+            for (uint32_t b = 0; b < 4; ++b) {
+                const uint32_t off = (&elem[i].x)[b];
+                place4[b] = off == ~0u ? ctx->sym_row : pair_place(order[off], kF32Run);
+                for (uint32_t sym = 0; sym < 8; ++sym) {
+                    if (off == ~0u || !valid(sym)) continue;
+                    const uint32_t k = rank[moved(cells[i], sym)] * 4 + sym_cell_byte((int)sym, (int)b);
+                    to[(size_t)sym * Kp + k] = (unsigned short)place4[b];
+                    from[(size_t)sym * E32 + order[off]] = k * ctx->sym_RT * 16 * (uint32_t)sizeof(float);
+                }
+            }
+            run[i] = make_uint2(place4[0] | (place4[1] << 16), place4[2] | (place4[3] << 16));
+        }
+        TRY(upload(ctx, &ctx->d_sym_run, run));
+        TRY(upload(ctx, &ctx->d_sym_to, to));
+        TRY(upload(ctx, &ctx->d_sym_from, from));
+    }
     const std::vector<uint32_t> outside = outside_elements(ctx, region);
     ctx->sym_outside = (uint32_t)outside.size();
     TRY(upload(ctx, &ctx->d_sym_upos, upos));
@@ -3545,12 +3636,21 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     TRY(dev_alloc(ctx, &ctx->d_sym_x, b * ctx->nrr_eff * Kp));
     TRY(dev_alloc(ctx, &ctx->d_sym_norm, b * ctx->sym_RT * 16 * 8));
     TRY(dev_alloc(ctx, &ctx->d_sym_best, b * ctx->N));
+    ctx->sym_f32 = f32;
+    if (f32) {
+        TRY(dev_alloc(ctx, &ctx->d_sym_err, b * ctx->sym_RT * 16));
+        TRY(dev_alloc(ctx, &ctx->d_sym_image, b));
+        TRY(dev_alloc(ctx, &ctx->d_sym_state, b + 1));
+        TRY(dev_alloc(ctx, &ctx->d_sym_turned, b * ctx->sym_RT * 16 * Kp));
+        HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_f32_rescue, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 2048));
+    }
     // (limits are per kernel, not per context)
-    HIP_TRY(ctx, hipFuncSetAttribute(sym_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
-    if (ctx->sym_prep_lds) HIP_TRY(ctx, hipFuncSetAttribute(sym_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max));
-    TRY(init_exchange(ctx, (size_t)2 * ctx->N * kSymStride, sym_kernel(ctx), kSymThreads, ctx->sym_lds));
+    const int most = (int)ctx->lds_max - (ctx->sym_f32 ? 2048 : 0);                // (those kernels' own arrays: up to 1.3 KB)
+    HIP_TRY(ctx, hipFuncSetAttribute(sym_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, most));
+    if (ctx->sym_prep_lds) HIP_TRY(ctx, hipFuncSetAttribute(sym_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, most));
+    TRY(init_exchange(ctx, (size_t)(f32 ? 4 : 2) * ctx->N * kSymStride, sym_kernel(ctx), kSymThreads, ctx->sym_lds));
     ctx->sym_tag0 = (ctx->exchange_tag - 1) % 0xfffeu + 1;
-    TRY(dev_alloc(ctx, &ctx->d_sym_keys, b * ctx->N));
+    TRY(dev_alloc(ctx, &ctx->d_sym_keys, b * ctx->N * (f32 ? f32_rescue_parts(ctx) : 1)));
     TRY(dev_alloc(ctx, &ctx->d_sym_rescue, b + 1));
     HIP_TRY(ctx, hipMemset(ctx->d_sym_rescue, 0, (b + 1) * sizeof(uint32_t)));
     ctx->sym_form = ctx->sym_train = true;
@@ -4612,7 +4712,7 @@ int init_ctx(pink_hip_ctx *ctx)
                 TRY(init_exchange(ctx, kSlotWords, (const void *)small_resident_kernel(ctx), kResidentThreads, (size_t)2 * nstored * ctx->S * sizeof(float)));
             }
         }
-        if (one_to_one && !ctx->small_train && !ctx->orbit_train) TRY(init_sym_train(ctx, region));
+        if (one_to_one && !ctx->small_train && !ctx->orbit_train && !ctx->f32gemm) TRY(init_sym_train(ctx, region));
         // one launch per image where the float32 distance kernel runs in its one-wave-per-SIMD form (see k_train_f32_dpp;
         // up to 256 neurons: measured with 512 allowed, 17 x 17 and 18 x 18 neurons at 720 variants train no faster this
         // way than with an update launch of their own -- with three to four waves per SIMD the launch saved is paid in
@@ -4741,9 +4841,17 @@ int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, 
     if (ctx->orbit_train) return run_orbit_train(ctx, dev_images, n_images, dev_bmu_out);
     TRY(choose_sym_form(ctx, n_images));
     if (ctx->sym_train) {
-        for (uint32_t done = 0; done < n_images; done += ctx->sym_B) {
-            const uint32_t B = std::min(ctx->sym_B, n_images - done);
+        for (uint32_t done = 0; done < n_images;) {
+            // (float32: whether the form suits the data, a small first group says -- ahead of the groups that would be queued behind it)
+            const bool probe = ctx->sym_f32 && !ctx->sym_proven;
+            const uint32_t B = std::min(probe ? std::min(ctx->sym_B, kF32Probe) : ctx->sym_B, n_images - done);
             TRY(run_sym_train(ctx, dev_images + (size_t)done * ctx->isz, B, dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group));
+            done += B;
+            if (!probe) continue;
+            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+            ctx->sym_proven = *(const volatile uint32_t *)ctx->h_resident_error == 0;
+            if (!ctx->sym_proven && done < n_images)
+                return train_queued(ctx, dev_images + (size_t)done * ctx->isz, n_images - done, dev_bmu_out ? dev_bmu_out + done : nullptr);
         }
         return PINK_HIP_OK;
     }

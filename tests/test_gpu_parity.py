@@ -639,6 +639,18 @@ RESIDENT_SYMMETRIC_SHAPES = [
     (520, 1, 12, 10, 20, True, 8, capi.CIRCULAR, capi.UINT16, 3),      # four neurons per block
     (601, 1, 30, 28, 8, True, 28, capi.QUADRATIC, capi.UINT8, 3),
     (2, 1, 208, 40, 60, True, 20, capi.QUADRATIC, capi.UINT8, 2),      # an image larger than the LDS
+    (3, 1, 22, 22, 1, False, 20, capi.QUADRATIC, capi.FLOAT, 5),
+    (1, 1, 24, 24, 4, True, 22, capi.QUADRATIC, capi.FLOAT, 5),
+    (7, 1, 26, 26, 4, True, 25, capi.CIRCULAR, capi.FLOAT, 6),
+    (9, 1, 30, 24, 68, True, 21, capi.QUADRATIC, capi.FLOAT, 5),
+    (6, 2, 26, 18, 132, True, 15, capi.QUADRATIC, capi.FLOAT, 4),
+    (5, 1, 24, 33, 200, False, 31, capi.CIRCULAR, capi.FLOAT, 4),
+    (4, 1, 30, 28, 448, True, 23, capi.QUADRATIC, capi.FLOAT, 3),      # seven tiles, the most
+    (3, 1, 60, 64, 40, True, 60, capi.QUADRATIC, capi.FLOAT, 3),       # runs in four blocks, three waves sum
+    (300, 1, 16, 12, 20, True, 11, capi.QUADRATIC, capi.FLOAT, 4),
+    (260, 1, 40, 36, 12, True, 33, capi.QUADRATIC, capi.FLOAT, 3),
+    (520, 1, 30, 26, 20, True, 25, capi.CIRCULAR, capi.FLOAT, 3),
+    (2, 1, 208, 40, 60, True, 20, capi.QUADRATIC, capi.FLOAT, 2),
 ]
 
 
@@ -676,6 +688,42 @@ def test_resident_symmetric_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, 
         assert np.array_equal(bits(som), bits(want)), max_batch
         assert np.array_equal(counts, np.bincount(obmu, minlength=N)), max_batch
         assert np.array_equal(bits(d1), bits(d2)) and np.array_equal(ssd1, ssd2) and np.array_equal(best1, best2)
+
+
+@pytest.mark.parametrize("kind", ["blank", "flat", "alike", "zero", "nan", "grown"])
+def test_resident_float_trainer_on_awkward_data(kind):
+    """Images and weights that leave many variants or several neurons to the float32 sums."""
+    say("resident float trainer", kind)
+    N, C_, I, D, nrot, ed, n = 12, 1, 40, 32, 180, 25, 50
+    rng = np.random.default_rng(5)
+    som0, imgs = rng.random((N, C_ * D * D), dtype=np.float32), rng.random((n, C_, I, I), dtype=np.float32)
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.MEXICAN_HAT if kind == "grown" else capi.GAUSSIAN, 1.0, 0.5)
+    if kind == "blank":
+        imgs[1::3] = 0.0
+    elif kind == "flat":
+        imgs[2:] = 0.25                                                # (all variants alike, image after image)
+    elif kind == "alike":
+        som0[3:9] = som0[3]                                            # (neurons that tie)
+    elif kind == "zero":
+        som0[:] = 0.0
+    elif kind == "nan":
+        imgs[4, 0, I // 2, I // 2] = np.nan
+    elif kind == "grown":
+        som0[::5] *= 3000.0
+    s = O.shape(N, C_, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT)
+    want = som0.copy()
+    want_bmu = O.train(s, want, imgs, F)
+    if kind == "nan":       # (no order among such distances: the kernel that sums every variant is the measure)
+        with capi.Context(N, C_, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT, F, kernel_choice=capi.KERNEL_VALU) as ctx:
+            ctx.set_som(som0)
+            want_bmu, want = ctx.train(imgs), ctx.get_som()
+    lost = np.isnan(want)
+    assert lost.any() == (kind == "nan")
+    with capi.Context(N, C_, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT, F) as ctx:
+        ctx.set_som(som0)
+        bmu = np.concatenate([ctx.train(imgs[:1]), ctx.train(imgs[1:])])
+        som = ctx.get_som()
+    assert np.array_equal(bmu, want_bmu) and np.array_equal(np.isnan(som), lost) and np.array_equal(bits(som)[~lost], bits(want)[~lost])
 
 
 def test_resident_symmetric_trainer_tries_again(monkeypatch):
@@ -800,8 +848,9 @@ SCREENED_TRAIN_SHAPES = [
 
 
 @pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,shape_,n,kind", SCREENED_TRAIN_SHAPES)
-def test_float_trainer_with_screened_distances(N, C_, I, D, nrot, flip, ed, shape_, n, kind):
+def test_float_trainer_with_screened_distances(monkeypatch, N, C_, I, D, nrot, flip, ed, shape_, n, kind):
     """Large float32 trainers sum the variants that a product of rounded values leaves: the oracle's bits, which sums them all."""
+    monkeypatch.setenv("PINK_HIP_RESIDENT_TRAINER", "0")
     say("screened float trainer", N, C_, I, D, nrot, flip, ed, shape_, n, kind)
     F = capi.make_update_factors(capi.CARTESIAN, [N], capi.MEXICAN_HAT if kind == "grown" else capi.GAUSSIAN, 1.0, 0.5)
     rng = np.random.default_rng(N + I)
