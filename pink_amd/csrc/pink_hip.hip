@@ -2490,6 +2490,7 @@ struct pink_hip_ctx {
     uint4 *d_orb_element = nullptr;
     uint32_t orb_cur = 0, orb_pitch = 0, orb_outside = 0;      // the set of norms that belongs to the operand
     uint32_t *d_orb_outside = nullptr, *d_orb_best = nullptr;
+    float *d_most = nullptr;                               // the group's images' largest absolute values
     float *d_orb_x = nullptr, *d_orb_values = nullptr;
     int *d_orb_part = nullptr;
     size_t orb_part_bytes = 0;
@@ -3212,12 +3213,12 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         Timed t(ctx, kClsRotate);
         SymPrep p{};
         p.images = dev_images; p.cos_t = ctx->d_cos; p.sin_t = ctx->d_sin; p.upos = ctx->d_sym_upos; p.smask = ctx->d_sym_mask;
-        p.opnd = ctx->d_sym_op; p.xrows = ctx->d_sym_x; p.norm = ctx->d_sym_norm;
+        p.opnd = ctx->d_sym_op; p.xrows = ctx->d_sym_x; p.norm = ctx->d_sym_norm; p.most = ctx->d_most;
         p.C = ctx->C; p.I = ctx->I; p.D = ctx->D; p.nrr = ctx->nrr_eff; p.RT = ctx->sym_RT; p.KS = ctx->sym_KS;
         p.all_sym = ctx->sym_all;
         // (an image in a large part of the LDS leaves room for few blocks on a CU: large ones then)
         const uint32_t threads = ctx->sym_prep_lds > 40 * 1024 || images * ctx->sym_RT < (uint32_t)ctx->num_cu ? 1024 : 256;
-        F32Prep pf{p.images, p.cos_t, p.sin_t, p.upos, p.smask, p.opnd, p.xrows, ctx->d_sym_err, (double *)ctx->d_sym_norm, ctx->d_sym_image, ctx->d_sym_state,
+        F32Prep pf{p.images, p.cos_t, p.sin_t, p.upos, p.smask, p.opnd, p.xrows, ctx->d_sym_err, (double *)ctx->d_sym_norm, ctx->d_sym_image, p.most, ctx->d_sym_state,
                    p.C, p.I, p.D, p.nrr, p.RT, p.KS, p.all_sym};
         void *args[] = {ctx->sym_f32 ? (void *)&pf : (void *)&p};
         HIP_TRY(ctx, hipLaunchKernel(sym_prepare_kernel(ctx), dim3(ctx->sym_RT, images), dim3(threads), args, ctx->sym_prep_lds, ctx->stream));
@@ -3277,10 +3278,10 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         Timed t(ctx, kClsUpdate);
         SymOutside o{};
         o.som = ctx->d_som; o.som_next = ctx->d_som_alt; o.images = dev_images; o.cos_t = ctx->d_cos; o.sin_t = ctx->d_sin;
-        o.factors = ctx->d_factors; o.best_variant = ctx->d_sym_best; o.bmu = dev_bmu; o.outside = ctx->d_sym_outside;
+        o.most = ctx->d_most; o.factors = ctx->d_factors; o.best_variant = ctx->d_sym_best; o.bmu = dev_bmu; o.outside = ctx->d_sym_outside;
         o.count = ctx->sym_outside; o.N = ctx->N; o.S = ctx->S; o.C = ctx->C; o.I = ctx->I;
         o.D = ctx->D; o.nrr = ctx->nrr_eff; o.num_rot = ctx->cfg.num_rot; o.images_n = images;
-        hipLaunchKernelGGL(k_sym_outside, dim3((ctx->sym_outside + 255) / 256, ctx->N), dim3(256), 0, ctx->stream, o);
+        hipLaunchKernelGGL(ctx->I == 1 ? k_sym_outside<true> : k_sym_outside<false>, dim3((ctx->sym_outside + 255) / 256, ctx->N), dim3(256), 0, ctx->stream, o);
         TRY(launch_check(ctx, "k_sym_outside"));
     }
     return resident_launched(ctx, dev_images, images, dev_bmu);
@@ -3354,7 +3355,7 @@ int free_all(pink_hip_ctx *ctx)
                     ctx->d_somP, ctx->d_somP_alt, ctx->d_bmu_group, ctx->d_rotT, ctx->d_bmu_scratch, ctx->d_dist, ctx->d_ssd, ctx->d_best,
                     ctx->d_Pa, ctx->d_Pb, ctx->d_na, ctx->d_nb, ctx->d_poff, ctx->d_need, ctx->d_inv,
                     ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4,
-                    ctx->d_orb_tables, ctx->d_orb_outside, ctx->d_orb_best, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
+                    ctx->d_orb_tables, ctx->d_orb_outside, ctx->d_orb_best, ctx->d_most, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
                     ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts, ctx->d_screen_choice, ctx->d_screen_bound, ctx->d_screen_moves, ctx->d_screen_range, ctx->d_coef_neuron, ctx->d_coef_image, ctx->d_coef_row, ctx->d_coef_words, ctx->d_coef_upper, ctx->d_sym_keys, ctx->d_sym_rescue, ctx->d_sym_err, ctx->d_sym_image, ctx->d_sym_run, ctx->d_sym_to, ctx->d_sym_from, ctx->d_sym_turned, ctx->d_sym_state};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu}) if (p) (void)hipFree(p);
@@ -3636,6 +3637,7 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     TRY(dev_alloc(ctx, &ctx->d_sym_x, b * ctx->nrr_eff * Kp));
     TRY(dev_alloc(ctx, &ctx->d_sym_norm, b * ctx->sym_RT * 16 * 8));
     TRY(dev_alloc(ctx, &ctx->d_sym_best, b * ctx->N));
+    if (!ctx->d_most) TRY(dev_alloc(ctx, &ctx->d_most, std::max<size_t>(b, kSymGroupMax)));
     ctx->sym_f32 = f32;
     if (f32) {
         TRY(dev_alloc(ctx, &ctx->d_sym_err, b * ctx->sym_RT * 16));
@@ -3645,7 +3647,7 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_f32_rescue, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 2048));
     }
     // (limits are per kernel, not per context)
-    const int most = (int)ctx->lds_max - (ctx->sym_f32 ? 2048 : 0);                // (those kernels' own arrays: up to 1.3 KB)
+    const int most = (int)ctx->lds_max - 2048;             // (the kernels' own arrays: up to 1.3 KB more than lds_max leaves them)
     HIP_TRY(ctx, hipFuncSetAttribute(sym_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, most));
     if (ctx->sym_prep_lds) HIP_TRY(ctx, hipFuncSetAttribute(sym_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, most));
     TRY(init_exchange(ctx, (size_t)(f32 ? 4 : 2) * ctx->N * kSymStride, sym_kernel(ctx), kSymThreads, ctx->sym_lds));
@@ -3992,7 +3994,7 @@ int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
     p.images = dev_images; p.index = ctx->d_orb_index; p.frac = ctx->d_orb_frac; p.mask = ctx->d_orb_mask;
     p.opnd = ctx->d_orb_rows; p.norm = ctx->d_orb_nb; p.key = ctx->d_key;
     p.xrows = ctx->d_orb_x; p.plane = orbit_rows_plane(ctx, B); p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.KS = ctx->orb_KS;
-    p.all_sym = ctx->orb_all; p.rl = ctx->orb_rl; p.pitch = ctx->orb_pitch;
+    p.all_sym = ctx->orb_all; p.rl = ctx->orb_rl; p.pitch = ctx->orb_pitch; p.most = ctx->d_most;
     const dim3 grid(B, (ctx->nrr_eff + (1u << p.rl) - 1) >> p.rl);
     const uint32_t threads = ctx->orb_prep_lds > 64 * 1024 || grid.x * grid.y < (uint32_t)ctx->num_cu ? 1024 : ctx->orb_prep_lds > 24 * 1024 ? 512 : 256;
     void *args[] = {&p};
@@ -4187,10 +4189,10 @@ int run_orbit_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_image
             Timed t(ctx, kClsUpdate);
             SymOutside o{};
             o.som = ctx->d_som; o.som_next = ctx->d_som; o.images = images; o.cos_t = ctx->d_cos; o.sin_t = ctx->d_sin;
-            o.factors = ctx->d_factors; o.best_variant = ctx->d_orb_best; o.bmu = bmu; o.outside = ctx->d_orb_outside;
+            o.most = ctx->d_most; o.factors = ctx->d_factors; o.best_variant = ctx->d_orb_best; o.bmu = bmu; o.outside = ctx->d_orb_outside;
             o.count = ctx->orb_outside; o.N = ctx->N; o.S = ctx->S; o.C = ctx->C; o.I = ctx->I;
             o.D = ctx->D; o.nrr = ctx->nrr_eff; o.num_rot = ctx->cfg.num_rot; o.images_n = B;
-            hipLaunchKernelGGL(k_sym_outside, dim3((ctx->orb_outside + 255) / 256, ctx->N), dim3(256), 0, ctx->stream, o);
+            hipLaunchKernelGGL(ctx->I == 1 ? k_sym_outside<true> : k_sym_outside<false>, dim3((ctx->orb_outside + 255) / 256, ctx->N), dim3(256), 0, ctx->stream, o);
             TRY(launch_check(ctx, "k_sym_outside"));
         }
     }
@@ -4565,6 +4567,7 @@ int init_ctx(pink_hip_ctx *ctx)
         else if (ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_x, B * ctx->nrr_eff * ctx->orb_KS * 32));
         if (ctx->trainer) {
             TRY(dev_alloc(ctx, &ctx->d_orb_best, B * ctx->N));
+            if (is_int(ctx) && !ctx->d_most) TRY(dev_alloc(ctx, &ctx->d_most, std::max<size_t>(B, kSymGroupMax)));
             const std::vector<uint32_t> outside = outside_elements(ctx, region);
             ctx->orb_outside = (uint32_t)outside.size();
             TRY(upload(ctx, &ctx->d_orb_outside, outside));

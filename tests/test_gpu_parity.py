@@ -726,6 +726,34 @@ def test_resident_float_trainer_on_awkward_data(kind):
     assert np.array_equal(bmu, want_bmu) and np.array_equal(np.isnan(som), lost) and np.array_equal(bits(som)[~lost], bits(want)[~lost])
 
 
+@pytest.mark.parametrize("N,I,D,nrot,ed,ed_type", [
+    (30, 24, 30, 20, 9, capi.UINT8),
+    (30, 24, 30, 20, 9, capi.UINT16),
+    (30, 40, 35, 20, 21, capi.FLOAT),
+    (3, 70, 110, 48, 95, capi.UINT16),                                 # (weights in orbit order)
+    (30, 1, 9, 4, 5, capi.UINT8),                                      # images of one pixel
+])
+def test_factors_that_move_some_elements_only(N, I, D, nrot, ed, ed_type):
+    """Elements outside the region are passed by where no element of a wave can move: factors down to nothing, small weights."""
+    say("factors that move some elements", N, I, D, nrot, ed, ed_type)
+    n = 6
+    rng = np.random.default_rng(N + I)
+    som0, imgs = rng.random((N, D * D), dtype=np.float32), rng.random((n, 1, I, I), dtype=np.float32)
+    som0[1::3] += np.float32(0.5)                                      # (no small weights)
+    som0[2::3, ::D] *= np.float32(1e-9)
+    som0[::4, 5] = 0.0
+    imgs[2] *= np.float32(-30.0)
+    imgs[3] = 0.0
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 1.5, 0.5) ** np.float32(1.3)
+    F[:, ::5] *= np.float32(3e-8)
+    F[:, 1::7] *= np.float32(-1e-7)
+    want = som0.copy()
+    want_bmu = O.train(O.shape(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, ed_type), want, imgs, F)
+    with capi.Context(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, ed_type, F) as ctx:
+        ctx.set_som(som0)
+        assert np.array_equal(ctx.train(imgs), want_bmu) and np.array_equal(bits(ctx.get_som()), bits(want))
+
+
 def test_resident_symmetric_trainer_tries_again(monkeypatch):
     """After a launch that gave up, the trainer takes the other form for some 256 images and is then resident again."""
     monkeypatch.setenv("PINK_HIP_RESIDENT_SPIN_LIMIT", "0")
