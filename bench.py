@@ -111,6 +111,11 @@ def screened(w, times, images):
     return w.ed_type == 0 and w.mode == "train" and groups > 0 and times["rotate"][0] == 2 * groups
 
 
+def resident_float(w, times, images):
+    """Whether a float32 trainer was resident in this run: groups of more images than any other form's, whose launch counts as one per image."""
+    return w.ed_type == 0 and w.mode == "train" and 0 < times["rotate"][0] * 64 < images and times["distance"][0] == images
+
+
 def small_resident(w):
     return w.ed_type == 2 and w.som_size <= 64 and w.R <= 32
 
@@ -118,6 +123,10 @@ def small_resident(w):
 def distance_path_name(w, path, times, images):
     """The kernel that computed the distances in this run, by the library's path and what was launched."""
     from pink_amd import capi
+    if resident_float(w, times, images):
+        return ("int8 MFMA product of 16-bit values inside the resident launch of a float32 trainer (one launch per group of images, counted "
+                "as one per image), then float32 sums in the CPU's order of the variants that can be a neuron's closest; a 64-bit word of "
+                "bounds per neuron and image exchanged through memory")
     if screened(w, times, images):
         return ("int8 MFMA product of 16-bit values for every (neuron, variant) pair, then float32 sums in the CPU's order of the "
                 "variants that can be a neuron's closest")
@@ -294,6 +303,11 @@ def run_workload(name, steps, warmup, n_images, kernel, cpu_budget_s, host_inclu
         achieved = alg["distance"]["ops"] * per_s / 1e12
         notes = ("float32 MFMA recast |a|^2 + |b|^2 - 2 a.b, requested with --kernel mfma_f32: not the CPU's summation "
                  "order (distances to a relative tolerance only); never the default")
+    elif dominant == "distance" and resident_float(w, times, prof_images):
+        bound, unit, peak = "mfma", "TOP/s", MFMA_INT8_PEAK_TOPS
+        achieved = alg["distance"]["ops"] * per_s / 1e12
+        notes = ("the whole step of an image, every pair's operations priced at the int8 peak: a chain of product, bounds, float32 sums "
+                 "beside the word exchange, update; four byte-plane products per pair element, counted once")
     elif dominant == "distance" and screened(w, times, prof_images):
         bound, unit, peak = "mfma", "TOP/s", MFMA_INT8_PEAK_TOPS
         achieved = alg["distance"]["ops"] * per_s / 1e12

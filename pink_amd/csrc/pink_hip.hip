@@ -2442,6 +2442,7 @@ struct pink_hip_ctx {
     uint32_t *d_sym_from = nullptr;
     float *d_sym_turned = nullptr;
     uint2 *d_sym_state = nullptr;
+    float *d_sym_norm_off = nullptr;
     bool sym_proven = false;                                // a resident launch has gone through since one gave up (float32)
     uint64_t sym_pause = 0, sym_pause_next = 256;          // images to train the other way after a launch gave up; ... the next time
     uint32_t *d_sym_rescue = nullptr;
@@ -3218,7 +3219,7 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         p.all_sym = ctx->sym_all;
         // (an image in a large part of the LDS leaves room for few blocks on a CU: large ones then)
         const uint32_t threads = ctx->sym_prep_lds > 40 * 1024 || images * ctx->sym_RT < (uint32_t)ctx->num_cu ? 1024 : 256;
-        F32Prep pf{p.images, p.cos_t, p.sin_t, p.upos, p.smask, p.opnd, p.xrows, ctx->d_sym_err, (double *)ctx->d_sym_norm, ctx->d_sym_image, p.most, ctx->d_sym_state,
+        F32Prep pf{p.images, p.cos_t, p.sin_t, p.upos, p.smask, p.opnd, p.xrows, ctx->d_sym_err, (double *)ctx->d_sym_norm, ctx->d_sym_norm_off, ctx->d_sym_image, p.most, ctx->d_sym_state,
                    p.C, p.I, p.D, p.nrr, p.RT, p.KS, p.all_sym};
         void *args[] = {ctx->sym_f32 ? (void *)&pf : (void *)&p};
         HIP_TRY(ctx, hipLaunchKernel(sym_prepare_kernel(ctx), dim3(ctx->sym_RT, images), dim3(threads), args, ctx->sym_prep_lds, ctx->stream));
@@ -3236,7 +3237,7 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         F32Rescue rescue{};
         F32Train &a = rescue.t;
         a.som = ctx->d_som; a.som_next = ctx->d_som_alt; a.opnd = ctx->d_sym_op; a.xrows = ctx->d_sym_x; a.norm = (const double *)ctx->d_sym_norm;
-        a.err = ctx->d_sym_err; a.image = ctx->d_sym_image;
+        a.norm_off = ctx->d_sym_norm_off; a.err = ctx->d_sym_err; a.image = ctx->d_sym_image;
         a.factors_t = ctx->d_factors_t; a.cell_elem = ctx->d_sym_elem; a.cell_at = ctx->d_sym_at; a.cell_run = ctx->d_sym_run; a.to = ctx->d_sym_to;
         a.state = ctx->d_sym_state;
         a.best_variant = ctx->d_sym_best; a.bmu_out = dev_bmu; a.slots = ctx->d_slots; a.error = ctx->d_resident_error;
@@ -3356,7 +3357,7 @@ int free_all(pink_hip_ctx *ctx)
                     ctx->d_Pa, ctx->d_Pb, ctx->d_na, ctx->d_nb, ctx->d_poff, ctx->d_need, ctx->d_inv,
                     ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4,
                     ctx->d_orb_tables, ctx->d_orb_outside, ctx->d_orb_best, ctx->d_most, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
-                    ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts, ctx->d_screen_choice, ctx->d_screen_bound, ctx->d_screen_moves, ctx->d_screen_range, ctx->d_coef_neuron, ctx->d_coef_image, ctx->d_coef_row, ctx->d_coef_words, ctx->d_coef_upper, ctx->d_sym_keys, ctx->d_sym_rescue, ctx->d_sym_err, ctx->d_sym_image, ctx->d_sym_run, ctx->d_sym_to, ctx->d_sym_from, ctx->d_sym_turned, ctx->d_sym_state};
+                    ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts, ctx->d_screen_choice, ctx->d_screen_bound, ctx->d_screen_moves, ctx->d_screen_range, ctx->d_coef_neuron, ctx->d_coef_image, ctx->d_coef_row, ctx->d_coef_words, ctx->d_coef_upper, ctx->d_sym_keys, ctx->d_sym_rescue, ctx->d_sym_err, ctx->d_sym_image, ctx->d_sym_run, ctx->d_sym_to, ctx->d_sym_from, ctx->d_sym_turned, ctx->d_sym_state, ctx->d_sym_norm_off};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu}) if (p) (void)hipFree(p);
     if (ctx->st_pin) (void)hipHostFree(ctx->st_pin);
@@ -3642,6 +3643,7 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     if (f32) {
         TRY(dev_alloc(ctx, &ctx->d_sym_err, b * ctx->sym_RT * 16));
         TRY(dev_alloc(ctx, &ctx->d_sym_image, b));
+        TRY(dev_alloc(ctx, &ctx->d_sym_norm_off, b * ctx->sym_RT * 16 * 8));
         TRY(dev_alloc(ctx, &ctx->d_sym_state, b + 1));
         TRY(dev_alloc(ctx, &ctx->d_sym_turned, b * ctx->sym_RT * 16 * Kp));
         HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_f32_rescue, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 2048));
