@@ -47,17 +47,17 @@ MEASURED_VALU_LANE_OPS_T = 50.0     # subtract / fma stream, eight waves per SIM
 # by what the same counter reads for a device-to-device copy of known size; (bytes, the summary
 # under profiles/ that holds the readings).  Not measured in the run that prints the line.
 COUNTER_TRAFFIC_PER_IMAGE = {
-    ("cfg0", "distance"): (12.280e6 + 3.239e6, "profiles/cfg0_train_f32_counters.txt"),   # with the update of the image before
-    ("cfg0", "update"): ((28.133e6 + 0.774e6 + 1.706e6 + 1.184e6) / 48, "profiles/cfg0_train_f32_counters.txt"),   # per group of 48
+    ("cfg0", "distance"): ((531.922e6 + 3.151e6) / 238, "profiles/cfg0_train_f32_counters.txt"),   # the resident launch, of 238 images on average
+    ("cfg0", "update"): ((31.326e6 + 0.516e6) / 238, "profiles/cfg0_train_f32_counters.txt"),     # elements outside the region
     ("cfg1", "rotate"): ((96.042e6 + 207.618e6) / 2048, "profiles/cfg1_map_u8_counters.txt"),
     ("cfg1", "distance"): ((214.632e6 + 1.639e6) / 2048, "profiles/cfg1_map_u8_counters.txt"),
     # the resident launch of 64 images and the one that brings the elements outside the region up to date
-    ("cfg2", "update"): ((819.878e6 + 7.440e6 + 206.588e6 + 12.635e6) / 64, "profiles/cfg2_train_u16_counters.txt"),
+    ("cfg2", "update"): ((819.876e6 + 7.440e6 + 141.852e6 + 13.839e6) / 64, "profiles/cfg2_train_u16_counters.txt"),
     # the product, the selection, the exact sums of variants and of neurons
-    ("cfg3", "distance"): (33.229e6 + 13.824e6 + 14.031e6 + 0.118e6 + 156.047e6 + 1.316e6 + 1.424e6 + 0.001e6,
+    ("cfg3", "distance"): (32.666e6 + 9.216e6 + 9.440e6 + 0.140e6 + 210.795e6 + 0.308e6 + 0.039e6,
                            "profiles/cfg3_train_f32_3ch_counters.txt"),
     # the operand rows per image and a sixteenth of the launch that brings the neurons' full images up to date
-    ("cfg3", "update"): (70.642e6 + 71.889e6 + (396.602e6 + 94.939e6) / 16, "profiles/cfg3_train_f32_3ch_counters.txt"),
+    ("cfg3", "update"): (39.981e6 + 40.509e6 + (294.450e6 + 55.482e6 + 94.359e6 + 0.051e6) / 16, "profiles/cfg3_train_f32_3ch_counters.txt"),
     ("cfg4", "update"): ((85.604e6 + 0.835e6) / 256, "profiles/cfg4_train_u8_counters.txt"),     # the resident launch of 256 images
 }
 

@@ -3239,7 +3239,7 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         a.som = ctx->d_som; a.som_next = ctx->d_som_alt; a.opnd = ctx->d_sym_op; a.xrows = ctx->d_sym_x; a.norm = (const double *)ctx->d_sym_norm;
         a.norm_off = ctx->d_sym_norm_off; a.err = ctx->d_sym_err; a.image = ctx->d_sym_image;
         a.factors_t = ctx->d_factors_t; a.cell_elem = ctx->d_sym_elem; a.cell_at = ctx->d_sym_at; a.cell_run = ctx->d_sym_run; a.to = ctx->d_sym_to;
-        a.state = ctx->d_sym_state;
+        a.state = ctx->d_sym_state; a.slow = ctx->h_resident_error + 1;
         a.best_variant = ctx->d_sym_best; a.bmu_out = dev_bmu; a.slots = ctx->d_slots; a.error = ctx->d_resident_error;
         a.launch = ++ctx->sym_launch;
         a.N = ctx->N; a.S = ctx->S; a.E = ctx->E; a.cells = ctx->sym_cells; a.KS = ctx->sym_KS; a.RT = ctx->sym_RT; a.nrr = ctx->nrr_eff;
@@ -3314,7 +3314,9 @@ int finish_resident(pink_hip_ctx *ctx)
 int choose_sym_form(pink_hip_ctx *ctx, uint32_t n_images)
 {
     if (!ctx->sym_form) return PINK_HIP_OK;
-    const uint32_t failed = *(const volatile uint32_t *)ctx->h_resident_error;
+    const volatile uint32_t *const word = ctx->h_resident_error;
+    uint32_t failed = word[0];
+    if (word[1] && (int32_t)(word[1] - ctx->sym_seen) > 0) failed = word[1];       // (float32: gone through, but slowly)
     if (ctx->sym_train && failed && (int32_t)(failed - ctx->sym_seen) > 0) {
         ctx->sym_seen = ctx->sym_launch;
         const size_t slots = (size_t)ctx->N * kSymStride;              // (16-byte words of both sets)
@@ -3426,11 +3428,11 @@ int init_exchange(pink_hip_ctx *ctx, size_t slot_words, const void *kernel, uint
     HIP_TRY(ctx, hipMemset(ctx->d_slots, 0, slot_words * sizeof(unsigned long long)));
     TRY(dev_alloc(ctx, &ctx->d_resident_error, 4));
     HIP_TRY(ctx, hipMemset(ctx->d_resident_error, 0, 4 * sizeof(uint32_t)));
-    if (hipHostMalloc((void **)&ctx->h_resident_error, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc((void **)&ctx->h_resident_error, 2 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
         ctx->h_resident_error = nullptr;
         return fail(ctx, PINK_HIP_ENOMEM, "pinned host allocation failed");
     }
-    *ctx->h_resident_error = 0;
+    ctx->h_resident_error[0] = ctx->h_resident_error[1] = 0;
     return PINK_HIP_OK;
 }
 
@@ -3548,10 +3550,11 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     // as few neurons per block as leave no more blocks than compute units: a block's part of an image shrinks with them
     uint32_t npb = 1;
     while (npb <= 4 && (ctx->N + npb - 1) / npb > (uint32_t)ctx->num_cu) npb *= 2;
-    // Float32, us an image (fields of spots, 720 variants; launch per image | resident): the exchange between the blocks, 4 us, is what
-    // short regions spend.  N 9: E 256 6.4 | 7.1, 576 9.1 | 7.7, 1936 22 | 13; N 100: 144 7.0 | 6.7, 1936 27 | 13; N 256: 144
-    // 9.1 | 7.2; N 484: 64 9.4 | 7.9; four neurons to a block, N 1024: 144 15 | 14, 576 28 | 21.
-    if (f32 && ctx->E < 400 && (npb > 2 || (uint64_t)ctx->N * ctx->E < 30000)) return PINK_HIP_OK;
+    // Float32, us an image (smooth fields; launch per image | resident): the exchange between the blocks, 4 us, is what short regions
+    // spend, and a launch per image takes longer with every pair.  N 9: E 256, 720 variants 6.4 | 7.1, 400 7.8 | 7.0, 1936 22 | 13; N 100: 144
+    // 7.0 | 6.7, 1936 27 | 13; N 256: 196, 56 variants 5.5 | 6.8, 256, 360 variants 6.9 | 6.3, 400, 8 variants 7.0 | 6.9; N 484:
+    // 256, 56 variants 8.0 | 9.3, 200 variants 9.3 | 8.8; four neurons to a block, N 1024: 144 15 | 14, 576 28 | 21.
+    if (f32 && ctx->E < 400 && (npb > 2 || (uint64_t)ctx->N * ctx->E * c.num_rot * (c.use_flip ? 2 : 1) < 15000000)) return PINK_HIP_OK;
     if (npb > 4) return PINK_HIP_OK;
     ctx->sym_npb = npb;
     ctx->sym_nit = (npb * ctx->sym_cells + kSymLanes - 1) / kSymLanes;
@@ -3860,7 +3863,7 @@ size_t orbit_image_bytes(const pink_hip_ctx *ctx)
                            (is_int(ctx) && !ctx->trainer ? (size_t)0 : is_int(ctx) ? (size_t)ctx->orb_KS * 128 : (size_t)ctx->orb_Ox * 32));
 }
 
-// Float32 mappers: whether a full launch group of images is screened (see k_screen_exact; few images are summed all the same,
+// Float32 mappers: whether a full launch group of images is screened (few images are summed all the same,
 // summed_images).  What summing a neuron's every variant takes grows with their
 // number, what is left to sum exactly does not: break-even lies near 100 variants (20 variants of 768 elements 10 % slower
 // with it, 8 of 1369 half as fast, 360 of 121 1.5 times as fast, 720 of 1024 3.8 times).  And what an image leaves in
@@ -4854,7 +4857,8 @@ int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, 
             done += B;
             if (!probe) continue;
             HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-            ctx->sym_proven = *(const volatile uint32_t *)ctx->h_resident_error == 0;
+            const volatile uint32_t *const word = ctx->h_resident_error;
+            ctx->sym_proven = word[0] == 0 && (word[1] == 0 || (int32_t)(word[1] - ctx->sym_seen) <= 0);
             if (!ctx->sym_proven && done < n_images)
                 return train_queued(ctx, dev_images + (size_t)done * ctx->isz, n_images - done, dev_bmu_out ? dev_bmu_out + done : nullptr);
         }

@@ -647,7 +647,7 @@ RESIDENT_SYMMETRIC_SHAPES = [
     (5, 1, 24, 33, 200, False, 31, capi.CIRCULAR, capi.FLOAT, 4),
     (4, 1, 30, 28, 448, True, 23, capi.QUADRATIC, capi.FLOAT, 3),      # seven tiles, the most
     (3, 1, 60, 64, 40, True, 60, capi.QUADRATIC, capi.FLOAT, 3),       # runs in four blocks, three waves sum
-    (300, 1, 16, 12, 20, True, 11, capi.QUADRATIC, capi.FLOAT, 4),
+    (300, 1, 16, 12, 208, True, 11, capi.QUADRATIC, capi.FLOAT, 4),
     (260, 1, 40, 36, 12, True, 33, capi.QUADRATIC, capi.FLOAT, 3),
     (520, 1, 30, 26, 20, True, 25, capi.CIRCULAR, capi.FLOAT, 3),
     (2, 1, 208, 40, 60, True, 20, capi.QUADRATIC, capi.FLOAT, 2),
