@@ -690,7 +690,7 @@ def test_resident_symmetric_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, 
         assert np.array_equal(bits(d1), bits(d2)) and np.array_equal(ssd1, ssd2) and np.array_equal(best1, best2)
 
 
-@pytest.mark.parametrize("kind", ["blank", "flat", "alike", "zero", "nan", "grown"])
+@pytest.mark.parametrize("kind", ["blank", "flat", "alike", "zero", "nan", "grown", "faint", "flux"])
 def test_resident_float_trainer_on_awkward_data(kind):
     """Images and weights that leave many variants or several neurons to the float32 sums."""
     say("resident float trainer", kind)
@@ -710,6 +710,10 @@ def test_resident_float_trainer_on_awkward_data(kind):
         imgs[4, 0, I // 2, I // 2] = np.nan
     elif kind == "grown":
         som0[::5] *= 3000.0
+    elif kind == "faint":
+        imgs *= np.float32(0.003)                                      # (the product's error is the smaller one)
+    elif kind == "flux":
+        imgs, som0 = imgs * np.float32(2e-20), som0 * np.float32(5e-19)       # (squares that are no float32 numbers)
     s = O.shape(N, C_, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT)
     want = som0.copy()
     want_bmu = O.train(s, want, imgs, F)
