@@ -758,6 +758,38 @@ def test_factors_that_move_some_elements_only(N, I, D, nrot, ed, ed_type):
         assert np.array_equal(ctx.train(imgs), want_bmu) and np.array_equal(bits(ctx.get_som()), bits(want))
 
 
+@pytest.mark.parametrize("N,I,D,nrot,ed,ed_type,pixel", [
+    (30, 24, 30, 20, 9, capi.UINT8, (1, 12)),
+    (30, 40, 35, 20, 21, capi.FLOAT, (3, 20)),
+    (3, 70, 110, 48, 95, capi.UINT16, None),                           # (weights in orbit order; no pixel beside the region)
+])
+def test_small_factors_on_weights_without_bounds(N, I, D, nrot, ed, ed_type, pixel):
+    """inf - (inf - x) f is no number under the smallest factor, nor is a difference that overflows small: such weights outside the
+    region are not passed by.  Factors of zero leave them."""
+    say("small factors on weights without bounds", N, I, D, nrot, ed, ed_type)
+    n = 5
+    rng = np.random.default_rng(N + I)
+    som0, imgs = rng.random((N, D, D), dtype=np.float32), rng.random((n, 1, I, I), dtype=np.float32)
+    m = (D - ed) // 2
+    outside = np.ones((D, D), bool)
+    outside[m:m + ed, m:m + ed] = False
+    for k, value in enumerate((np.inf, -np.inf, 3e38, -2e38, 9e37)):
+        som0[k::6, outside] = value
+    if pixel:
+        imgs[1, 0][pixel], imgs[3, 0][pixel] = -3e38, 2e38
+    F = np.full((N, N), 1e-8, np.float32)
+    F[:, 1::4] *= np.float32(-1.0)
+    F[:, 2::7] = 0.0
+    want = som0.reshape(N, -1).copy()
+    want_bmu = O.train(O.shape(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, ed_type), want, imgs, F)
+    lost = np.isnan(want)
+    assert lost.any() and np.isinf(want).any()
+    with capi.Context(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, ed_type, F) as ctx:
+        ctx.set_som(som0.reshape(N, -1))
+        bmu, som = ctx.train(imgs), ctx.get_som()
+    assert np.array_equal(bmu, want_bmu) and np.array_equal(np.isnan(som), lost) and np.array_equal(bits(som)[~lost], bits(want)[~lost])
+
+
 def test_resident_symmetric_trainer_tries_again(monkeypatch):
     """After a launch that gave up, the trainer takes the other form for some 256 images and is then resident again."""
     monkeypatch.setenv("PINK_HIP_RESIDENT_SPIN_LIMIT", "0")
