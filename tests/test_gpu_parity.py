@@ -978,6 +978,30 @@ def test_float_trainer_with_screened_distances(monkeypatch, N, C_, I, D, nrot, f
         assert np.array_equal(best[known], want_best[0][known]), max_batch
 
 
+def test_screened_float_trainer_after_an_image_without_bounds(monkeypatch):
+    """An image that holds a NaN and an infinity beside the region: the largest value is then no number, and the weight that the
+    infinity made infinite is moved by the smallest factor."""
+    monkeypatch.setenv("PINK_HIP_RESIDENT_TRAINER", "0")
+    say("screened float trainer after an image without bounds")
+    N, I, D, nrot, ed, n = 9, 100, 96, 360, 91, 17
+    rng = np.random.default_rng(3)
+    som0 = (0.1 + 0.5 * rng.random((N, D, D))).astype(np.float32)
+    imgs = np.full((n, 1, I, I), 0.3, np.float32)
+    imgs[:, 0, 2:98, 2:98] = som0[[0] + (n - 2) * [7] + [5]]           # (fifteen images are not screened behind the first)
+    imgs[0, 0, 2, 2], imgs[0, 0, 97, 97] = np.inf, np.nan
+    F = np.zeros((N, N), np.float32)
+    F[0], F[5] = 0.5, 1e-12
+    want = som0.reshape(N, -1).copy()
+    want_bmu = O.train(O.shape(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT), want, imgs, F)
+    assert want_bmu.tolist() == [0] + (n - 2) * [7] + [5]
+    lost = np.isnan(want)
+    assert lost.reshape(N, D, D)[0, 0, 0]
+    with capi.Context(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT, F, max_batch=n) as ctx:
+        ctx.set_som(som0.reshape(N, -1))
+        bmu, som = ctx.train(imgs), ctx.get_som()
+    assert np.array_equal(bmu, want_bmu) and np.array_equal(np.isnan(som), lost) and np.array_equal(bits(som)[~lost], bits(want)[~lost])
+
+
 @pytest.mark.parametrize("N,ed_type", [(9, capi.FLOAT), (9, capi.UINT8), (530, capi.UINT8)])
 def test_train_with_any_factor_matrix(N, ed_type):
     # the C interface takes any N x N matrix, not only the symmetric ones that a distance functor gives
