@@ -147,7 +147,7 @@ int pink_hip_train(pink_hip_ctx *ctx, const float *host_images, uint32_t n_image
 int pink_hip_update_counts(pink_hip_ctx *ctx, uint32_t *host_counts_out);
 /* Same with the images already on the device and the BMUs left on the device;
  * asynchronous on the context's stream (see pink_hip_synchronize), but for the first kind of
- * trainer below and the first images of the third.  These train a launch group of images in ONE
+ * trainer below and as far as is said of the third.  These train a launch group of images in ONE
  * launch whose blocks stay on the device and exchange one word per image, every wait bounded: they
  * need all their blocks on the device at once, which other work there may keep from them.
  *   - uint8, at most 64 neurons, 32 variants, 2048 elements per neuron, groups of up to 256
@@ -161,8 +161,10 @@ int pink_hip_update_counts(pink_hip_ctx *ctx, uint32_t *host_counts_out);
  *     happens), then the resident form.
  *   - float32, up to 1024 neurons that fit the LDS, regions that are not short: as these, and so
  *     after a launch that found the form slow on its images (variants too close to tell apart
- *     without summing them).  The host waits for the first group, of 32 images, and for the first
- *     one after such a launch.
+ *     without summing them), within the call too.  So that no more images than need be go that way,
+ *     a call returns with at most 32 images queued until that many have gone through well, at
+ *     first and after such a launch; then with at most three groups, or a quarter of the images
+ *     that went through well if that is more.
  * The environment variable PINK_HIP_RESIDENT_TRAINER=0, read when a context is created, selects
  * the other forms from the start. */
 int pink_hip_train_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out);

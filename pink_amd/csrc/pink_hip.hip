@@ -2109,16 +2109,20 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
 #include "f32_train.inc"
 
 // m_update_info[bmu]++ for the images of a group (Trainer.h:302-303), behind a resident launch: nothing when that launch
-// or one before it gave up and nobody rescued it.  The error word goes to the host with it, which looks when it next comes by.
+// or one before it gave up and nobody rescued it.  The error word goes to the host with it, which looks when it next comes by, and how many
+// images of the context's resident launches have been through.
 // Behind k_sym_rescue (one block, `rescue` its ticket and counts per image): what it and the next launch need is made ready again,
 // and how many groups are left to it before a resident launch is tried once more: one after a failure, twice as many after
 // each that follows without a success between (error: the launch that failed, groups left, groups next time).
 __global__ __launch_bounds__(256) void k_count_best_matches(const uint32_t *__restrict__ bmu, uint32_t images, uint32_t *__restrict__ counts,
-                                                            uint32_t *__restrict__ error, uint32_t *__restrict__ host_error,
+                                                            uint32_t *__restrict__ error, uint32_t *__restrict__ host, uint32_t through,
                                                             uint32_t *__restrict__ rescue, unsigned long long *__restrict__ slots, uint32_t slot_words)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, e = *error;
-    if (t == 0) *host_error = e;
+    if (t == 0) {                                         // (a slow launch's number, the word between them, comes from its own kernel)
+        host[0] = e;
+        __hip_atomic_store(&host[2], through, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     if (t < images && (e == 0 || rescue)) atomicAdd(&counts[bmu[t]], 1u);
     if (!rescue) return;
     __syncthreads();
@@ -2443,7 +2447,8 @@ struct pink_hip_ctx {
     float *d_sym_turned = nullptr;
     uint2 *d_sym_state = nullptr;
     float *d_sym_norm_off = nullptr;
-    bool sym_proven = false;                                // a resident launch has gone through since one gave up (float32)
+    uint32_t sym_sent = 0, sym_counted = 0;                // images of resident launches queued; of those through, looked at
+    uint64_t sym_good = 0;                                 // (float32) images through since a launch was slow or gave up
     uint64_t sym_pause = 0, sym_pause_next = 256;          // images to train the other way after a launch gave up; ... the next time
     uint32_t *d_sym_rescue = nullptr;
     unsigned long long *d_sym_keys = nullptr;
@@ -3112,8 +3117,9 @@ void swap_resident(pink_hip_ctx *ctx)
 int resident_launched(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, uint32_t *dev_bmu)
 {
     const bool rescued = ctx->sym_train;
+    ctx->sym_sent += images;
     hipLaunchKernelGGL(k_count_best_matches, dim3((images + 255) / 256), dim3(256), 0, ctx->stream, dev_bmu, images, ctx->d_counts,
-                       ctx->d_resident_error, ctx->h_resident_error, rescued ? ctx->d_sym_rescue : nullptr, ctx->d_slots,
+                       ctx->d_resident_error, ctx->h_resident_error, ctx->sym_sent, rescued ? ctx->d_sym_rescue : nullptr, ctx->d_slots,
                        rescued ? 2 * ctx->N * kSymStride : 0u);
     TRY(launch_check(ctx, "k_count_best_matches"));
     if (!rescued) ctx->resident_queued.push_back({dev_images, images, dev_bmu});
@@ -3308,29 +3314,61 @@ int finish_resident(pink_hip_ctx *ctx)
     return PINK_HIP_OK;
 }
 
-// Whether an integer trainer that can be resident is: after a launch gave up (k_sym_rescue has done its group and those queued
-// behind it) the next images go through the other form, then it is tried again.  The host's copy of the error word says so some
-// time after; a launch that failed before the slots were cleared is not counted twice.
-int choose_sym_form(pink_hip_ctx *ctx, uint32_t n_images)
+// Float32: whether the form suits the data its launches tell behind themselves, and groups queued by then go through it all the same, at
+// a third of the other form's rate where they give up.  So until kF32Probe images have gone through well no more than that
+// many are queued unseen; then three groups, or a quarter of the images that went through well: what groups queued too
+// many can cost (53 us an image) stays about what the others gained (4 to 14).  *count: the images to queue now.
+int await_resident(pink_hip_ctx *ctx, uint32_t *count)
+{
+    const volatile uint32_t *const word = ctx->h_resident_error;
+    for (;;) {
+        const uint32_t through = word[2];
+        std::atomic_thread_fence(std::memory_order_acquire);
+        for (const uint32_t launch : {(uint32_t)word[0], (uint32_t)word[1]})
+            if (launch && (int32_t)(launch - ctx->sym_seen) > 0) return PINK_HIP_OK;       // (choose_sym_form's)
+        if ((int32_t)(through - ctx->sym_counted) > 0) {
+            ctx->sym_good += through - ctx->sym_counted;
+            ctx->sym_counted = through;
+        }
+        const bool proven = ctx->sym_good >= kF32Probe;
+        const uint32_t unseen = ctx->sym_sent - through, next = std::min({*count, ctx->sym_B, proven ? ctx->sym_B : kF32Probe});
+        const uint64_t ahead = proven ? std::max<uint64_t>(3 * (uint64_t)ctx->sym_B, ctx->sym_good / 4) : kF32Probe;
+        if (unseen == 0 || unseen + next <= ahead) { *count = next; return PINK_HIP_OK; }
+        const hipError_t e = hipStreamQuery(ctx->stream);
+        (void)hipGetLastError();                          // (a stream that still runs is no error)
+        if (e != hipErrorNotReady) HIP_TRY(ctx, e);
+        std::this_thread::yield();
+    }
+}
+
+// Whether a trainer that can be resident is: after a launch gave up (k_sym_rescue or k_f32_rescue has done its group and those
+// queued behind it), or a float32 one went through slowly, the next images go through the other form, then it is tried again.  The
+// host's words say so some time after; a launch that failed before the slots were cleared is not counted twice.  *count: images to
+// train in the form chosen, then to be asked again.
+int choose_sym_form(pink_hip_ctx *ctx, uint32_t *count)
 {
     if (!ctx->sym_form) return PINK_HIP_OK;
     const volatile uint32_t *const word = ctx->h_resident_error;
+    if (!ctx->sym_train && ctx->sym_pause == 0) ctx->sym_train = true;
+    if (ctx->sym_train && ctx->sym_f32) TRY(await_resident(ctx, count));
     uint32_t failed = word[0];
-    if (word[1] && (int32_t)(word[1] - ctx->sym_seen) > 0) failed = word[1];       // (float32: gone through, but slowly)
+    if (word[1] && (int32_t)(word[1] - ctx->sym_seen) > 0) failed = word[1];       // (float32: by its data, or gone through but slowly)
     if (ctx->sym_train && failed && (int32_t)(failed - ctx->sym_seen) > 0) {
         ctx->sym_seen = ctx->sym_launch;
+        ctx->sym_counted = ctx->sym_sent;
+        ctx->sym_good = 0;
         const size_t slots = (size_t)ctx->N * kSymStride;              // (16-byte words of both sets)
         hipLaunchKernelGGL(k_fill_zero, dim3((uint32_t)((slots + 255) / 256)), dim3(256), 0, ctx->stream, (v4i *)ctx->d_slots, slots);
         hipLaunchKernelGGL(k_fill_zero, dim3(1), dim3(256), 0, ctx->stream, (v4i *)ctx->d_resident_error, (size_t)1);
         TRY(launch_check(ctx, "k_fill_zero"));
         TRY(run_pack_som(ctx));                            // the other form's operand of the SOM as it is now
-        ctx->sym_train = ctx->sym_proven = false;
+        ctx->sym_train = false;
         ctx->sym_pause = ctx->sym_pause_next;
         ctx->sym_pause_next = std::min<uint64_t>(4 * ctx->sym_pause_next, 1u << 20);
     }
     if (!ctx->sym_train) {
-        if (ctx->sym_pause == 0) ctx->sym_train = true;
-        else ctx->sym_pause -= std::min<uint64_t>(ctx->sym_pause, n_images);
+        if (ctx->sym_f32) *count = (uint32_t)std::min<uint64_t>(*count, ctx->sym_pause);
+        ctx->sym_pause -= std::min<uint64_t>(ctx->sym_pause, *count);
     }
     return PINK_HIP_OK;
 }
@@ -3428,11 +3466,11 @@ int init_exchange(pink_hip_ctx *ctx, size_t slot_words, const void *kernel, uint
     HIP_TRY(ctx, hipMemset(ctx->d_slots, 0, slot_words * sizeof(unsigned long long)));
     TRY(dev_alloc(ctx, &ctx->d_resident_error, 4));
     HIP_TRY(ctx, hipMemset(ctx->d_resident_error, 0, 4 * sizeof(uint32_t)));
-    if (hipHostMalloc((void **)&ctx->h_resident_error, 2 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc((void **)&ctx->h_resident_error, 3 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
         ctx->h_resident_error = nullptr;
         return fail(ctx, PINK_HIP_ENOMEM, "pinned host allocation failed");
     }
-    ctx->h_resident_error[0] = ctx->h_resident_error[1] = 0;
+    std::fill_n(ctx->h_resident_error, 3, 0u);
     return PINK_HIP_OK;
 }
 
@@ -4843,27 +4881,10 @@ int distance_group(pink_hip_ctx *ctx, const float *dev_images, uint32_t B, bool 
 
 int distance_group(pink_hip_ctx *ctx, const float *dev_images, uint32_t B) { return distance_group(ctx, dev_images, B, B <= ctx->sum_images); }
 
-// Training of images that are on the device, queued on the context's stream.
-int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
+// Training of images that are on the device, queued on the context's stream: in launch groups, a launch or more per image or a
+// resident launch of a small uint8 trainer for all of them.
+int train_in_turn(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
 {
-    if (ctx->orbit_train) return run_orbit_train(ctx, dev_images, n_images, dev_bmu_out);
-    TRY(choose_sym_form(ctx, n_images));
-    if (ctx->sym_train) {
-        for (uint32_t done = 0; done < n_images;) {
-            // (float32: whether the form suits the data, a small first group says -- ahead of the groups that would be queued behind it)
-            const bool probe = ctx->sym_f32 && !ctx->sym_proven;
-            const uint32_t B = std::min(probe ? std::min(ctx->sym_B, kF32Probe) : ctx->sym_B, n_images - done);
-            TRY(run_sym_train(ctx, dev_images + (size_t)done * ctx->isz, B, dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group));
-            done += B;
-            if (!probe) continue;
-            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-            const volatile uint32_t *const word = ctx->h_resident_error;
-            ctx->sym_proven = word[0] == 0 && (word[1] == 0 || (int32_t)(word[1] - ctx->sym_seen) <= 0);
-            if (!ctx->sym_proven && done < n_images)
-                return train_queued(ctx, dev_images + (size_t)done * ctx->isz, n_images - done, dev_bmu_out ? dev_bmu_out + done : nullptr);
-        }
-        return PINK_HIP_OK;
-    }
     // The variants of an image and their packed distance operand do not depend on the SOM: they
     // are produced for a group of images per launch.  Distance and update stay strictly sequential.
     for (uint32_t done = 0; done < n_images; done += ctx->Bcap) {
@@ -4913,6 +4934,22 @@ int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, 
             if (!ctx->d_inv || (ctx->gemm && !ctx->fused_som)) TRY(run_pack_som(ctx));
             else if (ctx->f32gemm) { Timed t(ctx, kClsPack); TRY(run_pack_frag_som(ctx)); }
         }
+    }
+    return PINK_HIP_OK;
+}
+
+// ... in the form that the context takes at present.
+int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
+{
+    if (ctx->orbit_train) return run_orbit_train(ctx, dev_images, n_images, dev_bmu_out);
+    for (uint32_t done = 0, count; done < n_images; done += count) {
+        count = n_images - done;
+        TRY(choose_sym_form(ctx, &count));
+        const float *images = dev_images + (size_t)done * ctx->isz;
+        uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : nullptr;
+        if (!ctx->sym_train) TRY(train_in_turn(ctx, images, count, bmu));
+        for (uint32_t b = 0; ctx->sym_train && b < count; b += ctx->sym_B)
+            TRY(run_sym_train(ctx, images + (size_t)b * ctx->isz, std::min(ctx->sym_B, count - b), bmu ? bmu + b : ctx->d_bmu_group));
     }
     return PINK_HIP_OK;
 }

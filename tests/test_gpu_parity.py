@@ -730,6 +730,95 @@ def test_resident_float_trainer_on_awkward_data(kind):
     assert np.array_equal(bmu, want_bmu) and np.array_equal(np.isnan(som), lost) and np.array_equal(bits(som)[~lost], bits(want)[~lost])
 
 
+class FloatTrainer:
+    """A resident float32 trainer beside one that sums every variant; counts the launch groups of a call."""
+    N, I, D, nrot, ed = 12, 40, 32, 180, 25
+
+    def __init__(self):
+        F = capi.make_update_factors(capi.CARTESIAN, [self.N], capi.GAUSSIAN, 1.0, 0.5)
+        self.ctx, self.plain = (capi.Context(self.N, 1, self.I, self.D, self.nrot, True, self.ed, capi.QUADRATIC, capi.FLOAT, F, kernel_choice=k)
+                                for k in (capi.KERNEL_AUTO, capi.KERNEL_VALU))
+        self.rng = np.random.default_rng(5)
+        som = self.rng.random((self.N, self.D ** 2), dtype=np.float32)
+        for c in (self.ctx, self.plain):
+            c.set_som(som)
+        self.ctx.set_profiling(True)
+
+    def images(self, n, flat=None):
+        imgs = self.rng.random((n, 1, self.I, self.I), dtype=np.float32)
+        if flat:
+            imgs[flat] = 0.25                                          # (all variants alike)
+        return imgs
+
+    def groups(self, imgs):
+        before = self.ctx.kernel_times()["rotate"][0]
+        assert np.array_equal(self.ctx.train(imgs), self.plain.train(imgs))
+        return self.ctx.kernel_times()["rotate"][0] - before
+
+    def check(self):
+        assert np.array_equal(bits(self.ctx.get_som()), bits(self.plain.get_som()))
+        assert np.array_equal(self.ctx.update_counts(), self.plain.update_counts())
+        self.ctx.close()
+        self.plain.close()
+
+
+def test_resident_float_trainer_is_tried_on_enough_images():
+    """One image that went through says little of the call behind it: flat images show within 32 of them, and the others take the
+    other form, whose launch groups are smaller."""
+    say("resident float trainer, one image first")
+    t = FloatTrainer()
+    assert t.groups(t.images(1)) == 1
+    groups = t.groups(t.images(300, slice(None)))
+    say("groups", groups)
+    t.check()
+    assert groups >= 6
+
+
+def test_resident_float_trainer_looks_up_during_a_call():
+    """A call that turns flat behind images that went through well leaves the resident form within a few groups."""
+    say("resident float trainer, a long call turns flat")
+    t = FloatTrainer()
+    t.groups(t.images(64))
+    groups = t.groups(t.images(3000, slice(300, None)))
+    say("groups", groups)
+    t.check()
+    assert groups >= 30
+
+
+def test_resident_float_trainer_leaves_what_is_slow_and_comes_back():
+    """A launch that spent too many sums without giving up: the next 256 images take the other form, then the form is tried again."""
+    say("resident float trainer, slow launches")
+    t = FloatTrainer()
+    t.groups(t.images(64))
+    proven = t.groups(t.images(150))
+    t.groups(t.images(90, slice(None, None, 3)))
+    away, back = t.groups(t.images(256)), t.groups(t.images(150))
+    say("groups", proven, away, back)
+    t.check()
+    assert proven == 1 and away >= 4 and back <= 2
+
+
+def test_resident_float_training_is_queued():
+    """pink_hip_train_device returns while the device still trains a context's first images."""
+    import time
+    from test_zz_no_alloc import Hip
+    N, I, D, n = 9, 64, 64, 32
+    F = capi.make_update_factors(capi.CARTESIAN, [3, 3], capi.GAUSSIAN, 1.1, 0.2)
+    hip = Hip()
+    imgs, bmu = hip.upload(np.random.default_rng(4).random((n, 1, I, I), dtype=np.float32)), hip.alloc(4 * n)
+    for _ in range(2):                                                 # (the first context loads the kernels)
+        with capi.Context(N, 1, I, D, 360, True, 64, capi.QUADRATIC, capi.FLOAT, F) as ctx:
+            ctx.set_som(np.random.default_rng(5).random((N, D * D), dtype=np.float32))
+            start = time.perf_counter()
+            ctx.train_device(imgs, n, bmu)
+            queued = time.perf_counter() - start
+            ctx.synchronize()
+            whole = time.perf_counter() - start
+    hip.release()
+    say("queued after", queued, "of", whole)
+    assert queued < 0.7 * whole
+
+
 @pytest.mark.parametrize("N,I,D,nrot,ed,ed_type", [
     (30, 24, 30, 20, 9, capi.UINT8),
     (30, 24, 30, 20, 9, capi.UINT16),
