@@ -2449,7 +2449,7 @@ struct pink_hip_ctx {
     float *d_sym_norm_off = nullptr;
     uint32_t sym_sent = 0, sym_counted = 0;                // images of resident launches queued; of those through, looked at
     uint64_t sym_good = 0;                                 // (float32) images through since a launch was slow or gave up
-    uint64_t sym_pause = 0, sym_pause_next = 256;          // images to train the other way after a launch gave up; ... the next time
+    uint64_t sym_pause = 0, sym_pause_next = kSymPause;    // images to train the other way after a launch gave up; ... the next time
     uint32_t *d_sym_rescue = nullptr;
     unsigned long long *d_sym_keys = nullptr;
     uint32_t sym_npb = 1, sym_nit = 0, sym_B = 0, sym_KS = 0, sym_RT = 0, sym_all = 0, sym_cells = 0, sym_outside = 0, sym_tag0 = 1;
@@ -3327,8 +3327,11 @@ int await_resident(pink_hip_ctx *ctx, uint32_t *count)
         for (const uint32_t launch : {(uint32_t)word[0], (uint32_t)word[1]})
             if (launch && (int32_t)(launch - ctx->sym_seen) > 0) return PINK_HIP_OK;       // (choose_sym_form's)
         if ((int32_t)(through - ctx->sym_counted) > 0) {
+            // (a launch is slow by its images: a thousand that were not, and what came before counts a quarter)
+            const uint64_t before = ctx->sym_good / kF32Forget;
             ctx->sym_good += through - ctx->sym_counted;
             ctx->sym_counted = through;
+            for (uint64_t k = before; k < ctx->sym_good / kF32Forget && ctx->sym_pause_next > kSymPause; ++k) ctx->sym_pause_next /= 4;
         }
         const bool proven = ctx->sym_good >= kF32Probe;
         const uint32_t unseen = ctx->sym_sent - through, next = std::min({*count, ctx->sym_B, proven ? ctx->sym_B : kF32Probe});

@@ -798,6 +798,28 @@ def test_resident_float_trainer_leaves_what_is_slow_and_comes_back():
     assert proven == 1 and away >= 4 and back <= 2
 
 
+def test_resident_float_trainer_forgets_slow_launches():
+    """The images that take the other form behind a slow launch are four times as many the next time, but not where a thousand went
+    through well between."""
+    say("resident float trainer, slow launches long apart")
+    t = FloatTrainer()
+    slow = slice(None, None, 3)
+    t.groups(t.images(64))
+    for between in (0, 1200):
+        t.groups(t.images(between))
+        t.groups(t.images(90, slow))
+        t.groups(t.images(256))
+        back = t.groups(t.images(150))
+        say("groups", back)
+        assert back <= 2
+    t.groups(t.images(90, slow))
+    t.groups(t.images(256))
+    still_away = t.groups(t.images(150))
+    say("groups", still_away)
+    t.check()
+    assert still_away > 2
+
+
 def test_resident_float_training_is_queued():
     """pink_hip_train_device returns while the device still trains a context's first images."""
     import time
