@@ -2487,6 +2487,10 @@ struct pink_hip_ctx {
     bool orbit_train = false;
     // ... and the float32 trainers that screen their distances: rows_f32_train's operands, the product's beside them
     bool screen_train = false;
+    // images of a call up to which a float32 trainer sums every variant all the same, beside the resident form and beside screening
+    uint32_t few_resident = 0, few_screened = 0;
+    // whether the operands of training in turn, and of those the product's, hold the weights as they are (a form keeps its own)
+    bool packed = false, screen_packed = false;
     uint32_t screen_set = 0;               // the counts that the last image took
     uint2 *d_screen_list = nullptr;
     uint32_t *d_screen_wide = nullptr, *d_screen_counts = nullptr, *d_screen_choice = nullptr;
@@ -2645,15 +2649,13 @@ int run_pack_frag_som(pink_hip_ctx *ctx)
 }
 
 int run_orbit_som(pink_hip_ctx *ctx);
-int run_screen_range(pink_hip_ctx *ctx);
+int run_screen_pack(pink_hip_ctx *ctx);
 
 int run_pack_som(pink_hip_ctx *ctx)
 {
+    ctx->packed = true;
+    if (ctx->screen_train) TRY(run_screen_pack(ctx));
     Timed t(ctx, kClsPack);
-    if (ctx->screen_train) {
-        TRY(run_orbit_som(ctx));
-        TRY(run_screen_range(ctx));
-    }
     if (ctx->orbit) {
         TRY(run_orbit_som(ctx));
         if (is_int(ctx)) return PINK_HIP_OK;              // (float32: the rows in the CPU's order too)
@@ -3031,7 +3033,7 @@ int run_update_rows(pink_hip_ctx *ctx, uint32_t slot, uint32_t *dev_bmu_out)
 }
 
 // The updates of the first `images` images of the current group applied to the neurons' full images, in order.
-int run_update_replay(pink_hip_ctx *ctx, uint32_t images, const uint32_t *dev_bmu)
+int run_update_replay(pink_hip_ctx *ctx, uint32_t images, const uint32_t *dev_bmu, bool screened)
 {
     Timed t(ctx, kClsUpdate);
     VariantPair vp{};
@@ -3042,7 +3044,7 @@ int run_update_replay(pink_hip_ctx *ctx, uint32_t images, const uint32_t *dev_bm
     hipLaunchKernelGGL(k_update_replay<EPT_>, dim3(ctx->N, (ctx->S + 256 * EPT_ - 1) / (256 * EPT_)), dim3(256), 0, ctx->stream, \
                        ctx->d_som, ctx->d_rot + (size_t)first * ctx->R * ctx->S, ctx->d_key + (size_t)first * ctx->N,            \
                        ctx->d_factors, dev_bmu + first, count, ctx->N, ctx->S, ctx->R, ctx->shift, vp,                                            \
-                       ctx->screen_train ? ctx->d_screen_moves + (size_t)first * ctx->N : nullptr)
+                       screened ? ctx->d_screen_moves + (size_t)first * ctx->N : nullptr)
         // (large SOMs: several elements per thread -- 1600 neurons of 3 x 70 x 70: 13.6 us per image with one, 10.2 with
         // two, 9.0 with four; small ones need the blocks -- 100 neurons of 45 x 45: 0.42, 0.46)
         const size_t weights = (size_t)ctx->N * ctx->S;
@@ -3216,6 +3218,7 @@ uint32_t f32_rescue_parts(const pink_hip_ctx *ctx) { return std::max(1u, (uint32
 // elements outside the region.
 int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, uint32_t *dev_bmu)
 {
+    ctx->packed = ctx->screen_packed = false;
     {
         Timed t(ctx, kClsRotate);
         SymPrep p{};
@@ -3364,7 +3367,6 @@ int choose_sym_form(pink_hip_ctx *ctx, uint32_t *count)
         hipLaunchKernelGGL(k_fill_zero, dim3((uint32_t)((slots + 255) / 256)), dim3(256), 0, ctx->stream, (v4i *)ctx->d_slots, slots);
         hipLaunchKernelGGL(k_fill_zero, dim3(1), dim3(256), 0, ctx->stream, (v4i *)ctx->d_resident_error, (size_t)1);
         TRY(launch_check(ctx, "k_fill_zero"));
-        TRY(run_pack_som(ctx));                            // the other form's operand of the SOM as it is now
         ctx->sym_train = false;
         ctx->sym_pause = ctx->sym_pause_next;
         ctx->sym_pause_next = std::min<uint64_t>(4 * ctx->sym_pause_next, 1u << 20);
@@ -3953,6 +3955,21 @@ bool orbit_trains(const pink_hip_ctx *ctx)
     return !resident;
 }
 
+// Float32 trainers: calls of few images.  Beside the resident form a launch per image saves the two launches behind a group, the neurons' way
+// into the LDS and back; beside screening five launches an image.  Images up to which it is no slower, from what a call takes
+// (us, 720 and 16 variants, a launch per image | resident: 100 neurons of 400 elements, 1 image 32 | 42 and 29 | 42, 3 images 56 | 59
+// and 46 | 58, 6 images 87 | 76 and 67 | 74; of 1024 elements 40 | 49 and 34 | 46, 3 images 80 | 72 and 60 | 64; 256 of 2025, 1 image
+// 69 | 63 and 45 | 61; 520 of 400 elements, four to a block, 720 variants, 2 images 61 | 78, 4 images 99 | 110; 720 variants, a launch per
+// image | screened: 9 of 8100 elements 126 | 148, 2 images 197 | 178; 100 of 16384 245 | 393, 3 images 650 | 583; 1600 of 1024
+// 96 | 80), over 4 to 1600 neurons, 225 to 16384 elements.
+void choose_few(pink_hip_ctx *ctx)
+{
+    const double E = ctx->E, R = ctx->R, NR = (double)ctx->N * ctx->R;
+    const auto up_to = [](double fixed, double per_image) { return (uint32_t)std::min(32.0, per_image > 0.0 ? fixed / per_image : 32.0); };
+    if (ctx->sym_f32) ctx->few_resident = up_to(1.5 + 4.0 * ctx->sym_npb + 0.0065 * E, E * (0.0038 + 2e-8 * NR + 3.4e-6 * R) - 0.6);
+    if (ctx->screen_train) ctx->few_screened = up_to(1.2 + 0.0116 * E, E * (0.0053 + 4.3e-8 * NR + 1.8e-6 * R) + 5.0);
+}
+
 int run_orbit_som(pink_hip_ctx *ctx)
 {
     const uint32_t Kp = ctx->orb_KS * 32;
@@ -3978,6 +3995,15 @@ int run_screen_range(pink_hip_ctx *ctx)
 {
     hipLaunchKernelGGL(k_screen_range, dim3(ctx->N), dim3(256), 0, ctx->stream, ctx->d_som, (WeightRange *)ctx->d_screen_range, ctx->S);
     return launch_check(ctx, "k_screen_range");
+}
+
+// ... and the product's operand.
+int run_screen_pack(pink_hip_ctx *ctx)
+{
+    Timed t(ctx, kClsPack);
+    ctx->screen_packed = true;
+    TRY(run_orbit_som(ctx));
+    return run_screen_range(ctx);
 }
 
 template <int MODE, int WM, int WN, int KC, int PD, int MINB>
@@ -4767,11 +4793,12 @@ int init_ctx(pink_hip_ctx *ctx)
         // way than with an update launch of their own -- with three to four waves per SIMD the launch saved is paid in
         // instructions)
         ctx->screen_train = ctx->screen_train && !ctx->f32gemm && ctx->d_somP && ctx->d_inv && B <= kReplayMax;
-        ctx->fused_f32_train = !ctx->screen_train && c.ed_type == PINK_HIP_FLOAT && !ctx->f32gemm && ctx->d_somP && ctx->d_inv && ctx->N <= 256 &&
+        ctx->fused_f32_train = c.ed_type == PINK_HIP_FLOAT && !ctx->f32gemm && ctx->d_somP && ctx->d_inv && ctx->N <= 256 &&
                                (size_t)(ctx->Rpad / kWave) * ((ctx->N + 3) / 4) <= (size_t)4 * ctx->num_cu;
-        ctx->rows_f32_train = !ctx->fused_f32_train && c.ed_type == PINK_HIP_FLOAT && !ctx->f32gemm && ctx->d_somP && ctx->d_inv &&
+        ctx->rows_f32_train = (!ctx->fused_f32_train || ctx->screen_train) && c.ed_type == PINK_HIP_FLOAT && !ctx->f32gemm && ctx->d_somP && ctx->d_inv &&
                               B <= kReplayMax;
         ctx->screen_train = ctx->screen_train && ctx->rows_f32_train;
+        choose_few(ctx);
         if (ctx->screen_train) {
             TRY(dev_alloc(ctx, (char **)&ctx->d_orb_rows, orbit_rows_bytes(ctx, B)));
             TRY(dev_alloc(ctx, (CoefRow **)&ctx->d_coef_row, B * ctx->nrr_eff));
@@ -4885,16 +4912,19 @@ int distance_group(pink_hip_ctx *ctx, const float *dev_images, uint32_t B, bool 
 int distance_group(pink_hip_ctx *ctx, const float *dev_images, uint32_t B) { return distance_group(ctx, dev_images, B, B <= ctx->sum_images); }
 
 // Training of images that are on the device, queued on the context's stream: in launch groups, a launch or more per image or a
-// resident launch of a small uint8 trainer for all of them.
-int train_in_turn(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
+// resident launch of a small uint8 trainer for all of them.  screened: float32 distances, where the context can.
+int train_in_turn(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out, bool screened)
 {
+    if (!ctx->packed) TRY(run_pack_som(ctx));
+    if (screened && !ctx->screen_packed) TRY(run_screen_pack(ctx));
+    ctx->screen_packed = screened;
     // The variants of an image and their packed distance operand do not depend on the SOM: they
     // are produced for a group of images per launch.  Distance and update stay strictly sequential.
     for (uint32_t done = 0; done < n_images; done += ctx->Bcap) {
         const uint32_t B = std::min(ctx->Bcap, n_images - done);
         TRY(run_rotate(ctx, dev_images + (size_t)done * ctx->isz, B, ctx->pair_variants ? kStorePair : kStoreAll));
         TRY(run_pack_rot(ctx, B));
-        if (ctx->fused_f32_train) {
+        if (ctx->fused_f32_train && !screened) {
             // every launch but the first applies the update of the image before it; the last image's update and,
             // ahead of it, all the others on the neurons' full images close the group
             uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group;
@@ -4903,15 +4933,15 @@ int train_in_turn(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images,
                 Timed t(ctx, kClsDist, B);
                 for (uint32_t b = 0; b < B; ++b) TRY(run_train_f32(ctx, b, b > 0, b > 0 ? bmu + b - 1 : nullptr));
             }
-            if (B > 1) TRY(run_update_replay(ctx, B - 1, bmu));
+            if (B > 1) TRY(run_update_replay(ctx, B - 1, bmu, false));
             TRY(run_update(ctx, B - 1, bmu + B - 1));
             continue;
         }
         if (ctx->rows_f32_train) {
-            if (ctx->screen_train) TRY(run_orbit_rows(ctx, dev_images + (size_t)done * ctx->isz, B));
+            if (screened) TRY(run_orbit_rows(ctx, dev_images + (size_t)done * ctx->isz, B));
             uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group;
             for (uint32_t b = 0; b < B; ++b) {
-                if (ctx->screen_train) {
+                if (screened) {
                     TRY(run_screen_keys(ctx, b));
                     TRY(run_screen_update(ctx, b, bmu + b));
                     continue;
@@ -4919,8 +4949,8 @@ int train_in_turn(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images,
                 TRY(run_dist(ctx, b, 1));
                 TRY(run_update_rows(ctx, b, bmu + b));
             }
-            TRY(run_update_replay(ctx, B, bmu));
-            if (ctx->screen_train) TRY(run_screen_range(ctx));
+            TRY(run_update_replay(ctx, B, bmu, screened));
+            if (screened) TRY(run_screen_range(ctx));
             continue;
         }
         if (ctx->resident_train) {
@@ -4947,12 +4977,14 @@ int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, 
     if (ctx->orbit_train) return run_orbit_train(ctx, dev_images, n_images, dev_bmu_out);
     for (uint32_t done = 0, count; done < n_images; done += count) {
         count = n_images - done;
-        TRY(choose_sym_form(ctx, &count));
+        const bool few = n_images <= ctx->few_resident;
+        if (!few) TRY(choose_sym_form(ctx, &count));
         const float *images = dev_images + (size_t)done * ctx->isz;
         uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : nullptr;
-        if (!ctx->sym_train) TRY(train_in_turn(ctx, images, count, bmu));
-        for (uint32_t b = 0; ctx->sym_train && b < count; b += ctx->sym_B)
-            TRY(run_sym_train(ctx, images + (size_t)b * ctx->isz, std::min(ctx->sym_B, count - b), bmu ? bmu + b : ctx->d_bmu_group));
+        if (few || !ctx->sym_train) TRY(train_in_turn(ctx, images, count, bmu, ctx->screen_train && !few && n_images > ctx->few_screened));
+        else
+            for (uint32_t b = 0; b < count; b += ctx->sym_B)
+                TRY(run_sym_train(ctx, images + (size_t)b * ctx->isz, std::min(ctx->sym_B, count - b), bmu ? bmu + b : ctx->d_bmu_group));
     }
     return PINK_HIP_OK;
 }
@@ -5535,7 +5567,7 @@ int pink_hip_distance(pink_hip_ctx *ctx, const float *host_image, float *host_di
     HIP_TRY(ctx, hipMalloc((void **)&d_img, (size_t)ctx->isz * sizeof(float)));
     hipError_t e = hipMemcpyAsync(d_img, host_image, (size_t)ctx->isz * sizeof(float), hipMemcpyHostToDevice, ctx->stream);
     int rc = PINK_HIP_OK;
-    if (e == hipSuccess && ctx->sym_train) rc = run_pack_som(ctx);        // (its training does not keep this operand)
+    if (e == hipSuccess && !ctx->packed) rc = run_pack_som(ctx);          // (resident training does not keep this operand)
     if (e == hipSuccess && rc == PINK_HIP_OK) rc = distance_group(ctx, d_img, 1);
     if (e == hipSuccess && rc == PINK_HIP_OK) rc = run_finalize(ctx, 1, ctx->d_dist, ctx->d_ssd, ctx->d_best, false);
     const size_t n = ctx->N;

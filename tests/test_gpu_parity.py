@@ -732,9 +732,8 @@ def test_resident_float_trainer_on_awkward_data(kind):
 
 class FloatTrainer:
     """A resident float32 trainer beside one that sums every variant; counts the launch groups of a call."""
-    N, I, D, nrot, ed = 12, 40, 32, 180, 25
-
-    def __init__(self):
+    def __init__(self, N=12, I=40, D=32, nrot=180, ed=25):
+        self.N, self.I, self.D, self.nrot, self.ed = N, I, D, nrot, ed
         F = capi.make_update_factors(capi.CARTESIAN, [self.N], capi.GAUSSIAN, 1.0, 0.5)
         self.ctx, self.plain = (capi.Context(self.N, 1, self.I, self.D, self.nrot, True, self.ed, capi.QUADRATIC, capi.FLOAT, F, kernel_choice=k)
                                 for k in (capi.KERNEL_AUTO, capi.KERNEL_VALU))
@@ -818,6 +817,52 @@ def test_resident_float_trainer_forgets_slow_launches():
     say("groups", still_away)
     t.check()
     assert still_away > 2
+
+
+@pytest.mark.parametrize("N,I,D,nrot,ed", [
+    (12, 40, 32, 180, 25),
+    (300, 30, 26, 60, 21),                                             # two neurons to a block
+    (200, 60, 50, 100, 45),                                            # resident, screened and summed
+    (9, 100, 96, 360, 91),                                             # screened and summed
+    (100, 24, 20, 360, 15),
+])
+def test_float_trainer_in_calls_of_every_size(N, I, D, nrot, ed):
+    """Calls of few images take a form of their own; every form goes on from the weights that another left."""
+    say("float trainer in calls of every size", N, I, D, nrot, ed)
+    t = FloatTrainer(N, I, D, nrot, ed)
+    for n in (1, 1, 33, 1, 2, 40, 3, 4, 36, 1, 6, 12, 34, 34, 5):
+        imgs = t.images(n)
+        t.groups(imgs)
+        if n < 34:
+            (d, _, best), (want_d, _, want_best) = t.ctx.distance(imgs[0]), t.plain.distance(imgs[0])
+            assert np.array_equal(best, want_best) and np.array_equal(bits(d), bits(want_d)), n
+    t.check()
+
+
+@pytest.mark.parametrize("N,I,D,nrot,ed", [(12, 40, 32, 180, 25), (9, 64, 51, 8, 45), (9, 180, 150, 8, 128)])
+def test_float_training_of_one_image_takes_no_longer_than_its_kernels(monkeypatch, N, I, D, nrot, ed):
+    """A call of one image: what sums every variant in a launch, not what launches a group or five kernels."""
+    import time
+    from test_zz_no_alloc import Hip
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 1.0, 0.5)
+    hip = Hip()
+    rng = np.random.default_rng(4)
+    imgs, som = hip.upload(rng.random((40, 1, I, I), dtype=np.float32)), rng.random((N, D * D), dtype=np.float32)
+    taken = []
+    for choice in (capi.KERNEL_VALU, capi.KERNEL_AUTO):
+        with capi.Context(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT, F, kernel_choice=choice) as ctx:
+            ctx.set_som(som)
+            ctx.train_device(imgs, 40)
+            times = []
+            for _ in range(60):
+                start = time.perf_counter()
+                ctx.train_device(imgs, 1)
+                ctx.synchronize()
+                times.append(time.perf_counter() - start)
+            taken.append(sorted(times)[30])
+    hip.release()
+    say("one image", taken)
+    assert taken[1] < 1.15 * taken[0]
 
 
 def test_resident_float_training_is_queued():
