@@ -165,6 +165,10 @@ int pink_hip_update_counts(pink_hip_ctx *ctx, uint32_t *host_counts_out);
  *     a call returns with at most 32 images queued until that many have gone through well, at
  *     first and after such a launch; then with at most three groups, or a quarter of the images
  *     that went through well if that is more.
+ *   - float32 beyond that, where the distances are screened: a launch group in which most variants
+ *     have to be summed image after image sends later images another way likewise.  A call returns
+ *     with at most eight groups (64 images each at most), or a quarter as above, queued; with 32
+ *     images where that has happened until as many have gone through well.
  * The environment variable PINK_HIP_RESIDENT_TRAINER=0, read when a context is created, selects
  * the other forms from the start. */
 int pink_hip_train_device(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out);

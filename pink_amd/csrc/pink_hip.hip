@@ -2338,6 +2338,15 @@ enum : uint32_t { kStoreNone = 0, kStoreAll = 1, kStorePair = 2 };
 
 }  // namespace
 
+// A form of training that does not suit all data, and what the host has seen of it.
+struct FormTrial {
+    uint32_t *word = nullptr;              // the host's, pinned: a launch that gave up, the last one that was slow, images gone through
+    uint32_t launch = 0, seen = 0;         // the last launch queued; the last one when it was left, so that none counts twice
+    uint32_t sent = 0, counted = 0;        // images queued; of those through, looked at
+    uint64_t good = 0;                     // images through since it was left
+    uint64_t pause = 0, pause_next = kSymPause;            // images to train the other way; ... the next time
+};
+
 struct pink_hip_ctx {
     pink_hip_config cfg{};
     uint32_t N = 0, C = 0, I = 0, D = 0, S = 0, R = 0, nrr = 0, E = 0, Epad = 0, Rpad = 0;
@@ -2436,7 +2445,7 @@ struct pink_hip_ctx {
     // integer trainers with the symmetries on the SOM side, resident over a launch group (k_train_sym_resident); the GEMM
     // path's operands are then made when something else wants them
     bool sym_form = false, sym_train = false;              // the context can; it does at present
-    uint32_t sym_launch = 0, sym_seen = 0;                 // the last resident launch queued; the last one before the slots were cleared
+    FormTrial sym_trial, screen_trial;                     // resident launches; groups of images that are screened (screen_train)
     bool sym_f32 = false;                                  // float32 (f32_train.inc)
     uint32_t sym_row = 0, sym_sum_waves = 0;
     float *d_sym_err = nullptr;
@@ -2447,9 +2456,6 @@ struct pink_hip_ctx {
     float *d_sym_turned = nullptr;
     uint2 *d_sym_state = nullptr;
     float *d_sym_norm_off = nullptr;
-    uint32_t sym_sent = 0, sym_counted = 0;                // images of resident launches queued; of those through, looked at
-    uint64_t sym_good = 0;                                 // (float32) images through since a launch was slow or gave up
-    uint64_t sym_pause = 0, sym_pause_next = kSymPause;    // images to train the other way after a launch gave up; ... the next time
     uint32_t *d_sym_rescue = nullptr;
     unsigned long long *d_sym_keys = nullptr;
     uint32_t sym_npb = 1, sym_nit = 0, sym_B = 0, sym_KS = 0, sym_RT = 0, sym_all = 0, sym_cells = 0, sym_outside = 0, sym_tag0 = 1;
@@ -3119,9 +3125,9 @@ void swap_resident(pink_hip_ctx *ctx)
 int resident_launched(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, uint32_t *dev_bmu)
 {
     const bool rescued = ctx->sym_train;
-    ctx->sym_sent += images;
+    ctx->sym_trial.sent += images;
     hipLaunchKernelGGL(k_count_best_matches, dim3((images + 255) / 256), dim3(256), 0, ctx->stream, dev_bmu, images, ctx->d_counts,
-                       ctx->d_resident_error, ctx->h_resident_error, ctx->sym_sent, rescued ? ctx->d_sym_rescue : nullptr, ctx->d_slots,
+                       ctx->d_resident_error, ctx->h_resident_error, ctx->sym_trial.sent, rescued ? ctx->d_sym_rescue : nullptr, ctx->d_slots,
                        rescued ? 2 * ctx->N * kSymStride : 0u);
     TRY(launch_check(ctx, "k_count_best_matches"));
     if (!rescued) ctx->resident_queued.push_back({dev_images, images, dev_bmu});
@@ -3250,7 +3256,7 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         a.factors_t = ctx->d_factors_t; a.cell_elem = ctx->d_sym_elem; a.cell_at = ctx->d_sym_at; a.cell_run = ctx->d_sym_run; a.to = ctx->d_sym_to;
         a.state = ctx->d_sym_state; a.slow = ctx->h_resident_error + 1;
         a.best_variant = ctx->d_sym_best; a.bmu_out = dev_bmu; a.slots = ctx->d_slots; a.error = ctx->d_resident_error;
-        a.launch = ++ctx->sym_launch;
+        a.launch = ++ctx->sym_trial.launch;
         a.N = ctx->N; a.S = ctx->S; a.E = ctx->E; a.cells = ctx->sym_cells; a.KS = ctx->sym_KS; a.RT = ctx->sym_RT; a.nrr = ctx->nrr_eff;
         a.num_rot = ctx->cfg.num_rot; a.use_flip = ctx->cfg.use_flip; a.images = images; a.tag0 = ctx->sym_tag0; a.spin_limit = ctx->spin_limit;
         a.row = ctx->sym_row; a.sum_waves = ctx->sym_sum_waves;
@@ -3273,7 +3279,7 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         a.som = ctx->d_som; a.som_next = ctx->d_som_alt; a.opnd = ctx->d_sym_op; a.xrows = ctx->d_sym_x; a.norm = ctx->d_sym_norm;
         a.factors_t = ctx->d_factors_t; a.cell_elem = ctx->d_sym_elem; a.cell_at = ctx->d_sym_at; a.best_variant = ctx->d_sym_best;
         a.bmu_out = dev_bmu; a.slots = ctx->d_slots; a.error = ctx->d_resident_error;
-        a.launch = ++ctx->sym_launch;
+        a.launch = ++ctx->sym_trial.launch;
         a.N = ctx->N; a.S = ctx->S; a.cells = ctx->sym_cells; a.KS = ctx->sym_KS; a.RT = ctx->sym_RT; a.nrr = ctx->nrr_eff;
         a.num_rot = ctx->cfg.num_rot; a.use_flip = ctx->cfg.use_flip; a.images = images; a.tag0 = ctx->sym_tag0; a.spin_limit = ctx->spin_limit;
         ctx->sym_tag0 = sym_tag(ctx->sym_tag0, images);
@@ -3317,28 +3323,44 @@ int finish_resident(pink_hip_ctx *ctx)
     return PINK_HIP_OK;
 }
 
-// Float32: whether the form suits the data its launches tell behind themselves, and groups queued by then go through it all the same, at
-// a third of the other form's rate where they give up.  So until kF32Probe images have gone through well no more than that
-// many are queued unseen; then three groups, or a quarter of the images that went through well: what groups queued too
-// many can cost (53 us an image) stays about what the others gained (4 to 14).  *count: the images to queue now.
-int await_resident(pink_hip_ctx *ctx, uint32_t *count)
+// The launch that the form is to be left for, if there is one.  The host's words know of it some time after.
+uint32_t trial_failed(const FormTrial &t)
 {
-    const volatile uint32_t *const word = ctx->h_resident_error;
+    const volatile uint32_t *const word = t.word;
+    for (int k = 0; k < 2; ++k)
+        if (const uint32_t launch = word[k]; launch && (int32_t)(launch - t.seen) > 0) return launch;
+    return 0;
+}
+void leave_form(FormTrial &t)
+{
+    t.seen = t.launch;
+    t.counted = t.sent;
+    t.good = 0;
+    t.pause = t.pause_next;
+    t.pause_next = std::min<uint64_t>(4 * t.pause_next, 1u << 20);
+}
+
+// Whether a form suits the data its launches tell behind themselves, and groups queued by then go through it all the same.  So until `probe`
+// images have gone through well no more than that many are queued unseen; then so many groups, or a quarter of the images that went
+// through well: what groups queued too many can cost (resident float32 trainers that give up: 53 us an image) stays about what the
+// others gained (4 to 14).  *count: the images to queue now.
+int await_trial(pink_hip_ctx *ctx, FormTrial &t, uint32_t probe, uint32_t groups, uint32_t group, uint32_t *count)
+{
+    constexpr uint32_t kForget = 1024;
     for (;;) {
-        const uint32_t through = word[2];
+        const uint32_t through = *(const volatile uint32_t *)&t.word[2];
         std::atomic_thread_fence(std::memory_order_acquire);
-        for (const uint32_t launch : {(uint32_t)word[0], (uint32_t)word[1]})
-            if (launch && (int32_t)(launch - ctx->sym_seen) > 0) return PINK_HIP_OK;       // (choose_sym_form's)
-        if ((int32_t)(through - ctx->sym_counted) > 0) {
+        if (trial_failed(t)) return PINK_HIP_OK;
+        if ((int32_t)(through - t.counted) > 0) {
             // (a launch is slow by its images: a thousand that were not, and what came before counts a quarter)
-            const uint64_t before = ctx->sym_good / kF32Forget;
-            ctx->sym_good += through - ctx->sym_counted;
-            ctx->sym_counted = through;
-            for (uint64_t k = before; k < ctx->sym_good / kF32Forget && ctx->sym_pause_next > kSymPause; ++k) ctx->sym_pause_next /= 4;
+            const uint64_t before = t.good / kForget;
+            t.good += through - t.counted;
+            t.counted = through;
+            for (uint64_t k = before; k < t.good / kForget && t.pause_next > kSymPause; ++k) t.pause_next /= 4;
         }
-        const bool proven = ctx->sym_good >= kF32Probe;
-        const uint32_t unseen = ctx->sym_sent - through, next = std::min({*count, ctx->sym_B, proven ? ctx->sym_B : kF32Probe});
-        const uint64_t ahead = proven ? std::max<uint64_t>(3 * (uint64_t)ctx->sym_B, ctx->sym_good / 4) : kF32Probe;
+        const bool proven = t.good >= probe;
+        const uint32_t unseen = t.sent - through, next = std::min({*count, group, proven ? group : probe});
+        const uint64_t ahead = proven ? std::max<uint64_t>((uint64_t)groups * group, t.good / 4) : probe;
         if (unseen == 0 || unseen + next <= ahead) { *count = next; return PINK_HIP_OK; }
         const hipError_t e = hipStreamQuery(ctx->stream);
         (void)hipGetLastError();                          // (a stream that still runs is no error)
@@ -3348,33 +3370,57 @@ int await_resident(pink_hip_ctx *ctx, uint32_t *count)
 }
 
 // Whether a trainer that can be resident is: after a launch gave up (k_sym_rescue or k_f32_rescue has done its group and those
-// queued behind it), or a float32 one went through slowly, the next images go through the other form, then it is tried again.  The
-// host's words say so some time after; a launch that failed before the slots were cleared is not counted twice.  *count: images to
-// train in the form chosen, then to be asked again.
+// queued behind it), or a float32 one went through slowly, the next images go through the other form, then it is tried again.
+// *count: images to train in the form chosen, then to be asked again.
 int choose_sym_form(pink_hip_ctx *ctx, uint32_t *count)
 {
-    if (!ctx->sym_form) return PINK_HIP_OK;
-    const volatile uint32_t *const word = ctx->h_resident_error;
-    if (!ctx->sym_train && ctx->sym_pause == 0) ctx->sym_train = true;
-    if (ctx->sym_train && ctx->sym_f32) TRY(await_resident(ctx, count));
-    uint32_t failed = word[0];
-    if (word[1] && (int32_t)(word[1] - ctx->sym_seen) > 0) failed = word[1];       // (float32: by its data, or gone through but slowly)
-    if (ctx->sym_train && failed && (int32_t)(failed - ctx->sym_seen) > 0) {
-        ctx->sym_seen = ctx->sym_launch;
-        ctx->sym_counted = ctx->sym_sent;
-        ctx->sym_good = 0;
+    FormTrial &t = ctx->sym_trial;
+    if (!ctx->sym_train && t.pause == 0) ctx->sym_train = true;
+    if (ctx->sym_train && ctx->sym_f32) TRY(await_trial(ctx, t, kF32Probe, 3, ctx->sym_B, count));
+    if (ctx->sym_train && trial_failed(t)) {
+        leave_form(t);
         const size_t slots = (size_t)ctx->N * kSymStride;              // (16-byte words of both sets)
         hipLaunchKernelGGL(k_fill_zero, dim3((uint32_t)((slots + 255) / 256)), dim3(256), 0, ctx->stream, (v4i *)ctx->d_slots, slots);
         hipLaunchKernelGGL(k_fill_zero, dim3(1), dim3(256), 0, ctx->stream, (v4i *)ctx->d_resident_error, (size_t)1);
         TRY(launch_check(ctx, "k_fill_zero"));
         ctx->sym_train = false;
-        ctx->sym_pause = ctx->sym_pause_next;
-        ctx->sym_pause_next = std::min<uint64_t>(4 * ctx->sym_pause_next, 1u << 20);
     }
     if (!ctx->sym_train) {
-        if (ctx->sym_f32) *count = (uint32_t)std::min<uint64_t>(*count, ctx->sym_pause);
-        ctx->sym_pause -= std::min<uint64_t>(ctx->sym_pause, *count);
+        if (ctx->sym_f32) *count = (uint32_t)std::min<uint64_t>(*count, t.pause);
+        t.pause -= std::min<uint64_t>(t.pause, *count);
     }
+    return PINK_HIP_OK;
+}
+
+// Whether a float32 trainer that screens its distances does: images that keep every variant of most neurons, one after the other
+// (flat ones), are summed faster by the kernels that sum every variant of all.  48 flat images, 720 variants, us, summed | through
+// the screening's lists: 9 neurons of 8100 elements 3990 | 6150, 256 of 4096 3350 | 7740, 484 of 4096 5210 | 5950.  (Calls go
+// eight groups ahead unseen: the loss is smaller than a resident launch's that gives up.)
+int choose_screened(pink_hip_ctx *ctx, uint32_t *count, bool *screened)
+{
+    FormTrial &t = ctx->screen_trial;
+    if (t.pause == 0) TRY(await_trial(ctx, t, t.seen ? kF32Probe : 0, 8, ctx->Bcap, count));
+    if (t.pause == 0 && trial_failed(t)) leave_form(t);
+    *screened = t.pause == 0;
+    if (*screened) return PINK_HIP_OK;
+    *count = (uint32_t)std::min<uint64_t>(*count, t.pause);
+    t.pause -= *count;
+    return PINK_HIP_OK;
+}
+
+enum class Form { resident, screened, in_turn };
+int choose_form(pink_hip_ctx *ctx, uint32_t call, uint32_t *count, Form *form)
+{
+    *form = Form::in_turn;
+    if (call <= ctx->few_resident) return PINK_HIP_OK;
+    if (ctx->sym_form) {
+        TRY(choose_sym_form(ctx, count));
+        if (ctx->sym_train) { *form = Form::resident; return PINK_HIP_OK; }
+    }
+    if (!ctx->screen_train || call <= ctx->few_screened) return PINK_HIP_OK;
+    bool screened = false;
+    TRY(choose_screened(ctx, count, &screened));
+    if (screened) *form = Form::screened;
     return PINK_HIP_OK;
 }
 
@@ -3407,6 +3453,7 @@ int free_all(pink_hip_ctx *ctx)
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu}) if (p) (void)hipFree(p);
     if (ctx->st_pin) (void)hipHostFree(ctx->st_pin);
     if (ctx->h_resident_error) (void)hipHostFree(ctx->h_resident_error);
+    if (ctx->screen_trial.word) (void)hipHostFree(ctx->screen_trial.word);
     for (int i = 0; i < 2; ++i) {
         if (ctx->pend_pin[i]) (void)hipHostFree(ctx->pend_pin[i]);
         if (ctx->pend_ev[i]) (void)hipEventDestroy(ctx->pend_ev[i]);
@@ -3476,6 +3523,7 @@ int init_exchange(pink_hip_ctx *ctx, size_t slot_words, const void *kernel, uint
         return fail(ctx, PINK_HIP_ENOMEM, "pinned host allocation failed");
     }
     std::fill_n(ctx->h_resident_error, 3, 0u);
+    ctx->sym_trial.word = ctx->h_resident_error;
     return PINK_HIP_OK;
 }
 
@@ -3991,9 +4039,10 @@ int run_orbit_som(pink_hip_ctx *ctx)
 }
 
 // (float32 trainers) what is known of the weights, from all of them.
-int run_screen_range(pink_hip_ctx *ctx)
+int run_screen_range(pink_hip_ctx *ctx, bool afresh)
 {
-    hipLaunchKernelGGL(k_screen_range, dim3(ctx->N), dim3(256), 0, ctx->stream, ctx->d_som, (WeightRange *)ctx->d_screen_range, ctx->S);
+    hipLaunchKernelGGL(k_screen_range, dim3(ctx->N), dim3(256), 0, ctx->stream, ctx->d_som, (WeightRange *)ctx->d_screen_range, ctx->S,
+                       ctx->screen_trial.word, ctx->screen_trial.sent, afresh ? ctx->d_screen_counts + 2 * kCounts : nullptr);
     return launch_check(ctx, "k_screen_range");
 }
 
@@ -4003,7 +4052,7 @@ int run_screen_pack(pink_hip_ctx *ctx)
     Timed t(ctx, kClsPack);
     ctx->screen_packed = true;
     TRY(run_orbit_som(ctx));
-    return run_screen_range(ctx);
+    return run_screen_range(ctx, true);
 }
 
 template <int MODE, int WM, int WN, int KC, int PD, int MINB>
@@ -4222,7 +4271,7 @@ int run_screen_update(pink_hip_ctx *ctx, uint32_t slot, uint32_t *dev_bmu_out)
     u.element = ctx->d_orb_element; u.weight = ctx->d_coef_weight; u.listed = ctx->d_screen_counts + kCounts * ctx->screen_set; u.skip = ctx->d_screen_counts + 2 * kCounts;
     u.opnd = ctx->d_orb_som; u.neuron = (CoefNeuron *)ctx->d_coef_neuron; u.key = ctx->d_key + (size_t)slot * ctx->N;
     u.bound = ctx->d_screen_bound; u.moves = ctx->d_screen_moves + (size_t)slot * ctx->N; u.choice = ctx->d_screen_choice;
-    u.range = (WeightRange *)ctx->d_screen_range; u.image = (const CoefImage *)ctx->d_coef_image + slot;
+    u.slow = ctx->screen_trial.word + 1; u.launch = ctx->screen_trial.launch; u.range = (WeightRange *)ctx->d_screen_range; u.image = (const CoefImage *)ctx->d_coef_image + slot;
     u.bmu_out = dev_bmu_out; u.counts = ctx->d_counts; u.N = ctx->N; u.Op = ctx->orb_KS * 4; u.Epad = ctx->Epad;
     const size_t row = (size_t)ctx->Epad * sizeof(float), both = row + (size_t)u.Op * 16;
     if (both + 1024 <= ctx->lds_max) hipLaunchKernelGGL(k_screen_update<true>, dim3(ctx->N), dim3(512), both, ctx->stream, u);
@@ -4809,7 +4858,12 @@ int init_ctx(pink_hip_ctx *ctx)
             TRY(dev_alloc(ctx, &ctx->d_screen_moves, B * ctx->N));
             TRY(dev_alloc(ctx, &ctx->d_screen_range, ctx->N));
             TRY(dev_alloc(ctx, &ctx->d_screen_choice, 2));
-            TRY(upload(ctx, &ctx->d_screen_counts, std::vector<uint32_t>(2 * kCounts + 1, 0u)));       // (two sets, images to skip)
+            TRY(upload(ctx, &ctx->d_screen_counts, std::vector<uint32_t>(2 * kCounts + 2, 0u)));       // (two sets, images to skip, looks in vain)
+            if (hipHostMalloc((void **)&ctx->screen_trial.word, 3 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+                ctx->screen_trial.word = nullptr;
+                return fail(ctx, PINK_HIP_ENOMEM, "pinned host allocation failed");
+            }
+            std::fill_n(ctx->screen_trial.word, 3, 0u);
             ctx->orb_part_bytes = std::max((size_t)24 << 20, (size_t)ctx->nrr_eff * ctx->N * 32);
             TRY(dev_alloc(ctx, (char **)&ctx->d_orb_part, ctx->orb_part_bytes));
             HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_screen_update<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 1024));
@@ -4938,7 +4992,11 @@ int train_in_turn(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images,
             continue;
         }
         if (ctx->rows_f32_train) {
-            if (screened) TRY(run_orbit_rows(ctx, dev_images + (size_t)done * ctx->isz, B));
+            if (screened) {
+                TRY(run_orbit_rows(ctx, dev_images + (size_t)done * ctx->isz, B));
+                ++ctx->screen_trial.launch;
+                ctx->screen_trial.sent += B;
+            }
             uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : ctx->d_bmu_group;
             for (uint32_t b = 0; b < B; ++b) {
                 if (screened) {
@@ -4950,7 +5008,7 @@ int train_in_turn(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images,
                 TRY(run_update_rows(ctx, b, bmu + b));
             }
             TRY(run_update_replay(ctx, B, bmu, screened));
-            if (screened) TRY(run_screen_range(ctx));
+            if (screened) TRY(run_screen_range(ctx, false));
             continue;
         }
         if (ctx->resident_train) {
@@ -4977,11 +5035,11 @@ int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, 
     if (ctx->orbit_train) return run_orbit_train(ctx, dev_images, n_images, dev_bmu_out);
     for (uint32_t done = 0, count; done < n_images; done += count) {
         count = n_images - done;
-        const bool few = n_images <= ctx->few_resident;
-        if (!few) TRY(choose_sym_form(ctx, &count));
+        Form form;
+        TRY(choose_form(ctx, n_images, &count, &form));
         const float *images = dev_images + (size_t)done * ctx->isz;
         uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : nullptr;
-        if (few || !ctx->sym_train) TRY(train_in_turn(ctx, images, count, bmu, ctx->screen_train && !few && n_images > ctx->few_screened));
+        if (form != Form::resident) TRY(train_in_turn(ctx, images, count, bmu, form == Form::screened));
         else
             for (uint32_t b = 0; b < count; b += ctx->sym_B)
                 TRY(run_sym_train(ctx, images + (size_t)b * ctx->isz, std::min(ctx->sym_B, count - b), bmu ? bmu + b : ctx->d_bmu_group));

@@ -749,10 +749,10 @@ class FloatTrainer:
             imgs[flat] = 0.25                                          # (all variants alike)
         return imgs
 
-    def groups(self, imgs):
-        before = self.ctx.kernel_times()["rotate"][0]
+    def groups(self, imgs, kernels="rotate"):
+        before = self.ctx.kernel_times()[kernels][0]
         assert np.array_equal(self.ctx.train(imgs), self.plain.train(imgs))
-        return self.ctx.kernel_times()["rotate"][0] - before
+        return self.ctx.kernel_times()[kernels][0] - before
 
     def check(self):
         assert np.array_equal(bits(self.ctx.get_som()), bits(self.plain.get_som()))
@@ -817,6 +817,21 @@ def test_resident_float_trainer_forgets_slow_launches():
     say("groups", still_away)
     t.check()
     assert still_away > 2
+
+
+@pytest.mark.parametrize("N,I,D,nrot,ed", [(9, 136, 96, 360, 91), (100, 80, 56, 360, 51)])
+def test_screened_float_trainer_leaves_flat_images_to_the_sums(monkeypatch, N, I, D, nrot, ed):
+    """Images that keep every variant, one after the other, go through the kernel that sums every variant and updates on the way, without
+    an update launch per image; images that do not are screened again after a while."""
+    monkeypatch.setenv("PINK_HIP_RESIDENT_TRAINER", "0")
+    say("screened float trainer, flat images", N, I, D, nrot, ed)
+    t = FloatTrainer(N, I, D, nrot, ed)
+    before = t.groups(t.images(60), "update")
+    flat = [t.groups(t.images(60, slice(None)), "update") for _ in range(4)]
+    away, back = t.groups(t.images(200), "update"), t.groups(t.images(150), "update")
+    say("update launches", before, flat, away, back)
+    t.check()
+    assert before >= 60 and flat[-1] < 30 and away < 150 and back >= 100
 
 
 @pytest.mark.parametrize("N,I,D,nrot,ed", [
