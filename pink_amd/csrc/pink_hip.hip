@@ -4640,7 +4640,9 @@ int init_ctx(pink_hip_ctx *ctx)
         size_t b = c.max_batch ? c.max_batch : ((ctx->mfma || ctx->mfma_sym || ctx->orbit) ? 2048 : 256);
         const size_t budget = (size_t)4 << 30;
         if (ctx->orbit) per_image = orbit_image_bytes(ctx);
-        while (b > 1 && b * per_image > budget) b >>= 1;
+        // (float32: the lists of the variants in question, which are mostly empty and no part of what the cache is to hold)
+        const size_t lists = ctx->orbit && !is_int(ctx) ? (size_t)ctx->N * (kPairKeep * sizeof(uint2) + 2 * sizeof(uint32_t)) : 0;
+        while (b > 1 && b * (per_image + lists) > budget) b >>= 1;
         if (ctx->orbit && !c.max_batch) {
             // the product reads a group's rows soon after they are written: within the last-level cache
             while (b > 16 && b * per_image > ((size_t)240 << 20)) b -= std::max<size_t>(1, b / 16);

@@ -430,6 +430,19 @@ def test_map_with_orbit_rows(N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, da
     assert np.array_equal(one_best, want_best[-1:]) and np.array_equal(bits(one_heat), bits(want_heat[-1:]))
 
 
+def test_memory_of_a_float_mapper_with_many_neurons():
+    """A launch group's buffers stay within some 4 GiB, the lists of variants in question among them."""
+    from test_zz_no_alloc import Hip
+    hip = Hip()
+    N, I, D, nrot, ed = 20000, 16, 12, 64, 6
+    with capi.Context(9, 1, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT):
+        before = hip.free_bytes()
+        with capi.Context(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT, max_batch=2048):
+            taken = before - hip.free_bytes()
+    say("bytes", taken)
+    assert taken < 5 << 30
+
+
 def _nearly_round(rng, n, C_, I, scale, noise=1e-3):
     """Images whose rotated copies differ by a thousandth: every variant's distance is close to every other's."""
     x = np.linspace(-1, 1, I)
