@@ -4171,8 +4171,9 @@ int run_coef_keys(pink_hip_ctx *ctx, uint32_t B)
     CoefPick q{};
     q.words = a.words; q.upper = a.upper; q.key = ctx->d_key; q.list = ctx->d_screen_list; q.list_count = ctx->d_screen_counts;
     q.wide = ctx->d_screen_wide; q.wide_count = ctx->d_screen_counts + 1; q.N = a.N; q.nrr = a.nrr; q.total = B * a.N;
-    if (q.total >= 512 * cu) hipLaunchKernelGGL(k_coef_pick<4>, dim3((q.total + 255) / 256), dim3(1024), 0, ctx->stream, q);
-    else hipLaunchKernelGGL(k_coef_pick<1>, dim3((q.total + 63) / 64), dim3(256), 0, ctx->stream, q);
+    const bool many = q.total >= 512 * cu, few_rows = q.nrr <= 32;
+    hipLaunchKernelGGL((many ? few_rows ? k_coef_pick<4, 8> : k_coef_pick<4, 24> : few_rows ? k_coef_pick<1, 8> : k_coef_pick<1, 24>),
+                       dim3((q.total + (many ? 255 : 63)) / (many ? 256 : 64)), dim3(many ? 1024 : 256), 0, ctx->stream, q);
     TRY(launch_check(ctx, "k_coef_pick"));
     CoefPairs x{};
     x.som_rows = (const float *)ctx->d_somP; x.xrows = ctx->d_orb_x; x.place = ctx->d_orb_place; x.list = q.list; x.list_count = q.list_count; x.key = q.key;
