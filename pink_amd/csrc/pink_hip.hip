@@ -3954,28 +3954,42 @@ size_t orbit_image_bytes(const pink_hip_ctx *ctx)
                            (is_int(ctx) && !ctx->trainer ? (size_t)0 : is_int(ctx) ? (size_t)ctx->orb_KS * 128 : (size_t)ctx->orb_Ox * 32));
 }
 
-// Float32 mappers: whether a full launch group of images is screened (few images are summed all the same,
-// summed_images).  What summing a neuron's every variant takes grows with their
-// number, what is left to sum exactly does not: break-even lies near 100 variants (20 variants of 768 elements 10 % slower
-// with it, 8 of 1369 half as fast, 360 of 121 1.5 times as fast, 720 of 1024 3.8 times).  And what an image leaves in
-// memory has to fit the scratch of pink_hip_map_device_static.
-bool orbit_screens(const pink_hip_ctx *ctx)
+// Float32 mappers: by how much an image of many takes longer where every variant is summed than where they are screened, in us: the sums
+// and the rotated variants in the order of the sums, less what screening takes for every row, neuron and pair that it leaves.  This
+// and what follows are fitted to 9 to 1600 neurons, 128 to 720 variants, 100 to 16384 elements, 1 to 512 images, smooth ones and noise.
+double screening_saves(const pink_hip_ctx *ctx)
 {
-    return ctx->R >= 128 && (size_t)ctx->nrr_eff * ctx->N * 8 * 4 + (size_t)ctx->nrr_eff * ctx->E * 12 <= ((size_t)24 << 20);
+    const double E = ctx->E, R = ctx->R, N = ctx->N;
+    return R * E * (7.6e-7 + 4.9e-8 * N) - N * (2.9e-7 * R + 6.4e-4 + 1e-6 * E) + 3e-4 * R + 1e-4 * E;
+}
+// ... and by how much longer a launch takes that screens, whatever its images: four launches more; the pass over the squares beside a
+// region that is not symmetric; images that do not fit the LDS.
+double screening_costs(const pink_hip_ctx *ctx)
+{
+    return 21.0 + 0.004 * std::max(0.0, ctx->E - 1000.0) + (ctx->orb_all ? 0.0 : 7.5) + (ctx->orb_prep_lds ? 0.0 : 0.009 * ctx->E);
 }
 
-// ... and the images of a launch up to which such a mapper sums every variant after all.  Screening launches three kernels more, and
-// the few sums that it leaves are one chain of E steps after all else: 9 + 0.021 E us.  The sums cost 29 ns per 10^6 neuron x
-// variant x element and the rotated variants 1.7 us per 10^6 variant x element more than screening them does.  Both fitted to
-// 9 to 1600 neurons, 128 to 720 variants, 400 to 4096 elements, 1 to 256 images; (summed / screened us) at 1024 elements, 720
-// variants: 9 neurons 16 images 60 / 66, 64 images 115 / 87; 100 neurons 1 image 35 / 62, 8 images 70 / 74, 16 images 105 / 78;
-// 1600 neurons 1 image 83 / 75.  A GiB at most for their rows.
+// Whether such a mapper screens launches of many images at all.  What summing a neuron's every variant takes grows with their number and length,
+// what screening takes hardly does: 128 variants of 121 elements, 1600 neurons, 512 images 690 us summed, 1000 screened; 720 of them
+// twice as fast screened.  Fewer than 16 base rotations the product's words are not made for.  And what an image leaves in memory has to
+// fit the scratch of pink_hip_map_device_static, in either form.
+bool orbit_screens(const pink_hip_ctx *ctx)
+{
+    const double saves = screening_saves(ctx);
+    const bool short_rows = saves * 512 < 21.0 && (size_t)ctx->R * (ctx->S + ctx->E + 64) * 4 <= ((size_t)16 << 20);
+    return ctx->R >= 128 && !short_rows && (size_t)ctx->nrr_eff * ctx->N * 8 * 4 + (size_t)ctx->nrr_eff * ctx->E * 12 <= ((size_t)24 << 20);
+}
+
+// ... and the images of a launch up to which it sums every variant after all.  (summed / screened us, smooth images, 720 variants: 9 neurons
+// of 225 elements, in a region that is not symmetric, 64 images 52 / 59, 256 images 131 / 75; 9 of 1024 16 images 58 / 66, 64 images 114 / 81; 100
+// of 1024 1 image 34 / 56, 4 images 52 / 59, 16 images 107 / 65; 100 of 4096 1 image 75 / 82, 4 images 128 / 88; 900 of 1024 1 image
+// 64 / 59; 100 of 16384, images beyond the LDS, 2 images 301 / 375, 4 images 483 / 402.)  A GiB at most for their rows.
 uint32_t summed_images(const pink_hip_ctx *ctx)
 {
-    const double variants = (double)ctx->R * ctx->E;
-    const double images = (9.0 + 0.021 * ctx->E) / (variants * (2.9e-8 * ctx->N + 1.7e-6));
+    const double saves = screening_saves(ctx), most = std::min<double>(ctx->Bcap, 4096.0);
+    const double images = saves * most > screening_costs(ctx) ? screening_costs(ctx) / saves + 0.1 : most;
     const size_t row_bytes = (size_t)ctx->Epad * ctx->Rpad * 4 + (ctx->fused_pack ? 0 : (size_t)ctx->R * ctx->S * 4);
-    return (uint32_t)std::min({images, (double)ctx->Bcap, (double)((size_t)1 << 30) / (double)row_bytes});
+    return (uint32_t)std::min(images, (double)((size_t)1 << 30) / (double)row_bytes);
 }
 
 // Trainers that take the orbits' product: integers where the resident form (init_sym_train) does not fit, which keep their
