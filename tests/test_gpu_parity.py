@@ -430,6 +430,59 @@ def test_map_with_orbit_rows(N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, da
     assert np.array_equal(one_best, want_best[-1:]) and np.array_equal(bits(one_heat), bits(want_heat[-1:]))
 
 
+@pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,n", [
+    (9, 1, 24, 18, 128, True, 13, 400),                                # regions that are not symmetric, shorter than a step of the product
+    (6, 3, 20, 15, 360, False, 9, 300),
+    (9, 1, 40, 30, 64, True, 16, 300),                                 # 16 base rotations, the fewest that are screened
+    (600, 1, 16, 12, 64, True, 10, 120),                               # summed however many images come
+    (520, 1, 30, 24, 360, True, 20, 270),                              # more pairs than one wave's blocks of the selection take
+])
+def test_map_of_many_images(N, C_, I, D, nrot, flip, ed, n):
+    """Float32 mappers on either side of the line where screening pays, and of the selection's forms."""
+    say("float mapper, many images", N, C_, I, D, nrot, flip, ed, n)
+    rng = np.random.default_rng(N + D)
+    imgs, som = rng.random((n, C_, I, I), dtype=np.float32), rng.random((N, C_ * D * D), dtype=np.float32)
+    few = min(n, 40)
+    want_heat, want_best = O.map_images(O.shape(N, C_, I, D, nrot, flip, ed, capi.QUADRATIC, capi.FLOAT), som, imgs[:few])
+    with capi.Context(N, C_, I, D, nrot, flip, ed, capi.QUADRATIC, capi.FLOAT) as ctx:
+        ctx.set_som(som)
+        heat, best = ctx.map(imgs)
+        parts = [ctx.map(imgs[i:i + 2]) for i in range(0, n, 2)]
+    assert np.array_equal(best[:few], want_best) and np.array_equal(bits(heat[:few]), bits(want_heat))
+    assert np.array_equal(best, np.concatenate([p[1] for p in parts])) and np.array_equal(bits(heat), bits(np.concatenate([p[0] for p in parts])))
+
+
+@pytest.mark.parametrize("N,I,D,nrot,ed,train", [
+    (40, 20, 14, 360, 10, False),
+    (40, 20, 14, 360, 9, False),                                       # not symmetric
+    (9, 100, 96, 360, 91, True),
+    (900, 40, 34, 360, 32, True),
+])
+def test_screening_with_infinities(monkeypatch, N, I, D, nrot, ed, train):
+    """Infinite pixels and weights bound nothing; against the kernel that sums every variant."""
+    monkeypatch.setenv("PINK_HIP_RESIDENT_TRAINER", "0")
+    say("screening with infinities", N, I, D, nrot, ed, train)
+    n = 12 if train else 150
+    rng = np.random.default_rng(N + ed)
+    som, imgs = rng.random((N, D, D), dtype=np.float32), rng.random((n, 1, I, I), dtype=np.float32)
+    imgs[3, 0, I // 2, I // 2], imgs[n // 2, 0, I // 2, I // 2 - 2] = np.inf, -np.inf
+    som[::5, D // 2, D // 2], som[3::5, D // 2, D // 2 + 1] = np.inf, -np.inf
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 1.0, 0.5) if train else None
+    got = []
+    for choice in (capi.KERNEL_VALU, capi.KERNEL_AUTO):
+        with capi.Context(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT, F, kernel_choice=choice) as ctx:
+            ctx.set_som(som.reshape(N, -1))
+            got.append(ctx.train(imgs) if train else ctx.map(imgs))
+            if train:
+                got[-1] = (ctx.get_som(), got[-1])
+    (want, want_which), (out, which) = got
+    lost = np.isnan(want)
+    assert lost.any() or not train
+    assert np.array_equal(np.isnan(out), lost) and np.array_equal(bits(out)[~lost], bits(want)[~lost])
+    known = np.ones(want_which.shape, bool) if train else ~lost
+    assert np.array_equal(which[known], want_which[known])
+
+
 def test_memory_of_a_float_mapper_with_many_neurons():
     """A launch group's buffers stay within some 4 GiB, the lists of variants in question among them."""
     from test_zz_no_alloc import Hip
@@ -743,6 +796,48 @@ def test_resident_float_trainer_on_awkward_data(kind):
     assert np.array_equal(bmu, want_bmu) and np.array_equal(np.isnan(som), lost) and np.array_equal(bits(som)[~lost], bits(want)[~lost])
 
 
+@pytest.mark.parametrize("kind", ["flat", "alike", "infinite image", "infinite weights", "nan", "grown"])
+@pytest.mark.parametrize("N,I,D,nrot,ed,shape_", [
+    (12, 40, 32, 180, 25, capi.QUADRATIC),
+    (12, 60, 50, 100, 44, capi.CIRCULAR),                              # rows of more than 1024 places
+    (150, 30, 25, 100, 22, capi.QUADRATIC),                            # more neurons than a request brings words of; not symmetric
+    (300, 30, 26, 60, 21, capi.QUADRATIC),                             # two neurons to a block
+    (520, 30, 26, 60, 25, capi.CIRCULAR),                              # four
+])
+def test_resident_float_trainer_on_awkward_data_over_shapes(N, I, D, nrot, ed, shape_, kind):
+    """... in every form of the exchange: lists past their length, neurons of several blocks that tie, what is no number; against the
+    kernel that sums every variant."""
+    say("resident float trainer", kind, N, I, D, nrot, ed, shape_)
+    n = 24
+    rng = np.random.default_rng(N + D)
+    som0, imgs = rng.random((N, D, D), dtype=np.float32), rng.random((n, 1, I, I), dtype=np.float32)
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.MEXICAN_HAT if kind == "grown" else capi.GAUSSIAN, 1.0, 0.5)
+    if kind == "flat":
+        imgs[1::3] = 0.25
+    elif kind == "alike":
+        som0[N // 4:N - 2] = som0[3]
+        F[F < 0.01] = 0.0                                              # (most of them stay alike)
+    elif kind == "infinite image":
+        imgs[3, 0, I // 2, I // 2], imgs[9, 0, I // 2 - 3, I // 2] = np.inf, -np.inf
+    elif kind == "infinite weights":
+        som0[::5, D // 2, D // 2], som0[3::5, D // 2, D // 2 + 1] = np.inf, -np.inf
+    elif kind == "nan":
+        imgs[5, 0, I // 2, I // 2 + 2] = np.nan
+    elif kind == "grown":
+        som0[::5] *= 3000.0
+    got = []
+    for choice in (capi.KERNEL_VALU, capi.KERNEL_AUTO):
+        with capi.Context(N, 1, I, D, nrot, True, ed, shape_, capi.FLOAT, F, kernel_choice=choice) as ctx:
+            ctx.set_som(som0.reshape(N, -1))
+            bmu = np.concatenate([ctx.train(imgs[:9]), ctx.train(imgs[9:])])
+            got.append((bmu, ctx.get_som(), ctx.update_counts()))
+    (want_bmu, want, want_counts), (bmu, som, counts) = got
+    lost = np.isnan(want)
+    assert lost.any() == (kind in ("infinite image", "infinite weights", "nan"))
+    assert np.array_equal(bmu, want_bmu) and np.array_equal(counts, want_counts)
+    assert np.array_equal(np.isnan(som), lost) and np.array_equal(bits(som)[~lost], bits(want)[~lost])
+
+
 class FloatTrainer:
     """A resident float32 trainer beside one that sums every variant; counts the launch groups of a call."""
     def __init__(self, N=12, I=40, D=32, nrot=180, ed=25):
@@ -1017,6 +1112,26 @@ def test_resident_trainers_side_by_side():
         t.join()
     for k, (_, _, want, bmu) in enumerate(work):
         assert np.array_equal(got[k][0], bmu) and np.array_equal(bits(got[k][1]), bits(want)), k
+
+
+def test_resident_float_trainers_side_by_side():
+    """... and float32 ones, each waiting for its own first images."""
+    import threading
+    trainers, done = [FloatTrainer(200, 40, 32, 36, 32) for _ in range(3)], []
+
+    def train(t):
+        for _ in range(3):
+            t.groups(t.images(40))
+        done.append(t)
+
+    threads = [threading.Thread(target=train, args=(t,)) for t in trainers]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert len(done) == len(trainers)
+    for t in trainers:
+        t.check()
 
 
 def test_resident_symmetric_training_is_queued():
