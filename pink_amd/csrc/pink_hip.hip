@@ -3331,13 +3331,16 @@ uint32_t trial_failed(const FormTrial &t)
         if (const uint32_t launch = word[k]; launch && (int32_t)(launch - t.seen) > 0) return launch;
     return 0;
 }
+// A launch that gave up cost its images several times over and is not tried again soon; one that went through slowly cost a part of their
+// time, and the data may have become easier since (images of unit length on random weights do so over some thousand images).
 void leave_form(FormTrial &t)
 {
+    const bool gave_up = *(const volatile uint32_t *)&t.word[0] != 0;
     t.seen = t.launch;
     t.counted = t.sent;
     t.good = 0;
     t.pause = t.pause_next;
-    t.pause_next = std::min<uint64_t>(4 * t.pause_next, 1u << 20);
+    t.pause_next = gave_up ? std::min<uint64_t>(4 * t.pause_next, 1u << 20) : std::max(t.pause_next, std::min<uint64_t>(2 * t.pause_next, 4 * kSymPause));
 }
 
 // Whether a form suits the data its launches tell behind themselves, and groups queued by then go through it all the same.  So until `probe`
@@ -3356,7 +3359,7 @@ int await_trial(pink_hip_ctx *ctx, FormTrial &t, uint32_t probe, uint32_t groups
             const uint64_t before = t.good / kForget;
             t.good += through - t.counted;
             t.counted = through;
-            for (uint64_t k = before; k < t.good / kForget && t.pause_next > kSymPause; ++k) t.pause_next /= 4;
+            for (uint64_t k = before; k < t.good / kForget && t.pause_next > kSymPause; ++k) t.pause_next = std::max(t.pause_next / 4, kSymPause);
         }
         const bool proven = t.good >= probe;
         const uint32_t unseen = t.sent - through, next = std::min({*count, group, proven ? group : probe});
