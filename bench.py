@@ -307,7 +307,8 @@ def run_workload(name, steps, warmup, n_images, kernel, cpu_budget_s, host_inclu
         bound, unit, peak = "mfma", "TOP/s", MFMA_INT8_PEAK_TOPS
         achieved = alg["distance"]["ops"] * per_s / 1e12
         notes = ("the whole step of an image, every pair's operations priced at the int8 peak: a chain of product, bounds, float32 sums "
-                 "beside the word exchange, update; four byte-plane products per pair element, counted once")
+                 "beside the word exchange, update; four byte-plane products per pair element, counted once; bound by that chain, not "
+                 "by the matrix cores: no roofline claimed")
     elif dominant == "distance" and screened(w, times, prof_images):
         bound, unit, peak = "mfma", "TOP/s", MFMA_INT8_PEAK_TOPS
         achieved = alg["distance"]["ops"] * per_s / 1e12

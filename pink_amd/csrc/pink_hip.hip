@@ -3647,7 +3647,9 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     // Float32, us an image (smooth fields; launch per image | resident): the exchange between the blocks, 4 us, is what short regions
     // spend, and a launch per image takes longer with every pair.  N 9: E 256, 720 variants 6.4 | 7.1, 400 7.8 | 7.0, 1936 22 | 13; N 100: 144
     // 7.0 | 6.7, 1936 27 | 13; N 256: 196, 56 variants 5.5 | 6.8, 256, 360 variants 6.9 | 6.3, 400, 8 variants 7.0 | 6.9; N 484:
-    // 256, 56 variants 8.0 | 9.3, 200 variants 9.3 | 8.8; four neurons to a block, N 1024: 144 15 | 14, 576 28 | 21.
+    // 256, 56 variants 8.0 | 9.3, 200 variants 9.3 | 8.8; four neurons to a block, N 1024: 144 15 | 14, 576 28 | 21.  From 400 elements on it
+    // holds with few neurons and variants too: 16 variants, N 4: 400 6.5 | 6.5, 576 7.6 | 6.6, N 36: 400 7.0 | 6.3 (500 images; 32 images
+    // of N 4, 400 elements 7.0 | 7.4; calls of fewer: choose_few).
     if (f32 && ctx->E < 400 && (npb > 2 || (uint64_t)ctx->N * ctx->E * c.num_rot * (c.use_flip ? 2 : 1) < 15000000)) return PINK_HIP_OK;
     if (npb > 4) return PINK_HIP_OK;
     ctx->sym_npb = npb;
