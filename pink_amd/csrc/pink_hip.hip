@@ -3987,14 +3987,18 @@ bool orbit_screens(const pink_hip_ctx *ctx)
 
 // ... and the images of a launch up to which it sums every variant after all.  (summed / screened us, smooth images, 720 variants: 9 neurons
 // of 225 elements, in a region that is not symmetric, 64 images 52 / 59, 256 images 131 / 75; 9 of 1024 16 images 58 / 66, 64 images 114 / 81; 100
-// of 1024 1 image 34 / 56, 4 images 52 / 59, 16 images 107 / 65; 100 of 4096 1 image 75 / 82, 4 images 128 / 88; 900 of 1024 1 image
-// 64 / 59; 100 of 16384, images beyond the LDS, 2 images 301 / 375, 4 images 483 / 402.)  A GiB at most for their rows.
+// of 1024 1 image 34 / 56, 4 images 52 / 59, 16 images 107 / 65; 100 of 16384, images beyond the LDS, 2 images 301 / 375, 4 images
+// 483 / 402.)  Images that keep every variant (flat ones) go through k_screen_wide, which few of them do not fill the chip for: up to so
+// many images (the second line) they would take more than twice what their sums do, up to four times (100 neurons of 3600 elements,
+// flat, 1 image 70 / 218, 4 images 118 / 234, 8 images 158 / 234, 32 images 518 / 544; 400 of 1936 1 image 72 / 164, 4 images 167 / 304).  A GiB at
+// most for their rows.
 uint32_t summed_images(const pink_hip_ctx *ctx)
 {
     const double saves = screening_saves(ctx), most = std::min<double>(ctx->Bcap, 4096.0);
-    const double images = saves * most > screening_costs(ctx) ? screening_costs(ctx) / saves + 0.1 : most;
+    double images = saves * most > screening_costs(ctx) ? screening_costs(ctx) / saves + 0.1 : most;
+    images = std::max(images, (9.0 + 0.021 * ctx->E) / ((double)ctx->R * ctx->E * (2.9e-8 * ctx->N + 1.7e-6)));
     const size_t row_bytes = (size_t)ctx->Epad * ctx->Rpad * 4 + (ctx->fused_pack ? 0 : (size_t)ctx->R * ctx->S * 4);
-    return (uint32_t)std::min(images, (double)((size_t)1 << 30) / (double)row_bytes);
+    return (uint32_t)std::min({images, (double)ctx->Bcap, (double)((size_t)1 << 30) / (double)row_bytes});
 }
 
 // Trainers that take the orbits' product: integers where the resident form (init_sym_train) does not fit, which keep their
