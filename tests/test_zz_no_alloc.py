@@ -153,3 +153,23 @@ def test_static_scratch_refusals():
             mp.map_device_static(imgs, 0, heat)          # no images: nothing to do
     finally:
         hip.release()
+
+
+@pytest.mark.parametrize("N,I,D,nrot,ed,n", [
+    (600, 16, 12, 64, 10, 70),                             # rows so short that screening never pays
+    (300, 210, 260, 64, 8, 5),                             # ... of neurons whose variants beside them do not fit the array
+])
+def test_static_scratch_of_short_rows(N, I, D, nrot, ed, n):
+    hip = Hip()
+    rng = np.random.default_rng(N)
+    try:
+        imgs = hip.upload(rng.random((n, 1, I, I), dtype=np.float32))
+        heat, best = hip.alloc(n * N * 4), hip.alloc(n * N * 4)
+        with capi.Context(N, 1, I, D, nrot, True, ed, capi.QUADRATIC, capi.FLOAT) as ctx:
+            ctx.set_som(rng.random((N, D * D), dtype=np.float32))
+            want = _run(ctx, ctx.map_device, imgs, n, heat, best, hip)
+            for m in (n, 1):
+                got = _run(ctx, ctx.map_device_static, imgs, m, heat, best, hip)
+                assert np.array_equal(got[0], want[0][:m]) and np.array_equal(got[1], want[1][:m])
+    finally:
+        hip.release()
