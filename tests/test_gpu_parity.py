@@ -985,7 +985,7 @@ def test_float_training_of_one_image_takes_no_longer_than_its_kernels(monkeypatc
             taken.append(sorted(times)[30])
     hip.release()
     say("one image", taken)
-    assert taken[1] < 1.15 * taken[0]
+    assert taken[1] < 1.2 * taken[0]
 
 
 def test_resident_float_training_is_queued():
