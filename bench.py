@@ -37,7 +37,7 @@ FP32_PEAK_TFLOPS = 157.3       # MI355X fp32 (vector with packed FMA, and fp32 M
 
 DTYPE_NAME = {0: "f32", 1: "u16", 2: "u8"}
 
-# Peaks measured on an MI355X of this pool with small microbenchmarks (independent MFMA / fma
+# Peaks measured on an MI355X with small microbenchmarks (independent MFMA / fma
 # streams on all CUs): the clock settles near 2.0-2.2 GHz under load.  Reported next to the
 # published figures, never instead of them.
 MEASURED_INT8_MFMA_TOPS = 4130.0
@@ -319,7 +319,7 @@ def run_workload(name, steps, warmup, n_images, kernel, cpu_budget_s, host_inclu
         # direct float32 form on the vector ALU: subtract + fma per pair element, counted as 2 ops
         bound, unit, peak = "valu", "TFLOP/s", FP32_PEAK_TFLOPS
         achieved = alg["distance"]["ops"] * per_s / 1e12
-        second_peak = ("non-packed vector-ALU stream measured on this pool (subtract + fma, eight waves per SIMD)",
+        second_peak = ("non-packed vector-ALU stream measured on an MI355X (subtract + fma, eight waves per SIMD)",
                        MEASURED_VALU_LANE_OPS_T)
         notes = ("compute bound on the vector ALU: bit-faithful sequential fma per (neuron, rotation), one subtract + "
                  "one fma per pair element (counted as 2 operations); non-packed instructions (packed FP32 is disabled in "
@@ -333,8 +333,8 @@ def run_workload(name, steps, warmup, n_images, kernel, cpu_budget_s, host_inclu
     elif dominant == "distance" and path in (capi.KERNEL_MFMA_SYM, capi.KERNEL_MFMA_GEMM, capi.KERNEL_MFMA):
         bound, unit, peak = "mfma", "TOP/s", MFMA_INT8_PEAK_TOPS
         achieved = alg["distance"]["ops"] * per_s / 1e12
-        second_peak = ("int8 MFMA stream measured on this pool (all SIMDs issuing)", MEASURED_INT8_MFMA_TOPS)
-        notes = "int8 MFMA; measured MFMA peak on this pool %.0f TOP/s" % MEASURED_INT8_MFMA_TOPS
+        second_peak = ("int8 MFMA stream measured on an MI355X (all SIMDs issuing)", MEASURED_INT8_MFMA_TOPS)
+        notes = "int8 MFMA; measured MFMA peak %.0f TOP/s" % MEASURED_INT8_MFMA_TOPS
         if w.ed_type == capi.UINT16:
             notes += "; uint16 runs four byte-plane products per pair element, counted once"
     else:
