@@ -2103,15 +2103,17 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
 }
 
 #include "ordered_sum.inc"
+#include "orbit_values.inc"
 #include "sym_train.inc"
 #include "orbit_gemm.inc"
+#include "orbit_train.inc"
 #include "coef_gemm.inc"
 #include "f32_train.inc"
 
 // m_update_info[bmu]++ for the images of a group (Trainer.h:302-303), behind a resident launch: nothing when that launch
 // or one before it gave up and nobody rescued it.  The error word goes to the host with it, which looks when it next comes by, and how many
 // images of the context's resident launches have been through.
-// Behind k_sym_rescue (one block, `rescue` its ticket and counts per image): what it and the next launch need is made ready again,
+// Behind k_orbit_rescue (one block, `rescue` its ticket and counts per image): what it and the next launch need is made ready again,
 // and how many groups are left to it before a resident launch is tried once more: one after a failure, twice as many after
 // each that follows without a success between (error: the launch that failed, groups left, groups next time).
 __global__ __launch_bounds__(256) void k_count_best_matches(const uint32_t *__restrict__ bmu, uint32_t images, uint32_t *__restrict__ counts,
@@ -2442,7 +2444,7 @@ struct pink_hip_ctx {
     hipEvent_t resident_done = nullptr;
     struct ResidentGroup { const float *images; uint32_t count; uint32_t *bmu; };
     std::vector<ResidentGroup> resident_queued;   // groups whose resident launches the host has not checked yet
-    // integer trainers with the symmetries on the SOM side, resident over a launch group (k_train_sym_resident); the GEMM
+    // integer trainers with the symmetries on the SOM side, resident over a launch group (k_train_orbit_resident); the GEMM
     // path's operands are then made when something else wants them
     bool sym_form = false, sym_train = false;              // the context can; it does at present
     FormTrial sym_trial, screen_trial;                     // resident launches; groups of images that are screened (screen_train)
@@ -2458,7 +2460,9 @@ struct pink_hip_ctx {
     float *d_sym_norm_off = nullptr;
     uint32_t *d_sym_rescue = nullptr;
     unsigned long long *d_sym_keys = nullptr;
-    uint32_t sym_npb = 1, sym_nit = 0, sym_B = 0, sym_KS = 0, sym_RT = 0, sym_all = 0, sym_cells = 0, sym_outside = 0, sym_tag0 = 1;
+    OrbitTrainPlan sym_plan;
+    uint32_t *d_sym_element = nullptr, *d_sym_sel = nullptr;
+    uint32_t sym_orbits = 0, sym_npb = 1, sym_nit = 0, sym_B = 0, sym_KS = 0, sym_RT = 0, sym_all = 0, sym_cells = 0, sym_outside = 0, sym_tag0 = 1;
     size_t sym_lds = 0, sym_prep_lds = 0;
     uint32_t *d_sym_upos = nullptr, *d_sym_outside = nullptr, *d_sym_best = nullptr;
     uint4 *d_sym_elem = nullptr, *d_sym_at = nullptr;
@@ -3122,13 +3126,14 @@ void swap_resident(pink_hip_ctx *ctx)
     ctx->na_cur ^= 1;
 }
 
+size_t sym_slot_words(const pink_hip_ctx *ctx);
 int resident_launched(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, uint32_t *dev_bmu)
 {
     const bool rescued = ctx->sym_train;
     ctx->sym_trial.sent += images;
     hipLaunchKernelGGL(k_count_best_matches, dim3((images + 255) / 256), dim3(256), 0, ctx->stream, dev_bmu, images, ctx->d_counts,
                        ctx->d_resident_error, ctx->h_resident_error, ctx->sym_trial.sent, rescued ? ctx->d_sym_rescue : nullptr, ctx->d_slots,
-                       rescued ? 2 * ctx->N * kSymStride : 0u);
+                       rescued ? (uint32_t)sym_slot_words(ctx) : 0u);
     TRY(launch_check(ctx, "k_count_best_matches"));
     if (!rescued) ctx->resident_queued.push_back({dev_images, images, dev_bmu});
     swap_resident(ctx);
@@ -3183,17 +3188,18 @@ int run_train_small_resident(pink_hip_ctx *ctx, const float *dev_images, uint32_
     return resident_launched(ctx, dev_images, images, dev_bmu);
 }
 
-template <bool U16, int NPB>
-const void *sym_kernel_of(uint32_t cells)
+template <bool U16, int NPB, int TPW>
+const void *orbit_train_kernel_of(uint32_t nit)
 {
-    return cells <= 1 ? (const void *)k_train_sym_resident<U16, NPB, 1> : cells <= 2 ? (const void *)k_train_sym_resident<U16, NPB, 2>
-         : (const void *)k_train_sym_resident<U16, NPB, kSymMaxCells>;
+    return nit <= 1 ? (const void *)k_train_orbit_resident<U16, NPB, 1, TPW> : nit <= 2 ? (const void *)k_train_orbit_resident<U16, NPB, 2, TPW>
+         : nit <= 4 ? (const void *)k_train_orbit_resident<U16, NPB, 4, TPW> : (const void *)k_train_orbit_resident<U16, NPB, kOrbTrainMaxNit, TPW>;
 }
 
-template <bool U16>
-const void *sym_kernel_for(uint32_t npb, uint32_t cells)
+const void *orbit_train_kernel(bool u16, const OrbitTrainPlan &p)
 {
-    return npb == 1 ? sym_kernel_of<U16, 1>(cells) : npb == 2 ? sym_kernel_of<U16, 2>(cells) : sym_kernel_of<U16, 4>(cells);
+    if (u16) return p.npb <= 2 ? orbit_train_kernel_of<true, 2, 1>(p.nit) : orbit_train_kernel_of<true, 4, 1>(p.nit);
+    if (p.tpw == 1) return p.npb <= 2 ? orbit_train_kernel_of<false, 2, 1>(p.nit) : orbit_train_kernel_of<false, 4, 1>(p.nit);
+    return p.npb <= 2 ? orbit_train_kernel_of<false, 2, 3>(p.nit) : orbit_train_kernel_of<false, 4, 3>(p.nit);
 }
 
 template <int NPB>
@@ -3206,19 +3212,43 @@ const void *f32_kernel_of(uint32_t cells)
 const void *sym_kernel(const pink_hip_ctx *ctx)
 {
     if (ctx->sym_f32) return ctx->sym_npb == 1 ? f32_kernel_of<1>(ctx->sym_nit) : ctx->sym_npb == 2 ? f32_kernel_of<2>(ctx->sym_nit) : f32_kernel_of<4>(ctx->sym_nit);
-    return ctx->cfg.ed_type == PINK_HIP_UINT16 ? sym_kernel_for<true>(ctx->sym_npb, ctx->sym_nit) : sym_kernel_for<false>(ctx->sym_npb, ctx->sym_nit);
-}
-
-const void *sym_prepare_kernel(const pink_hip_ctx *ctx)
-{
-    if (ctx->sym_f32) return ctx->sym_prep_lds ? (const void *)k_f32_prepare<true> : (const void *)k_f32_prepare<false>;
-    if (ctx->cfg.ed_type == PINK_HIP_UINT16)
-        return ctx->sym_prep_lds ? (const void *)k_sym_prepare<true, true> : (const void *)k_sym_prepare<true, false>;
-    return ctx->sym_prep_lds ? (const void *)k_sym_prepare<false, true> : (const void *)k_sym_prepare<false, false>;
+    return orbit_train_kernel(ctx->cfg.ed_type == PINK_HIP_UINT16, ctx->sym_plan);
 }
 
 // Items of k_f32_rescue per image and neuron: as many as find a compute unit.
 uint32_t f32_rescue_parts(const pink_hip_ctx *ctx) { return std::max(1u, (uint32_t)ctx->num_cu / ctx->N); }
+
+template <int MODE>
+const void *orbit_prepare_for(bool tile, bool x)
+{
+    if (x) return tile ? (const void *)k_orbit_prepare<MODE, true, true> : (const void *)k_orbit_prepare<MODE, false, true>;
+    return tile ? (const void *)k_orbit_prepare<MODE, true, false> : (const void *)k_orbit_prepare<MODE, false, false>;
+}
+const void *orbit_prepare_kernel(const pink_hip_ctx *ctx)
+{
+    const bool tile = ctx->orb_prep_lds != 0;
+    switch (ctx->orb_mode) {
+    case ORB_U8: return orbit_prepare_for<ORB_U8>(tile, ctx->trainer);
+    case ORB_U16: return orbit_prepare_for<ORB_U16>(tile, ctx->trainer);
+    default:
+        if (ctx->trainer) return tile ? (const void *)k_coef_prepare<true, false> : (const void *)k_coef_prepare<false, false>;
+        return tile ? (const void *)k_coef_prepare<true, true> : (const void *)k_coef_prepare<false, true>;
+    }
+}
+
+int launch_orbit_prepare(pink_hip_ctx *ctx, OrbitPrep &p, uint32_t images)
+{
+    const dim3 grid(images, (ctx->nrr_eff + (1u << p.rl) - 1) >> p.rl);
+    const uint32_t threads = ctx->orb_prep_lds > 64 * 1024 || grid.x * grid.y < (uint32_t)ctx->num_cu ? 1024 : ctx->orb_prep_lds > 24 * 1024 ? 512 : 256;
+    void *args[] = {&p};
+    HIP_TRY(ctx, hipLaunchKernel(orbit_prepare_kernel(ctx), grid, dim3(threads), args, ctx->orb_prep_lds, ctx->stream));
+    return PINK_HIP_OK;
+}
+
+// Blocks of a resident launch.
+uint32_t sym_blocks(const pink_hip_ctx *ctx) { return (ctx->N + ctx->sym_npb - 1) / ctx->sym_npb * ctx->sym_plan.splits; }
+// 64-bit words of the slots they exchange words through, the two sets that carry tags.
+size_t sym_slot_words(const pink_hip_ctx *ctx) { return ctx->sym_f32 ? (size_t)2 * ctx->N * kSymStride : orbit_train_slots(sym_blocks(ctx)); }
 
 // A launch group of an integer trainer with the symmetries on the SOM side: base rotations, the resident launch, the
 // elements outside the region.
@@ -3227,19 +3257,24 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
     ctx->packed = ctx->screen_packed = false;
     {
         Timed t(ctx, kClsRotate);
-        SymPrep p{};
-        p.images = dev_images; p.cos_t = ctx->d_cos; p.sin_t = ctx->d_sin; p.upos = ctx->d_sym_upos; p.smask = ctx->d_sym_mask;
-        p.opnd = ctx->d_sym_op; p.xrows = ctx->d_sym_x; p.norm = ctx->d_sym_norm; p.most = ctx->d_most;
-        p.C = ctx->C; p.I = ctx->I; p.D = ctx->D; p.nrr = ctx->nrr_eff; p.RT = ctx->sym_RT; p.KS = ctx->sym_KS;
-        p.all_sym = ctx->sym_all;
-        // (an image in a large part of the LDS leaves room for few blocks on a CU: large ones then)
-        const uint32_t threads = ctx->sym_prep_lds > 40 * 1024 || images * ctx->sym_RT < (uint32_t)ctx->num_cu ? 1024 : 256;
-        F32Prep pf{p.images, p.cos_t, p.sin_t, p.upos, p.smask, p.opnd, p.xrows, ctx->d_sym_err, (double *)ctx->d_sym_norm, ctx->d_sym_norm_off, ctx->d_sym_image, p.most, ctx->d_sym_state,
-                   p.C, p.I, p.D, p.nrr, p.RT, p.KS, p.all_sym};
-        void *args[] = {ctx->sym_f32 ? (void *)&pf : (void *)&p};
-        HIP_TRY(ctx, hipLaunchKernel(sym_prepare_kernel(ctx), dim3(ctx->sym_RT, images), dim3(threads), args, ctx->sym_prep_lds, ctx->stream));
+        if (ctx->sym_f32) {
+            const F32Prep p{dev_images, ctx->d_cos, ctx->d_sin, ctx->d_sym_upos, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_err, (double *)ctx->d_sym_norm,
+                            ctx->d_sym_norm_off, ctx->d_sym_image, ctx->d_most, ctx->d_sym_state, ctx->C, ctx->I, ctx->D, ctx->nrr_eff, ctx->sym_RT, ctx->sym_KS, ctx->sym_all};
+            // (an image in a large part of the LDS leaves room for few blocks on a CU: large ones then)
+            const dim3 grid(ctx->sym_RT, images), threads(ctx->sym_prep_lds > 40 * 1024 || images * ctx->sym_RT < (uint32_t)ctx->num_cu ? 1024 : 256);
+            if (ctx->sym_prep_lds) hipLaunchKernelGGL(k_f32_prepare<true>, grid, threads, ctx->sym_prep_lds, ctx->stream, p);
+            else hipLaunchKernelGGL(k_f32_prepare<false>, grid, threads, 0, ctx->stream, p);
+            TRY(launch_check(ctx, "k_f32_prepare"));
+        } else {
+            OrbitPrep p{};
+            p.images = dev_images; p.index = ctx->d_orb_index; p.frac = ctx->d_orb_frac; p.mask = ctx->d_sym_mask;
+            p.opnd = ctx->d_sym_op; p.norm = ctx->d_sym_norm; p.xrows = ctx->d_sym_x; p.most = ctx->d_most;
+            p.plane = (size_t)images * ctx->sym_RT * ctx->sym_KS * 64; p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.KS = 2 * ctx->sym_KS;
+            p.all_sym = ctx->sym_all; p.rl = ctx->orb_rl; p.pitch = p.norm_pitch = ctx->sym_RT * 16; p.tl = 4;
+            TRY(launch_orbit_prepare(ctx, p, images));
+        }
     }
-    const uint32_t blocks = (ctx->N + ctx->sym_npb - 1) / ctx->sym_npb;
+    const uint32_t blocks = sym_blocks(ctx);
     auto resident = [&](void *arg) {
         return launch_resident(ctx, blocks, [&] {
             void *args[] = {arg};
@@ -3274,21 +3309,22 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         TRY(launch_check(ctx, "k_f32_rescue"));
     } else {
         Timed t(ctx, kClsUpdate);
-        SymRescue rescue{};
-        SymTrain &a = rescue.t;
+        OrbitRescue rescue{};
+        OrbitTrain &a = rescue.t;
         a.som = ctx->d_som; a.som_next = ctx->d_som_alt; a.opnd = ctx->d_sym_op; a.xrows = ctx->d_sym_x; a.norm = ctx->d_sym_norm;
-        a.factors_t = ctx->d_factors_t; a.cell_elem = ctx->d_sym_elem; a.cell_at = ctx->d_sym_at; a.best_variant = ctx->d_sym_best;
+        a.factors_t = ctx->d_factors_t; a.elem = ctx->d_sym_element; a.selectors = ctx->d_sym_sel; a.moves = ctx->d_sym_sel + 16; a.best_variant = ctx->d_sym_best;
         a.bmu_out = dev_bmu; a.slots = ctx->d_slots; a.error = ctx->d_resident_error;
         a.launch = ++ctx->sym_trial.launch;
-        a.N = ctx->N; a.S = ctx->S; a.cells = ctx->sym_cells; a.KS = ctx->sym_KS; a.RT = ctx->sym_RT; a.nrr = ctx->nrr_eff;
+        a.N = ctx->N; a.S = ctx->S; a.orbits = ctx->sym_orbits; a.KS = ctx->sym_KS; a.RT = ctx->sym_RT; a.nrr = ctx->nrr_eff;
         a.num_rot = ctx->cfg.num_rot; a.use_flip = ctx->cfg.use_flip; a.images = images; a.tag0 = ctx->sym_tag0; a.spin_limit = ctx->spin_limit;
+        a.npb = ctx->sym_npb; a.splits = ctx->sym_plan.splits; a.groups = blocks / a.splits; a.abreast = ctx->sym_plan.abreast;
         ctx->sym_tag0 = sym_tag(ctx->sym_tag0, images);
         TRY(resident(&a));
         rescue.keys = ctx->d_sym_keys; rescue.ticket = ctx->d_sym_rescue; rescue.done = ctx->d_sym_rescue + 1;
-        const size_t lds = (size_t)ctx->sym_cells * (sizeof(uint2) + 1);
-        if (ctx->cfg.ed_type == PINK_HIP_UINT16) hipLaunchKernelGGL(k_sym_rescue<true>, rescuers, dim3(kRescueThreads), lds, ctx->stream, rescue);
-        else hipLaunchKernelGGL(k_sym_rescue<false>, rescuers, dim3(kRescueThreads), lds, ctx->stream, rescue);
-        TRY(launch_check(ctx, "k_sym_rescue"));
+        const size_t lds = (size_t)ctx->sym_orbits * (sizeof(uint4) + 1);
+        if (ctx->cfg.ed_type == PINK_HIP_UINT16) hipLaunchKernelGGL(k_orbit_rescue<true>, rescuers, dim3(kRescueThreads), lds, ctx->stream, rescue);
+        else hipLaunchKernelGGL(k_orbit_rescue<false>, rescuers, dim3(kRescueThreads), lds, ctx->stream, rescue);
+        TRY(launch_check(ctx, "k_orbit_rescue"));
     }
     if (ctx->sym_outside) {
         Timed t(ctx, kClsUpdate);
@@ -3372,7 +3408,7 @@ int await_trial(pink_hip_ctx *ctx, FormTrial &t, uint32_t probe, uint32_t groups
     }
 }
 
-// Whether a trainer that can be resident is: after a launch gave up (k_sym_rescue or k_f32_rescue has done its group and those
+// Whether a trainer that can be resident is: after a launch gave up (k_orbit_rescue or k_f32_rescue has done its group and those
 // queued behind it), or a float32 one went through slowly, the next images go through the other form, then it is tried again.
 // *count: images to train in the form chosen, then to be asked again.
 int choose_sym_form(pink_hip_ctx *ctx, uint32_t *count)
@@ -3382,7 +3418,7 @@ int choose_sym_form(pink_hip_ctx *ctx, uint32_t *count)
     if (ctx->sym_train && ctx->sym_f32) TRY(await_trial(ctx, t, kF32Probe, 3, ctx->sym_B, count));
     if (ctx->sym_train && trial_failed(t)) {
         leave_form(t);
-        const size_t slots = (size_t)ctx->N * kSymStride;              // (16-byte words of both sets)
+        const size_t slots = sym_slot_words(ctx) / 2;                  // (16-byte words)
         hipLaunchKernelGGL(k_fill_zero, dim3((uint32_t)((slots + 255) / 256)), dim3(256), 0, ctx->stream, (v4i *)ctx->d_slots, slots);
         hipLaunchKernelGGL(k_fill_zero, dim3(1), dim3(256), 0, ctx->stream, (v4i *)ctx->d_resident_error, (size_t)1);
         TRY(launch_check(ctx, "k_fill_zero"));
@@ -3449,7 +3485,7 @@ int free_all(pink_hip_ctx *ctx)
     void *bufs[] = {ctx->d_som, ctx->d_rot, ctx->d_cos, ctx->d_sin, ctx->d_factors, ctx->d_factors_t, ctx->d_region, ctx->d_key,
                     ctx->d_somP, ctx->d_somP_alt, ctx->d_bmu_group, ctx->d_rotT, ctx->d_bmu_scratch, ctx->d_dist, ctx->d_ssd, ctx->d_best,
                     ctx->d_Pa, ctx->d_Pb, ctx->d_na, ctx->d_nb, ctx->d_poff, ctx->d_need, ctx->d_inv,
-                    ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4,
+                    ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_element, ctx->d_sym_sel, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4,
                     ctx->d_orb_tables, ctx->d_orb_outside, ctx->d_orb_best, ctx->d_most, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
                     ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts, ctx->d_screen_choice, ctx->d_screen_bound, ctx->d_screen_moves, ctx->d_screen_range, ctx->d_coef_neuron, ctx->d_coef_image, ctx->d_coef_row, ctx->d_coef_words, ctx->d_coef_upper, ctx->d_sym_keys, ctx->d_sym_rescue, ctx->d_sym_err, ctx->d_sym_image, ctx->d_sym_run, ctx->d_sym_to, ctx->d_sym_from, ctx->d_sym_turned, ctx->d_sym_state, ctx->d_sym_norm_off};
     for (void *p : bufs) if (p) (void)hipFree(p);
@@ -3588,14 +3624,143 @@ std::vector<uint32_t> outside_elements(const pink_hip_ctx *ctx, const std::vecto
     return outside;
 }
 
-// Integer trainers whose neurons' eight symmetric operand rows fit the LDS of as many blocks as there are compute units:
+// The orbits of a region under the symmetries (see orbit_gemm.inc).  Coordinates run to an even bound, the middle of an odd one twice:
+// place X of pixel x, and back.
+struct OrbitGrid {
+    uint32_t D, Ds;
+    std::vector<uint32_t> orbit_of, reps;                   // per place; an orbit's first place
+    uint32_t place(uint32_t x) const { return x + ((D & 1) && x > D / 2 ? 1u : 0u); }
+    uint32_t pixel(uint32_t X) const { return X - ((D & 1) && X > D / 2 ? 1u : 0u); }
+    uint32_t at(uint32_t off) const { return off / (D * D) * Ds * Ds + place((off % (D * D)) / D) * Ds + place(off % D); }
+    uint32_t moved(uint32_t at, uint32_t sym) const         // place ch * Ds * Ds + X * Ds + Y under a symmetry
+    {
+        int x, y;
+        orbit_apply((int)sym, (int)((at % (Ds * Ds)) / Ds), (int)(at % Ds), (int)Ds - 1, x, y);
+        return at / (Ds * Ds) * (Ds * Ds) + (uint32_t)x * Ds + (uint32_t)y;
+    }
+    // In the order of their first places, 8 x 8 places at a time (neighbouring pieces of a row then read neighbouring pixels).
+    OrbitGrid(uint32_t D_, uint32_t C, const std::vector<uint32_t> &region) : D(D_), Ds(D_ + (D_ & 1)), orbit_of((size_t)C * Ds * Ds, ~0u)
+    {
+        for (uint32_t off : region) {
+            uint32_t first = at(off);
+            for (uint32_t sym = 1; sym < 8; ++sym) first = std::min(first, moved(at(off), sym));
+            if (orbit_of[first] == ~0u) { orbit_of[first] = 0; reps.push_back(first); }
+        }
+        uint32_t corner = Ds;                               // (of the region)
+        for (uint32_t off : region) corner = std::min({corner, place((off % (D * D)) / D), place(off % D)});
+        auto key = [&](uint32_t p) {
+            const uint64_t ch = p / (Ds * Ds), x = (p % (Ds * Ds)) / Ds + 8 - corner % 8, y = p % Ds + 8 - corner % 8;
+            return (ch << 48) | ((x / 8) << 32) | ((y / 8) << 16) | ((x % 8) << 8) | (y % 8);
+        };
+        std::sort(reps.begin(), reps.end(), [&](uint32_t l, uint32_t r) { return key(l) < key(r); });
+        for (uint32_t o = 0; o < reps.size(); ++o)
+            for (uint32_t sym = 0; sym < 8; ++sym) orbit_of[moved(reps[o], sym)] = o;
+    }
+};
+
+// How many neurons a block of a resident integer trainer holds and between how many blocks the rows are shared out: what is expected to
+// take least.  In clocks of an image: a block's rows through its CU's 64 bytes a clock, its waves' instructions or the matrix pipes; a round of
+// tiles, whose shares of k meet in the LDS; an update of 64 orbits a wave; the words of the blocks that hold the same neurons.  Fitted to
+// every plan of 29 shapes (15 to 1024 neurons of 169 to 10000 elements, 4 to 720 variants): off by 3.2 % in the mean, the plan taken 1.4 %
+// slower than the fastest in the mean and 6.6 % at most, where plans are up to four times apart.  npb 0: no way to hold the neurons.
+OrbitTrainPlan plan_orbit_train(uint32_t N, uint32_t E, uint32_t orbits, uint32_t nrr, bool u16, uint32_t units, size_t lds_max)
+{
+    const uint32_t RT = (nrr + 15) / 16, KS = round_up((orbits * 8 + 63) / 64, 2), planes = u16 ? 2 : 1, accs = u16 ? 3 : 1, products = u16 ? 4 : 1;
+    const double most = (double)E * (u16 ? 65535.0 * 65535.0 : 255.0 * 255.0);
+    OrbitTrainPlan best;
+    double best_cost = 0.0;
+    for (uint32_t npb = 1; npb <= 4; ++npb) {
+        const uint32_t groups = (N + npb - 1) / npb, columns = npb > 2 ? 2 : 1, nit = (npb * ((orbits + 63) / 64) + kOrbTrainWorkers - 1) / kOrbTrainWorkers;
+        if (nit > kOrbTrainMaxNit || most >= (double)(1ull << (48 - orbit_train_bits(npb)))) break;
+        uint32_t tiles_before = 0;
+        for (uint32_t splits = 1; splits <= std::min(kOrbTrainSplits, RT) && groups * splits <= units; ++splits) {
+            const uint32_t tiles = (RT + splits - 1) / splits;
+            if (tiles == tiles_before) continue;
+            tiles_before = tiles;
+            for (uint32_t abreast = 1; abreast <= 8; abreast *= 2)
+                for (uint32_t tpw = 1; tpw <= (u16 ? 1u : 3u); tpw += 2) {
+                    const size_t lds = orbit_train_lds(npb, orbits, u16, N, tpw);
+                    if (lds + 2048 > lds_max) continue;
+                    const uint32_t rounds = (tiles + abreast * tpw - 1) / (abreast * tpw), shares = kSymWaves / abreast;
+                    const double stream = rounds * abreast * tpw * 16.0 * KS * planes;
+                    const double issue = rounds * (KS / 2.0 / shares) * (columns * planes * 10.0 + tpw * planes * 4.0 + tpw * columns * products * 2.0 + 10.0) * 8.6;
+                    const double matrix = rounds * abreast * tpw * (double)columns * KS * products * 4.0;
+                    const double cost = 1.155 * std::max({stream, issue, matrix}) + rounds * (2850.0 + 110.0 * tpw * columns * accs + 10.0 * accs * shares * ((abreast * tpw * columns + 7) / 8)) +
+                                        nit * (u16 ? 2070.0 : 1594.0) + (splits > 1 ? 1000.0 : 0.0) + 100.0 * (abreast - 1) + 3.0 * groups * splits;
+                    if (!best.npb || cost < best_cost) {
+                        best.npb = npb; best.splits = splits; best.abreast = abreast; best.tpw = tpw; best.nit = nit; best.lds = lds;
+                        best_cost = cost;
+                    }
+                }
+        }
+    }
+    return best;
+}
+
+int orbit_samples(pink_hip_ctx *ctx, const uint32_t *d_upos, uint32_t Kp);
+int finish_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, const std::vector<uint32_t> &upos, const std::vector<unsigned char> &mask);
+
+// Integer trainers whose neurons fit the blocks of a resident launch: the resident form with the symmetries on the SOM side (orbit_train.inc).
+// (region: distinct elements, in the CPU's order.)
+int init_orbit_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
+{
+    const pink_hip_config &c = ctx->cfg;
+    if (!ctx->gemm || !ctx->fused_som || c.kernel_choice != PINK_HIP_KERNEL_AUTO || ctx->N > kSymMaxNeurons || ctx->D >= 4095 || ctx->C >= 256 || !resident_allowed())
+        return PINK_HIP_OK;
+    const OrbitGrid grid(ctx->D, ctx->C, region);
+    const bool u16 = c.ed_type != PINK_HIP_UINT8;
+    ctx->sym_plan = plan_orbit_train(ctx->N, ctx->E, (uint32_t)grid.reps.size(), ctx->nrr_eff, u16, (uint32_t)ctx->num_cu, ctx->lds_max);
+    if (!ctx->sym_plan.npb) { ctx->sym_plan = {}; return PINK_HIP_OK; }
+    ctx->sym_orbits = (uint32_t)grid.reps.size();
+    ctx->sym_npb = ctx->sym_plan.npb;
+    ctx->sym_lds = ctx->sym_plan.lds;
+    ctx->sym_RT = (ctx->nrr_eff + 15) / 16;
+    ctx->sym_KS = round_up((ctx->sym_orbits * 8 + 63) / 64, 2);
+    const uint32_t Kp = ctx->sym_KS * 64, D = ctx->D, Ds = grid.Ds;
+    std::vector<uint32_t> upos(Kp, ~0u), elem((size_t)ctx->sym_orbits * 8, ~0u), sel(16 + 64);
+    std::vector<unsigned char> mask((size_t)8 * Kp, 0);
+    std::vector<char> inside(ctx->S, 0);
+    for (uint32_t off : region) inside[off] = 1;
+    for (uint32_t o = 0; o < ctx->sym_orbits; ++o)
+        for (uint32_t p = 0; p < 8; ++p) {
+            const uint32_t at = grid.moved(grid.reps[o], p);
+            upos[o * 8 + p] = (at / (Ds * Ds) << 24) | (grid.pixel((at % (Ds * Ds)) / Ds) << 12) | grid.pixel(at % Ds);
+        }
+    auto valid = [&](uint32_t sym) { return (c.num_rot != 1 || (sym & 3) == 0) && (c.use_flip || sym < 4); };
+    ctx->sym_all = 1;                                       // the pixels of P_s are the same for every s, or not
+    for (uint32_t off : region) {
+        const uint32_t at = grid.at(off), o = grid.orbit_of[at];
+        uint32_t p = 0;
+        while (grid.moved(grid.reps[o], p) != at) ++p;
+        elem[o * 8 + p] = off;
+        for (uint32_t sym = 0; sym < 8; ++sym)
+            if (valid(sym)) {
+                const uint32_t k = o * 8 + orbit_moves((int)sym, (int)p), pos = upos[k];
+                mask[(size_t)sym * Kp + k] = 0xff;
+                if (!inside[(pos >> 24) * D * D + ((pos >> 12) & 0xfffu) * D + (pos & 0xfffu)]) ctx->sym_all = 0;
+            }
+    }
+    for (uint32_t s = 0; s < 8; ++s) {
+        sel[2 * s] = orbit_selector((int)s, 0);
+        sel[2 * s + 1] = orbit_selector((int)s, 1);
+        for (uint32_t q = 0; q < 8; ++q) sel[16 + s * 8 + q] = orbit_moves((int)s, (int)q) * (Kp / 8) * (uint32_t)sizeof(float);
+    }
+    TRY(upload(ctx, &ctx->d_sym_element, elem));
+    TRY(upload(ctx, &ctx->d_sym_sel, sel));
+    const void *rescue = u16 ? (const void *)k_orbit_rescue<true> : (const void *)k_orbit_rescue<false>;
+    HIP_TRY(ctx, hipFuncSetAttribute(rescue, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 2048));
+    return finish_sym_train(ctx, region, upos, mask);
+}
+
+// Float32 trainers whose neurons' eight symmetric operand rows fit the LDS of as many blocks as there are compute units:
 // the resident form with the symmetries on the SOM side.  (region: distinct elements, in the CPU's order.)
 int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
 {
     const pink_hip_config &c = ctx->cfg;
     const uint32_t D = ctx->D, DD = D * D;
     const bool f32 = c.ed_type == PINK_HIP_FLOAT;
-    if ((f32 ? !ctx->d_inv : !ctx->gemm || !ctx->fused_som) || c.kernel_choice != PINK_HIP_KERNEL_AUTO || ctx->N > kSymMaxNeurons || D >= 4096 || ctx->C >= 256 ||
+    if (!f32) return init_orbit_train(ctx, region);
+    if (!ctx->d_inv || c.kernel_choice != PINK_HIP_KERNEL_AUTO || ctx->N > kSymMaxNeurons || D >= 4096 || ctx->C >= 256 ||
         !resident_allowed())
         return PINK_HIP_OK;
     // Coordinates run to an even bound, the middle of an odd one twice (see sym_train.inc): place X of pixel x, and back.
@@ -3639,8 +3804,7 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     // every share of k a multiple of four k-steps
     ctx->sym_KS = round_up(((uint32_t)all.size() * 4 + 63) / 64, 4 * sym_shares(ctx->sym_RT));
     const uint32_t Kp = ctx->sym_KS * 64;
-    if (Kp > kSymMaxK || (f32 && ctx->sym_RT > kSymWorkers)) return PINK_HIP_OK;
-    const bool u16 = c.ed_type != PINK_HIP_UINT8;           // (two planes)
+    if (Kp > kSymMaxK || ctx->sym_RT > kSymWorkers) return PINK_HIP_OK;
     // as few neurons per block as leave no more blocks than compute units: a block's part of an image shrinks with them
     uint32_t npb = 1;
     while (npb <= 4 && (ctx->N + npb - 1) / npb > (uint32_t)ctx->num_cu) npb *= 2;
@@ -3650,23 +3814,18 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     // 256, 56 variants 8.0 | 9.3, 200 variants 9.3 | 8.8; four neurons to a block, N 1024: 144 15 | 14, 576 28 | 21.  From 400 elements on it
     // holds with few neurons and variants too: 16 variants, N 4: 400 6.5 | 6.5, 576 7.6 | 6.6, N 36: 400 7.0 | 6.3 (500 images; 32 images
     // of N 4, 400 elements 7.0 | 7.4; calls of fewer: choose_few).
-    if (f32 && ctx->E < 400 && (npb > 2 || (uint64_t)ctx->N * ctx->E * c.num_rot * (c.use_flip ? 2 : 1) < 15000000)) return PINK_HIP_OK;
+    if (ctx->E < 400 && (npb > 2 || (uint64_t)ctx->N * ctx->E * c.num_rot * (c.use_flip ? 2 : 1) < 15000000)) return PINK_HIP_OK;
     if (npb > 4) return PINK_HIP_OK;
     ctx->sym_npb = npb;
     ctx->sym_nit = (npb * ctx->sym_cells + kSymLanes - 1) / kSymLanes;
-    ctx->sym_lds = f32 ? f32_lds_bytes(npb, ctx->sym_KS, ctx->N, ctx->sym_RT, ctx->E) : sym_lds_bytes(npb, ctx->sym_KS, u16, ctx->N, ctx->sym_RT);
-    if (f32) {
-        // the rest of the LDS for the rows of waves that sum, two of them at least
-        ctx->sym_row = f32_row(ctx->E);
-        const size_t row = (size_t)(ctx->sym_row + 4) * sizeof(float);
-        if (ctx->sym_lds + 2 * row + 4096 > ctx->lds_max || ctx->sym_row >= 65536) return PINK_HIP_OK;
-        ctx->sym_sum_waves = (uint32_t)std::min<size_t>(kSymWorkers, (ctx->lds_max - 4096 - ctx->sym_lds) / row);
-        ctx->sym_lds += ctx->sym_sum_waves * row;
-    }
+    ctx->sym_lds = f32_lds_bytes(npb, ctx->sym_KS, ctx->N, ctx->sym_RT, ctx->E);
+    // the rest of the LDS for the rows of waves that sum, two of them at least
+    ctx->sym_row = f32_row(ctx->E);
+    const size_t row = (size_t)(ctx->sym_row + 4) * sizeof(float);
+    if (ctx->sym_lds + 2 * row + 4096 > ctx->lds_max || ctx->sym_row >= 65536) return PINK_HIP_OK;
+    ctx->sym_sum_waves = (uint32_t)std::min<size_t>(kSymWorkers, (ctx->lds_max - 4096 - ctx->sym_lds) / row);
+    ctx->sym_lds += ctx->sym_sum_waves * row;
     if (ctx->sym_nit > kSymMaxCells || ctx->sym_lds + 2048 > ctx->lds_max) return PINK_HIP_OK;
-    const size_t image_lds = (size_t)ctx->C * ctx->I * ctx->I * sizeof(float);
-    ctx->sym_prep_lds = image_lds <= 150 * 1024 ? image_lds : 0;
-
     // position k of a row: element 2 r + c of cell k / 4
     std::vector<uint32_t> rank(cells_all, 0), upos(Kp, ~0u);
     for (uint32_t i = 0; i < all.size(); ++i) rank[all[i]] = i;
@@ -3695,50 +3854,65 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         }
         at[i] = make_uint4(a16[0] | (a16[1] << 16), a16[2] | (a16[3] << 16), a16[4] | (a16[5] << 16), a16[6] | (a16[7] << 16));
     }
-    if (f32) {
-        // where the elements' runs are: of a cell, and of a base rotation's values under a symmetry
-        std::vector<uint32_t> order(ctx->S, ~0u);
-        for (uint32_t e = 0; e < region.size(); ++e) order[region[e]] = e;
-        std::vector<uint2> run(cells.size());
-        std::vector<unsigned short> to((size_t)8 * Kp, (unsigned short)ctx->sym_row);
-        const uint32_t E32 = round_up(ctx->E, kF32Ahead);
-        std::vector<uint32_t> from((size_t)8 * E32, 0);
-        for (uint32_t i = 0; i < cells.size(); ++i) {
-            uint32_t place4[4];
-            for (uint32_t b = 0; b < 4; ++b) {
-                const uint32_t off = (&elem[i].x)[b];
-                place4[b] = off == ~0u ? ctx->sym_row : pair_place(order[off], kF32Run);
-                for (uint32_t sym = 0; sym < 8; ++sym) {
-                    if (off == ~0u || !valid(sym)) continue;
-                    const uint32_t k = rank[moved(cells[i], sym)] * 4 + sym_cell_byte((int)sym, (int)b);
-                    to[(size_t)sym * Kp + k] = (unsigned short)place4[b];
-                    from[(size_t)sym * E32 + order[off]] = k * ctx->sym_RT * 16 * (uint32_t)sizeof(float);
-                }
+    // where the elements' runs are: of a cell, and of a base rotation's values under a symmetry
+    std::vector<uint32_t> order(ctx->S, ~0u);
+    for (uint32_t e = 0; e < region.size(); ++e) order[region[e]] = e;
+    std::vector<uint2> run(cells.size());
+    std::vector<unsigned short> to((size_t)8 * Kp, (unsigned short)ctx->sym_row);
+    const uint32_t E32 = round_up(ctx->E, kF32Ahead);
+    std::vector<uint32_t> from((size_t)8 * E32, 0);
+    for (uint32_t i = 0; i < cells.size(); ++i) {
+        uint32_t place4[4];
+        for (uint32_t b = 0; b < 4; ++b) {
+            const uint32_t off = (&elem[i].x)[b];
+            place4[b] = off == ~0u ? ctx->sym_row : pair_place(order[off], kF32Run);
+            for (uint32_t sym = 0; sym < 8; ++sym) {
+                if (off == ~0u || !valid(sym)) continue;
+                const uint32_t k = rank[moved(cells[i], sym)] * 4 + sym_cell_byte((int)sym, (int)b);
+                to[(size_t)sym * Kp + k] = (unsigned short)place4[b];
+                from[(size_t)sym * E32 + order[off]] = k * ctx->sym_RT * 16 * (uint32_t)sizeof(float);
             }
-            run[i] = make_uint2(place4[0] | (place4[1] << 16), place4[2] | (place4[3] << 16));
         }
-        TRY(upload(ctx, &ctx->d_sym_run, run));
-        TRY(upload(ctx, &ctx->d_sym_to, to));
-        TRY(upload(ctx, &ctx->d_sym_from, from));
+        run[i] = make_uint2(place4[0] | (place4[1] << 16), place4[2] | (place4[3] << 16));
     }
+    TRY(upload(ctx, &ctx->d_sym_run, run));
+    TRY(upload(ctx, &ctx->d_sym_to, to));
+    TRY(upload(ctx, &ctx->d_sym_from, from));
+    TRY(upload(ctx, &ctx->d_sym_elem, elem));
+    TRY(upload(ctx, &ctx->d_sym_at, at));
+    ctx->sym_f32 = true;
+    return finish_sym_train(ctx, region, upos, mask);
+}
+
+// What the resident forms share: the operand's tables, the buffers of a group, the exchange.
+int finish_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, const std::vector<uint32_t> &upos, const std::vector<unsigned char> &mask)
+{
+    const pink_hip_config &c = ctx->cfg;
+    const bool f32 = ctx->sym_f32, u16 = c.ed_type != PINK_HIP_UINT8;       // (two planes)
+    const uint32_t Kp = ctx->sym_KS * 64;
     const std::vector<uint32_t> outside = outside_elements(ctx, region);
     ctx->sym_outside = (uint32_t)outside.size();
     TRY(upload(ctx, &ctx->d_sym_upos, upos));
-    TRY(upload(ctx, &ctx->d_sym_elem, elem));
     TRY(upload(ctx, &ctx->d_sym_outside, outside));
-    TRY(upload(ctx, &ctx->d_sym_at, at));
     TRY(upload(ctx, (unsigned char **)&ctx->d_sym_mask, mask));
+    if (f32) {
+        const size_t image_lds = (size_t)ctx->C * ctx->I * ctx->I * sizeof(float);
+        ctx->sym_prep_lds = image_lds <= 150 * 1024 ? image_lds : 0;
+        HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_f32_prepare<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 2048));
+    } else {
+        ctx->orb_mode = u16 ? ORB_U16 : ORB_U8;
+        TRY(orbit_samples(ctx, ctx->d_sym_upos, Kp));
+    }
     // a group's operand and rows are written by one launch and read by the next: within the last-level cache
     const size_t op_image = (size_t)(u16 ? 2 : 1) * ctx->sym_RT * ctx->sym_KS * 1024, x_image = (size_t)ctx->nrr_eff * Kp * sizeof(float);
     size_t b = c.max_batch ? std::min<size_t>(c.max_batch, kSymGroupMax) : kSymGroupMax;
     while (b > 8 && b * (op_image + x_image) > ((size_t)192 << 20)) --b;
     ctx->sym_B = (uint32_t)b;
     TRY(dev_alloc(ctx, &ctx->d_sym_op, b * op_image / 16));
-    TRY(dev_alloc(ctx, &ctx->d_sym_x, b * ctx->nrr_eff * Kp));
+    TRY(dev_alloc(ctx, &ctx->d_sym_x, b * ctx->nrr_eff * Kp + 64));       // (a chunk of 64 orbits may read past the last)
     TRY(dev_alloc(ctx, &ctx->d_sym_norm, b * ctx->sym_RT * 16 * 8));
     TRY(dev_alloc(ctx, &ctx->d_sym_best, b * ctx->N));
     if (!ctx->d_most) TRY(dev_alloc(ctx, &ctx->d_most, std::max<size_t>(b, kSymGroupMax)));
-    ctx->sym_f32 = f32;
     if (f32) {
         TRY(dev_alloc(ctx, &ctx->d_sym_err, b * ctx->sym_RT * 16));
         TRY(dev_alloc(ctx, &ctx->d_sym_image, b));
@@ -3750,8 +3924,7 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     // (limits are per kernel, not per context)
     const int most = (int)ctx->lds_max - 2048;             // (the kernels' own arrays: up to 1.3 KB more than lds_max leaves them)
     HIP_TRY(ctx, hipFuncSetAttribute(sym_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, most));
-    if (ctx->sym_prep_lds) HIP_TRY(ctx, hipFuncSetAttribute(sym_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, most));
-    TRY(init_exchange(ctx, (size_t)(f32 ? 4 : 2) * ctx->N * kSymStride, sym_kernel(ctx), kSymThreads, ctx->sym_lds));
+    TRY(init_exchange(ctx, sym_slot_words(ctx) * (f32 ? 2 : 1), sym_kernel(ctx), kSymThreads, ctx->sym_lds));
     ctx->sym_tag0 = (ctx->exchange_tag - 1) % 0xfffeu + 1;
     TRY(dev_alloc(ctx, &ctx->d_sym_keys, b * ctx->N * (f32 ? f32_rescue_parts(ctx) : 1)));
     TRY(dev_alloc(ctx, &ctx->d_sym_rescue, b + 1));
@@ -3760,57 +3933,46 @@ int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     return PINK_HIP_OK;
 }
 
-template <int MODE>
-const void *orbit_prepare_for(bool tile, bool x)
+// Where the samples of the base rotations lie, for rows of Kp places (d_upos).
+int orbit_samples(pink_hip_ctx *ctx, const uint32_t *d_upos, uint32_t Kp)
 {
-    if (x) return tile ? (const void *)k_orbit_prepare<MODE, true, true> : (const void *)k_orbit_prepare<MODE, false, true>;
-    return tile ? (const void *)k_orbit_prepare<MODE, true, false> : (const void *)k_orbit_prepare<MODE, false, false>;
-}
-const void *orbit_prepare_kernel(const pink_hip_ctx *ctx)
-{
-    const bool tile = ctx->orb_prep_lds != 0;
-    switch (ctx->orb_mode) {
-    case ORB_U8: return orbit_prepare_for<ORB_U8>(tile, ctx->trainer);
-    case ORB_U16: return orbit_prepare_for<ORB_U16>(tile, ctx->trainer);
-    default:
-        if (ctx->trainer) return tile ? (const void *)k_coef_prepare<true, false> : (const void *)k_coef_prepare<false, false>;
-        return tile ? (const void *)k_coef_prepare<true, true> : (const void *)k_coef_prepare<false, true>;
-    }
+    const bool f32 = ctx->orb_mode == ORB_F32;
+    const size_t image_lds = (size_t)ctx->C * orbit_tile(ctx->I) * sizeof(float);
+    ctx->orb_prep_lds = image_lds <= 120 * 1024 ? image_lds : 0;
+    if (ctx->orb_prep_lds)
+        HIP_TRY(ctx, hipFuncSetAttribute(orbit_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024));
+    // as many base rotations per wave as there are, up to 16; four for a trainer's few
+    // images of long rows, two where the image comes out of memory: a wave's pixels are neighbours then, and a call with one
+    // image has blocks for a part of the chip
+    ctx->orb_rl = 0;
+    while ((1u << ctx->orb_rl) < ctx->nrr_eff && ctx->orb_rl < (!ctx->orb_prep_lds ? 1u : ctx->trainer && Kp >= 4096 ? 2u : 4u)) ++ctx->orb_rl;
+    const uint32_t blocks = (ctx->nrr_eff + (1u << ctx->orb_rl) - 1) >> ctx->orb_rl, groups = orbit_piece_groups(Kp / 16, ctx->orb_rl);
+    const uint32_t tiles = (ctx->nrr_eff + 15) / 16;
+    const size_t entries = f32 ? (size_t)tiles * Kp * 16 : (size_t)blocks * groups * 1024;
+    TRY(dev_alloc(ctx, &ctx->d_orb_index, entries));
+    TRY(dev_alloc(ctx, &ctx->d_orb_frac, entries));
+    OrbitTable t{};
+    t.cos_t = ctx->d_cos; t.sin_t = ctx->d_sin; t.upos = d_upos; t.index = ctx->d_orb_index; t.frac = ctx->d_orb_frac;
+    t.stride = ctx->orb_prep_lds ? orbit_stride(ctx->I) : ctx->I;
+    t.channel = ctx->orb_prep_lds ? orbit_tile(ctx->I) : ctx->I * ctx->I;
+    t.I = ctx->I; t.D = ctx->D; t.nrr = ctx->nrr_eff; t.pieces = Kp / 16; t.rl = ctx->orb_rl;
+    if (f32) hipLaunchKernelGGL(k_coef_table, dim3((uint32_t)(entries / 256)), dim3(256), 0, ctx->stream, t, Kp / 512);
+    else hipLaunchKernelGGL(k_orbit_table, dim3((groups * 1024 + 255) / 256, blocks), dim3(256), 0, ctx->stream, t);
+    return launch_check(ctx, "k_orbit_table");
 }
 
 // The tables of the orbit order (see orbit_gemm.inc) and the SOM's operand.  (region: distinct elements, in the CPU's order.)
 int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
 {
     const pink_hip_config &c = ctx->cfg;
-    const uint32_t D = ctx->D, DD = D * D, odd = D & 1, mid = D / 2, Ds = D + odd;
-    auto place = [&](uint32_t x) { return x + (odd && x > mid ? 1u : 0u); };
-    auto pixel = [&](uint32_t X) { return X - (odd && X > mid ? 1u : 0u); };
-    auto moved = [&](uint32_t at, uint32_t sym) {           // place ch * Ds * Ds + X * Ds + Y under a symmetry
-        int x, y;
-        orbit_apply((int)sym, (int)((at % (Ds * Ds)) / Ds), (int)(at % Ds), (int)Ds - 1, x, y);
-        return at / (Ds * Ds) * (Ds * Ds) + (uint32_t)x * Ds + (uint32_t)y;
-    };
+    const OrbitGrid grid(ctx->D, ctx->C, region);
+    const uint32_t D = ctx->D, DD = D * D, Ds = grid.Ds;
+    const std::vector<uint32_t> &reps = grid.reps, &orbit_of = grid.orbit_of;
+    auto pixel = [&](uint32_t X) { return grid.pixel(X); };
+    auto moved = [&](uint32_t at, uint32_t sym) { return grid.moved(at, sym); };
     ctx->orb_mode = c.ed_type == PINK_HIP_UINT8 ? ORB_U8 : c.ed_type == PINK_HIP_UINT16 ? ORB_U16 : ORB_F32;
     ctx->orb_ns = c.use_flip ? 8 : 4;
     ctx->orb_valid = (c.num_rot == 1 ? 0x11u : 0xffu) & (c.use_flip ? 0xffu : 0x0fu);
-    // the orbits of the region's places, in the order of their first places, 8 x 8 places at a time (neighbouring pieces of a
-    // row then read neighbouring pixels)
-    std::vector<uint32_t> orbit_of((size_t)ctx->C * Ds * Ds, ~0u), reps;
-    for (uint32_t off : region) {
-        const uint32_t at = off / DD * Ds * Ds + place((off % DD) / D) * Ds + place(off % D);
-        uint32_t first = at;
-        for (uint32_t sym = 1; sym < 8; ++sym) first = std::min(first, moved(at, sym));
-        if (orbit_of[first] == ~0u) { orbit_of[first] = 0; reps.push_back(first); }
-    }
-    uint32_t corner = Ds;                                   // (of the region)
-    for (uint32_t off : region) corner = std::min({corner, place((off % DD) / D), place(off % D)});
-    auto key = [&](uint32_t at) {
-        const uint64_t ch = at / (Ds * Ds), x = (at % (Ds * Ds)) / Ds + 8 - corner % 8, y = at % Ds + 8 - corner % 8;
-        return (ch << 48) | ((x / 8) << 32) | ((y / 8) << 16) | ((x % 8) << 8) | (y % 8);
-    };
-    std::sort(reps.begin(), reps.end(), [&](uint32_t l, uint32_t r) { return key(l) < key(r); });
-    for (uint32_t o = 0; o < reps.size(); ++o)
-        for (uint32_t sym = 0; sym < 8; ++sym) orbit_of[moved(reps[o], sym)] = o;
     const bool f32 = ctx->orb_mode == ORB_F32;
     ctx->orb_KS = round_up(((uint32_t)reps.size() * 8 + 31) / 32, f32 ? 16u : ctx->orb_mode == ORB_U8 ? 4u : 2u);       // (k_coef_gemm's steps, k_orbit_gemm's KC)
     const uint32_t Kp = ctx->orb_KS * 32;
@@ -3831,7 +3993,7 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     ctx->orb_all = 1;
     std::vector<unsigned char> mask((size_t)8 * Kp, 0);
     for (uint32_t e = 0; e < region.size(); ++e) {
-        const uint32_t off = region[e], at = off / DD * Ds * Ds + place((off % DD) / D) * Ds + place(off % D), o = orbit_of[at];
+        const uint32_t off = region[e], at = grid.at(off), o = orbit_of[at];
         uint32_t p = 0;
         while (moved(reps[o], p) != at) ++p;
         elem[o * 8 + p] = off;
@@ -3887,15 +4049,6 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     if (f32) TRY(dev_alloc(ctx, (CoefNeuron **)&ctx->d_coef_neuron, ctx->N));
     else TRY(dev_alloc(ctx, &ctx->d_orb_na, 3 * (size_t)ctx->N));        // (a trainer's three sets take turns)
     if (!f32 && ctx->trainer) TRY(dev_alloc(ctx, &ctx->d_orb_values, (size_t)ctx->N * Kp));
-    const size_t image_lds = (size_t)ctx->C * orbit_tile(ctx->I) * sizeof(float);
-    ctx->orb_prep_lds = image_lds <= 120 * 1024 ? image_lds : 0;
-    if (ctx->orb_prep_lds)
-        HIP_TRY(ctx, hipFuncSetAttribute(orbit_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024));
-    // as many base rotations per wave as there are, up to 16; four for a trainer's few
-    // images of long rows, two where the image comes out of memory: a wave's pixels are neighbours then, and a call with one
-    // image has blocks for a part of the chip
-    ctx->orb_rl = 0;
-    while ((1u << ctx->orb_rl) < ctx->nrr_eff && ctx->orb_rl < (!ctx->orb_prep_lds ? 1u : ctx->trainer && Kp >= 4096 ? 2u : 4u)) ++ctx->orb_rl;
     if (f32) {
         tables.add(&ctx->d_coef_weight, weight);
         if (ctx->trainer) {
@@ -3923,21 +4076,7 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         }
     }
     TRY(tables.commit(ctx, &ctx->d_orb_tables));
-    {
-        const uint32_t blocks = (ctx->nrr_eff + (1u << ctx->orb_rl) - 1) >> ctx->orb_rl, groups = orbit_piece_groups(Kp / 16, ctx->orb_rl);
-        const uint32_t tiles = (ctx->nrr_eff + 15) / 16;
-        const size_t entries = f32 ? (size_t)tiles * Kp * 16 : (size_t)blocks * groups * 1024;
-        TRY(dev_alloc(ctx, &ctx->d_orb_index, entries));
-        TRY(dev_alloc(ctx, &ctx->d_orb_frac, entries));
-        OrbitTable t{};
-        t.cos_t = ctx->d_cos; t.sin_t = ctx->d_sin; t.upos = d_upos; t.index = ctx->d_orb_index; t.frac = ctx->d_orb_frac;
-        t.stride = ctx->orb_prep_lds ? orbit_stride(ctx->I) : ctx->I;
-        t.channel = ctx->orb_prep_lds ? orbit_tile(ctx->I) : ctx->I * ctx->I;
-        t.I = ctx->I; t.D = D; t.nrr = ctx->nrr_eff; t.pieces = Kp / 16; t.rl = ctx->orb_rl;
-        if (f32) hipLaunchKernelGGL(k_coef_table, dim3((uint32_t)(entries / 256)), dim3(256), 0, ctx->stream, t, Kp / 512);
-        else hipLaunchKernelGGL(k_orbit_table, dim3((groups * 1024 + 255) / 256, blocks), dim3(256), 0, ctx->stream, t);
-        TRY(launch_check(ctx, "k_orbit_table"));
-    }
+    TRY(orbit_samples(ctx, d_upos, Kp));
     ctx->orb_pitch = ctx->trainer ? round_up(ctx->nrr_eff, f32 ? 16 : 32) : ctx->nrr_eff;
     ctx->screen_train = ctx->trainer && f32;
     ctx->orbit = !ctx->screen_train;
@@ -4009,7 +4148,7 @@ uint32_t summed_images(const pink_hip_ctx *ctx)
 // 25 / 27, 256 720 4096 80 / 41, 484 720 1024 34 / 30, 900 720 576 32 / 30, 1600 720 576 45 / 31, 1600 720 4096 255 / 58, 9 80 8100 72 / 28,
 // 900 80 8100 88 / 39.)  Very long rows leave many variants in question, whose rows come from memory again and again: 100 720 16384
 // 193 / 111, 49 720 29241 315 / 204, but 256 720 16384 297 / 325, 256 720 28900 544 / 719.
-bool orbit_trains(const pink_hip_ctx *ctx)
+bool orbit_trains(const pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
 {
     if (!is_int(ctx)) {
         const double E = ctx->E, NR = (double)ctx->N * ctx->R;
@@ -4018,12 +4157,9 @@ bool orbit_trains(const pink_hip_ctx *ctx)
     }
     // (below a dozen base rotations the product's tiles of 64 rows are mostly empty)
     if (!ctx->gemm || ctx->E < 1024 || ctx->nrr_eff < 12 || !resident_allowed()) return false;
-    uint32_t npb = 1;
-    while (npb <= 4 && (ctx->N + npb - 1) / npb > (uint32_t)ctx->num_cu) npb *= 2;
-    const uint32_t RT = (ctx->nrr_eff + 15) / 16, KS = round_up((ctx->E + 63) / 64, 4 * sym_shares(RT));
-    const bool resident = ctx->N <= kSymMaxNeurons && KS * 64 <= kSymMaxK && npb <= 4 && npb * (ctx->E / 4) <= kSymMaxCells * kSymLanes &&
-                          sym_lds_bytes(npb, KS, ctx->cfg.ed_type == PINK_HIP_UINT16, ctx->N, RT) + 2048 <= ctx->lds_max;
-    return !resident;
+    return ctx->N > kSymMaxNeurons ||
+           !plan_orbit_train(ctx->N, ctx->E, (uint32_t)OrbitGrid(ctx->D, ctx->C, region).reps.size(), ctx->nrr_eff, ctx->cfg.ed_type == PINK_HIP_UINT16,
+                             (uint32_t)ctx->num_cu, ctx->lds_max).npb;
 }
 
 // Float32 trainers: calls of few images.  Beside the resident form a launch per image saves the two launches behind a group, the neurons' way
@@ -4138,12 +4274,8 @@ int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
     p.images = dev_images; p.index = ctx->d_orb_index; p.frac = ctx->d_orb_frac; p.mask = ctx->d_orb_mask;
     p.opnd = ctx->d_orb_rows; p.norm = ctx->d_orb_nb; p.key = ctx->d_key;
     p.xrows = ctx->d_orb_x; p.plane = orbit_rows_plane(ctx, B); p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.KS = ctx->orb_KS;
-    p.all_sym = ctx->orb_all; p.rl = ctx->orb_rl; p.pitch = ctx->orb_pitch; p.most = ctx->d_most;
-    const dim3 grid(B, (ctx->nrr_eff + (1u << p.rl) - 1) >> p.rl);
-    const uint32_t threads = ctx->orb_prep_lds > 64 * 1024 || grid.x * grid.y < (uint32_t)ctx->num_cu ? 1024 : ctx->orb_prep_lds > 24 * 1024 ? 512 : 256;
-    void *args[] = {&p};
-    HIP_TRY(ctx, hipLaunchKernel(orbit_prepare_kernel(ctx), grid, dim3(threads), args, ctx->orb_prep_lds, ctx->stream));
-    return PINK_HIP_OK;
+    p.all_sym = ctx->orb_all; p.rl = ctx->orb_rl; p.pitch = ctx->orb_pitch; p.most = ctx->d_most; p.norm_pitch = ctx->nrr_eff; p.tl = 5;
+    return launch_orbit_prepare(ctx, p, B);
 }
 
 // How a float32 product is cut into splits: as many as fill the chip twice, of at least two steps, as far as the buffer goes.
@@ -4558,7 +4690,7 @@ int init_ctx(pink_hip_ctx *ctx)
         std::vector<char> seen(ctx->S, 0);
         for (uint32_t off : region) { if (seen[off]) distinct = false; seen[off] = 1; }
         const bool fits = distinct && c.kernel_choice == PINK_HIP_KERNEL_AUTO && ctx->D < 4095 && ctx->C < 256;
-        if (fits && (ctx->trainer ? orbit_trains(ctx) : is_int(ctx) ? !ctx->mfma_sym : orbit_screens(ctx))) {
+        if (fits && (ctx->trainer ? orbit_trains(ctx, region) : is_int(ctx) ? !ctx->mfma_sym : orbit_screens(ctx))) {
             TRY(init_orbit(ctx, region));
             if (ctx->orbit) ctx->mfma = false;
             if (ctx->orbit && is_int(ctx)) ctx->gemm = true;               // (the matrix cores, for pink_hip_distance_kernel)

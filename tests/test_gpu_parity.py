@@ -756,6 +756,35 @@ def test_resident_symmetric_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, 
         assert np.array_equal(bits(d1), bits(d2)) and np.array_equal(ssd1, ssd2) and np.array_equal(best1, best2)
 
 
+# (neurons of a block x blocks that share out an image's rows; tiles of a wave; chunks of 64 orbits of a neuron, of a wave)
+RESIDENT_INTEGER_PLANS = [
+    (90, 1, 40, 40, 360, True, 34, capi.QUADRATIC, capi.UINT8, 3),       # 2 x 3, two groups of waves
+    (91, 1, 40, 40, 360, True, 35, capi.QUADRATIC, capi.UINT16, 3),      # the last block holds one neuron; an odd region in an even neuron
+    (130, 1, 30, 30, 360, True, 21, capi.QUADRATIC, capi.UINT8, 3),      # 2 x 1, three tiles to a wave
+    (331, 1, 60, 60, 240, True, 55, capi.CIRCULAR, capi.UINT16, 2),      # 2 x 1, four groups of waves
+    (331, 1, 90, 80, 360, True, 75, capi.CIRCULAR, capi.UINT16, 2),      # 4 x 3: nine chunks of a neuron, up to six of a wave
+    (60, 2, 36, 36, 500, True, 24, capi.QUADRATIC, capi.UINT16, 3),      # 2 x 8, the most
+    (5, 1, 20, 20, 1000, True, 15, capi.QUADRATIC, capi.UINT16, 3),      # 2 x 8, two tiles each; 250 rotations are not whole tiles
+    (255, 1, 30, 30, 720, False, 20, capi.CIRCULAR, capi.UINT8, 3),      # twelve tiles, four groups of waves
+    (10, 1, 100, 100, 200, True, 91, capi.QUADRATIC, capi.UINT8, 2),     # 1 x 4, seventeen chunks
+    (12, 1, 100, 100, 80, False, 98, capi.QUADRATIC, capi.UINT16, 2),
+    (200, 1, 120, 120, 24, True, 98, capi.QUADRATIC, capi.UINT8, 2),     # twenty chunks
+    (6, 1, 150, 150, 40, True, 146, capi.QUADRATIC, capi.UINT8, 2),      # 43 chunks
+    (6, 1, 150, 150, 40, True, 143, capi.QUADRATIC, capi.UINT8, 2),      # 42, six to a wave
+    (513, 1, 60, 60, 24, True, 50, capi.QUADRATIC, capi.UINT8, 2),       # 3 x 1
+    (1023, 1, 20, 18, 12, True, 17, capi.QUADRATIC, capi.UINT16, 3),     # 4 x 1, the last block holds three
+    (40, 1, 23, 22, 36, True, 22, capi.QUADRATIC, capi.UINT16, 3),       # 66 orbits: a chunk and two more
+    (40, 1, 23, 21, 36, True, 21, capi.QUADRATIC, capi.UINT8, 3),        # an odd neuron: the middle twice
+]
+
+
+@pytest.mark.parametrize("form", ["resident", "gives up", "tags wrap"])
+@pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,shape_,ed_type,n", RESIDENT_INTEGER_PLANS)
+def test_resident_integer_trainer_plans(monkeypatch, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, form):
+    """How the neurons and an image's rows are dealt to the blocks, at the edges of chunks, tiles, groups of waves and blocks."""
+    test_resident_symmetric_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, form)
+
+
 @pytest.mark.parametrize("kind", ["blank", "flat", "alike", "zero", "nan", "grown", "faint", "flux"])
 def test_resident_float_trainer_on_awkward_data(kind):
     """Images and weights that leave many variants or several neurons to the float32 sums."""
