@@ -2462,7 +2462,8 @@ struct pink_hip_ctx {
     unsigned long long *d_sym_keys = nullptr;
     OrbitTrainPlan sym_plan;
     uint32_t *d_sym_element = nullptr, *d_sym_sel = nullptr;
-    uint32_t sym_orbits = 0, sym_npb = 1, sym_nit = 0, sym_B = 0, sym_KS = 0, sym_RT = 0, sym_all = 0, sym_cells = 0, sym_outside = 0, sym_tag0 = 1;
+    uint32_t orb_table_groups = 0;                          // of the samples' table, per row block
+    uint32_t sym_orbits = 0, sym_reached = 0, sym_npb = 1, sym_nit = 0, sym_B = 0, sym_KS = 0, sym_RT = 0, sym_all = 0, sym_cells = 0, sym_outside = 0, sym_tag0 = 1;
     size_t sym_lds = 0, sym_prep_lds = 0;
     uint32_t *d_sym_upos = nullptr, *d_sym_outside = nullptr, *d_sym_best = nullptr;
     uint4 *d_sym_elem = nullptr, *d_sym_at = nullptr;
@@ -3192,7 +3193,8 @@ template <bool U16, int NPB, int TPW>
 const void *orbit_train_kernel_of(uint32_t nit)
 {
     return nit <= 1 ? (const void *)k_train_orbit_resident<U16, NPB, 1, TPW> : nit <= 2 ? (const void *)k_train_orbit_resident<U16, NPB, 2, TPW>
-         : nit <= 4 ? (const void *)k_train_orbit_resident<U16, NPB, 4, TPW> : (const void *)k_train_orbit_resident<U16, NPB, kOrbTrainMaxNit, TPW>;
+         : nit <= 4 ? (const void *)k_train_orbit_resident<U16, NPB, 4, TPW> : nit <= kOrbTrainAllNit || NPB > 2 ? (const void *)k_train_orbit_resident<U16, NPB, 6, TPW>
+         : (const void *)k_train_orbit_resident<U16, 2, kOrbTrainMaxNit, TPW>;
 }
 
 const void *orbit_train_kernel(bool u16, const OrbitTrainPlan &p)
@@ -3238,6 +3240,7 @@ const void *orbit_prepare_kernel(const pink_hip_ctx *ctx)
 
 int launch_orbit_prepare(pink_hip_ctx *ctx, OrbitPrep &p, uint32_t images)
 {
+    p.table_groups = ctx->orb_table_groups;
     const dim3 grid(images, (ctx->nrr_eff + (1u << p.rl) - 1) >> p.rl);
     const uint32_t threads = ctx->orb_prep_lds > 64 * 1024 || grid.x * grid.y < (uint32_t)ctx->num_cu ? 1024 : ctx->orb_prep_lds > 24 * 1024 ? 512 : 256;
     void *args[] = {&p};
@@ -3315,7 +3318,7 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
         a.factors_t = ctx->d_factors_t; a.elem = ctx->d_sym_element; a.selectors = ctx->d_sym_sel; a.moves = ctx->d_sym_sel + 16; a.best_variant = ctx->d_sym_best;
         a.bmu_out = dev_bmu; a.slots = ctx->d_slots; a.error = ctx->d_resident_error;
         a.launch = ++ctx->sym_trial.launch;
-        a.N = ctx->N; a.S = ctx->S; a.orbits = ctx->sym_orbits; a.KS = ctx->sym_KS; a.RT = ctx->sym_RT; a.nrr = ctx->nrr_eff;
+        a.N = ctx->N; a.S = ctx->S; a.orbits = ctx->sym_orbits; a.reached = ctx->sym_reached; a.KS = ctx->sym_KS; a.RT = ctx->sym_RT; a.nrr = ctx->nrr_eff;
         a.num_rot = ctx->cfg.num_rot; a.use_flip = ctx->cfg.use_flip; a.images = images; a.tag0 = ctx->sym_tag0; a.spin_limit = ctx->spin_limit;
         a.npb = ctx->sym_npb; a.splits = ctx->sym_plan.splits; a.groups = blocks / a.splits; a.abreast = ctx->sym_plan.abreast;
         ctx->sym_tag0 = sym_tag(ctx->sym_tag0, images);
@@ -3627,7 +3630,7 @@ std::vector<uint32_t> outside_elements(const pink_hip_ctx *ctx, const std::vecto
 // The orbits of a region under the symmetries (see orbit_gemm.inc).  Coordinates run to an even bound, the middle of an odd one twice:
 // place X of pixel x, and back.
 struct OrbitGrid {
-    uint32_t D, Ds;
+    uint32_t D, Ds, reached = 0;                            // (orbits that rotations of the image can reach; they come first)
     std::vector<uint32_t> orbit_of, reps;                   // per place; an orbit's first place
     uint32_t place(uint32_t x) const { return x + ((D & 1) && x > D / 2 ? 1u : 0u); }
     uint32_t pixel(uint32_t X) const { return X - ((D & 1) && X > D / 2 ? 1u : 0u); }
@@ -3639,7 +3642,7 @@ struct OrbitGrid {
         return at / (Ds * Ds) * (Ds * Ds) + (uint32_t)x * Ds + (uint32_t)y;
     }
     // In the order of their first places, 8 x 8 places at a time (neighbouring pieces of a row then read neighbouring pixels).
-    OrbitGrid(uint32_t D_, uint32_t C, const std::vector<uint32_t> &region) : D(D_), Ds(D_ + (D_ & 1)), orbit_of((size_t)C * Ds * Ds, ~0u)
+    OrbitGrid(uint32_t D_, uint32_t C, uint32_t I, const std::vector<uint32_t> &region) : D(D_), Ds(D_ + (D_ & 1)), orbit_of((size_t)C * Ds * Ds, ~0u)
     {
         for (uint32_t off : region) {
             uint32_t first = at(off);
@@ -3653,33 +3656,51 @@ struct OrbitGrid {
             return (ch << 48) | ((x / 8) << 32) | ((y / 8) << 16) | ((x % 8) << 8) | (y % 8);
         };
         std::sort(reps.begin(), reps.end(), [&](uint32_t l, uint32_t r) { return key(l) < key(r); });
+        // half the image's diagonal, and two pixels for the crop's shift, the places of an odd neuron and the roundings of a rotation
+        const double most = (I - 1) * 0.70711 + 2.0, middle = (D - 1) * 0.5;
+        reached = (uint32_t)(std::stable_partition(reps.begin(), reps.end(), [&](uint32_t p) {
+            const double x = pixel((p % (Ds * Ds)) / Ds) - middle, y = pixel(p % Ds) - middle;
+            return x * x + y * y <= most * most;
+        }) - reps.begin());
         for (uint32_t o = 0; o < reps.size(); ++o)
             for (uint32_t sym = 0; sym < 8; ++sym) orbit_of[moved(reps[o], sym)] = o;
     }
 };
+
+// Orbits that a resident integer trainer takes for reached: whole chunks of 64, if not all.  (All of them where the sums of what is not
+// reached, 16 bits squared, could pass 2^31.)
+uint32_t orbit_train_reached(const pink_hip_ctx *ctx, const OrbitGrid &grid)
+{
+    const uint32_t all = (uint32_t)grid.reps.size();
+    return ctx->cfg.ed_type == PINK_HIP_UINT16 && ctx->E > 33025 ? all : std::min(all, round_up(std::max(1u, grid.reached), 64));
+}
 
 // How many neurons a block of a resident integer trainer holds and between how many blocks the rows are shared out: what is expected to
 // take least.  In clocks of an image: a block's rows through its CU's 64 bytes a clock, its waves' instructions or the matrix pipes; a round of
 // tiles, whose shares of k meet in the LDS; an update of 64 orbits a wave; the words of the blocks that hold the same neurons.  Fitted to
 // every plan of 29 shapes (15 to 1024 neurons of 169 to 10000 elements, 4 to 720 variants): off by 3.2 % in the mean, the plan taken 1.4 %
 // slower than the fastest in the mean and 6.6 % at most, where plans are up to four times apart.  npb 0: no way to hold the neurons.
-OrbitTrainPlan plan_orbit_train(uint32_t N, uint32_t E, uint32_t orbits, uint32_t nrr, bool u16, uint32_t units, size_t lds_max)
+OrbitTrainPlan plan_orbit_train(uint32_t N, uint32_t E, uint32_t orbits, uint32_t reached, uint32_t nrr, bool u16, uint32_t units, size_t lds_max)
 {
-    const uint32_t RT = (nrr + 15) / 16, KS = round_up((orbits * 8 + 63) / 64, 2), planes = u16 ? 2 : 1, accs = u16 ? 3 : 1, products = u16 ? 4 : 1;
+    const uint32_t RT = (nrr + 15) / 16, planes = u16 ? 2 : 1, accs = u16 ? 3 : 1, products = u16 ? 4 : 1;
     const double most = (double)E * (u16 ? 65535.0 * 65535.0 : 255.0 * 255.0);
     OrbitTrainPlan best;
     double best_cost = 0.0;
     for (uint32_t npb = 1; npb <= 4; ++npb) {
         const uint32_t groups = (N + npb - 1) / npb, columns = npb > 2 ? 2 : 1, nit = (npb * ((orbits + 63) / 64) + kOrbTrainWorkers - 1) / kOrbTrainWorkers;
-        if (nit > kOrbTrainMaxNit || most >= (double)(1ull << (48 - orbit_train_bits(npb)))) break;
+        const uint32_t streamed = nit > kOrbTrainAllNit ? reached : orbits, KS = round_up((streamed * 8 + 63) / 64, 2);
+        if (nit > (npb > 2 ? kOrbTrainAllNit : kOrbTrainMaxNit) || most >= (double)(1ull << (48 - orbit_train_bits(npb)))) break;
         uint32_t tiles_before = 0;
         for (uint32_t splits = 1; splits <= std::min(kOrbTrainSplits, RT) && groups * splits <= units; ++splits) {
             const uint32_t tiles = (RT + splits - 1) / splits;
             if (tiles == tiles_before) continue;
+            // (more than six orbits a thread: rows that a compute unit takes longer to pull through than the orbits' product takes for an image,
+            // 15 us for three tiles of 33488 uint8 elements)
+            if (nit > kOrbTrainAllNit && tiles * KS * planes > 1600) continue;
             tiles_before = tiles;
             for (uint32_t abreast = 1; abreast <= 8; abreast *= 2)
                 for (uint32_t tpw = 1; tpw <= (u16 ? 1u : 3u); tpw += 2) {
-                    const size_t lds = orbit_train_lds(npb, orbits, u16, N, tpw);
+                    const size_t lds = orbit_train_lds(npb, orbits, streamed, u16, N, tpw);
                     if (lds + 2048 > lds_max) continue;
                     const uint32_t rounds = (tiles + abreast * tpw - 1) / (abreast * tpw), shares = kSymWaves / abreast;
                     const double stream = rounds * abreast * tpw * 16.0 * KS * planes;
@@ -3688,7 +3709,7 @@ OrbitTrainPlan plan_orbit_train(uint32_t N, uint32_t E, uint32_t orbits, uint32_
                     const double cost = 1.155 * std::max({stream, issue, matrix}) + rounds * (2850.0 + 110.0 * tpw * columns * accs + 10.0 * accs * shares * ((abreast * tpw * columns + 7) / 8)) +
                                         nit * (u16 ? 2070.0 : 1594.0) + (splits > 1 ? 1000.0 : 0.0) + 100.0 * (abreast - 1) + 3.0 * groups * splits;
                     if (!best.npb || cost < best_cost) {
-                        best.npb = npb; best.splits = splits; best.abreast = abreast; best.tpw = tpw; best.nit = nit; best.lds = lds;
+                        best.npb = npb; best.splits = splits; best.abreast = abreast; best.tpw = tpw; best.nit = nit; best.lds = lds; best.reached = streamed;
                         best_cost = cost;
                     }
                 }
@@ -3697,7 +3718,7 @@ OrbitTrainPlan plan_orbit_train(uint32_t N, uint32_t E, uint32_t orbits, uint32_
     return best;
 }
 
-int orbit_samples(pink_hip_ctx *ctx, const uint32_t *d_upos, uint32_t Kp);
+int orbit_samples(pink_hip_ctx *ctx, const uint32_t *d_upos, uint32_t Kp, uint32_t images);
 int finish_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, const std::vector<uint32_t> &upos, const std::vector<unsigned char> &mask);
 
 // Integer trainers whose neurons fit the blocks of a resident launch: the resident form with the symmetries on the SOM side (orbit_train.inc).
@@ -3705,23 +3726,24 @@ int finish_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, con
 int init_orbit_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
 {
     const pink_hip_config &c = ctx->cfg;
-    if (!ctx->gemm || !ctx->fused_som || c.kernel_choice != PINK_HIP_KERNEL_AUTO || ctx->N > kSymMaxNeurons || ctx->D >= 4095 || ctx->C >= 256 || !resident_allowed())
+    if (!ctx->gemm || (!ctx->fused_som && !ctx->orbit_train) || c.kernel_choice != PINK_HIP_KERNEL_AUTO || ctx->N > kSymMaxNeurons || ctx->D >= 4095 || ctx->C >= 256 || !resident_allowed())
         return PINK_HIP_OK;
-    const OrbitGrid grid(ctx->D, ctx->C, region);
+    const OrbitGrid grid(ctx->D, ctx->C, ctx->I, region);
     const bool u16 = c.ed_type != PINK_HIP_UINT8;
-    ctx->sym_plan = plan_orbit_train(ctx->N, ctx->E, (uint32_t)grid.reps.size(), ctx->nrr_eff, u16, (uint32_t)ctx->num_cu, ctx->lds_max);
+    ctx->sym_plan = plan_orbit_train(ctx->N, ctx->E, (uint32_t)grid.reps.size(), orbit_train_reached(ctx, grid), ctx->nrr_eff, u16, (uint32_t)ctx->num_cu, ctx->lds_max);
     if (!ctx->sym_plan.npb) { ctx->sym_plan = {}; return PINK_HIP_OK; }
     ctx->sym_orbits = (uint32_t)grid.reps.size();
+    ctx->sym_reached = ctx->sym_plan.reached;
     ctx->sym_npb = ctx->sym_plan.npb;
     ctx->sym_lds = ctx->sym_plan.lds;
     ctx->sym_RT = (ctx->nrr_eff + 15) / 16;
-    ctx->sym_KS = round_up((ctx->sym_orbits * 8 + 63) / 64, 2);
+    ctx->sym_KS = round_up((ctx->sym_reached * 8 + 63) / 64, 2);
     const uint32_t Kp = ctx->sym_KS * 64, D = ctx->D, Ds = grid.Ds;
     std::vector<uint32_t> upos(Kp, ~0u), elem((size_t)ctx->sym_orbits * 8, ~0u), sel(16 + 64);
     std::vector<unsigned char> mask((size_t)8 * Kp, 0);
     std::vector<char> inside(ctx->S, 0);
     for (uint32_t off : region) inside[off] = 1;
-    for (uint32_t o = 0; o < ctx->sym_orbits; ++o)
+    for (uint32_t o = 0; o < ctx->sym_reached; ++o)
         for (uint32_t p = 0; p < 8; ++p) {
             const uint32_t at = grid.moved(grid.reps[o], p);
             upos[o * 8 + p] = (at / (Ds * Ds) << 24) | (grid.pixel((at % (Ds * Ds)) / Ds) << 12) | grid.pixel(at % Ds);
@@ -3733,7 +3755,7 @@ int init_orbit_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         uint32_t p = 0;
         while (grid.moved(grid.reps[o], p) != at) ++p;
         elem[o * 8 + p] = off;
-        for (uint32_t sym = 0; sym < 8; ++sym)
+        for (uint32_t sym = 0; sym < 8 && o < ctx->sym_reached; ++sym)
             if (valid(sym)) {
                 const uint32_t k = o * 8 + orbit_moves((int)sym, (int)p), pos = upos[k];
                 mask[(size_t)sym * Kp + k] = 0xff;
@@ -3895,19 +3917,19 @@ int finish_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, con
     TRY(upload(ctx, &ctx->d_sym_upos, upos));
     TRY(upload(ctx, &ctx->d_sym_outside, outside));
     TRY(upload(ctx, (unsigned char **)&ctx->d_sym_mask, mask));
+    // a group's operand and rows are written by one launch and read by the next: within the last-level cache
+    const size_t op_image = (size_t)(u16 ? 2 : 1) * ctx->sym_RT * ctx->sym_KS * 1024, x_image = (size_t)ctx->nrr_eff * Kp * sizeof(float);
+    size_t b = c.max_batch ? std::min<size_t>(c.max_batch, kSymGroupMax) : kSymGroupMax;
+    while (b > 8 && b * (op_image + x_image) > ((size_t)192 << 20)) --b;
+    ctx->sym_B = (uint32_t)b;
     if (f32) {
         const size_t image_lds = (size_t)ctx->C * ctx->I * ctx->I * sizeof(float);
         ctx->sym_prep_lds = image_lds <= 150 * 1024 ? image_lds : 0;
         HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_f32_prepare<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 2048));
     } else {
         ctx->orb_mode = u16 ? ORB_U16 : ORB_U8;
-        TRY(orbit_samples(ctx, ctx->d_sym_upos, Kp));
+        if (!ctx->orbit_train) TRY(orbit_samples(ctx, ctx->d_sym_upos, Kp, (uint32_t)b));        // (else init_orbit's: the same places)
     }
-    // a group's operand and rows are written by one launch and read by the next: within the last-level cache
-    const size_t op_image = (size_t)(u16 ? 2 : 1) * ctx->sym_RT * ctx->sym_KS * 1024, x_image = (size_t)ctx->nrr_eff * Kp * sizeof(float);
-    size_t b = c.max_batch ? std::min<size_t>(c.max_batch, kSymGroupMax) : kSymGroupMax;
-    while (b > 8 && b * (op_image + x_image) > ((size_t)192 << 20)) --b;
-    ctx->sym_B = (uint32_t)b;
     TRY(dev_alloc(ctx, &ctx->d_sym_op, b * op_image / 16));
     TRY(dev_alloc(ctx, &ctx->d_sym_x, b * ctx->nrr_eff * Kp + 64));       // (a chunk of 64 orbits may read past the last)
     TRY(dev_alloc(ctx, &ctx->d_sym_norm, b * ctx->sym_RT * 16 * 8));
@@ -3934,19 +3956,23 @@ int finish_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, con
 }
 
 // Where the samples of the base rotations lie, for rows of Kp places (d_upos).
-int orbit_samples(pink_hip_ctx *ctx, const uint32_t *d_upos, uint32_t Kp)
+int orbit_samples(pink_hip_ctx *ctx, const uint32_t *d_upos, uint32_t Kp, uint32_t images)
 {
     const bool f32 = ctx->orb_mode == ORB_F32;
     const size_t image_lds = (size_t)ctx->C * orbit_tile(ctx->I) * sizeof(float);
     ctx->orb_prep_lds = image_lds <= 120 * 1024 ? image_lds : 0;
     if (ctx->orb_prep_lds)
         HIP_TRY(ctx, hipFuncSetAttribute(orbit_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024));
-    // as many base rotations per wave as there are, up to 16; four for a trainer's few
-    // images of long rows, two where the image comes out of memory: a wave's pixels are neighbours then, and a call with one
-    // image has blocks for a part of the chip
+    // as many base rotations per wave as there are, up to 16; two where the image comes out of memory: a wave's pixels are neighbours
+    // then; four for a trainer's few images of long rows, which have blocks for a part of the chip (us per image, 4 | 8 | 16 rotations:
+    // 30 images of 25 rows of 42440 elements 3.6 | 6.2 | -, 12 of 90 rows of 33488 14.5 | 12.8 | 23.6; groups of 67 images of 4480 elements
+    // 2.0 | 1.7 | 1.5, of 167 of 2304 0.63 | 0.53 | 0.52)
+    const auto row_blocks = [&](uint32_t rl) { return (ctx->nrr_eff + (1u << rl) - 1) >> rl; };
+    const uint32_t most = !ctx->orb_prep_lds ? 1u : ctx->trainer && Kp >= 4096 && images * row_blocks(4) < (uint32_t)ctx->num_cu / 2 ? 2u : 4u;
     ctx->orb_rl = 0;
-    while ((1u << ctx->orb_rl) < ctx->nrr_eff && ctx->orb_rl < (!ctx->orb_prep_lds ? 1u : ctx->trainer && Kp >= 4096 ? 2u : 4u)) ++ctx->orb_rl;
-    const uint32_t blocks = (ctx->nrr_eff + (1u << ctx->orb_rl) - 1) >> ctx->orb_rl, groups = orbit_piece_groups(Kp / 16, ctx->orb_rl);
+    while (ctx->orb_rl < most && row_blocks(ctx->orb_rl) > 1) ++ctx->orb_rl;
+    const uint32_t blocks = row_blocks(ctx->orb_rl), groups = orbit_piece_groups(Kp / 16, ctx->orb_rl);
+    ctx->orb_table_groups = groups;
     const uint32_t tiles = (ctx->nrr_eff + 15) / 16;
     const size_t entries = f32 ? (size_t)tiles * Kp * 16 : (size_t)blocks * groups * 1024;
     TRY(dev_alloc(ctx, &ctx->d_orb_index, entries));
@@ -3965,7 +3991,7 @@ int orbit_samples(pink_hip_ctx *ctx, const uint32_t *d_upos, uint32_t Kp)
 int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
 {
     const pink_hip_config &c = ctx->cfg;
-    const OrbitGrid grid(ctx->D, ctx->C, region);
+    const OrbitGrid grid(ctx->D, ctx->C, ctx->I, region);
     const uint32_t D = ctx->D, DD = D * D, Ds = grid.Ds;
     const std::vector<uint32_t> &reps = grid.reps, &orbit_of = grid.orbit_of;
     auto pixel = [&](uint32_t X) { return grid.pixel(X); };
@@ -3974,7 +4000,8 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     ctx->orb_ns = c.use_flip ? 8 : 4;
     ctx->orb_valid = (c.num_rot == 1 ? 0x11u : 0xffu) & (c.use_flip ? 0xffu : 0x0fu);
     const bool f32 = ctx->orb_mode == ORB_F32;
-    ctx->orb_KS = round_up(((uint32_t)reps.size() * 8 + 31) / 32, f32 ? 16u : ctx->orb_mode == ORB_U8 ? 4u : 2u);       // (k_coef_gemm's steps, k_orbit_gemm's KC)
+    // (k_coef_gemm's steps, k_orbit_gemm's KC; a trainer's rows are those of init_orbit_train too)
+    ctx->orb_KS = round_up(((uint32_t)reps.size() * 8 + 31) / 32, f32 ? 16u : ctx->orb_mode == ORB_U8 || ctx->trainer ? 4u : 2u);
     const uint32_t Kp = ctx->orb_KS * 32;
     ctx->orb_Ox = round_up((uint32_t)reps.size(), 16);
     if (f32 && Kp > 65536) return PINK_HIP_OK;      // (positions in a row are 16 bits there)
@@ -4076,7 +4103,7 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         }
     }
     TRY(tables.commit(ctx, &ctx->d_orb_tables));
-    TRY(orbit_samples(ctx, d_upos, Kp));
+    TRY(orbit_samples(ctx, d_upos, Kp, 1));
     ctx->orb_pitch = ctx->trainer ? round_up(ctx->nrr_eff, f32 ? 16 : 32) : ctx->nrr_eff;
     ctx->screen_train = ctx->trainer && f32;
     ctx->orbit = !ctx->screen_train;
@@ -4140,8 +4167,7 @@ uint32_t summed_images(const pink_hip_ctx *ctx)
     return (uint32_t)std::min({images, (double)ctx->Bcap, (double)((size_t)1 << 30) / (double)row_bytes});
 }
 
-// Trainers that take the orbits' product: integers where the resident form (init_sym_train) does not fit, which keep their
-// weights in that order too; float32 where every variant's sum costs more than the product and the sums that it leaves.
+// Trainers that take the orbits' product, integers where they are not resident (init_orbit_train), which keep their weights in that order too; float32 where every variant's sum costs more than the product and the sums that it leaves.
 // Summing all: a chain of E steps and, with more neurons than fill the chip, its share of the vector ALUs, E (0.0095 + 4.6e-8 N R) us
 // per image; screening: five dependent launches and what grows with the elements, 22 + 0.0035 E.  (summed / screened
 // us at N R E: 9 720 2304 25 / 30, 9 720 4096 42 / 35, 9 720 16384 167 / 77, 100 720 2304 31 / 31, 100 720 4096 50 / 38, 256 720 1024
@@ -4157,8 +4183,10 @@ bool orbit_trains(const pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     }
     // (below a dozen base rotations the product's tiles of 64 rows are mostly empty)
     if (!ctx->gemm || ctx->E < 1024 || ctx->nrr_eff < 12 || !resident_allowed()) return false;
-    return ctx->N > kSymMaxNeurons ||
-           !plan_orbit_train(ctx->N, ctx->E, (uint32_t)OrbitGrid(ctx->D, ctx->C, region).reps.size(), ctx->nrr_eff, ctx->cfg.ed_type == PINK_HIP_UINT16,
+    const OrbitGrid grid(ctx->D, ctx->C, ctx->I, region);
+    // (the rows of every variant, which the other form in turn writes and reads, are 8 MB an image and more)
+    return ctx->N > kSymMaxNeurons || (uint64_t)ctx->R * ctx->Epad * (ctx->cfg.ed_type == PINK_HIP_UINT16 ? 2 : 1) > (8u << 20) ||
+           !plan_orbit_train(ctx->N, ctx->E, (uint32_t)grid.reps.size(), orbit_train_reached(ctx, grid), ctx->nrr_eff, ctx->cfg.ed_type == PINK_HIP_UINT16,
                              (uint32_t)ctx->num_cu, ctx->lds_max).npb;
 }
 
@@ -4995,7 +5023,7 @@ int init_ctx(pink_hip_ctx *ctx)
                 TRY(init_exchange(ctx, kSlotWords, (const void *)small_resident_kernel(ctx), kResidentThreads, (size_t)2 * nstored * ctx->S * sizeof(float)));
             }
         }
-        if (one_to_one && !ctx->small_train && !ctx->orbit_train && !ctx->f32gemm) TRY(init_sym_train(ctx, region));
+        if (one_to_one && !ctx->small_train && !ctx->f32gemm) TRY(init_sym_train(ctx, region));
         // one launch per image where the float32 distance kernel runs in its one-wave-per-SIMD form (see k_train_f32_dpp;
         // up to 256 neurons: measured with 512 allowed, 17 x 17 and 18 x 18 neurons at 720 variants train no faster this
         // way than with an update launch of their own -- with three to four waves per SIMD the launch saved is paid in
@@ -5191,14 +5219,17 @@ int train_in_turn(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images,
 // ... in the form that the context takes at present.
 int train_queued(pink_hip_ctx *ctx, const float *dev_images, uint32_t n_images, uint32_t *dev_bmu_out)
 {
-    if (ctx->orbit_train) return run_orbit_train(ctx, dev_images, n_images, dev_bmu_out);
+    if (ctx->orbit_train && !ctx->sym_form) return run_orbit_train(ctx, dev_images, n_images, dev_bmu_out);
     for (uint32_t done = 0, count; done < n_images; done += count) {
         count = n_images - done;
         Form form;
         TRY(choose_form(ctx, n_images, &count, &form));
         const float *images = dev_images + (size_t)done * ctx->isz;
         uint32_t *bmu = dev_bmu_out ? dev_bmu_out + done : nullptr;
-        if (form != Form::resident) TRY(train_in_turn(ctx, images, count, bmu, form == Form::screened));
+        if (form != Form::resident && ctx->orbit_train) {
+            if (!ctx->packed) TRY(run_pack_som(ctx));
+            TRY(run_orbit_train(ctx, images, count, bmu));
+        } else if (form != Form::resident) TRY(train_in_turn(ctx, images, count, bmu, form == Form::screened));
         else
             for (uint32_t b = 0; b < count; b += ctx->sym_B)
                 TRY(run_sym_train(ctx, images + (size_t)b * ctx->isz, std::min(ctx->sym_B, count - b), bmu ? bmu + b : ctx->d_bmu_group));

@@ -775,6 +775,13 @@ RESIDENT_INTEGER_PLANS = [
     (1023, 1, 20, 18, 12, True, 17, capi.QUADRATIC, capi.UINT16, 3),     # 4 x 1, the last block holds three
     (40, 1, 23, 22, 36, True, 22, capi.QUADRATIC, capi.UINT16, 3),       # 66 orbits: a chunk and two more
     (40, 1, 23, 21, 36, True, 21, capi.QUADRATIC, capi.UINT8, 3),        # an odd neuron: the middle twice
+    (12, 1, 30, 70, 80, True, 60, capi.QUADRATIC, capi.UINT8, 3),        # places that no rotation of the image reaches: three of eight chunks
+    (500, 1, 30, 71, 40, True, 61, capi.CIRCULAR, capi.UINT16, 3),
+    (400, 1, 20, 60, 24, False, 49, capi.QUADRATIC, capi.UINT16, 2),
+    (9, 1, 64, 200, 48, True, 181, capi.QUADRATIC, capi.UINT8, 2),       # ten chunks to a thread
+    (9, 1, 64, 200, 48, True, 180, capi.QUADRATIC, capi.UINT16, 2),
+    (3, 1, 40, 190, 16, True, 186, capi.QUADRATIC, capi.UINT16, 2),      # all of them: their squares pass 2^31
+    (60, 1, 100, 140, 36, True, 130, capi.QUADRATIC, capi.UINT8, 2),     # 34 chunks, 31 reached
 ]
 
 
