@@ -1862,11 +1862,16 @@ __global__ __launch_bounds__(256) void k_train_small_u8(float *__restrict__ som,
 // The same trainers with the kernel RESIDENT over a whole launch group: one block per neuron keeps its neuron
 // -- weights in registers, its row of the SOM operand and the norm in LDS -- over all images of the group and
 // computes only its own neuron's distances (the MFMA's 32 columns all hold the one neuron).  Per image the
-// blocks exchange one 64-bit word each, (tag, smallest distance of the neuron), through slots a cache line
-// apart: a block stores its word and its first wave polls the N slots until all carry the image's tag.  Nothing
-// else crosses between blocks, so no fences: the payload rides in the atomic word.  Two sets of slots take turns
-// (a block can be at most one image ahead of another).  The exchange costs about 1.4 us, where a launch boundary
-// with the distance matrix worked out again in every block costs 5.
+// blocks exchange one 64-bit word each, (tag, smallest distance of the neuron): a block stores its word and a wave polls
+// the N blocks' until all carry the image's tag.  Nothing else crosses between blocks, so no fences: the payload rides in
+// the atomic word.  Two sets of words take turns (a block can be at most one image ahead of another).
+// An image is one chain of latencies, and all of it is what the kernel is bound by (64 neurons of 28 x 28, 8 variants, 1.83 -> 1.48 us; 32
+// variants 2.98 -> 1.71; 0.8 of it the exchange).  Where one wave can hold the image's rows (FT tiles of 16 rows x FK k-steps of 64
+// bytes, v_mfma_i32_16x16x64_i8: half the cycles of the 32-row form for up to 16 variants), it multiplies alone and has the neuron's
+// distances in its accumulators and its norm beside them: eight waves' parts meet in the LDS behind a barrier, 0.62 us to the word.
+// Another wave polls and asks for nothing else: a word comes back behind what its wave asked for before.  The values of the
+// neuron's best variant come out of memory while the words travel (staging every variant in the LDS an image ahead: 1.52; 1.6 with 16
+// variants).  Neurons of more than 1024 elements and 16 variants keep the eight waves: their rows do not fit one wave's registers.
 // Every wait is bounded: a wave that does not see all words within `spin_limit` polls raises `error` and marks its
 // block's slots, polling waves leave when they see such a mark, a block that leaves stops publishing, so every
 // block leaves.  The group's
@@ -1874,8 +1879,14 @@ __global__ __launch_bounds__(256) void k_train_small_u8(float *__restrict__ som,
 // that follow one that gave up leave at once, so its inputs stay as they were.  The host looks at `error` after the last
 // of the launches it queued and trains the groups again, image by image, from the one that gave up.
 // ---------------------------------------------------------------------------------
-constexpr uint32_t kSlotStride = 16;                      // 64-bit words between two blocks' slots (128 bytes)
-constexpr uint32_t kSlotWords = 2 * 64 * kSlotStride;     // two sets of 64 slots
+// A word that every block waits for is written kCopies times, block b reads copy b % kCopies, its words 16 bytes apart: a poll holds up the
+// stores to what it reads, so as few blocks as possible ask for a line, and none before the words can be there (await_others; requests for
+// words that are there already are not repeated).  The exchange alone, us, 64 / 150 / 250 blocks: one copy 64 bytes apart, polled at
+// once 1.08 / 1.27 / 1.41, after 768 clocks 0.93 / 1.14 / 1.25; eight copies 0.77 / 0.95 / 0.98; blocks that are 0 to 500 clocks late 1.27 / 1.54 / 1.77
+// and 1.07 / 1.15 / 1.17; one copy without space between the words, polled at once, 1.83 / 1.96 / 2.03.
+constexpr uint32_t kCopies = 8, kCopyStride = 2;
+__device__ __forceinline__ void await_others() { __builtin_amdgcn_s_sleep(12); }
+constexpr uint32_t kSlotWords = 2 * 64 * kCopies * kCopyStride;       // two sets of kCopies words of 64 blocks
 constexpr uint32_t kGaveUpTag = 0xffffffffu;              // in a slot: its block has left the launch
 
 struct ResidentTrain {
@@ -1887,7 +1898,7 @@ struct ResidentTrain {
     unsigned long long *slots;
     uint32_t *error;                // 0, or the number (from 1) of the launch that gave up, among those the host has not checked yet
     uint32_t launch;                // this launch's number
-    uint32_t N, S, R, KS, nstored, images, tag0, spin_limit;
+    uint32_t N, S, R, KS, images, tag0, spin_limit;
     uint32_t rot_stride, pb_stride, nb_stride;      // per image: floats, 16-byte words, norms
     VariantPair vp;
 };
@@ -1895,7 +1906,8 @@ struct ResidentTrain {
 // Eight waves per block: two share a SIMD without slowing each other, so each wave's part of every step is half as long.
 constexpr uint32_t kResidentThreads = 512, kResidentWaves = kResidentThreads / 64;
 
-template <int EPT, int KSW, int SV>    // elements of the neuron, k-steps and variant elements (first batch) per thread
+// Elements of the neuron per thread; tiles and k-steps of the wave that multiplies alone, or 0 and the 32-byte k-steps a wave holds at a time.
+template <int EPT, int FT, int FK>
 __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__restrict__ som, float *__restrict__ som_next,
                                                                  const float *__restrict__ rot, const v4i *__restrict__ Pa,
                                                                  signed char *__restrict__ Pa_next, const v4i *__restrict__ Pb,
@@ -1903,14 +1915,17 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
                                                                  const unsigned long long *__restrict__ src4,
                                                                  const uint32_t *__restrict__ kbyte, ResidentTrain a)
 {
-    extern __shared__ float s_var[];                      // the stored variants of this image and of the next one
     __shared__ v4i s_op[128 + 1];                         // this neuron's operand row: [k-step][half of the k-step]; one spare
-    __shared__ v4i s_part[kResidentWaves][2][4];          // [wave][half][16 accumulators]
+    constexpr bool ALONE = FT != 0;
+    constexpr int KSW = FK;
+    constexpr uint32_t COPIES = ALONE ? kCopies : 1, STRIDE = kCopies * kCopyStride / COPIES;     // of a block's word; 64-bit words from one block's to the next
+    __shared__ v4i s_part[ALONE ? 1 : kResidentWaves][2][4];     // [wave][half][16 accumulators]
+    __shared__ uint32_t s_best;                           // the key of the wave that multiplies alone
     __shared__ int s_sq[kResidentWaves];
     __shared__ uint2 s_bmu_f;                             // the best match (all ones: leave) and this neuron's factor for it
     uint32_t &s_bmu = s_bmu_f.x;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = blockIdx.x;
-    const uint32_t N = a.N, S = a.S, KS = a.KS, n_var = a.nstored * S;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = FT ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)) : tid >> 6, n = blockIdx.x;
+    const uint32_t N = a.N, S = a.S, KS = a.KS;
     // (a launch that follows one that gave up leaves at once; one thread looks, so the whole block decides alike)
     if (tid == 0) s_bmu = __hip_atomic_load(a.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
@@ -1941,7 +1956,6 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
     const uint32_t row = lane & 31;                       // the operand row whose key this lane works out
     const uint32_t var_row = a.variant[row];
     const uint32_t acc_half = (row >> 2) & 1, acc_j = ((row >> 3) << 2) | (row & 3);     // where the MFMA leaves row `row`
-    for (uint32_t t = tid; t < n_var; t += kResidentThreads) s_var[t] = rot[t];
     // variant r of an image: which stored variant it is read from and how (rows / columns reversed), worked out once
     // by lane r: offset of the stored variant in floats << 8 | shift into the packed source positions
     uint32_t dec_lane;
@@ -1950,101 +1964,158 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
         const uint32_t q = rem / a.vp.nrr, b0 = rem - q * a.vp.nrr;
         dec_lane = ((((q & 1) * a.vp.nrr + b0) * S) << 8) | (16 * (2 * (flip ^ (q >> 1)) + (q >> 1)));
     }
-    v4i fb[KSW];
+    v4i fb[ALONE ? 1 : KSW];
     auto load_fragments = [&](const v4i *pb, uint32_t first) {
 #pragma unroll
         for (int u = 0; u < KSW; ++u) fb[u] = pb[(size_t)min(first + kResidentWaves * u, KS - 1) * 64 + lane];
     };
-    load_fragments(Pb, wave);
-    int nb_row = (int)a.nb[row];
-    // the variants of the image after next wait in registers for a whole image (asked for during one exchange,
-    // put into LDS during the next)
-    float sv[SV];
-    auto load_variants = [&](const float *src) {
+    // rows of the wave that multiplies alone: lane l holds row l % 16 of a tile, bytes 16 (l / 16) .. of a k-step; norms and variants of the rows 4 (l / 16) .., as the MFMA leaves them
+    constexpr int T = ALONE ? FT : 1, K = ALONE ? FK : 1;
+    v4i rows[T][K];
+    uint32_t row_var[T][4];
+    int row_norm[T][4], nb_row = 0;
+    auto load_rows = [&](const v4i *pb, const long long *nb) {
+        const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc((void *)pb, 0, (int)(KS * 1024), 0x00027000);      // (past the end: zeros)
 #pragma unroll
-        for (int u = 0; u < SV; ++u) sv[u] = src[min(tid + kResidentThreads * u, n_var - 1)];
+        for (int t = 0; t < T; ++t) {
+#pragma unroll
+            for (int u = 0; u < K; ++u)
+                rows[t][u] = __builtin_amdgcn_raw_buffer_load_b128(from, (int)((lane >> 4) * 512 + (lane & 15) * 16 + 256 * t + 2048 * u), 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) row_norm[t][r] = (int)nb[16 * t + (lane >> 4) * 4 + r];
+        }
     };
-    if (a.images > 1) load_variants(rot + a.rot_stride);
+    const bool multiplier = ALONE && wave == 0, poller = wave == (ALONE ? 1 : 0);
+    if (multiplier) {
+        load_rows(Pb, a.nb);
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) row_var[t][r] = 16 * t + (lane >> 4) * 4 + r < a.R ? a.variant[16 * t + (lane >> 4) * 4 + r] : 0xffffffffu;      // (no match)
+    }
+    if constexpr (!ALONE) { load_fragments(Pb, wave); nb_row = (int)a.nb[row]; }
     __syncthreads();
 
     for (uint32_t i = 0; i < a.images; ++i) {
         const bool more = i + 1 < a.images;
         const v4i *pb = Pb + (size_t)i * a.pb_stride;
-        float *var_cur = s_var + (i & 1) * n_var, *var_next = s_var + ((i + 1) & 1) * n_var;
         if (i + 2 == a.images) PROBE(kProbeResident, n, 0);
 
         // (1) this neuron against all variants: this wave's k-steps (the operand row out of LDS first: a lone
         // wave waits out every LDS read it issues between two MFMAs)
         // (the first batch whatever KS: a wave with no k-step of its own multiplies by the zero k-steps)
-        v16i acc = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        for (uint32_t first = wave;;) {
-            v4i fa[KSW];
-#pragma unroll
-            for (int u = 0; u < KSW; ++u) fa[u] = s_op[min(first + kResidentWaves * u, 63u) * 2 + (lane >> 5)];
-#pragma unroll
-            for (int u = 0; u < KSW; ++u) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[u], fa[u], acc, 0, 0, 0);
-            first += kResidentWaves * KSW;
-            if (first >= KS) break;
-            load_fragments(pb, first);
-        }
-        if (i + 2 == a.images) PROBE(kProbeResident, n, 1);
-        if ((lane & 31) == 0) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                s_part[wave][lane >> 5][g] = (v4i){acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
-        }
-        __syncthreads();
-        if (i + 2 == a.images) PROBE(kProbeResident, n, 2);
-
-        // (2) the neuron's key (every wave for itself) and its word into the exchange
-        const int *part = (const int *)&s_part[0][acc_half][0] + acc_j;
-        int dot = 0;                                          // the waves' k ranges
-#pragma unroll
-        for (uint32_t w = 0; w < kResidentWaves; ++w) dot += part[32 * w];
-        const uint32_t key = row < a.R ? ((uint32_t)(na + nb_row - 2 * dot) << 5) | var_row : 0xffffffffu;
-        const uint32_t best = wave_min_u32_dpp(key);
         const uint32_t tag = a.tag0 + i;
-        unsigned long long *set = a.slots + (size_t)(i & 1) * 64 * kSlotStride;
-        if (tid == 0)
-            __hip_atomic_store(set + (size_t)n * kSlotStride, ((unsigned long long)tag << 32) | (best >> 5), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        if (i + 2 == a.images) PROBE(kProbeResident, n, 3);
-
-        // (3) while the words travel: the next image's variants into LDS, the requests for the image after it, and the
-        // part of the update that does not need the best match (the neuron's own best variant is known)
-        if (more) {
+        // (copies for the form whose polls come back at once; the other's, behind what its waves have asked for, are no faster for them)
+        unsigned long long *set = a.slots + (size_t)(i & 1) * 64 * kCopies * kCopyStride;
+        auto publish = [&](uint32_t key) {                // (a copy per lane)
+            if (lane < COPIES)
+                __hip_atomic_store(set + (lane * 64 + n) * STRIDE, ((unsigned long long)tag << 32) | (key >> 5), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        uint32_t best = 0;
+        if constexpr (ALONE) {
+            if (multiplier) {
+                // (two accumulators a tile: no MFMA waits for the one before)
+                constexpr int B = K < 16 ? K : 8;         // (more pieces: eight of the neuron's at a time, the next eight on their way)
+                v4i op[2][B], acc[T][2];
+                auto read = [&](int u0) {
 #pragma unroll
-            for (int u = 0; u < SV; ++u) {
-                const uint32_t t = tid + kResidentThreads * u;
-                if (t < n_var) var_next[t] = sv[u];
+                    for (int u = u0; u < u0 + B && u < K; ++u) op[u / B & 1][u % B] = s_op[4 * u + (lane >> 4)];
+                };
+                read(0);
+#pragma unroll
+                for (int t = 0; t < T; ++t) acc[t][0] = acc[t][1] = (v4i){0, 0, 0, 0};
+                int sq[4] = {0, 0, 0, 0};                 // (the neuron's norm beside the products)
+#pragma unroll
+                for (int u = 0; u < K; ++u) {
+                    if (u % B == 0) read(u + B);
+                    const v4i p = op[u / B & 1][u % B];
+#pragma unroll
+                    for (int t = 0; t < T; ++t) acc[t][u & 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(rows[t][u], p, acc[t][u & 1], 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sq[r] = __builtin_amdgcn_sdot4(p[r], p[r], sq[r], false);
+                }
+                // (the 16 lanes of a row hold the same)
+                const int part = sq[0] + sq[1] + sq[2] + sq[3];
+                na = __builtin_amdgcn_readlane(part, 0) + __builtin_amdgcn_readlane(part, 16) + __builtin_amdgcn_readlane(part, 32) + __builtin_amdgcn_readlane(part, 48);
+                if (i + 2 == a.images) PROBE(kProbeResident, n, 1);
+                uint32_t key = 0xffffffffu;
+#pragma unroll
+                for (int t = 0; t < T; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) key = min(key, ((uint32_t)(na + row_norm[t][r] - 2 * (acc[t][0][r] + acc[t][1][r])) << 5) | row_var[t][r]);
+                best = min(min((uint32_t)__builtin_amdgcn_readlane((int)key, 0), (uint32_t)__builtin_amdgcn_readlane((int)key, 16)), min((uint32_t)__builtin_amdgcn_readlane((int)key, 32), (uint32_t)__builtin_amdgcn_readlane((int)key, 48)));
+                publish(best);
+                if (lane == 0) s_best = best;
+                if (more) load_rows(pb + a.pb_stride, a.nb + (size_t)(i + 1) * a.nb_stride);
+                if (i + 2 == a.images) PROBE(kProbeResident, n, 2);
             }
-            for (uint32_t t = tid + kResidentThreads * SV; t < n_var; t += kResidentThreads) var_next[t] = rot[(size_t)(i + 1) * a.rot_stride + t];
-            load_fragments(pb + a.pb_stride, wave);
-            nb_row = (int)a.nb[(size_t)(i + 1) * a.nb_stride + row];
-            if (i + 2 < a.images) load_variants(rot + (size_t)(i + 2) * a.rot_stride);
+        } else {
+            v16i acc = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+            for (uint32_t first = wave;;) {
+                v4i fa[KSW];
+#pragma unroll
+                for (int u = 0; u < KSW; ++u) fa[u] = s_op[min(first + kResidentWaves * u, 63u) * 2 + (lane >> 5)];
+#pragma unroll
+                for (int u = 0; u < KSW; ++u) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[u], fa[u], acc, 0, 0, 0);
+                first += kResidentWaves * KSW;
+                if (first >= KS) break;
+                load_fragments(pb, first);
+            }
+            if (i + 2 == a.images) PROBE(kProbeResident, n, 1);
+            if ((lane & 31) == 0) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    s_part[wave][lane >> 5][g] = (v4i){acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+            }
+            __syncthreads();
+            if (i + 2 == a.images) PROBE(kProbeResident, n, 2);
+
+            // (2) the neuron's key (every wave for itself) and its word into the exchange
+            const int *part = (const int *)&s_part[0][acc_half][0] + acc_j;
+            int dot = 0;                                      // the waves' k ranges
+#pragma unroll
+            for (uint32_t w = 0; w < kResidentWaves; ++w) dot += part[32 * w];
+            const uint32_t key = row < a.R ? ((uint32_t)(na + nb_row - 2 * dot) << 5) | var_row : 0xffffffffu;
+            best = wave_min_u32_dpp(key);
+            if (wave == 0) publish(best);
+            if (i + 2 == a.images) PROBE(kProbeResident, n, 3);
+        }
+
+        // (3) while the words travel: the requests for the next image, and the part of the update that does not need the best match (the
+        // neuron's own best variant is known)
+        if constexpr (!ALONE)
+            if (more) {
+                load_fragments(pb + a.pb_stride, wave);
+                nb_row = (int)a.nb[(size_t)(i + 1) * a.nb_stride + row];
+            }
+        if constexpr (ALONE) {
+            __syncthreads();
+            best = s_best;
+            if (i + 2 == a.images) PROBE(kProbeResident, n, 3);
         }
         const uint32_t dec = (uint32_t)__builtin_amdgcn_readlane((int)dec_lane, (int)(best & 31u));
-        const float *x = var_cur + (dec >> 8);
+        const float *x = rot + (size_t)i * a.rot_stride + (dec >> 8);
         const uint32_t shift = dec & 0xffu;
         float diff[EPT];
 #pragma unroll
         for (int u = 0; u < EPT; ++u) diff[u] = __fsub_rn(wv[u], x[(uint32_t)(sp[u] >> shift) & 0xffffu]);
 
-        // (4) the first wave waits for all words
-        if (wave == 0) {
-            unsigned long long v = 0;
+        // (4) a wave waits for all words
+        if (poller) {
+            const unsigned long long *words = set + (n % COPIES) * 64 * STRIDE;
+            unsigned long long v = lane < N ? 0 : (unsigned long long)tag << 32;
+            if constexpr (ALONE) __builtin_amdgcn_s_sleep(6);
             uint32_t spins = 0;
             bool all_in = false, gave_up = false;
-            // (one load per poll: a block that gives up says so in its own slots, with a tag no image has)
+            // (one load per poll: a block that gives up says so in its own words, with a tag no image has)
             while (!all_in && !gave_up) {
-                v = lane < N ? __hip_atomic_load(set + (size_t)lane * kSlotStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                             : (unsigned long long)tag << 32;
+                if (ALONE ? (uint32_t)(v >> 32) != tag : lane < N) v = __hip_atomic_load(words + lane * STRIDE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 all_in = __all((uint32_t)(v >> 32) == tag) != 0;
                 if (!all_in) gave_up = __any(++spins > a.spin_limit || (uint32_t)(v >> 32) == kGaveUpTag) != 0;
             }
             if (gave_up) {
-                if (lane < 2)
-                    __hip_atomic_store(a.slots + ((size_t)lane * 64 + n) * kSlotStride, (unsigned long long)kGaveUpTag << 32, __ATOMIC_RELAXED,
+                if (lane < 2 * COPIES)
+                    __hip_atomic_store(a.slots + ((lane % 2) * COPIES + lane / 2) * 64 * STRIDE + n * STRIDE, (unsigned long long)kGaveUpTag << 32, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
                 if (lane == 0) {
                     __hip_atomic_store(a.error, a.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2076,15 +2147,17 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
                 wv[u] = nv;
                 const int h = quantise(nv, 255.0f) - 128;
                 ((signed char *)s_op)[cb[u]] = (signed char)h;
-                sq += (h * h) & (int)in_region[u];
+                if constexpr (!ALONE) sq += (h * h) & (int)in_region[u];
             }
-            sq = wave_sum_i32_dpp(sq);
-            if (lane == 0) s_sq[wave] = sq;
+            if constexpr (!ALONE) {
+                sq = wave_sum_i32_dpp(sq);
+                if (lane == 0) s_sq[wave] = sq;
+            }
         }
         if (i + 2 == a.images) PROBE(kProbeResident, n, 6);
         __syncthreads();
         if (i + 2 == a.images) PROBE(kProbeResident, n, 7);
-        if (f != 0.0f) {
+        if (!ALONE && f != 0.0f) {
             na = 0;
 #pragma unroll
             for (uint32_t w = 0; w < kResidentWaves; ++w) na += s_sq[w];
@@ -2099,6 +2172,13 @@ __global__ __launch_bounds__(512) void k_train_small_u8_resident(const float *__
     }
     if (tid < 2 * KS)
         *(v4i *)(Pa_next + ((((size_t)(n >> 5) * KS) * 64 + (n & 31)) << 4) + (size_t)(tid >> 1) * 1024 + (tid & 1) * 512) = s_op[tid];
+    if constexpr (ALONE) {
+        const v4i lo = s_op[lane], hi = s_op[64 + lane];
+        na = 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) na = __builtin_amdgcn_sdot4(hi[r], hi[r], __builtin_amdgcn_sdot4(lo[r], lo[r], na, false), false);
+        na = wave_sum_i32_dpp(na);
+    }
     if (tid == 0) a.na_next[n] = (long long)na;
 }
 
@@ -3141,12 +3221,14 @@ int resident_launched(pink_hip_ctx *ctx, const float *dev_images, uint32_t image
     return PINK_HIP_OK;
 }
 
-// (elements of a neuron per thread, k-steps per wave in one batch, variant elements per thread in registers)
-decltype(&k_train_small_u8_resident<2, 4, 4>) small_resident_kernel(const pink_hip_ctx *ctx)
+// (us per image, eight waves | one, 64 neurons: 784 elements 8 variants 1.83 | 1.48, 32 variants 2.98 | 1.71; 1024 elements 32 variants 3.80 | 2.25;
+// 2025 elements 8 variants 2.44 | 2.15)
+decltype(&k_train_small_u8_resident<2, 1, 8>) small_resident_kernel(const pink_hip_ctx *ctx)
 {
-    const uint32_t nstored = std::min(2 * std::max(ctx->nrr, 1u), ctx->R);
-    if (ctx->S <= 1024 && (size_t)nstored * ctx->S <= 4 * kResidentThreads) return k_train_small_u8_resident<2, 4, 4>;
-    return ctx->S <= 1024 ? k_train_small_u8_resident<2, 4, 8> : k_train_small_u8_resident<4, 8, 8>;
+    const uint32_t steps = (ctx->gKS + 1) / 2;
+    if (ctx->S > 1024) return ctx->R <= 16 ? k_train_small_u8_resident<4, 1, 32> : k_train_small_u8_resident<4, 0, 8>;
+    if (ctx->R > 16) return steps <= 8 ? k_train_small_u8_resident<2, 2, 8> : steps <= 13 ? k_train_small_u8_resident<2, 2, 13> : k_train_small_u8_resident<2, 2, 16>;
+    return steps <= 8 ? k_train_small_u8_resident<2, 1, 8> : steps <= 13 ? k_train_small_u8_resident<2, 1, 13> : k_train_small_u8_resident<2, 1, 16>;
 }
 
 // The first `images` images of the current group in one resident launch (small uint8 trainers), queued: whether every
@@ -3168,7 +3250,6 @@ int run_train_small_resident(pink_hip_ctx *ctx, const float *dev_images, uint32_
     a.error = ctx->d_resident_error;
     a.launch = (uint32_t)ctx->resident_queued.size() + 1;
     a.N = ctx->N; a.S = ctx->S; a.R = ctx->R; a.KS = ctx->gKS;
-    a.nstored = std::min(2 * std::max(ctx->nrr, 1u), ctx->R);
     a.images = images; a.tag0 = ctx->exchange_tag; a.spin_limit = ctx->spin_limit;
     a.rot_stride = ctx->R * ctx->S;
     a.pb_stride = (ctx->Rp / 32) * ctx->gKS * 64;
@@ -3177,11 +3258,10 @@ int run_train_small_resident(pink_hip_ctx *ctx, const float *dev_images, uint32_
     ctx->exchange_tag += images;
     const v4i *pa = cur_gPa(ctx);
     signed char *pa_next = (signed char *)(ctx->pa_cur ? ctx->d_gPa : ctx->d_gPa_alt);
-    const size_t lds = (size_t)2 * a.nstored * ctx->S * sizeof(float);
     {
         Timed t(ctx, kClsUpdate);
         TRY(launch_resident(ctx, ctx->N, [&] {
-            hipLaunchKernelGGL(small_resident_kernel(ctx), dim3(ctx->N), dim3(kResidentThreads), lds, ctx->stream, ctx->d_som,
+            hipLaunchKernelGGL(small_resident_kernel(ctx), dim3(ctx->N), dim3(kResidentThreads), 0, ctx->stream, ctx->d_som,
                                ctx->d_som_alt, ctx->d_rot, pa, pa_next, ctx->d_gPb, ctx->d_factors, ctx->d_src4, ctx->d_kbyte, a);
             return launch_check(ctx, "k_train_small_u8_resident");
         }));
@@ -5020,7 +5100,7 @@ int init_ctx(pink_hip_ctx *ctx)
             ctx->resident_train = ctx->N <= (uint32_t)ctx->num_cu && resident_allowed();
             if (ctx->resident_train) {
                 HIP_TRY(ctx, hipFuncSetAttribute((const void *)small_resident_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
-                TRY(init_exchange(ctx, kSlotWords, (const void *)small_resident_kernel(ctx), kResidentThreads, (size_t)2 * nstored * ctx->S * sizeof(float)));
+                TRY(init_exchange(ctx, kSlotWords, (const void *)small_resident_kernel(ctx), kResidentThreads, 0));
             }
         }
         if (one_to_one && !ctx->small_train && !ctx->f32gemm) TRY(init_sym_train(ctx, region));

@@ -649,6 +649,13 @@ SMALL_UINT8_SHAPES = [s for s in FUSED_TRAIN_SHAPES if s[8] == capi.UINT8 and s[
     (64, 1, 28, 28, 4, True, 28, capi.QUADRATIC, capi.UINT8, 40),     # the 8 x 8 MNIST-sized trainer of the benchmark set
     (1, 1, 16, 16, 4, True, 12, capi.QUADRATIC, capi.UINT8, 9),       # one neuron: an exchange with itself
     (64, 1, 45, 45, 4, False, 45, capi.QUADRATIC, capi.UINT8, 6),     # 2025 elements: four per thread, 64 k-steps
+    (9, 1, 32, 32, 4, True, 31, capi.QUADRATIC, capi.UINT8, 6),       # 961: sixteen 64-byte k-steps of a tile
+    (5, 1, 22, 22, 16, True, 22, capi.CIRCULAR, capi.UINT8, 6),       # two tiles: six,
+    (5, 1, 29, 28, 16, True, 27, capi.QUADRATIC, capi.UINT8, 6),      # twelve,
+    (5, 1, 32, 32, 16, True, 32, capi.QUADRATIC, capi.UINT8, 6),      # sixteen
+    (4, 1, 20, 20, 20, False, 19, capi.QUADRATIC, capi.UINT8, 6),     # the second with four rows
+    (3, 1, 33, 33, 4, True, 33, capi.QUADRATIC, capi.UINT8, 5),       # 1089 elements: one tile
+    (4, 1, 36, 36, 12, True, 36, capi.QUADRATIC, capi.UINT8, 5),      # 1296 and two tiles: eight waves
 ]
 
 
