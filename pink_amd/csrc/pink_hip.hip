@@ -2542,7 +2542,7 @@ struct pink_hip_ctx {
     unsigned long long *d_sym_keys = nullptr;
     OrbitTrainPlan sym_plan;
     uint32_t *d_sym_element = nullptr, *d_sym_sel = nullptr;
-    uint32_t orb_table_groups = 0;                          // of the samples' table, per row block
+    uint32_t orb_table_groups[2] = {0, 0}, orb_few = 0;     // of the samples' table, per row block; images up to which there is another one
     uint32_t sym_orbits = 0, sym_reached = 0, sym_npb = 1, sym_nit = 0, sym_B = 0, sym_KS = 0, sym_RT = 0, sym_all = 0, sym_cells = 0, sym_outside = 0, sym_tag0 = 1;
     size_t sym_lds = 0, sym_prep_lds = 0;
     uint32_t *d_sym_upos = nullptr, *d_sym_outside = nullptr, *d_sym_best = nullptr;
@@ -2560,11 +2560,12 @@ struct pink_hip_ctx {
     int orb_mode = 0;
     uint32_t orb_KS = 0, orb_all = 0, orb_ns = 8, orb_valid = 0;
     size_t orb_prep_lds = 0;
+    uint32_t orb_lo = 0, orb_size = 0;                      // the rows and columns of an image that its preparation keeps in the LDS
     uint32_t sum_images = 0;               // float32: launches of at most so many images sum every variant (summed_images)
     uint32_t orb_rl = 0, orb_Ox = 0;       // (float32) orbits, a multiple of 16
     char *d_orb_tables = nullptr;          // ... the tables below that init_orbit makes on the host
-    uint32_t *d_orb_elem = nullptr, *d_orb_sel = nullptr, *d_orb_index = nullptr;
-    float2 *d_orb_frac = nullptr;
+    uint32_t *d_orb_elem = nullptr, *d_orb_sel = nullptr, *d_orb_index[2] = {nullptr, nullptr};
+    float2 *d_orb_frac[2] = {nullptr, nullptr};
     unsigned short *d_orb_place = nullptr;
     float *d_coef_weight = nullptr;        // (float32, coef_gemm.inc)
     unsigned char *d_coef_outside = nullptr;
@@ -3300,31 +3301,36 @@ const void *sym_kernel(const pink_hip_ctx *ctx)
 // Items of k_f32_rescue per image and neuron: as many as find a compute unit.
 uint32_t f32_rescue_parts(const pink_hip_ctx *ctx) { return std::max(1u, (uint32_t)ctx->num_cu / ctx->N); }
 
-template <int MODE>
-const void *orbit_prepare_for(bool tile, bool x)
+template <int MODE, bool TILE>
+const void *orbit_prepare_for(bool x, bool all)
 {
-    if (x) return tile ? (const void *)k_orbit_prepare<MODE, true, true> : (const void *)k_orbit_prepare<MODE, false, true>;
-    return tile ? (const void *)k_orbit_prepare<MODE, true, false> : (const void *)k_orbit_prepare<MODE, false, false>;
+    if (x) return all ? (const void *)k_orbit_prepare<MODE, TILE, true, true> : (const void *)k_orbit_prepare<MODE, TILE, true, false>;
+    return all ? (const void *)k_orbit_prepare<MODE, TILE, false, true> : (const void *)k_orbit_prepare<MODE, TILE, false, false>;
 }
-const void *orbit_prepare_kernel(const pink_hip_ctx *ctx)
+const void *orbit_prepare_kernel(const pink_hip_ctx *ctx, bool all)
+{
+    const bool tile = ctx->orb_prep_lds != 0, x = ctx->trainer;
+    if (ctx->orb_mode == ORB_U8) return tile ? orbit_prepare_for<ORB_U8, true>(x, all) : orbit_prepare_for<ORB_U8, false>(x, all);
+    return tile ? orbit_prepare_for<ORB_U16, true>(x, all) : orbit_prepare_for<ORB_U16, false>(x, all);
+}
+const void *coef_prepare_kernel(const pink_hip_ctx *ctx)
 {
     const bool tile = ctx->orb_prep_lds != 0;
-    switch (ctx->orb_mode) {
-    case ORB_U8: return orbit_prepare_for<ORB_U8>(tile, ctx->trainer);
-    case ORB_U16: return orbit_prepare_for<ORB_U16>(tile, ctx->trainer);
-    default:
-        if (ctx->trainer) return tile ? (const void *)k_coef_prepare<true, false> : (const void *)k_coef_prepare<false, false>;
-        return tile ? (const void *)k_coef_prepare<true, true> : (const void *)k_coef_prepare<false, true>;
-    }
+    if (ctx->trainer) return tile ? (const void *)k_coef_prepare<true, false> : (const void *)k_coef_prepare<false, false>;
+    return tile ? (const void *)k_coef_prepare<true, true> : (const void *)k_coef_prepare<false, true>;
 }
 
 int launch_orbit_prepare(pink_hip_ctx *ctx, OrbitPrep &p, uint32_t images)
 {
-    p.table_groups = ctx->orb_table_groups;
+    // A mapper's images that would have blocks for less than half of the chip: four base rotations a wave, not 16 (us per call of 2, 8, 40 and 200
+    // images, 90 rotations of 4480 uint16 elements: 62 | 78, 93 | 106, 273 | 261, 1270 | 1210)
+    const int few = images <= ctx->orb_few ? 1 : 0;
+    p.index = ctx->d_orb_index[few]; p.frac = ctx->d_orb_frac[few]; p.table_groups = ctx->orb_table_groups[few]; p.rl = few ? 2u : ctx->orb_rl;
+    p.lo = ctx->orb_lo; p.size = ctx->orb_size;
     const dim3 grid(images, (ctx->nrr_eff + (1u << p.rl) - 1) >> p.rl);
     const uint32_t threads = ctx->orb_prep_lds > 64 * 1024 || grid.x * grid.y < (uint32_t)ctx->num_cu ? 1024 : ctx->orb_prep_lds > 24 * 1024 ? 512 : 256;
     void *args[] = {&p};
-    HIP_TRY(ctx, hipLaunchKernel(orbit_prepare_kernel(ctx), grid, dim3(threads), args, ctx->orb_prep_lds, ctx->stream));
+    HIP_TRY(ctx, hipLaunchKernel(orbit_prepare_kernel(ctx, p.all_sym), grid, dim3(threads), args, ctx->orb_prep_lds, ctx->stream));
     return PINK_HIP_OK;
 }
 
@@ -3350,10 +3356,10 @@ int run_sym_train(pink_hip_ctx *ctx, const float *dev_images, uint32_t images, u
             TRY(launch_check(ctx, "k_f32_prepare"));
         } else {
             OrbitPrep p{};
-            p.images = dev_images; p.index = ctx->d_orb_index; p.frac = ctx->d_orb_frac; p.mask = ctx->d_sym_mask;
+            p.pixels = dev_images; p.mask = ctx->d_sym_mask;
             p.opnd = ctx->d_sym_op; p.norm = ctx->d_sym_norm; p.xrows = ctx->d_sym_x; p.most = ctx->d_most;
             p.plane = (size_t)images * ctx->sym_RT * ctx->sym_KS * 64; p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.KS = 2 * ctx->sym_KS;
-            p.all_sym = ctx->sym_all; p.rl = ctx->orb_rl; p.pitch = p.norm_pitch = ctx->sym_RT * 16; p.tl = 4;
+            p.all_sym = ctx->sym_all; p.pitch = p.norm_pitch = ctx->sym_RT * 16; p.tl = 4;
             TRY(launch_orbit_prepare(ctx, p, images));
         }
     }
@@ -3569,7 +3575,7 @@ int free_all(pink_hip_ctx *ctx)
                     ctx->d_somP, ctx->d_somP_alt, ctx->d_bmu_group, ctx->d_rotT, ctx->d_bmu_scratch, ctx->d_dist, ctx->d_ssd, ctx->d_best,
                     ctx->d_Pa, ctx->d_Pb, ctx->d_na, ctx->d_nb, ctx->d_poff, ctx->d_need, ctx->d_inv,
                     ctx->d_upos, ctx->d_aoff, ctx->d_kmask, ctx->d_gPa, ctx->d_gPa_alt, ctx->d_som_alt, ctx->d_slots, ctx->d_resident_error, ctx->d_src4, ctx->d_kbyte, ctx->d_gPb, ctx->d_gna, ctx->d_gnb, ctx->d_rtab, ctx->d_symoff, ctx->d_sym_upos, ctx->d_sym_element, ctx->d_sym_sel, ctx->d_sym_elem, ctx->d_sym_outside, ctx->d_sym_best, ctx->d_sym_at, ctx->d_sym_mask, ctx->d_sym_op, ctx->d_sym_x, ctx->d_sym_norm, ctx->d_grow, ctx->d_gvariant, ctx->d_region4,
-                    ctx->d_orb_tables, ctx->d_orb_outside, ctx->d_orb_best, ctx->d_most, ctx->d_orb_index, ctx->d_orb_frac, ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
+                    ctx->d_orb_tables, ctx->d_orb_outside, ctx->d_orb_best, ctx->d_most, ctx->d_orb_index[0], ctx->d_orb_index[1], ctx->d_orb_frac[0], ctx->d_orb_frac[1], ctx->d_orb_x, ctx->d_orb_values, ctx->d_orb_part, ctx->d_orb_som, ctx->d_orb_rows, ctx->d_orb_na, ctx->d_orb_nb,
                     ctx->d_screen_list, ctx->d_screen_wide, ctx->d_screen_counts, ctx->d_screen_choice, ctx->d_screen_bound, ctx->d_screen_moves, ctx->d_screen_range, ctx->d_coef_neuron, ctx->d_coef_image, ctx->d_coef_row, ctx->d_coef_words, ctx->d_coef_upper, ctx->d_sym_keys, ctx->d_sym_rescue, ctx->d_sym_err, ctx->d_sym_image, ctx->d_sym_run, ctx->d_sym_to, ctx->d_sym_from, ctx->d_sym_turned, ctx->d_sym_state, ctx->d_sym_norm_off};
     for (void *p : bufs) if (p) (void)hipFree(p);
     for (void *p : {(void *)ctx->st_img, (void *)ctx->st_heat, (void *)ctx->st_best, (void *)ctx->st_bmu}) if (p) (void)hipFree(p);
@@ -3798,8 +3804,9 @@ OrbitTrainPlan plan_orbit_train(uint32_t N, uint32_t E, uint32_t orbits, uint32_
     return best;
 }
 
-int orbit_samples(pink_hip_ctx *ctx, const uint32_t *d_upos, uint32_t Kp, uint32_t images);
+int orbit_samples(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, const uint32_t *d_upos, uint32_t Kp, uint32_t images, bool all);
 int finish_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, const std::vector<uint32_t> &upos, const std::vector<unsigned char> &mask);
+void add_partly(std::vector<unsigned char> &mask, uint32_t Kp);
 
 // Integer trainers whose neurons fit the blocks of a resident launch: the resident form with the symmetries on the SOM side (orbit_train.inc).
 // (region: distinct elements, in the CPU's order.)
@@ -3851,6 +3858,7 @@ int init_orbit_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     TRY(upload(ctx, &ctx->d_sym_sel, sel));
     const void *rescue = u16 ? (const void *)k_orbit_rescue<true> : (const void *)k_orbit_rescue<false>;
     HIP_TRY(ctx, hipFuncSetAttribute(rescue, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 2048));
+    add_partly(mask, Kp);
     return finish_sym_train(ctx, region, upos, mask);
 }
 
@@ -4008,7 +4016,7 @@ int finish_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, con
         HIP_TRY(ctx, hipFuncSetAttribute((const void *)k_f32_prepare<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_max - 2048));
     } else {
         ctx->orb_mode = u16 ? ORB_U16 : ORB_U8;
-        if (!ctx->orbit_train) TRY(orbit_samples(ctx, ctx->d_sym_upos, Kp, (uint32_t)b));        // (else init_orbit's: the same places)
+        if (!ctx->orbit_train) TRY(orbit_samples(ctx, region, ctx->d_sym_upos, Kp, (uint32_t)b, ctx->sym_all));        // (else init_orbit's: the same places)
     }
     TRY(dev_alloc(ctx, &ctx->d_sym_op, b * op_image / 16));
     TRY(dev_alloc(ctx, &ctx->d_sym_x, b * ctx->nrr_eff * Kp + 64));       // (a chunk of 64 orbits may read past the last)
@@ -4035,35 +4043,63 @@ int finish_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, con
     return PINK_HIP_OK;
 }
 
+// Behind the masks of the eight symmetries (see k_orbit_prepare): the pieces of 16 places in which they differ.
+void add_partly(std::vector<unsigned char> &mask, uint32_t Kp)
+{
+    for (uint32_t piece = 0; piece < Kp / 16; ++piece) {
+        unsigned char differ = 0;
+        for (uint32_t s = 1; s < 8; ++s)
+            for (uint32_t k = piece * 16; k < piece * 16 + 16; ++k) differ |= mask[(size_t)s * Kp + k] ^ mask[k];
+        mask.push_back(differ);
+    }
+}
+
 // Where the samples of the base rotations lie, for rows of Kp places (d_upos).
-int orbit_samples(pink_hip_ctx *ctx, const uint32_t *d_upos, uint32_t Kp, uint32_t images)
+int orbit_samples(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, const uint32_t *d_upos, uint32_t Kp, uint32_t images, bool all)
 {
     const bool f32 = ctx->orb_mode == ORB_F32;
-    const size_t image_lds = (size_t)ctx->C * orbit_tile(ctx->I) * sizeof(float);
+    // the rows and columns of the image that samples lie in: as far from its middle as the region's elements from the neuron's, and a pixel and
+    // a half for the crop's shift and the roundings of a rotation
+    double far = 0.0;
+    for (uint32_t off : region) {
+        const double x = (off % (ctx->D * ctx->D)) / ctx->D - (ctx->D - 1) * 0.5, y = off % ctx->D - (ctx->D - 1) * 0.5;
+        far = std::max(far, x * x + y * y);
+    }
+    const double middle = (ctx->I - 1) * 0.5, reach = std::sqrt(far) + 1.5;
+    ctx->orb_lo = f32 ? 0u : (uint32_t)std::max(0.0, std::floor(middle - reach));
+    ctx->orb_size = f32 ? ctx->I + 1 : (uint32_t)std::min<double>(ctx->I, std::ceil(middle + reach) + 1.0) - ctx->orb_lo + 1;
+    const uint32_t stride = f32 ? orbit_stride(ctx->I) : ctx->orb_size | 1u;
+    const size_t image_lds = (size_t)ctx->C * ctx->orb_size * stride * sizeof(float);
     ctx->orb_prep_lds = image_lds <= 120 * 1024 ? image_lds : 0;
     if (ctx->orb_prep_lds)
-        HIP_TRY(ctx, hipFuncSetAttribute(orbit_prepare_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024));
+        HIP_TRY(ctx, hipFuncSetAttribute(f32 ? coef_prepare_kernel(ctx) : orbit_prepare_kernel(ctx, all), hipFuncAttributeMaxDynamicSharedMemorySize, 120 * 1024));
+    else
+        ctx->orb_lo = 0;
     // as many base rotations per wave as there are, up to 16; two where the image comes out of memory: a wave's pixels are neighbours
-    // then; four for a trainer's few images of long rows, which have blocks for a part of the chip (us per image, 4 | 8 | 16 rotations:
-    // 30 images of 25 rows of 42440 elements 3.6 | 6.2 | -, 12 of 90 rows of 33488 14.5 | 12.8 | 23.6; groups of 67 images of 4480 elements
-    // 2.0 | 1.7 | 1.5, of 167 of 2304 0.63 | 0.53 | 0.52)
+    // then; eight for a trainer, whose rows' float values leave in 64 bytes in a row so, four for its few images of long rows, which have
+    // blocks for a part of the chip (us per launch, 4 | 8 | 16 rotations: 67 images of 90 rows of 2304 elements 54 | 49 | 54, uint16 of 4480
+    // 73 | 65 | 75, 30 of 25 rows of 42440 74 | 133 | -; a mapper's 150 of 4480 119 | 107 | 94)
     const auto row_blocks = [&](uint32_t rl) { return (ctx->nrr_eff + (1u << rl) - 1) >> rl; };
-    const uint32_t most = !ctx->orb_prep_lds ? 1u : ctx->trainer && Kp >= 4096 && images * row_blocks(4) < (uint32_t)ctx->num_cu / 2 ? 2u : 4u;
+    const uint32_t most = !ctx->orb_prep_lds ? 1u : !ctx->trainer ? 4u : Kp >= 4096 && images * row_blocks(3) < (uint32_t)ctx->num_cu / 2 ? 2u : 3u;
     ctx->orb_rl = 0;
     while (ctx->orb_rl < most && row_blocks(ctx->orb_rl) > 1) ++ctx->orb_rl;
-    const uint32_t blocks = row_blocks(ctx->orb_rl), groups = orbit_piece_groups(Kp / 16, ctx->orb_rl);
-    ctx->orb_table_groups = groups;
-    const uint32_t tiles = (ctx->nrr_eff + 15) / 16;
-    const size_t entries = f32 ? (size_t)tiles * Kp * 16 : (size_t)blocks * groups * 1024;
-    TRY(dev_alloc(ctx, &ctx->d_orb_index, entries));
-    TRY(dev_alloc(ctx, &ctx->d_orb_frac, entries));
-    OrbitTable t{};
-    t.cos_t = ctx->d_cos; t.sin_t = ctx->d_sin; t.upos = d_upos; t.index = ctx->d_orb_index; t.frac = ctx->d_orb_frac;
-    t.stride = ctx->orb_prep_lds ? orbit_stride(ctx->I) : ctx->I;
-    t.channel = ctx->orb_prep_lds ? orbit_tile(ctx->I) : ctx->I * ctx->I;
-    t.I = ctx->I; t.D = ctx->D; t.nrr = ctx->nrr_eff; t.pieces = Kp / 16; t.rl = ctx->orb_rl;
-    if (f32) hipLaunchKernelGGL(k_coef_table, dim3((uint32_t)(entries / 256)), dim3(256), 0, ctx->stream, t, Kp / 512);
-    else hipLaunchKernelGGL(k_orbit_table, dim3((groups * 1024 + 255) / 256, blocks), dim3(256), 0, ctx->stream, t);
+    // (a mapper's calls with few images: a table of their own; see launch_orbit_prepare)
+    ctx->orb_few = !f32 && !ctx->trainer && ctx->orb_rl > 2 ? ctx->num_cu / (2 * row_blocks(ctx->orb_rl)) : 0;
+    for (int few = 0; few < (ctx->orb_few ? 2 : 1); ++few) {
+        const uint32_t rl = few ? 2u : ctx->orb_rl, blocks = row_blocks(rl), groups = orbit_piece_groups(Kp / 16, rl), tiles = (ctx->nrr_eff + 15) / 16;
+        const size_t entries = f32 ? (size_t)tiles * Kp * 16 : (size_t)blocks * groups * 1024;
+        TRY(dev_alloc(ctx, &ctx->d_orb_index[few], entries));
+        TRY(dev_alloc(ctx, &ctx->d_orb_frac[few], entries));
+        ctx->orb_table_groups[few] = groups;
+        OrbitTable t{};
+        t.cos_t = ctx->d_cos; t.sin_t = ctx->d_sin; t.upos = d_upos; t.index = ctx->d_orb_index[few]; t.frac = ctx->d_orb_frac[few];
+        t.stride = ctx->orb_prep_lds ? stride : ctx->I;
+        t.channel = ctx->orb_prep_lds ? ctx->orb_size * stride : ctx->I * ctx->I;
+        t.lo = ctx->orb_lo; t.x = !f32 && ctx->trainer;
+        t.I = ctx->I; t.D = ctx->D; t.nrr = ctx->nrr_eff; t.pieces = Kp / 16; t.rl = rl;
+        if (f32) hipLaunchKernelGGL(k_coef_table, dim3((uint32_t)(entries / 256)), dim3(256), 0, ctx->stream, t, Kp / 512);
+        else hipLaunchKernelGGL(k_orbit_table, dim3((groups * 1024 + 255) / 256, blocks), dim3(256), 0, ctx->stream, t);
+    }
     return launch_check(ctx, "k_orbit_table");
 }
 
@@ -4150,6 +4186,7 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     tables.add(&ctx->d_orb_elem, elem);
     tables.add(&d_upos, upos);
     tables.add(&ctx->d_orb_sel, sel);
+    if (!f32) add_partly(mask, Kp);
     tables.add(&ctx->d_orb_mask, mask.data(), mask.size());
     const uint32_t planes = ctx->orb_mode == ORB_U8 ? 1 : 2;
     TRY(dev_alloc(ctx, &ctx->d_orb_som, (size_t)planes * ctx->N * Kp / 16));
@@ -4183,7 +4220,7 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
         }
     }
     TRY(tables.commit(ctx, &ctx->d_orb_tables));
-    TRY(orbit_samples(ctx, d_upos, Kp, 1));
+    TRY(orbit_samples(ctx, region, d_upos, Kp, 1, ctx->orb_all));
     ctx->orb_pitch = ctx->trainer ? round_up(ctx->nrr_eff, f32 ? 16 : 32) : ctx->nrr_eff;
     ctx->screen_train = ctx->trainer && f32;
     ctx->orbit = !ctx->screen_train;
@@ -4358,7 +4395,7 @@ int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
     Timed t(ctx, kClsRotate);
     if (ctx->orb_mode == ORB_F32) {
         CoefPrep p{};
-        p.images = dev_images; p.index = ctx->d_orb_index; p.frac = ctx->d_orb_frac; p.weight = ctx->d_coef_weight; p.outside = ctx->d_coef_outside;
+        p.images = dev_images; p.index = ctx->d_orb_index[0]; p.frac = ctx->d_orb_frac[0]; p.weight = ctx->d_coef_weight; p.outside = ctx->d_coef_outside;
         p.opnd = (uint32_t *)ctx->d_orb_rows; p.row = (CoefRow *)ctx->d_coef_row; p.image = (CoefImage *)ctx->d_coef_image; p.xrows = ctx->d_orb_x;
         if (!ctx->trainer) { p.wide_count = ctx->d_screen_counts + 1; p.list_count = ctx->d_screen_counts; p.upper = ctx->d_coef_upper; }
         p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.Op = ctx->orb_KS * 4; p.Ox = ctx->orb_Ox; p.all_sym = ctx->orb_all; p.pitch = ctx->orb_pitch;
@@ -4370,7 +4407,7 @@ int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
         if (large) p.tiles = std::min(p.tiles, (2 * coef_prepare_waves(true) + quarters - 1) / quarters);
         const uint32_t waves = std::min(large || B * tiles < 2 * (uint32_t)ctx->num_cu ? coef_prepare_waves(ctx->orb_prep_lds != 0) : 4u, quarters * p.tiles);
         void *args[] = {&p};
-        HIP_TRY(ctx, hipLaunchKernel(orbit_prepare_kernel(ctx), dim3(B, (tiles + p.tiles - 1) / p.tiles), dim3(64 * waves), args, ctx->orb_prep_lds, ctx->stream));
+        HIP_TRY(ctx, hipLaunchKernel(coef_prepare_kernel(ctx), dim3(B, (tiles + p.tiles - 1) / p.tiles), dim3(64 * waves), args, ctx->orb_prep_lds, ctx->stream));
         if (ctx->coef_beside) {
             const CoefBeside e{ctx->d_orb_x, ctx->d_coef_beside, p.row, ctx->coef_beside, B * ctx->nrr_eff, p.Ox * 8};
             hipLaunchKernelGGL(k_coef_beside, dim3((e.rows + 3) / 4), dim3(256), 0, ctx->stream, e);
@@ -4379,10 +4416,10 @@ int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
         return PINK_HIP_OK;
     }
     OrbitPrep p{};
-    p.images = dev_images; p.index = ctx->d_orb_index; p.frac = ctx->d_orb_frac; p.mask = ctx->d_orb_mask;
+    p.pixels = dev_images; p.mask = ctx->d_orb_mask;
     p.opnd = ctx->d_orb_rows; p.norm = ctx->d_orb_nb; p.key = ctx->d_key;
     p.xrows = ctx->d_orb_x; p.plane = orbit_rows_plane(ctx, B); p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.KS = ctx->orb_KS;
-    p.all_sym = ctx->orb_all; p.rl = ctx->orb_rl; p.pitch = ctx->orb_pitch; p.most = ctx->d_most; p.norm_pitch = ctx->nrr_eff; p.tl = 5;
+    p.all_sym = ctx->orb_all; p.pitch = ctx->orb_pitch; p.most = ctx->d_most; p.norm_pitch = ctx->nrr_eff; p.tl = 5;
     return launch_orbit_prepare(ctx, p, B);
 }
 

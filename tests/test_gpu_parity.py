@@ -380,6 +380,9 @@ ORBIT_MAP_SHAPES = [
     (3, 1, 180, 254, 8, True, 181, capi.QUADRATIC, capi.UINT8, 1, "noise"),   # an image beyond the LDS, k in splits
     (90, 1, 16, 12, 360, True, 8, capi.QUADRATIC, capi.UINT16, 300, "noise"), # the large tiles
     (340, 1, 70, 64, 360, True, 60, capi.CIRCULAR, capi.UINT8, 4, "noise"),
+    (4, 1, 1, 6, 12, True, 5, capi.QUADRATIC, capi.UINT16, 3, "noise"),       # an image of a pixel
+    (6, 2, 61, 40, 68, True, 25, capi.QUADRATIC, capi.UINT16, 5, "noise"),    # a window of the image; pieces partly outside the region
+    (5, 1, 250, 64, 40, False, 37, capi.CIRCULAR, capi.UINT8, 4, "noise"),    # ... of an image beyond the LDS
     (9, 1, 24, 18, 128, True, 13, capi.QUADRATIC, capi.FLOAT, 5, "noise"),    # 13 rows and columns: bands and patches cut short
     (6, 3, 20, 15, 360, False, 9, capi.QUADRATIC, capi.FLOAT, 3, "noise"),
     (37, 1, 30, 30, 456, True, 30, capi.CIRCULAR, capi.FLOAT, 6, "noise"),    # 114 rows: more than the kept ones
@@ -789,6 +792,9 @@ RESIDENT_INTEGER_PLANS = [
     (9, 1, 64, 200, 48, True, 180, capi.QUADRATIC, capi.UINT16, 2),
     (3, 1, 40, 190, 16, True, 186, capi.QUADRATIC, capi.UINT16, 2),      # all of them: their squares pass 2^31
     (60, 1, 100, 140, 36, True, 130, capi.QUADRATIC, capi.UINT8, 2),     # 34 chunks, 31 reached
+    (8, 2, 61, 40, 68, True, 25, capi.QUADRATIC, capi.UINT16, 3),        # a window of the image; a region that symmetries move by a pixel
+    (8, 1, 5, 9, 12, True, 8, capi.QUADRATIC, capi.UINT8, 3),            # an image smaller than its window; one piece of most rows
+    (8, 1, 200, 64, 40, False, 37, capi.CIRCULAR, capi.UINT8, 3),
 ]
 
 
@@ -1205,6 +1211,8 @@ ORBIT_TRAIN_SHAPES = [
     (4, 2, 64, 90, 132, True, 70, capi.QUADRATIC, capi.UINT8, 3),      # two channels
     (1030, 1, 40, 36, 48, True, 33, capi.QUADRATIC, capi.UINT16, 3),   # more neurons than the resident form takes
     (2, 1, 190, 120, 60, True, 110, capi.CIRCULAR, capi.UINT16, 3),    # an image beyond the LDS
+    (2, 1, 260, 200, 24, True, 190, capi.QUADRATIC, capi.UINT16, 2),   # ... and its window too
+    (1030, 1, 1, 3, 8, True, 3, capi.QUADRATIC, capi.UINT8, 2),        # an image of a pixel
 ]
 
 
