@@ -52,13 +52,13 @@ COUNTER_TRAFFIC_PER_IMAGE = {
     ("cfg1", "rotate"): ((96.042e6 + 207.618e6) / 2048, "profiles/cfg1_map_u8_counters.txt"),
     ("cfg1", "distance"): ((214.632e6 + 1.639e6) / 2048, "profiles/cfg1_map_u8_counters.txt"),
     # the resident launch of 64 images and the one that brings the elements outside the region up to date
-    ("cfg2", "update"): ((819.876e6 + 7.440e6 + 141.852e6 + 13.839e6) / 64, "profiles/cfg2_train_u16_counters.txt"),
+    ("cfg2", "update"): ((1143.018e6 + 11.723e6 + 159.882e6 + 13.821e6) / 64, "profiles/cfg2_train_u16_counters.txt"),
     # the product, the selection, the exact sums of variants and of neurons
     ("cfg3", "distance"): (32.666e6 + 9.216e6 + 9.440e6 + 0.140e6 + 210.795e6 + 0.308e6 + 0.039e6,
                            "profiles/cfg3_train_f32_3ch_counters.txt"),
     # the operand rows per image and a sixteenth of the launch that brings the neurons' full images up to date
     ("cfg3", "update"): (39.981e6 + 40.509e6 + (294.450e6 + 55.482e6 + 94.359e6 + 0.051e6) / 16, "profiles/cfg3_train_f32_3ch_counters.txt"),
-    ("cfg4", "update"): ((85.604e6 + 0.835e6) / 256, "profiles/cfg4_train_u8_counters.txt"),     # the resident launch of 256 images
+    ("cfg4", "update"): ((43.423e6 + 4.505e6) / 256, "profiles/cfg4_train_u8_counters.txt"),     # the resident launch of 256 images
 }
 
 # Images per step of the workloads that ride along in `all_configs` (the headline workload always
@@ -351,7 +351,7 @@ def run_workload(name, steps, warmup, n_images, kernel, cpu_budget_s, host_inclu
         elif dominant == "update" and times["distance"][0] == 0:
             notes = ("a small uint8 trainer: distances, best match and update of a whole group of images in one resident "
                      "launch (class 'update'), one block per neuron; per image the blocks exchange one 64-bit word each "
-                     "through memory (store, then polls: about 0.9 us) around about 1 us of lone-wave instruction issue; "
+                     "through memory (store, then polls: about 0.8 us) between one wave's product and the update; "
                      "bound by that chain, not by HBM: no roofline claimed")
     traffic = COUNTER_TRAFFIC_PER_IMAGE.get((name, dominant))
     roofline = {

@@ -770,11 +770,12 @@ def test_resident_symmetric_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, 
 RESIDENT_INTEGER_PLANS = [
     (90, 1, 40, 40, 360, True, 34, capi.QUADRATIC, capi.UINT8, 3),       # 2 x 3, two groups of waves
     (91, 1, 40, 40, 360, True, 35, capi.QUADRATIC, capi.UINT16, 3),      # the last block holds one neuron; an odd region in an even neuron
-    (130, 1, 30, 30, 360, True, 21, capi.QUADRATIC, capi.UINT8, 3),      # 2 x 1, three tiles to a wave
+    (130, 1, 30, 30, 360, True, 21, capi.QUADRATIC, capi.UINT8, 3),      # 1 x 1, two groups of waves, three tiles to a wave
     (331, 1, 60, 60, 240, True, 55, capi.CIRCULAR, capi.UINT16, 2),      # 2 x 1, four groups of waves
     (331, 1, 90, 80, 360, True, 75, capi.CIRCULAR, capi.UINT16, 2),      # 4 x 3: nine chunks of a neuron, up to six of a wave
-    (60, 2, 36, 36, 500, True, 24, capi.QUADRATIC, capi.UINT16, 3),      # 2 x 8, the most
-    (5, 1, 20, 20, 1000, True, 15, capi.QUADRATIC, capi.UINT16, 3),      # 2 x 8, two tiles each; 250 rotations are not whole tiles
+    (60, 2, 36, 36, 500, True, 24, capi.QUADRATIC, capi.UINT16, 3),      # 2 x 4
+    (5, 1, 20, 20, 1000, True, 15, capi.QUADRATIC, capi.UINT16, 3),      # 1 x 4, four tiles each; 250 rotations are not whole tiles
+    (4, 1, 24, 24, 2400, True, 19, capi.QUADRATIC, capi.UINT16, 2),      # 1 x 5, eight groups of waves
     (255, 1, 30, 30, 720, False, 20, capi.CIRCULAR, capi.UINT8, 3),      # twelve tiles, four groups of waves
     (10, 1, 100, 100, 200, True, 91, capi.QUADRATIC, capi.UINT8, 2),     # 1 x 4, seventeen chunks
     (12, 1, 100, 100, 80, False, 98, capi.QUADRATIC, capi.UINT16, 2),
