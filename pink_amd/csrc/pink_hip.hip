@@ -41,6 +41,7 @@
 
 #include "mfma_u8_sym.h"
 #include "pink_hip.h"
+#include "orbit_train_plan.h"
 #include "resident_use.h"
 
 // Scratch of pink_hip_map_device_static, the entry point for callers that cannot allocate: the
@@ -3761,49 +3762,6 @@ uint32_t orbit_train_reached(const pink_hip_ctx *ctx, const OrbitGrid &grid)
     return ctx->cfg.ed_type == PINK_HIP_UINT16 && ctx->E > 33025 ? all : std::min(all, round_up(std::max(1u, grid.reached), 64));
 }
 
-// How many neurons a block of a resident integer trainer holds and between how many blocks the rows are shared out: what is expected to
-// take least.  In clocks of an image: a block's rows through its CU's 64 bytes a clock, its waves' instructions or the matrix pipes; a round of
-// tiles, whose shares of k meet in the LDS; an update of 64 orbits a wave; the words of the blocks that hold the same neurons.  Fitted to
-// every plan of 40 shapes (8 to 1024 neurons of 128 to 10000 elements, 4 to 720 variants): off by 3.2 % in the mean, the plan taken 1.1 %
-// slower than the fastest in the mean and 4.9 % at most, where plans are up to four times apart.  npb 0: no way to hold the neurons.
-OrbitTrainPlan plan_orbit_train(uint32_t N, uint32_t E, uint32_t orbits, uint32_t reached, uint32_t nrr, bool u16, uint32_t units, size_t lds_max)
-{
-    const uint32_t RT = (nrr + 15) / 16, planes = u16 ? 2 : 1, accs = u16 ? 3 : 1, products = u16 ? 4 : 1;
-    const double most = (double)E * (u16 ? 65535.0 * 65535.0 : 255.0 * 255.0);
-    OrbitTrainPlan best;
-    double best_cost = 0.0;
-    for (uint32_t npb = 1; npb <= 4; ++npb) {
-        const uint32_t groups = (N + npb - 1) / npb, columns = npb > 2 ? 2 : 1, nit = (npb * ((orbits + 63) / 64) + kOrbTrainWorkers - 1) / kOrbTrainWorkers;
-        const uint32_t streamed = nit > kOrbTrainAllNit ? reached : orbits, KS = round_up((streamed * 8 + 63) / 64, 2);
-        if (nit > (npb > 2 ? kOrbTrainAllNit : kOrbTrainMaxNit) || most >= (double)(1ull << (48 - orbit_train_bits(npb)))) break;
-        uint32_t tiles_before = 0;
-        for (uint32_t splits = 1; splits <= std::min(kOrbTrainSplits, RT) && groups * splits <= units; ++splits) {
-            const uint32_t tiles = (RT + splits - 1) / splits;
-            if (tiles == tiles_before) continue;
-            // (more than six orbits a thread: rows that a compute unit takes longer to pull through than the orbits' product takes for an image,
-            // 15 us for three tiles of 33488 uint8 elements)
-            if (nit > kOrbTrainAllNit && tiles * KS * planes > 1600) continue;
-            tiles_before = tiles;
-            for (uint32_t abreast = 1; abreast <= 8; abreast *= 2)
-                for (uint32_t tpw = 1; tpw <= (u16 ? 1u : 3u); tpw += 2) {
-                    const size_t lds = orbit_train_lds(npb, orbits, streamed, u16, N, tpw);
-                    if (lds + 2048 > lds_max) continue;
-                    const uint32_t rounds = (tiles + abreast * tpw - 1) / (abreast * tpw), shares = kSymWaves / abreast;
-                    const double stream = rounds * abreast * tpw * 16.0 * KS * planes;
-                    const double issue = rounds * (KS / 2.0 / shares) * (columns * planes * 10.0 + tpw * planes * 4.0 + tpw * columns * products * 2.0 + 10.0) * 8.6;
-                    const double matrix = rounds * abreast * tpw * (double)columns * KS * products * 4.0;
-                    const double cost = 1.155 * std::max({stream, issue, matrix}) + rounds * (2850.0 + 110.0 * tpw * columns * accs + 10.0 * accs * shares * ((abreast * tpw * columns + 7) / 8)) +
-                                        nit * (u16 ? 2070.0 : 1594.0) + (npb - 1) * (u16 ? 100.0 : 200.0) + (splits > 1 ? 100.0 + 300.0 * splits : 0.0) + 150.0 * (abreast - 1) + 3.0 * groups * splits;
-                    if (!best.npb || cost < best_cost) {
-                        best.npb = npb; best.splits = splits; best.abreast = abreast; best.tpw = tpw; best.nit = nit; best.lds = lds; best.reached = streamed;
-                        best_cost = cost;
-                    }
-                }
-        }
-    }
-    return best;
-}
-
 int orbit_samples(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, const uint32_t *d_upos, uint32_t Kp, uint32_t images, bool all);
 int finish_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, const std::vector<uint32_t> &upos, const std::vector<unsigned char> &mask);
 void add_partly(std::vector<unsigned char> &mask, uint32_t Kp);
@@ -3824,7 +3782,7 @@ int init_orbit_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     ctx->sym_npb = ctx->sym_plan.npb;
     ctx->sym_lds = ctx->sym_plan.lds;
     ctx->sym_RT = (ctx->nrr_eff + 15) / 16;
-    ctx->sym_KS = round_up((ctx->sym_reached * 8 + 63) / 64, 2);
+    ctx->sym_KS = orbit_train_steps(ctx->sym_reached);
     const uint32_t Kp = ctx->sym_KS * 64, D = ctx->D, Ds = grid.Ds;
     std::vector<uint32_t> upos(Kp, ~0u), elem((size_t)ctx->sym_orbits * 8, ~0u), sel(16 + 64);
     std::vector<unsigned char> mask((size_t)8 * Kp, 0);
@@ -4005,10 +3963,8 @@ int finish_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, con
     TRY(upload(ctx, &ctx->d_sym_upos, upos));
     TRY(upload(ctx, &ctx->d_sym_outside, outside));
     TRY(upload(ctx, (unsigned char **)&ctx->d_sym_mask, mask));
-    // a group's operand and rows are written by one launch and read by the next: within the last-level cache
-    const size_t op_image = (size_t)(u16 ? 2 : 1) * ctx->sym_RT * ctx->sym_KS * 1024, x_image = (size_t)ctx->nrr_eff * Kp * sizeof(float);
-    size_t b = c.max_batch ? std::min<size_t>(c.max_batch, kSymGroupMax) : kSymGroupMax;
-    while (b > 8 && b * (op_image + x_image) > ((size_t)192 << 20)) --b;
+    const size_t op_image = orbit_train_operand(ctx->nrr_eff, ctx->sym_KS, u16), x_image = (size_t)ctx->nrr_eff * Kp * sizeof(float);
+    const size_t b = resident_group(c.max_batch, op_image, x_image);
     ctx->sym_B = (uint32_t)b;
     if (f32) {
         const size_t image_lds = (size_t)ctx->C * ctx->I * ctx->I * sizeof(float);

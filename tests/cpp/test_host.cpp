@@ -5,6 +5,7 @@
 // Usage: test_host args   -> argument validation only (no device needed)
 //        test_host gpu    -> everything
 #define PINK_HIP_STANDALONE
+#include "../../pink_amd/csrc/orbit_train_plan.h"
 #include "../../pink_amd/csrc/resident_use.h"
 #include "pink_hip_som.h"
 
@@ -42,6 +43,29 @@ static void test_arguments()
     EXPECT(!throws_pink([&] { Trainer2(som, f, 0, 720, false, 1.0, Interpolation::BILINEAR, 2); }));
     EXPECT(throws_pink([] { HexagonalLayout(HexagonalLayout::DimensionType{{4, 4}}); }));
     EXPECT(HexagonalLayout(HexagonalLayout::DimensionType{{21, 21}}).size() == 331);
+}
+
+// A resident integer trainer's group of images: its operand is counted in 32 bits, and what is not wanted of it is asked for 2^31 bytes
+// behind its start.  (Base rotations up to those of 65536 variants, orbits up to those that a block can hold.)
+static void test_resident_groups()
+{
+    int planned = 0;
+    for (bool u16 : {false, true})
+        for (uint32_t N : {1u, 4u, 100u})
+            for (uint32_t orbits : {136u, 2080u, 2688u, 4465u})
+                for (uint32_t nrr : {1u, 90u, 8191u, 12000u, 16384u})
+                    for (uint32_t max_batch : {0u, 3u, 256u}) {
+                        OrbitTrainPlan const p = plan_orbit_train(N, orbits * 8 - 64, orbits, orbits, nrr, u16, 256, 159 * 1024);
+                        if (!p.npb) continue;
+                        ++planned;
+                        uint32_t const KS = orbit_train_steps(p.reached);
+                        size_t const op = orbit_train_operand(nrr, KS, u16);
+                        uint32_t const b = resident_group(max_batch, op, (size_t)nrr * KS * 64 * sizeof(float));
+                        EXPECT(b >= 1 && b <= (max_batch ? max_batch : 256));
+                        EXPECT(b * op < kOrbTrainOperand);
+                        if (b < 8 && (!max_batch || b < max_batch)) EXPECT((b + 1) * op >= kOrbTrainOperand);
+                    }
+    EXPECT(planned > 200);
 }
 
 static void test_trainer()
@@ -151,6 +175,7 @@ int main(int argc, char** argv)
 {
     bool const gpu = argc > 1 and std::strcmp(argv[1], "gpu") == 0;
     test_arguments();
+    test_resident_groups();
     test_resident_rule();
     if (gpu) {
         test_trainer();
