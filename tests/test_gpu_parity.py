@@ -791,7 +791,7 @@ RESIDENT_INTEGER_PLANS = [
     (400, 1, 20, 60, 24, False, 49, capi.QUADRATIC, capi.UINT16, 2),
     (9, 1, 64, 200, 48, True, 181, capi.QUADRATIC, capi.UINT8, 2),       # ten chunks to a thread
     (9, 1, 64, 200, 48, True, 180, capi.QUADRATIC, capi.UINT16, 2),
-    (3, 1, 40, 190, 16, True, 186, capi.QUADRATIC, capi.UINT16, 2),      # all of them: their squares pass 2^31
+    (3, 1, 40, 190, 16, True, 186, capi.QUADRATIC, capi.UINT16, 2),      # all of them: saturated, their squares could pass 2^31
     (60, 1, 100, 140, 36, True, 130, capi.QUADRATIC, capi.UINT8, 2),     # 34 chunks, 31 reached
     (8, 2, 61, 40, 68, True, 25, capi.QUADRATIC, capi.UINT16, 3),        # a window of the image; a region that symmetries move by a pixel
     (8, 1, 5, 9, 12, True, 8, capi.QUADRATIC, capi.UINT8, 3),            # an image smaller than its window; one piece of most rows
@@ -804,6 +804,82 @@ RESIDENT_INTEGER_PLANS = [
 def test_resident_integer_trainer_plans(monkeypatch, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, form):
     """How the neurons and an image's rows are dealt to the blocks, at the edges of chunks, tiles, groups of waves and blocks."""
     test_resident_symmetric_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, form)
+
+
+def awkward(kind, rng, som, imgs):
+    """Values that the integer conversions send to the ends of their range, in images and in the weights of the middle of a neuron; in place."""
+    if kind == "outside":
+        som *= 4
+        som -= 1.5
+        imgs *= 4
+        imgs -= 1.5
+        return
+    for a in (som, imgs):
+        mid = a.shape[-1] // 2
+        for value in {"infinite": (np.inf, -np.inf), "nan": (np.nan, -np.nan), "saturated": ()}[kind]:
+            picked = rng.integers(0, a.shape[0], 2)
+            a[picked, ..., mid + rng.integers(-2, 3, 2), mid + rng.integers(-2, 3, 2)] = value
+    if kind == "saturated":                                            # (squares as large as they can be, but the closest neuron's)
+        som[1:] = 1.0 + 1e20 * som[1:]
+        som[0] = 0.9
+
+
+AWKWARD_INTEGER_TRAINERS = [(kind,) + shape for kind in ("outside", "infinite", "nan") for shape in (
+    (9, 1, 28, 28, 4, True, 28, capi.QUADRATIC, capi.UINT8, 6),        # eight symmetries, one wave multiplies
+    (20, 1, 24, 18, 40, True, 16, capi.QUADRATIC, capi.UINT8, 6),
+    (20, 1, 24, 18, 40, True, 16, capi.CIRCULAR, capi.UINT16, 6),
+    (300, 1, 16, 12, 68, True, 11, capi.QUADRATIC, capi.UINT16, 4),    # two neurons to a block
+    (9, 1, 64, 200, 48, True, 181, capi.QUADRATIC, capi.UINT8, 2),     # ten orbits a thread, places that no rotation reaches
+    (9, 1, 64, 200, 48, True, 180, capi.QUADRATIC, capi.UINT16, 2),
+)] + [("saturated",) + shape for shape in (
+    (3, 1, 40, 190, 16, True, 186, capi.QUADRATIC, capi.UINT8, 2),     # unreached squares up to 2.2e9 beside reached ones: past 2^31
+    (3, 1, 40, 190, 16, True, 181, capi.QUADRATIC, capi.UINT16, 2),    # ... up to 32 761 times 255^2 in each of three sums: just below it
+    (3, 1, 40, 190, 16, True, 186, capi.QUADRATIC, capi.UINT16, 2),    # they would pass it: all places are taken for reached
+)]
+
+
+@pytest.mark.parametrize("form", ["resident", "gives up", "off"])
+@pytest.mark.parametrize("kind,N,C_,I,D,nrot,flip,ed,shape_,ed_type,n", AWKWARD_INTEGER_TRAINERS)
+def test_integer_trainers_on_awkward_values(monkeypatch, kind, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, form):
+    """Values outside [0, 1], infinite ones and none at all quantise to the ends of the range (no number: 0) in every form of a trainer."""
+    say("awkward integer trainer", kind, form, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n)
+    if form == "gives up":
+        monkeypatch.setenv("PINK_HIP_RESIDENT_SPIN_LIMIT", "0")
+    if form == "off":
+        monkeypatch.setenv("PINK_HIP_RESIDENT_TRAINER", "0")
+    rng = np.random.default_rng(N + I + nrot)
+    som0, imgs = rng.random((N, C_, D, D), dtype=np.float32), rng.random((n, C_, I, I), dtype=np.float32)
+    awkward(kind, rng, som0, imgs)
+    som0 = som0.reshape(N, -1)
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 1.0, 0.5)
+    F[F < 0.01] = 0.0
+    want = som0.copy()
+    obmu = O.train(O.shape(N, C_, I, D, nrot, flip, ed, shape_, ed_type), want, imgs, F)
+    lost = np.isnan(want)
+    with capi.Context(N, C_, I, D, nrot, flip, ed, shape_, ed_type, F) as ctx:
+        ctx.set_som(som0)
+        bmu = np.concatenate([ctx.train(imgs[:1]), ctx.train(imgs[1:])])
+        som = ctx.get_som()
+    assert np.array_equal(bmu, obmu)
+    assert np.array_equal(np.isnan(som), lost) and np.array_equal(bits(som)[~lost], bits(want)[~lost])
+
+
+@pytest.mark.parametrize("kind", ["outside", "infinite", "nan"])
+@pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,shape_,ed_type,n", [
+    (20, 1, 24, 18, 40, True, 16, capi.QUADRATIC, capi.UINT16, 6),
+    (5, 1, 250, 64, 40, False, 37, capi.CIRCULAR, capi.UINT8, 4),      # uint8 beyond the other product's images,
+    (3, 1, 180, 254, 8, True, 181, capi.QUADRATIC, capi.UINT8, 3),     # ... and regions
+])
+def test_orbit_mappers_on_awkward_values(N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, kind):
+    say("awkward integer mapper", kind, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n)
+    rng = np.random.default_rng(N + I + nrot)
+    som, imgs = rng.random((N, C_, D, D), dtype=np.float32), rng.random((n, C_, I, I), dtype=np.float32)
+    awkward(kind, rng, som, imgs)
+    oheat, obest = O.map_images(O.shape(N, C_, I, D, nrot, flip, ed, shape_, ed_type), som, imgs)
+    with capi.Context(N, C_, I, D, nrot, flip, ed, shape_, ed_type) as ctx:
+        ctx.set_som(som.reshape(N, -1))
+        heat, best = ctx.map(imgs)
+    assert np.array_equal(bits(heat), bits(oheat)) and np.array_equal(best, obest)
 
 
 @pytest.mark.parametrize("kind", ["blank", "flat", "alike", "zero", "nan", "grown", "faint", "flux"])
