@@ -66,6 +66,11 @@ static void test_resident_groups()
                         if (b < 8 && (!max_batch || b < max_batch)) EXPECT((b + 1) * op >= kOrbTrainOperand);
                     }
     EXPECT(planned > 200);
+    // short rows of uint16 in six tiles: a tile to a wave, and one exchange an image (three blocks that share them out took up to 7 % longer)
+    for (uint32_t N : {4u, 25u, 49u}) {
+        OrbitTrainPlan const p = plan_orbit_train(N, 64, 10, 10, 90, true, 256, 159 * 1024);
+        EXPECT(p.npb == 1 && p.splits == 1 && p.abreast == 8);
+    }
 }
 
 static void test_trainer()
