@@ -37,10 +37,10 @@ constexpr size_t orbit_train_operand(uint32_t nrr, uint32_t KS, bool u16) { retu
 
 // How many neurons a block of a resident integer trainer holds and between how many blocks the rows are shared out: what is expected to
 // take least.  In clocks of an image: a block's rows through its CU's 64 bytes a clock, its waves' instructions or the matrix pipes; a round of
-// tiles, whose shares of k meet in the LDS; an update of 64 orbits a wave; the words of the blocks that hold the same neurons.  Fitted to
-// every plan of 40 shapes (8 to 1024 neurons of 128 to 10000 elements, 4 to 720 variants): off by 3.2 % in the mean.  Beside every plan of 79
-// shapes (1 to 1024 neurons of 36 to 8281 elements, 40 to 720 rotations), up to four times apart, the plan taken is 0.7 % slower than the
-// fastest in the mean, most with 512 uint16 and 256 uint8 neurons of 2025 elements (7.5 and 6.2 %).  npb 0: no way to hold the neurons.
+// tiles, whose shares of k meet in the LDS; an update of 64 orbits a wave; two column tiles of uint16; the words of the blocks that hold the
+// same neurons.  Fitted to every plan of 116 shapes (1 to 1024 neurons of 36 to 8281 elements, 40 to 720 rotations), up to four times apart:
+// the plan taken is 0.3 % slower than the fastest in the mean, most with 256 uint8 neurons of 2025 elements (6.2 %).  npb 0: no way to hold the
+// neurons.
 inline OrbitTrainPlan plan_orbit_train(uint32_t N, uint32_t E, uint32_t orbits, uint32_t reached, uint32_t nrr, bool u16, uint32_t units, size_t lds_max)
 {
     const uint32_t RT = (nrr + 15) / 16, planes = u16 ? 2 : 1, accs = u16 ? 3 : 1, products = u16 ? 4 : 1;
@@ -68,8 +68,8 @@ inline OrbitTrainPlan plan_orbit_train(uint32_t N, uint32_t E, uint32_t orbits, 
                     const double stream = rounds * abreast * tpw * 16.0 * KS * planes;
                     const double issue = rounds * (KS / 2.0 / shares) * (columns * planes * 10.0 + tpw * planes * 4.0 + tpw * columns * products * 2.0 + 10.0) * 8.6;
                     const double matrix = rounds * abreast * tpw * (double)columns * KS * products * 4.0;
-                    const double cost = 1.155 * std::max({stream, issue, matrix}) + rounds * (2850.0 + 110.0 * tpw * columns * accs + 10.0 * accs * shares * ((abreast * tpw * columns + 7) / 8)) +
-                                        nit * (u16 ? 2070.0 : 1594.0) + (npb - 1) * (u16 ? 100.0 : 200.0) + (splits > 1 ? 100.0 + 300.0 * splits : 0.0) + (u16 ? 75.0 : 175.0) * (abreast - 1) + 3.0 * groups * splits;
+                    const double cost = (u16 ? 1.24 : 1.155) * std::max({stream, issue, matrix}) + rounds * (2850.0 + 110.0 * tpw * columns * accs + 10.0 * accs * shares * ((abreast * tpw * columns + 7) / 8)) +
+                                        nit * (u16 ? 2070.0 : 1594.0) + (npb - 1) * (u16 ? 100.0 : 200.0) + (u16 && npb > 2 ? 1400.0 : 0.0) + (splits > 1 ? 100.0 + 300.0 * splits : 0.0) + (u16 ? 75.0 : 175.0) * (abreast - 1) + 3.0 * groups * splits;
                     if (!best.npb || cost < best_cost) {
                         best.npb = npb; best.splits = splits; best.abreast = abreast; best.tpw = tpw; best.nit = nit; best.lds = lds; best.reached = streamed;
                         best_cost = cost;

@@ -71,6 +71,9 @@ static void test_resident_groups()
         OrbitTrainPlan const p = plan_orbit_train(N, 64, 10, 10, 90, true, 256, 159 * 1024);
         EXPECT(p.npb == 1 && p.splits == 1 && p.abreast == 8);
     }
+    // two uint16 neurons a block while there are blocks for it (four and half of the rows: 400 neurons of 1600 elements 10 % longer), four beyond
+    for (uint32_t N : {400u, 512u}) EXPECT(plan_orbit_train(N, 1600, 210, 210, 90, true, 256, 159 * 1024).npb == 2);
+    EXPECT(plan_orbit_train(1024, 256, 36, 36, 90, true, 256, 159 * 1024).npb == 4);
 }
 
 static void test_trainer()

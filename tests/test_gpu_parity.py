@@ -783,6 +783,8 @@ RESIDENT_INTEGER_PLANS = [
     (6, 1, 150, 150, 40, True, 146, capi.QUADRATIC, capi.UINT8, 2),      # 43 chunks
     (6, 1, 150, 150, 40, True, 143, capi.QUADRATIC, capi.UINT8, 2),      # 42, six to a wave
     (513, 1, 60, 60, 24, True, 50, capi.QUADRATIC, capi.UINT8, 2),       # 3 x 1
+    (625, 1, 34, 34, 360, True, 24, capi.QUADRATIC, capi.UINT8, 2),      # ... three tiles to a wave
+    (331, 1, 90, 90, 360, True, 64, capi.QUADRATIC, capi.UINT8, 2),      # 3 x 2, the last block holds one neuron
     (1023, 1, 20, 18, 12, True, 17, capi.QUADRATIC, capi.UINT16, 3),     # 4 x 1, the last block holds three
     (40, 1, 23, 22, 36, True, 22, capi.QUADRATIC, capi.UINT16, 3),       # 66 orbits: a chunk and two more
     (40, 1, 23, 21, 36, True, 21, capi.QUADRATIC, capi.UINT8, 3),        # an odd neuron: the middle twice
