@@ -32,6 +32,7 @@
 #include <new>
 #include <string>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include <condition_variable>
@@ -3719,6 +3720,8 @@ std::vector<uint32_t> outside_elements(const pink_hip_ctx *ctx, const std::vecto
 struct OrbitGrid {
     uint32_t D, Ds, reached = 0;                            // (orbits that rotations of the image can reach; they come first)
     std::vector<uint32_t> orbit_of, reps;                   // per place; an orbit's first place
+    std::vector<unsigned char> slot_of;                     // per place: the symmetry that takes the first place there (the lowest of them)
+    uint32_t moves[8][8];                                   // where a slot goes under a symmetry
     uint32_t place(uint32_t x) const { return x + ((D & 1) && x > D / 2 ? 1u : 0u); }
     uint32_t pixel(uint32_t X) const { return X - ((D & 1) && X > D / 2 ? 1u : 0u); }
     uint32_t at(uint32_t off) const { return off / (D * D) * Ds * Ds + place((off % (D * D)) / D) * Ds + place(off % D); }
@@ -3729,8 +3732,10 @@ struct OrbitGrid {
         return at / (Ds * Ds) * (Ds * Ds) + (uint32_t)x * Ds + (uint32_t)y;
     }
     // In the order of their first places, 8 x 8 places at a time (neighbouring pieces of a row then read neighbouring pixels).
-    OrbitGrid(uint32_t D_, uint32_t C, uint32_t I, const std::vector<uint32_t> &region) : D(D_), Ds(D_ + (D_ & 1)), orbit_of((size_t)C * Ds * Ds, ~0u)
+    OrbitGrid(uint32_t D_, uint32_t C, uint32_t I, const std::vector<uint32_t> &region) : D(D_), Ds(D_ + (D_ & 1)), orbit_of((size_t)C * Ds * Ds, ~0u), slot_of((size_t)C * Ds * Ds, 0)
     {
+        for (uint32_t sym = 0; sym < 8; ++sym)
+            for (uint32_t to = 0; to < 8; ++to) moves[sym][orbit_source((int)sym, (int)to)] = to;
         for (uint32_t off : region) {
             uint32_t first = at(off);
             for (uint32_t sym = 1; sym < 8; ++sym) first = std::min(first, moved(at(off), sym));
@@ -3738,11 +3743,13 @@ struct OrbitGrid {
         }
         uint32_t corner = Ds;                               // (of the region)
         for (uint32_t off : region) corner = std::min({corner, place((off % (D * D)) / D), place(off % D)});
-        auto key = [&](uint32_t p) {
+        std::vector<std::pair<uint64_t, uint32_t>> keys;
+        for (uint32_t p : reps) {
             const uint64_t ch = p / (Ds * Ds), x = (p % (Ds * Ds)) / Ds + 8 - corner % 8, y = p % Ds + 8 - corner % 8;
-            return (ch << 48) | ((x / 8) << 32) | ((y / 8) << 16) | ((x % 8) << 8) | (y % 8);
-        };
-        std::sort(reps.begin(), reps.end(), [&](uint32_t l, uint32_t r) { return key(l) < key(r); });
+            keys.push_back({(ch << 48) | ((x / 8) << 32) | ((y / 8) << 16) | ((x % 8) << 8) | (y % 8), p});
+        }
+        std::sort(keys.begin(), keys.end());
+        for (uint32_t o = 0; o < reps.size(); ++o) reps[o] = keys[o].second;
         // half the image's diagonal, and two pixels for the crop's shift, the places of an odd neuron and the roundings of a rotation
         const double most = (I - 1) * 0.70711 + 2.0, middle = (D - 1) * 0.5;
         reached = (uint32_t)(std::stable_partition(reps.begin(), reps.end(), [&](uint32_t p) {
@@ -3750,7 +3757,23 @@ struct OrbitGrid {
             return x * x + y * y <= most * most;
         }) - reps.begin());
         for (uint32_t o = 0; o < reps.size(); ++o)
-            for (uint32_t sym = 0; sym < 8; ++sym) orbit_of[moved(reps[o], sym)] = o;
+            for (uint32_t sym = 8; sym-- > 0;) {
+                const uint32_t p = moved(reps[o], sym);
+                orbit_of[p] = o;
+                slot_of[p] = (unsigned char)sym;
+            }
+    }
+};
+
+// The orbits of a context's region, made when they are first asked for: up to three of its forms are considered or set up from them.
+struct RegionOrbits {
+    const pink_hip_ctx *ctx;
+    const std::vector<uint32_t> &region;                    // distinct elements, in the CPU's order
+    std::unique_ptr<OrbitGrid> made;
+    const OrbitGrid &grid()
+    {
+        if (!made) made.reset(new OrbitGrid(ctx->D, ctx->C, ctx->I, region));
+        return *made;
     }
 };
 
@@ -3767,13 +3790,13 @@ int finish_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, con
 void add_partly(std::vector<unsigned char> &mask, uint32_t Kp);
 
 // Integer trainers whose neurons fit the blocks of a resident launch: the resident form with the symmetries on the SOM side (orbit_train.inc).
-// (region: distinct elements, in the CPU's order.)
-int init_orbit_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
+int init_orbit_train(pink_hip_ctx *ctx, RegionOrbits &orbits)
 {
     const pink_hip_config &c = ctx->cfg;
     if (!ctx->gemm || (!ctx->fused_som && !ctx->orbit_train) || c.kernel_choice != PINK_HIP_KERNEL_AUTO || ctx->N > kSymMaxNeurons || ctx->D >= 4095 || ctx->C >= 256 || !resident_allowed())
         return PINK_HIP_OK;
-    const OrbitGrid grid(ctx->D, ctx->C, ctx->I, region);
+    const OrbitGrid &grid = orbits.grid();
+    const std::vector<uint32_t> &region = orbits.region;
     const bool u16 = c.ed_type != PINK_HIP_UINT8;
     ctx->sym_plan = plan_orbit_train(ctx->N, ctx->E, (uint32_t)grid.reps.size(), orbit_train_reached(ctx, grid), ctx->nrr_eff, u16, (uint32_t)ctx->num_cu, ctx->lds_max);
     if (!ctx->sym_plan.npb) { ctx->sym_plan = {}; return PINK_HIP_OK; }
@@ -3796,13 +3819,11 @@ int init_orbit_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     auto valid = [&](uint32_t sym) { return (c.num_rot != 1 || (sym & 3) == 0) && (c.use_flip || sym < 4); };
     ctx->sym_all = 1;                                       // the pixels of P_s are the same for every s, or not
     for (uint32_t off : region) {
-        const uint32_t at = grid.at(off), o = grid.orbit_of[at];
-        uint32_t p = 0;
-        while (grid.moved(grid.reps[o], p) != at) ++p;
+        const uint32_t at = grid.at(off), o = grid.orbit_of[at], p = grid.slot_of[at];
         elem[o * 8 + p] = off;
         for (uint32_t sym = 0; sym < 8 && o < ctx->sym_reached; ++sym)
             if (valid(sym)) {
-                const uint32_t k = o * 8 + orbit_moves((int)sym, (int)p), pos = upos[k];
+                const uint32_t k = o * 8 + grid.moves[sym][p], pos = upos[k];
                 mask[(size_t)sym * Kp + k] = 0xff;
                 if (!inside[(pos >> 24) * D * D + ((pos >> 12) & 0xfffu) * D + (pos & 0xfffu)]) ctx->sym_all = 0;
             }
@@ -3810,7 +3831,7 @@ int init_orbit_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     for (uint32_t s = 0; s < 8; ++s) {
         sel[2 * s] = orbit_selector((int)s, 0);
         sel[2 * s + 1] = orbit_selector((int)s, 1);
-        for (uint32_t q = 0; q < 8; ++q) sel[16 + s * 8 + q] = orbit_moves((int)s, (int)q) * (Kp / 8) * (uint32_t)sizeof(float);
+        for (uint32_t q = 0; q < 8; ++q) sel[16 + s * 8 + q] = grid.moves[s][q] * (Kp / 8) * (uint32_t)sizeof(float);
     }
     TRY(upload(ctx, &ctx->d_sym_element, elem));
     TRY(upload(ctx, &ctx->d_sym_sel, sel));
@@ -3821,13 +3842,14 @@ int init_orbit_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
 }
 
 // Float32 trainers whose neurons' eight symmetric operand rows fit the LDS of as many blocks as there are compute units:
-// the resident form with the symmetries on the SOM side.  (region: distinct elements, in the CPU's order.)
-int init_sym_train(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
+// the resident form with the symmetries on the SOM side.
+int init_sym_train(pink_hip_ctx *ctx, RegionOrbits &orbits)
 {
     const pink_hip_config &c = ctx->cfg;
     const uint32_t D = ctx->D, DD = D * D;
     const bool f32 = c.ed_type == PINK_HIP_FLOAT;
-    if (!f32) return init_orbit_train(ctx, region);
+    if (!f32) return init_orbit_train(ctx, orbits);
+    const std::vector<uint32_t> &region = orbits.region;
     if (!ctx->d_inv || c.kernel_choice != PINK_HIP_KERNEL_AUTO || ctx->N > kSymMaxNeurons || D >= 4096 || ctx->C >= 256 ||
         !resident_allowed())
         return PINK_HIP_OK;
@@ -4059,11 +4081,12 @@ int orbit_samples(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, const 
     return launch_check(ctx, "k_orbit_table");
 }
 
-// The tables of the orbit order (see orbit_gemm.inc) and the SOM's operand.  (region: distinct elements, in the CPU's order.)
-int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
+// The tables of the orbit order (see orbit_gemm.inc) and the SOM's operand.
+int init_orbit(pink_hip_ctx *ctx, RegionOrbits &orbits)
 {
     const pink_hip_config &c = ctx->cfg;
-    const OrbitGrid grid(ctx->D, ctx->C, ctx->I, region);
+    const OrbitGrid &grid = orbits.grid();
+    const std::vector<uint32_t> &region = orbits.region;
     const uint32_t D = ctx->D, DD = D * D, Ds = grid.Ds;
     const std::vector<uint32_t> &reps = grid.reps, &orbit_of = grid.orbit_of;
     auto pixel = [&](uint32_t X) { return grid.pixel(X); };
@@ -4084,17 +4107,13 @@ int init_orbit(pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
             const uint32_t at = moved(reps[o], p);
             upos[o * 8 + p] = (at / (Ds * Ds) << 24) | (pixel((at % (Ds * Ds)) / Ds) << 12) | pixel(at % Ds);
         }
-    uint32_t moves[8][8];                                   // where a slot goes under a symmetry
-    for (uint32_t sym = 0; sym < 8; ++sym)
-        for (uint32_t to = 0; to < 8; ++to) moves[sym][orbit_source((int)sym, (int)to)] = to;
+    const auto &moves = grid.moves;
     std::vector<uint32_t> in_region(ctx->S, 0);             // (place in the CPU's order + 1)
     for (uint32_t e = 0; e < region.size(); ++e) in_region[region[e]] = e + 1;
     ctx->orb_all = 1;
     std::vector<unsigned char> mask((size_t)8 * Kp, 0);
     for (uint32_t e = 0; e < region.size(); ++e) {
-        const uint32_t off = region[e], at = grid.at(off), o = orbit_of[at];
-        uint32_t p = 0;
-        while (moved(reps[o], p) != at) ++p;
+        const uint32_t off = region[e], at = grid.at(off), o = orbit_of[at], p = grid.slot_of[at];
         elem[o * 8 + p] = off;
         for (uint32_t sym = 0; sym < 8; ++sym)
             if ((ctx->orb_valid >> sym) & 1) {
@@ -4247,7 +4266,7 @@ uint32_t summed_images(const pink_hip_ctx *ctx)
 // 25 / 27, 256 720 4096 80 / 41, 484 720 1024 34 / 30, 900 720 576 32 / 30, 1600 720 576 45 / 31, 1600 720 4096 255 / 58, 9 80 8100 72 / 28,
 // 900 80 8100 88 / 39.)  Very long rows leave many variants in question, whose rows come from memory again and again: 100 720 16384
 // 193 / 111, 49 720 29241 315 / 204, but 256 720 16384 297 / 325, 256 720 28900 544 / 719.
-bool orbit_trains(const pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
+bool orbit_trains(const pink_hip_ctx *ctx, RegionOrbits &orbits)
 {
     if (!is_int(ctx)) {
         const double E = ctx->E, NR = (double)ctx->N * ctx->R;
@@ -4256,7 +4275,7 @@ bool orbit_trains(const pink_hip_ctx *ctx, const std::vector<uint32_t> &region)
     }
     // (below a dozen base rotations the product's tiles of 64 rows are mostly empty)
     if (!ctx->gemm || ctx->E < 1024 || ctx->nrr_eff < 12 || !resident_allowed()) return false;
-    const OrbitGrid grid(ctx->D, ctx->C, ctx->I, region);
+    const OrbitGrid &grid = orbits.grid();
     // (the rows of every variant, which the other form in turn writes and reads, are 8 MB an image and more)
     return ctx->N > kSymMaxNeurons || (uint64_t)ctx->R * ctx->Epad * (ctx->cfg.ed_type == PINK_HIP_UINT16 ? 2 : 1) > (8u << 20) ||
            !plan_orbit_train(ctx->N, ctx->E, (uint32_t)grid.reps.size(), orbit_train_reached(ctx, grid), ctx->nrr_eff, ctx->cfg.ed_type == PINK_HIP_UINT16,
@@ -4786,13 +4805,14 @@ int init_ctx(pink_hip_ctx *ctx)
     }
 
     // Mappers: rows of many images against the SOM, symmetries on the SOM side (orbit_gemm.inc).
+    RegionOrbits orbits{ctx, region, nullptr};
     {
         bool distinct = true;
         std::vector<char> seen(ctx->S, 0);
         for (uint32_t off : region) { if (seen[off]) distinct = false; seen[off] = 1; }
         const bool fits = distinct && c.kernel_choice == PINK_HIP_KERNEL_AUTO && ctx->D < 4095 && ctx->C < 256;
-        if (fits && (ctx->trainer ? orbit_trains(ctx, region) : is_int(ctx) ? !ctx->mfma_sym : orbit_screens(ctx))) {
-            TRY(init_orbit(ctx, region));
+        if (fits && (ctx->trainer ? orbit_trains(ctx, orbits) : is_int(ctx) ? !ctx->mfma_sym : orbit_screens(ctx))) {
+            TRY(init_orbit(ctx, orbits));
             if (ctx->orbit) ctx->mfma = false;
             if (ctx->orbit && is_int(ctx)) ctx->gemm = true;               // (the matrix cores, for pink_hip_distance_kernel)
         }
@@ -5096,7 +5116,7 @@ int init_ctx(pink_hip_ctx *ctx)
                 TRY(init_exchange(ctx, kSlotWords, (const void *)small_resident_kernel(ctx), kResidentThreads, 0));
             }
         }
-        if (one_to_one && !ctx->small_train && !ctx->f32gemm) TRY(init_sym_train(ctx, region));
+        if (one_to_one && !ctx->small_train && !ctx->f32gemm) TRY(init_sym_train(ctx, orbits));
         // one launch per image where the float32 distance kernel runs in its one-wave-per-SIMD form (see k_train_f32_dpp;
         // up to 256 neurons: measured with 512 allowed, 17 x 17 and 18 x 18 neurons at 720 variants train no faster this
         // way than with an update launch of their own -- with three to four waves per SIMD the launch saved is paid in
