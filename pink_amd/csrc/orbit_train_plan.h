@@ -56,8 +56,10 @@ inline OrbitTrainPlan plan_orbit_train(uint32_t N, uint32_t E, uint32_t orbits, 
         for (uint32_t splits = 1; splits <= std::min(kOrbTrainSplits, RT) && groups * splits <= units; ++splits) {
             const uint32_t tiles = (RT + splits - 1) / splits;
             if (tiles == tiles_before) continue;
-            // (more than six orbits a thread: rows that a compute unit takes longer to pull through than the orbits' product takes for an image,
-            // 15 us for three tiles of 33488 uint8 elements)
+            // (More than six orbits a thread: rows that a compute unit takes longer to pull through than the orbits' product takes for an image.  Us an
+            // image with everything, resident | image by image, neurons of 181 x 181 and images of 256 x 256 pixels, by tiles x KS x planes: 1048, 60
+            // and 100 uint8 neurons 44.7 | 46.3 and 41.5 | 43.4, 60 uint16 39.0 | 49.1; 1572, 100 and 200 uint8 52.6 | 52.3 and 44.6 | 43.6; 2096, 100 uint8
+            // 74.8 | 62.0, 60 and 100 uint16 61.2 | 60.1 and 49.6 | 52.4; 3144, 100 and 200 uint8 89.1 | 82.3 and 75.8 | 62.9, 100 uint16 77.5 | 69.3.)
             if (nit > kOrbTrainAllNit && tiles * KS * planes > 1600) continue;
             tiles_before = tiles;
             for (uint32_t abreast = 1; abreast <= 8; abreast *= 2)

@@ -1863,7 +1863,7 @@ __global__ __launch_bounds__(256) void k_train_small_u8(float *__restrict__ som,
 // ---------------------------------------------------------------------------------
 // The same trainers with the kernel RESIDENT over a whole launch group: one block per neuron keeps its neuron
 // -- weights in registers, its row of the SOM operand and the norm in LDS -- over all images of the group and
-// computes only its own neuron's distances (the MFMA's 32 columns all hold the one neuron).  Per image the
+// computes only its own neuron's distances (every column of the matrix instruction holds the one neuron).  Per image the
 // blocks exchange one 64-bit word each, (tag, smallest distance of the neuron): a block stores its word and a wave polls
 // the N blocks' until all carry the image's tag.  Nothing else crosses between blocks, so no fences: the payload rides in
 // the atomic word.  Two sets of words take turns (a block can be at most one image ahead of another).
@@ -1871,8 +1871,8 @@ __global__ __launch_bounds__(256) void k_train_small_u8(float *__restrict__ som,
 // variants 2.98 -> 1.71; 0.8 of it the exchange).  Where one wave can hold the image's rows (FT tiles of 16 rows x FK k-steps of 64
 // bytes, v_mfma_i32_16x16x64_i8: half the cycles of the 32-row form for up to 16 variants), it multiplies alone and has the neuron's
 // distances in its accumulators and its norm beside them: eight waves' parts meet in the LDS behind a barrier, 0.62 us to the word.
-// Another wave polls and asks for nothing else: a word comes back behind what its wave asked for before.  The values of the
-// neuron's best variant come out of memory while the words travel (staging every variant in the LDS an image ahead: 1.52; 1.6 with 16
+// Another wave polls: the next image's rows, which a word would come back behind, are not its requests (its share of the best variant's values
+// are).  Those values come out of memory while the words travel (staging every variant in the LDS an image ahead: 1.52; 1.6 with 16
 // variants).  Neurons of more than 1024 elements and 16 variants keep the eight waves: their rows do not fit one wave's registers.
 // Every wait is bounded: a wave that does not see all words within `spin_limit` polls raises `error` and marks its
 // block's slots, polling waves leave when they see such a mark, a block that leaves stops publishing, so every
@@ -3225,7 +3225,9 @@ int resident_launched(pink_hip_ctx *ctx, const float *dev_images, uint32_t image
 }
 
 // (us per image, eight waves | one, 64 neurons: 784 elements 8 variants 1.83 | 1.48, 32 variants 2.98 | 1.71; 1024 elements 32 variants 3.80 | 2.25;
-// 2025 elements 8 variants 2.44 | 2.15)
+// 2025 elements 8 variants 2.44 | 2.15.  The wave's k-steps are held in registers and multiplied whether there are values or not, so there is a
+// kernel for half of the range and one in between; 8 | 13 | 16 steps: 484 elements 8 variants 1.34 | 1.43 | 1.53, 32 variants 1.44 | 1.62 | 2.09, where
+// the last spills eight registers; 784 elements - | 1.44 | 1.55 and - | 1.65 | 2.14; 1024 elements - | - | 1.73 and 2.18)
 decltype(&k_train_small_u8_resident<2, 1, 8>) small_resident_kernel(const pink_hip_ctx *ctx)
 {
     const uint32_t steps = (ctx->gKS + 1) / 2;
@@ -4056,7 +4058,9 @@ int orbit_samples(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, const 
     // as many base rotations per wave as there are, up to 16; two where the image comes out of memory: a wave's pixels are neighbours
     // then; eight for a trainer, whose rows' float values leave in 64 bytes in a row so, four for its few images of long rows, which have
     // blocks for a part of the chip (us per launch, 4 | 8 | 16 rotations: 67 images of 90 rows of 2304 elements 54 | 49 | 54, uint16 of 4480
-    // 73 | 65 | 75, 30 of 25 rows of 42440 74 | 133 | -; a mapper's 150 of 4480 119 | 107 | 94)
+    // 73 | 65 | 75, 30 of 25 rows of 42440 74 | 133 | -; a mapper's 150 of 4480 119 | 107 | 94).  Where long rows train resident too, their groups of
+    // eight to 256 images read the same table: us an image with everything, 4 | 8, rows of 33488: 90 uint8 rows of 256 x 256 pixels 52.5 | 55.2, of
+    // 100 x 100 23.6 | 24.8, of 64 x 64 14.5 | 14.5, 45 uint16 rows of 256 x 256 39.2 | 47.1, of 100 x 100 19.9 | 19.7
     const auto row_blocks = [&](uint32_t rl) { return (ctx->nrr_eff + (1u << rl) - 1) >> rl; };
     const uint32_t most = !ctx->orb_prep_lds ? 1u : !ctx->trainer ? 4u : Kp >= 4096 && images * row_blocks(3) < (uint32_t)ctx->num_cu / 2 ? 2u : 3u;
     ctx->orb_rl = 0;
@@ -4195,7 +4199,7 @@ int init_orbit(pink_hip_ctx *ctx, RegionOrbits &orbits)
         }
     }
     TRY(tables.commit(ctx, &ctx->d_orb_tables));
-    TRY(orbit_samples(ctx, region, d_upos, Kp, 1, ctx->orb_all));
+    TRY(orbit_samples(ctx, region, d_upos, Kp, 1, ctx->orb_all));           // (rows of many elements: four base rotations a wave, see there)
     ctx->orb_pitch = ctx->trainer ? round_up(ctx->nrr_eff, f32 ? 16 : 32) : ctx->nrr_eff;
     ctx->screen_train = ctx->trainer && f32;
     ctx->orbit = !ctx->screen_train;
@@ -5112,7 +5116,6 @@ int init_ctx(pink_hip_ctx *ctx)
             // resident over a launch group: every block needs a compute unit of its own for the whole launch
             ctx->resident_train = ctx->N <= (uint32_t)ctx->num_cu && resident_allowed();
             if (ctx->resident_train) {
-                HIP_TRY(ctx, hipFuncSetAttribute((const void *)small_resident_kernel(ctx), hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
                 TRY(init_exchange(ctx, kSlotWords, (const void *)small_resident_kernel(ctx), kResidentThreads, 0));
             }
         }
