@@ -733,7 +733,7 @@ RESIDENT_SYMMETRIC_SHAPES = [
 @pytest.mark.parametrize("form", ["resident", "gives up", "tags wrap"])
 @pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,shape_,ed_type,n", RESIDENT_SYMMETRIC_SHAPES)
 def test_resident_symmetric_trainer_forms(monkeypatch, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n, form):
-    """Integer trainers keep their neurons' eight symmetric operand rows on the device over a launch group (see
+    """Trainers with the symmetries on the SOM side keep their neurons on the device over a launch group (see
     test_small_uint8_trainer_forms for the exchange between the blocks).  What a launch that gives up leaves undone, and the groups
     queued behind it, the launch that follows it trains; the next call takes the other form."""
     say("resident symmetric trainer", form, N, C_, I, D, nrot, flip, ed, shape_, ed_type, n)
