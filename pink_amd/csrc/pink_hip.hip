@@ -3330,7 +3330,7 @@ int launch_orbit_prepare(pink_hip_ctx *ctx, OrbitPrep &p, uint32_t images)
     // images, 90 rotations of 4480 uint16 elements: 62 | 78, 93 | 106, 273 | 261, 1270 | 1210)
     const int few = images <= ctx->orb_few ? 1 : 0;
     p.index = ctx->d_orb_index[few]; p.frac = ctx->d_orb_frac[few]; p.table_groups = ctx->orb_table_groups[few]; p.rl = few ? 2u : ctx->orb_rl;
-    p.lo = ctx->orb_lo; p.size = ctx->orb_size;
+    p.lo = ctx->orb_lo; p.size = ctx->orb_size; p.over = orbit_over(ctx->orb_size);
     const dim3 grid(images, (ctx->nrr_eff + (1u << p.rl) - 1) >> p.rl);
     const uint32_t threads = ctx->orb_prep_lds > 64 * 1024 || grid.x * grid.y < (uint32_t)ctx->num_cu ? 1024 : ctx->orb_prep_lds > 24 * 1024 ? 512 : 256;
     void *args[] = {&p};
@@ -4377,7 +4377,7 @@ int run_orbit_rows(pink_hip_ctx *ctx, const float *dev_images, uint32_t B)
         p.images = dev_images; p.index = ctx->d_orb_index[0]; p.frac = ctx->d_orb_frac[0]; p.weight = ctx->d_coef_weight; p.outside = ctx->d_coef_outside;
         p.opnd = (uint32_t *)ctx->d_orb_rows; p.row = (CoefRow *)ctx->d_coef_row; p.image = (CoefImage *)ctx->d_coef_image; p.xrows = ctx->d_orb_x;
         if (!ctx->trainer) { p.wide_count = ctx->d_screen_counts + 1; p.list_count = ctx->d_screen_counts; p.upper = ctx->d_coef_upper; }
-        p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.Op = ctx->orb_KS * 4; p.Ox = ctx->orb_Ox; p.all_sym = ctx->orb_all; p.pitch = ctx->orb_pitch;
+        p.C = ctx->C; p.I = ctx->I; p.N = ctx->N; p.nrr = ctx->nrr_eff; p.Op = ctx->orb_KS * 4; p.Ox = ctx->orb_Ox; p.all_sym = ctx->orb_all; p.pitch = ctx->orb_pitch; p.over = orbit_over(ctx->I + 1);
         // Large images: a block has a CU to itself and takes all its waves.  Others: four waves, so that blocks that load, work and store share a
         // CU, and as many tiles as leave a dozen waves per CU (an image is loaded once for them).
         const bool large = ctx->orb_prep_lds > 50 * 1024 || !ctx->orb_prep_lds;
