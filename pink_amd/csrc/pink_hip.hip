@@ -4065,8 +4065,9 @@ int orbit_samples(pink_hip_ctx *ctx, const std::vector<uint32_t> &region, const 
     const uint32_t most = !ctx->orb_prep_lds ? 1u : !ctx->trainer ? 4u : Kp >= 4096 && images * row_blocks(3) < (uint32_t)ctx->num_cu / 2 ? 2u : 3u;
     ctx->orb_rl = 0;
     while (ctx->orb_rl < most && row_blocks(ctx->orb_rl) > 1) ++ctx->orb_rl;
-    // (a mapper's calls with few images: a table of their own; see launch_orbit_prepare)
-    ctx->orb_few = !f32 && !ctx->trainer && ctx->orb_rl > 2 ? ctx->num_cu / (2 * row_blocks(ctx->orb_rl)) : 0;
+    // (a mapper's calls with few images: a table of their own; see launch_orbit_prepare.  Short rows have work for one turn of a block's waves either
+    // way: us per call, 4 | 16 rotations, 10 of 256 elements 24.1 | 23.7 (1 image) and 26.5 | 25.5 (4), of 484 25.5 | 26.3 and 26.3 | 27.2)
+    ctx->orb_few = !f32 && !ctx->trainer && ctx->orb_rl > 2 && Kp >= 512 ? ctx->num_cu / (2 * row_blocks(ctx->orb_rl)) : 0;
     for (int few = 0; few < (ctx->orb_few ? 2 : 1); ++few) {
         const uint32_t rl = few ? 2u : ctx->orb_rl, blocks = row_blocks(rl), groups = orbit_piece_groups(Kp / 16, rl), tiles = (ctx->nrr_eff + 15) / 16;
         const size_t entries = f32 ? (size_t)tiles * Kp * 16 : (size_t)blocks * groups * 1024;
