@@ -866,6 +866,21 @@ def test_integer_trainers_on_awkward_values(monkeypatch, kind, N, C_, I, D, nrot
     assert np.array_equal(np.isnan(som), lost) and np.array_equal(bits(som)[~lost], bits(want)[~lost])
 
 
+def test_resident_integer_trainer_of_the_most_rotations():
+    """A group's operand is counted in 32 bits: an image's is 272 MB here, so seven make a group, where there were always eight."""
+    N, I, nrot, n = 4, 90, 65536, 8
+    say("resident integer trainer, 65536 rotations")
+    rng = np.random.default_rng(3)
+    som0, imgs = rng.random((N, I * I), dtype=np.float32), rng.random((n, I * I), dtype=np.float32)
+    F = capi.make_update_factors(capi.CARTESIAN, [N], capi.GAUSSIAN, 1.0, 0.5)
+    want = som0.copy()
+    obmu = O.train(O.shape(N, 1, I, I, nrot, False, I, capi.QUADRATIC, capi.UINT16), want, imgs, F)
+    with capi.Context(N, 1, I, I, nrot, False, I, capi.QUADRATIC, capi.UINT16, F) as ctx:
+        ctx.set_som(som0)
+        bmu, som = ctx.train(imgs), ctx.get_som()
+    assert np.array_equal(bmu, obmu) and np.array_equal(bits(som).ravel(), bits(want).ravel())
+
+
 @pytest.mark.parametrize("kind", ["outside", "infinite", "nan"])
 @pytest.mark.parametrize("N,C_,I,D,nrot,flip,ed,shape_,ed_type,n", [
     (20, 1, 24, 18, 40, True, 16, capi.QUADRATIC, capi.UINT16, 6),
